@@ -1,0 +1,124 @@
+"""The searches that leave out what a bound rules out give the full search's
+bits: hex levels score only the sub-tets that can decide a candidate
+(csrc/dmo_kernels.hip).  Positions bit-exact against the oracle, which scores
+everything, on the forms where a bound or a selection could go wrong: exact
+and near ties (regular and barely jittered meshes), inverted and flat
+elements, frames far from the origin, tiny and huge scales (thresholds and
+margins far apart), wide and single-level windows, every nq, both extents and
+hex metrics, rings of more elements than lanes.
+"""
+import numpy as np
+import pytest
+
+from volumesurfacediscretemeshoptimization_amd import (DMOHexClass, DMOMeshHexFactory, DMOMeshTetFactory, DMOTetClass,
+                                                       synth)
+
+pytestmark = pytest.mark.gpu
+
+FACTORY = {"tet": DMOMeshTetFactory, "hex": DMOMeshHexFactory}
+CLASS = {"tet": DMOTetClass, "hex": DMOHexClass}
+
+
+def _compare(oracle, kind, xyz, cells, iters=3, nq=8, depth=3, grid_scale=0.5, extent=-1, hex_metric=0):
+    g = FACTORY[kind].create(xyz, cells)
+    opt = CLASS[kind](g, n_iter=iters, nq=nq, depth=depth, gridScale=grid_scale, extent_mode=extent,
+                      fixed_boundary=True, quality_guard=False, hex_metric=hex_metric)
+    o = oracle.OracleMesh(kind, xyz, cells)
+    o.hex_metric = hex_metric
+    moved = 0
+    try:
+        for it in range(iters):
+            before = g.positions(original_order=False)
+            opt.doIteration()
+            o.iterate(nq=nq, depth=depth, grid_scale=grid_scale, extent=None if extent < 0 else extent)
+            gp, op = g.positions(original_order=False), o.positions()
+            bad = (gp.view(np.uint32) != op.view(np.uint32)).any(axis=1)
+            assert not bad.any(), (it, int(bad.sum()), np.nonzero(bad)[0][:5], gp[bad][:2], op[bad][:2])
+            moved += int((gp != before).any(axis=1).sum())
+        return moved
+    finally:
+        opt.close()
+        g.close()
+
+
+def _cube(kind, n, seed, jitter):
+    return (synth.tet_cube if kind == "tet" else synth.hex_cube)(n, seed=seed, jitter=jitter)
+
+
+@pytest.mark.parametrize("kind", ["tet", "hex"])
+@pytest.mark.parametrize("jitter", [0.0, 1e-6, 1e-3, 0.15, 0.3, 0.49])
+def test_jitters(oracle, kind, jitter):
+    xyz, cells = _cube(kind, 7, 71, jitter)
+    _compare(oracle, kind, xyz, cells, iters=4)
+
+
+@pytest.mark.parametrize("kind", ["tet", "hex"])
+@pytest.mark.parametrize("scale,shift", [(1.0, 1000.0), (1e-3, 50.0), (1e-6, 0.0), (1e-12, 0.0), (1e5, 0.0), (1e12, 0.0),
+                                         (1.0, 1e6)])
+def test_scales_and_offsets(oracle, kind, scale, shift):
+    xyz, cells = _cube(kind, 6, 72, 0.3)
+    xyz = (xyz.astype(np.float64) * scale + shift).astype(np.float32)
+    _compare(oracle, kind, xyz, cells)
+
+
+@pytest.mark.parametrize("kind", ["tet", "hex"])
+@pytest.mark.parametrize("nq", [2, 4, 6, 8])
+@pytest.mark.parametrize("depth,grid_scale", [(1, 0.5), (3, 2.5), (7, 0.5), (3, 0.01)])
+def test_grids(oracle, kind, nq, depth, grid_scale):
+    xyz, cells = _cube(kind, 6, 73, 0.3)
+    _compare(oracle, kind, xyz, cells, nq=nq, depth=depth, grid_scale=grid_scale)
+
+
+@pytest.mark.parametrize("kind,extent,metric", [("tet", 1, 0), ("hex", 0, 0), ("hex", -1, 1), ("hex", 0, 1)])
+def test_extents_and_metrics(oracle, kind, extent, metric):
+    xyz, cells = _cube(kind, 7, 74, 0.35)
+    assert _compare(oracle, kind, xyz, cells, extent=extent, hex_metric=metric) > 100
+
+
+@pytest.mark.parametrize("kind", ["tet", "hex"])
+def test_stretched_and_flat(oracle, kind):
+    """elements 1000 times wider than high, and a layer squeezed flat"""
+    xyz, cells = _cube(kind, 6, 75, 0.3)
+    _compare(oracle, kind, xyz * np.array([1.0, 1.0, 1e-3], np.float32), cells)
+    flat = xyz.copy()
+    flat[(flat[:, 2] > 0.3) & (flat[:, 2] < 0.6), 2] = 0.5
+    _compare(oracle, kind, flat, cells)
+
+
+def _hex_fan(k, seed):
+    """k quads around an axis in 2 layers: the axis' middle vertex has 2k hexes"""
+    r = np.random.RandomState(seed)
+    t = 2.0 * np.pi * np.arange(2 * k) / (2 * k)
+    rad = np.where(np.arange(2 * k) % 2 == 0, 1.0, 1.3)
+    layer = np.concatenate([[[0.0, 0.0]], np.stack([rad * np.cos(t), rad * np.sin(t)], axis=1)])
+    z = 3.0 / k
+    xyz = np.concatenate([np.column_stack([layer, np.full(len(layer), h * z)]) for h in range(3)])
+    xyz[2 * k + 1] += r.uniform(-0.2, 0.2, 3) * z
+    m = 2 * k + 1
+    cells = []
+    for h in range(2):
+        for i in range(k):
+            q = [0, 1 + 2 * i, 2 + 2 * i, 1 + (2 * i + 2) % (2 * k)]
+            cells.append([v + (h + 1) * m for v in q] + [v + h * m for v in q])
+    return xyz.astype(np.float32), np.array(cells, np.int32)
+
+
+@pytest.mark.parametrize("k", [3, 6, 7, 8, 9, 20, 32])
+def test_hex_rings(oracle, k):
+    """rings of 6 to 64 hexes (the oracle's largest): 64 p-free sub-tets at k =
+    8, 60 / 70 p-dependent ones at k = 6 / 7, an element per lane at k = 32"""
+    xyz, cells = _hex_fan(k, 5)
+    for metric in (0, 1):
+        _compare(oracle, "hex", xyz, cells, iters=2, hex_metric=metric)
+
+
+@pytest.mark.parametrize("k", [3, 12, 31, 32, 33, 100, 256])
+def test_tet_rings(oracle, k):
+    """a bipyramid's centre with 2k tets, up to 512 (the oracle's largest)"""
+    t = 2.0 * np.pi * np.arange(k) / k
+    pts = [[0.05, -0.03, 0.02]] + [[np.cos(a), np.sin(a), 0.0] for a in t] + [[0.0, 0.0, 1.0], [0.0, 0.0, -1.0]]
+    cells = []
+    for i in range(k):
+        j = (i + 1) % k
+        cells += [[0, 1 + i, 1 + j, k + 1], [0, 1 + j, 1 + i, k + 2]]
+    assert _compare(oracle, "tet", np.array(pts, np.float32), np.array(cells, np.int32), iters=2) > 0

@@ -303,7 +303,7 @@ void record_iteration(vsdmo_batch* b)
         }
         auto plain = [&](int lo, int qend, int end) {
             launch_batch_round(b->p.nq, b->p.waves_per_vertex, a, b->rowHex.p, b->ringHex.p, b->items.p, lo, qend, end,
-                               b->ctr.p + r, b->grid[r], b->lds, s);
+                               b->ctr.p + r, b->grid[r], b->lds, b->maxRingHex, s);
         };
         if (lh && !lt) {   // hexes learned, tets plain: the tets, then the triangles
             plain(off, midT, midT);

@@ -170,7 +170,7 @@ void launch_search_split(int kind, int nq, const SearchArgs& a, int tail, int ri
 // items [lo, mid) from the atomic counter *ctr and stride over the flat
 // items [mid, hi) (the one-block-per-item schedule is launch_batch_typed)
 void launch_batch_round(int nq, int w, const SearchArgs& a, const int* rowHex, const int* valHex, const int* items,
-                        int lo, int mid, int hi, int* ctr, int grid, size_t lds, hipStream_t s);
+                        int lo, int mid, int hi, int* ctr, int grid, size_t lds, int hexCap, hipStream_t s);
 int batch_round_blocks_per_cu(int nq, int w, size_t lds);
 void launch_fill_int(int* p, int n, int v, hipStream_t s);
 // one block per item of items[lo, hi), all of element type `type` (0 tet,

@@ -46,6 +46,48 @@ __device__ __forceinline__ void wave_argmax(float& best, int& idx)
     }
 }
 
+// Reductions over the wave whose result is uniform (an SGPR): DPP moves inside
+// the rows of 16 lanes, two row broadcasts, lane 63 holds the result.  The
+// ds_bpermute of a shuffle costs an LDS round trip per step.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_move(float v)
+{
+    const int i = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ float lane_f(float v, int lane)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+}
+__device__ __forceinline__ float wave_max_u(float v)
+{
+    v = fmaxf(v, dpp_move<0x111, 0xf>(v));   // row_shr 1, 2, 4, 8
+    v = fmaxf(v, dpp_move<0x112, 0xf>(v));
+    v = fmaxf(v, dpp_move<0x114, 0xf>(v));
+    v = fmaxf(v, dpp_move<0x118, 0xf>(v));
+    v = fmaxf(v, dpp_move<0x142, 0xa>(v));   // row_bcast 15 into rows 1, 3
+    v = fmaxf(v, dpp_move<0x143, 0xc>(v));   // row_bcast 31 into rows 2, 3
+    return lane_f(v, 63);
+}
+__device__ __forceinline__ float wave_min_u(float v)
+{
+    v = fminf(v, dpp_move<0x111, 0xf>(v));
+    v = fminf(v, dpp_move<0x112, 0xf>(v));
+    v = fminf(v, dpp_move<0x114, 0xf>(v));
+    v = fminf(v, dpp_move<0x118, 0xf>(v));
+    v = fminf(v, dpp_move<0x142, 0xa>(v));
+    v = fminf(v, dpp_move<0x143, 0xc>(v));
+    return lane_f(v, 63);
+}
+// LDS written by some lanes of the wave, read by others of the same wave: its
+// LDS operations complete in order, the fence keeps the compiler's order
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
 // Block-level reductions for W waves per vertex (blockDim = 64*W).  With
 // W = 1 they are the wave shuffles alone; otherwise the per-wave results are
 // combined through LDS.  max/min and the (score, index) argmax are order
@@ -314,23 +356,70 @@ __device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, TetC* s_tc, 
 // ------------------------------------------------------------------ hexes
 struct HexLds { float cd[4], cF[4]; HexP hp[5]; };
 
+// LDS of a hex vertex search per ring element: the constants and the codes of
+// the element's sub-tets in the list of those a level scores
+constexpr size_t kHexLdsPer = sizeof(HexLds) + 5 * sizeof(int);
+// rounded up for a wave's slice of a block's LDS
+__host__ __device__ constexpr size_t hex_wave_lds(int ringCap) { return (kHexLdsPer * (size_t)ringCap + 15) / 16 * 16; }
+__device__ __forceinline__ int* hex_act(unsigned char* lds, int ringCap)
+{
+    return reinterpret_cast<int*>(lds + sizeof(HexLds) * (size_t)ringCap);
+}
+
 // staged state of a hex vertex search (as TetFrame), plus the accumulator of
 // the 4 sub-tets per ring element that do not contain the moving vertex
 struct HexFrame {
     float x0x, x0y, x0z, ex, ey, ez, sg, epsD, epsF;
     int n;
     bool corner8;   // the principal-axes sub-tet (slot 4 of HexP) left out
+    bool inRange;   // hex_stage: every p-free pair is in sel_range
     HexAcc acc0;
 };
 
-template <int W>
-__device__ HexFrame hex_stage(const SearchArgs& a, int vid, bool emin, HexLds* s_hx, RedLds<W>& rd)
+// The canonical selection compares ratios det^2 / F^3 in FP32 products; it
+// picks by the true ratios wherever they differ by more than its rounding, as
+// long as no product leaves the normal range.  kSelF / kSelD bound F and det
+// from below for that (det^2 F^3 >= 2^-108), kSel is the relative distance
+// (on det / F^1.5) beyond which a ratio counts as clearly larger: 2^-10,
+// against the selection's ~2^-22 per comparison.
+constexpr float kSelF = 0x1p-13f, kSelD = 0x1p-24f, kSelY = 0x1p-15f, kSel = 0x1p-10f;
+constexpr float kSelMax = 0x1p16f;   // and from above: no product overflows
+__device__ __forceinline__ bool sel_range(float det, float F)
 {
-    constexpr int T = 64 * W;
-    const int tid = (W == 1) ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
+    return det >= kSelD && det <= kSelMax && F >= kSelF && F <= kSelMax;   // false for NaN
+}
+
+// The running selection over up to 64 (det, F) pairs held one per lane (lane
+// order = selection order; have: the lane holds one), continued from acc:
+// the pair with the smallest ratio, found by one reduction.  Where several
+// lie within kSel of it, those alone are taken in order: a clearly larger one
+// never ends up selected, whatever its place.  Every lane calls it; at least
+// one holds a pair, and all pairs are in sel_range (as is acc's when it has one).
+__device__ __forceinline__ void select_lanes(float& bd2, float& bF3, bool hasAcc, bool have, float det, float F)
+{
+    const float d2 = det * det, F3 = (F * F) * F;
+    const float y = have ? d2 * __builtin_amdgcn_rcpf(F3) : FLT_MAX;
+    const float ya = hasAcc ? bd2 * __builtin_amdgcn_rcpf(bF3) : FLT_MAX;
+    const float lim = fminf(wave_min_u(y), ya) * (1.0f + 2.0f * kSel);
+    unsigned long long band = __ballot(have && y <= lim);
+    if (!(ya <= lim)) { bd2 = 1.0f; bF3 = 0.0f; }   // replaced by the band's first
+    while (band) {
+        const int l = __builtin_ctzll(band);
+        band &= band - 1;
+        const float ld = lane_f(d2, l), lF = lane_f(F3, l);
+        const bool take = ld * bF3 < bd2 * lF;
+        bd2 = take ? ld : bd2;
+        bF3 = take ? lF : bF3;
+    }
+}
+
+// One-wave staging of vid's ring: constants in LDS, the p-free accumulator.
+__device__ HexFrame hex_stage(const SearchArgs& a, int vid, bool emin, HexLds* s_hx)
+{
+    const int lane = (int)(threadIdx.x & 63);
     HexFrame f;
-    const int r0 = a.ringRow[vid];
-    f.n = a.ringRow[vid + 1] - r0;
+    const int r0 = uniform(a.ringRow[vid]);
+    f.n = uniform(a.ringRow[vid + 1]) - r0;
     f.x0x = a.x[vid]; f.x0y = a.y[vid]; f.x0z = a.z[vid];
     f.corner8 = a.hexCorner8 != 0;
     float ex = emin ? FLT_MAX : -FLT_MAX, ey = ex, ez = ex, mabs = 0.0f;
@@ -341,12 +430,12 @@ __device__ HexFrame hex_stage(const SearchArgs& a, int vid, bool emin, HexLds* s
         ez = emin ? fminf(ez, dz) : fmaxf(ez, dz);
         mabs = fmaxf(mabs, fmaxf(dx, fmaxf(dy, dz)));
     };
-    // the thread's first element keeps its corner offsets in registers for
-    // the constants (the positions are read once; tet_stage)
-    const bool own0 = tid < f.n;
+    // the lane's first element keeps its corner offsets in registers for
+    // the constants (the positions are read once)
+    const bool own0 = lane < f.n;
     float d0[7][3];
     if (own0) {
-        const int* h = a.ringVal + (size_t)(r0 + tid) * 7;
+        const int* h = a.ringVal + (size_t)(r0 + lane) * 7;
 #pragma unroll
         for (int t = 0; t < 7; ++t) {
             const int v = h[t];
@@ -354,16 +443,16 @@ __device__ HexFrame hex_stage(const SearchArgs& a, int vid, bool emin, HexLds* s
             extent(d0[t][0], d0[t][1], d0[t][2]);
         }
     }
-    for (int e = tid + T; e < f.n; e += T) {
+    for (int e = lane + 64; e < f.n; e += 64) {
         const int* h = a.ringVal + (size_t)(r0 + e) * 7;
         for (int t = 0; t < 7; ++t) {
             const int v = h[t];
             extent(a.x[v] - f.x0x, a.y[v] - f.x0y, a.z[v] - f.x0z);
         }
     }
-    block_extents<W>(emin, ex, ey, ez, mabs, rd);
-    f.ex = ex; f.ey = ey; f.ez = ez;
-    f.sg = pow2_scale(mabs);
+    if (emin) { f.ex = wave_min_u(ex); f.ey = wave_min_u(ey); f.ez = wave_min_u(ez); }
+    else { f.ex = wave_max_u(ex); f.ey = wave_max_u(ey); f.ez = wave_max_u(ez); }
+    f.sg = pow2_scale(wave_max_u(mabs));
     const float s2 = f.sg * f.sg, s3 = s2 * f.sg;
     f.epsD = kHexEps * s3; f.epsF = kHexEps * s2;
     if (own0) {
@@ -373,9 +462,9 @@ __device__ HexFrame hex_stage(const SearchArgs& a, int vid, bool emin, HexLds* s
         for (int t = 0; t < 7; ++t) r[t + 1] = { d0[t][0] * f.sg, d0[t][1] * f.sg, d0[t][2] * f.sg };
         HexLds L;
         hex_consts(r, L.cd, L.cF, L.hp);
-        s_hx[tid] = L;
+        s_hx[lane] = L;
     }
-    for (int e = tid + T; e < f.n; e += T) {
+    for (int e = lane + 64; e < f.n; e += 64) {
         const int* h = a.ringVal + (size_t)(r0 + e) * 7;
         f3 r[8];
         r[0] = { 0.0f, 0.0f, 0.0f };
@@ -387,12 +476,27 @@ __device__ HexFrame hex_stage(const SearchArgs& a, int vid, bool emin, HexLds* s
         hex_consts(r, L.cd, L.cF, L.hp);
         s_hx[e] = L;
     }
-    __syncthreads();
-    // p-free sub-tets of the whole ring, in ring order
+    wave_lds_fence();
+    // p-free sub-tets of the whole ring, in ring order: one pair per lane
+    // where the ring has at most 16 hexes
     f.acc0 = hex_acc0();
-    for (int e = 0; e < f.n; ++e)
+    f.inRange = false;
+    if (f.n > 0 && 4 * f.n <= 64) {
+        const bool have = lane < 4 * f.n;
+        const int e = have ? lane >> 2 : 0;
+        const float det = s_hx[e].cd[lane & 3], F = s_hx[e].cF[lane & 3];
+        f.inRange = __ballot(have && !sel_range(det, F)) == 0ull;
+        if (f.inRange) {
+            f.acc0.dmin = wave_min_u(have ? det : FLT_MAX);
+            f.acc0.fmin = wave_min_u(have ? F : FLT_MAX);
+            select_lanes(f.acc0.bd2, f.acc0.bF3, false, have, det, F);
+        }
+    }
+    if (!f.inRange) {
+        for (int e = 0; e < f.n; ++e)
 #pragma unroll
-        for (int sIdx = 0; sIdx < 4; ++sIdx) hex_acc_add(f.acc0, s_hx[e].cd[sIdx], s_hx[e].cF[sIdx]);
+            for (int sIdx = 0; sIdx < 4; ++sIdx) hex_acc_add(f.acc0, s_hx[e].cd[sIdx], s_hx[e].cF[sIdx]);
+    }
     return f;
 }
 
@@ -407,124 +511,226 @@ __device__ __forceinline__ bool hex_pinned(const HexFrame& f)
     return f.acc0.dmin < f.epsD || f.acc0.fmin < f.epsF;
 }
 
-// the p-dependent sub-tets of the ring at one point: NS = 5 (the nine-tet
-// metric) or 4 (eight corners).  The slot count is a template argument so
-// that the callers branch on the metric once, outside the element loop (a
-// branch inside it holds the LDS reads of the last slot back)
-template <int NS>
-__device__ __forceinline__ void hex_ring_add(HexAcc& acc, const HexLds* s_hx, int n, float px, float py, float pz)
+// ring element of the p-dependent sub-tet t (5 or 4 per element; t < 2^14)
+__device__ __forceinline__ int sub_elem(int t, bool corner8)
 {
-    const float Q1 = fmaf(pz, pz, py * py), Q3 = 3.0f * Q1, t3 = 3.0f * px;
-    for (int e = 0; e < n; ++e)
-#pragma unroll
-        for (int sIdx = 0; sIdx < NS; ++sIdx) {
-            const HexP h = s_hx[e].hp[sIdx];
-            const bool a3 = (sIdx == 1 || sIdx == 4);
-            float Tyz = fmaf(h.gy, py, fmaf(h.gz, pz, h.D));
-            float Ryz = fmaf(h.sy, py, fmaf(h.sz, pz, h.K + (a3 ? Q3 : Q1)));
-            hex_acc_add(acc, fmaf(h.gx, px, Tyz), fmaf(px, (a3 ? t3 : px) + h.sx, Ryz));
-        }
+    return corner8 ? t >> 2 : (int)(((unsigned)t * 52429u) >> 18);
 }
 
-__device__ __forceinline__ float hex_score(const HexFrame& f, const HexLds* s_hx, float px, float py, float pz)
+// the p-dependent sub-tets of the ring at the start position (p = 0: det = D,
+// |J|^2 = K exactly), in ring order
+__device__ __forceinline__ float hex_start_score(const HexFrame& f, const HexLds* s_hx)
 {
+    const int lane = (int)(threadIdx.x & 63), ns = f.corner8 ? 4 : 5;
     HexAcc acc = f.acc0;
-    if (f.corner8) hex_ring_add<4>(acc, s_hx, f.n, px, py, pz);
-    else hex_ring_add<5>(acc, s_hx, f.n, px, py, pz);
+    if (f.inRange && ns * f.n <= 64) {
+        const bool have = lane < ns * f.n;
+        const int e = have ? sub_elem(lane, f.corner8) : 0, s = have ? lane - e * ns : 0;
+        const float det = s_hx[e].hp[s].D, F = s_hx[e].hp[s].K;
+        if (__ballot(have && !sel_range(det, F)) == 0ull) {
+            acc.dmin = fminf(acc.dmin, wave_min_u(have ? det : FLT_MAX));
+            acc.fmin = fminf(acc.fmin, wave_min_u(have ? F : FLT_MAX));
+            select_lanes(acc.bd2, acc.bF3, true, have, det, F);
+            return hex_acc_score(acc, f.epsD, f.epsF);
+        }
+    }
+    for (int e = 0; e < f.n; ++e)
+        for (int s = 0; s < ns; ++s) hex_acc_add(acc, s_hx[e].hp[s].D, s_hx[e].hp[s].K);
     return hex_acc_score(acc, f.epsD, f.epsF);
 }
 
-// the p-dependent sub-tets of the ring for the CPL candidates px[i] of a lane
-// (shared y, z): NS slots per element as in hex_ring_add
-template <int NS, int CPL>
-__device__ __forceinline__ void hex_ring_add_cpl(HexAcc* acc, const HexLds* s_hx, int n, const float* px,
-                                                 const float* t3, float py, float pz)
+// What a level can say about one p-dependent sub-tet over its whole window (a
+// box of half-widths H around c, frame coordinates): with |J|^2 = alpha (|p -
+// g|^2 + kn), bounds of det / F^1.5 from above (ub) and below (lb) for every
+// candidate, and whether det and F of every candidate stay clear of the
+// metric's thresholds (clear) and of the selection's (sel).  The margins cover
+// the rounding of the candidates' canonical evaluation: md, mf bound its
+// absolute error (2^-18 of the sum of the terms' magnitudes, against a few
+// 2^-24).
+struct HexBound { float ub, lb; bool clear, sel; };
+__device__ __forceinline__ HexBound hex_bound(const HexP& h, bool a3, float cx, float cy, float cz, float Hx, float Hy,
+                                              float Hz, float epsD, float epsF)
 {
-    const float Q1 = fmaf(pz, pz, py * py), Q3 = 3.0f * Q1;
-    // two elements per iteration at 8 candidates per lane: the minima of
-    // consecutive elements fold into v_min3 without canonicalising the
-    // accumulator each time (533 -> 506 VALU per element); at fewer
-    // candidates per lane the register growth costs more than it saves
-    constexpr int kUnrollE = CPL >= 8 ? 2 : 1;
-#pragma unroll kUnrollE
-    for (int e = 0; e < n; ++e) {
-#pragma unroll
-        for (int sIdx = 0; sIdx < NS; ++sIdx) {
-            const HexP h = s_hx[e].hp[sIdx];
-            const bool a3 = (sIdx == 1 || sIdx == 4);
-            const float Tyz = fmaf(h.gy, py, fmaf(h.gz, pz, h.D));
-            const float Ryz = fmaf(h.sy, py, fmaf(h.sz, pz, h.K + (a3 ? Q3 : Q1)));
-#pragma unroll
-            for (int i = 0; i < CPL; ++i)
-                hex_acc_add(acc[i], fmaf(h.gx, px[i], Tyz), fmaf(px[i], (a3 ? t3[i] : px[i]) + h.sx, Ryz));
-        }
-    }
+    constexpr float kR = 0x1p-18f;
+    const float ia = a3 ? 1.0f / 3.0f : 1.0f, al = a3 ? 3.0f : 1.0f;
+    const float iy = a3 ? 0.19245009f : 1.0f;   // alpha^-1.5
+    const float gx = -0.5f * ia * h.sx, gy = -0.5f * ia * h.sy, gz = -0.5f * ia * h.sz;
+    const float Px = fabsf(cx) + Hx, Py = fabsf(cy) + Hy, Pz = fabsf(cz) + Hz;
+    const float kn = ia * h.K - fmaf(gx, gx, fmaf(gy, gy, gz * gz));
+    const float mf = kR * (ia * h.K + fmaf(Px, Px + 2.0f * fabsf(gx), fmaf(Py, Py + 2.0f * fabsf(gy), Pz * (Pz + 2.0f * fabsf(gz)))));
+    const float wx = fabsf(cx - gx), wy = fabsf(cy - gy), wz = fabsf(cz - gz);
+    const float lx = fmaxf(wx - Hx, 0.0f), ly = fmaxf(wy - Hy, 0.0f), lz = fmaxf(wz - Hz, 0.0f);
+    const float ux = wx + Hx, uy = wy + Hy, uz = wz + Hz;
+    const float Fl = (kn - mf) + fmaf(lx, lx, fmaf(ly, ly, lz * lz));
+    const float Fu = (kn + mf) + fmaf(ux, ux, fmaf(uy, uy, uz * uz));
+    const float nx = fabsf(h.gx), ny = fabsf(h.gy), nz = fabsf(h.gz);
+    const float dc = fmaf(h.gx, cx, fmaf(h.gy, cy, fmaf(h.gz, cz, h.D)));
+    const float A = fmaf(nx, Hx, fmaf(ny, Hy, nz * Hz));
+    const float md = kR * (fabsf(h.D) + fmaf(nx, Px, fmaf(ny, Py, nz * Pz)));
+    const float dhi = (dc + A) + md, dlo = (dc - A) - md;
+    const float ru = __builtin_amdgcn_rsqf(Fl), rl = __builtin_amdgcn_rsqf(Fu);
+    HexBound b;
+    b.ub = ((dhi * ru) * (ru * ru)) * iy;   // NaN where Fl <= 0: no bound
+    b.lb = ((dlo * rl) * (rl * rl)) * iy;
+    b.sel = al * Fl >= kSelF;
+    b.clear = dlo >= 1.001f * epsD && al * Fl >= 1.001f * epsF;
+    return b;
 }
 
-// the nested grid search of a hex vertex (lane layout as tet_levels)
-template <int NQ, int W>
-__device__ bool hex_levels(const SearchArgs& a, const HexFrame& f, const HexLds* s_hx, RedLds<W>& rd, float qcur,
-                           float& cx, float& cy, float& cz)
+// one p-dependent sub-tet for the CPL candidates px[i] of a lane (shared y, z)
+template <bool A3, int CPL>
+__device__ __forceinline__ void hex_add_cpl(HexAcc* acc, const HexP& h, const float* px, const float* t3, float py,
+                                            float pz, float Q1, float Q3)
 {
-    constexpr int CPL = NQ / W;
-    static_assert(NQ % W == 0, "nq must be a multiple of the waves per vertex");
-    const int tid = (W == 1) ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
-    const int lane = tid & 63, i0 = (tid >> 6) * CPL;
+    const float Tyz = fmaf(h.gy, py, fmaf(h.gz, pz, h.D));
+    const float Ryz = fmaf(h.sy, py, fmaf(h.sz, pz, h.K + (A3 ? Q3 : Q1)));
+#pragma unroll
+    for (int i = 0; i < CPL; ++i)
+        hex_acc_add(acc[i], fmaf(h.gx, px[i], Tyz), fmaf(px[i], (A3 ? t3[i] : px[i]) + h.sx, Ryz));
+}
+
+// The nested grid search of a hex vertex, one wave: lane l = j + nq*k owns the
+// candidates (i, j, k), i = 0..nq-1 (index i + nq*l; the lowest index wins).
+//
+// Every level first bounds each sub-tet over its whole window, one sub-tet
+// per lane.  U, the smallest upper bound (the p-free sub-tets' minimum
+// included), bounds every candidate's minimum; a sub-tet whose lower bound is
+// clearly above U, and whose det and F are clear of the thresholds, is never
+// the one a candidate's selection ends with, so the candidates are scored over
+// the others alone, in ring order: the same bits.  On 48^3 cubes 0.5-3 of the
+// 40 sub-tets are left (the windows are scaled by the smallest one-ring offset
+// and the p-free sub-tets cap the minimum).  With none left every candidate
+// scores exactly the cap, and with U clearly below the current score none is
+// better: the level is decided without scoring.  Rings or frames outside the
+// bounds' range score every sub-tet.
+//
+// Bound by VALU issue and, now, by the staging: 15,000 -> ~2,700 VALU
+// instructions per vertex.
+template <int NQ>
+__device__ void hex_vertex(const SearchArgs& a, int vid, bool emin, HexLds* s_hx, int* s_act)
+{
+    const int lane = (int)(threadIdx.x & 63);
+    const HexFrame f = hex_stage(a, vid, emin, s_hx);
+    if (hex_pinned(f)) return;   // uniform: every lane holds the same frame
+    const int ns = f.corner8 ? 4 : 5, nSub = ns * f.n;
+    float qcur = hex_start_score(f, s_hx);
+    const float S0 = hex_acc_score(f.acc0, f.epsD, f.epsF);   // the score of a candidate that selects none
+    // the cap's det / F^1.5
+    const float capY = f.inRange ? __builtin_amdgcn_sqrtf(f.acc0.bd2 * __builtin_amdgcn_rcpf(f.acc0.bF3)) : FLT_MAX;
+    float cx = f.x0x, cy = f.x0y, cz = f.x0z, ds = a.gridScale;
     const int j = lane % NQ, k = lane / NQ;
     const bool active = lane < NQ * NQ;
-    float ds = a.gridScale;
     bool moved = false;
-    for (int d = 0; d < a.depth; ++d) {
+    for (int d = 0; d < a.depth; ++d, ds = ds * a.shrink) {
         const float gxM = cx + ds * f.ex, gxm = cx - ds * f.ex;
         const float gyM = cy + ds * f.ey, gym = cy - ds * f.ey;
         const float gzM = cz + ds * f.ez, gzm = cz - ds * f.ez;
+        // window box in frame coordinates, widened by the rounding of the
+        // candidates' world coordinates
+        const float wx = (cx - f.x0x) * f.sg, wy = (cy - f.x0y) * f.sg, wz = (cz - f.x0z) * f.sg;
+        const float Hx = 1.001f * (ds * f.ex) * f.sg + 0x1p-20f * (fabsf(cx) + ds * f.ex) * f.sg;
+        const float Hy = 1.001f * (ds * f.ey) * f.sg + 0x1p-20f * (fabsf(cy) + ds * f.ey) * f.sg;
+        const float Hz = 1.001f * (ds * f.ez) * f.sg + 0x1p-20f * (fabsf(cz) + ds * f.ez) * f.sg;
+        auto bound = [&](int t) {
+            const int e = sub_elem(t, f.corner8), s = t - e * ns;
+            return hex_bound(s_hx[e].hp[s], s == 1 || s == 4, wx, wy, wz, Hx, Hy, Hz, f.epsD, f.epsF);
+        };
+        float u = FLT_MAX;
+        bool sel = true;
+        HexBound b0{ FLT_MAX, FLT_MAX, true, true };
+        for (int t = lane; t < nSub; t += 64) {
+            const HexBound b = bound(t);
+            if (t == lane) b0 = b;
+            u = fminf(u, b.ub);
+            sel = sel && b.sel;
+        }
+        const float U = fminf(wave_min_u(u), capY);
+        if (U < 0.0f) continue;   // a determinant below 0 all over the window: every candidate scores 0
+        const bool fast = f.inRange && __ballot(!sel) == 0ull && U >= kSelY;
+        const float tq = qcur * (1.0f / 3.0f), yq = tq * __builtin_amdgcn_sqrtf(tq);   // qcur's det / F^1.5
+        if (fast && U * (1.0f + kSel) < yq * (1.0f - kSel)) continue;   // no candidate reaches qcur
+        int nAct = 0;
+        for (int t0 = 0; t0 < nSub; t0 += 64) {
+            const int t = t0 + lane;
+            const int e = sub_elem(t, f.corner8), s = t - e * ns;
+            bool keep = t < nSub;
+            if (keep && fast) {
+                const HexBound b = t0 == 0 ? b0 : bound(t);
+                keep = !(b.clear && b.lb * (1.0f - kSel) > U * (1.0f + 2.0f * kSel));
+            }
+            const unsigned long long bal = __ballot(keep);
+            if (keep)
+                s_act[nAct + __popcll(bal & ((1ull << lane) - 1ull))] = (e << 4) | (s << 1) | (s == 1 || s == 4 ? 1 : 0);
+            nAct += __popcll(bal);
+        }
+        if (nAct == 0) {   // every candidate scores S0: the first one, if that is better
+            if (qcur < S0) {
+                cx = grid_coord(a.aff, 0, NQ, gxm, gxM);
+                cy = grid_coord(a.aff, 0, NQ, gym, gyM);
+                cz = grid_coord(a.aff, 0, NQ, gzm, gzM);
+                qcur = S0;
+                moved = true;
+            }
+            continue;
+        }
+        wave_lds_fence();
         const float py = (grid_coord(a.aff, j, NQ, gym, gyM) - f.x0y) * f.sg;
         const float pz = (grid_coord(a.aff, k, NQ, gzm, gzM) - f.x0z) * f.sg;
-        float px[CPL], t3[CPL];
+        float px[NQ], t3[NQ];
 #pragma unroll
-        for (int i = 0; i < CPL; ++i) {
-            px[i] = (grid_coord(a.aff, i0 + i, NQ, gxm, gxM) - f.x0x) * f.sg;
+        for (int i = 0; i < NQ; ++i) {
+            px[i] = (grid_coord(a.aff, i, NQ, gxm, gxM) - f.x0x) * f.sg;
             t3[i] = 3.0f * px[i];
         }
-        HexAcc acc[CPL];
+        const float Q1 = fmaf(pz, pz, py * py), Q3 = 3.0f * Q1;
+        HexAcc acc[NQ];
 #pragma unroll
-        for (int i = 0; i < CPL; ++i) acc[i] = f.acc0;
-        if (a.hexCorner8) hex_ring_add_cpl<4, CPL>(acc, s_hx, f.n, px, t3, py, pz);   // uniform: a kernel argument
-        else hex_ring_add_cpl<5, CPL>(acc, s_hx, f.n, px, t3, py, pz);
+        for (int i = 0; i < NQ; ++i) acc[i] = f.acc0;
+        for (int q = 0; q < nAct; ++q) {
+            const int code = uniform(s_act[q]);
+            const HexP h = s_hx[code >> 4].hp[(code >> 1) & 7];
+            if (code & 1) hex_add_cpl<true, NQ>(acc, h, px, t3, py, pz, Q1, Q3);
+            else hex_add_cpl<false, NQ>(acc, h, px, t3, py, pz, Q1, Q3);
+        }
+        wave_lds_fence();   // the next level rewrites the list
+        // scores: only of candidates whose ratio is within rounding of the
+        // best one's (a clearly smaller ratio has a smaller score), and none
+        // where the accumulator is still the cap's
+        float y[NQ], ym = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) {
+            y[i] = (acc[i].dmin < f.epsD || acc[i].fmin < f.epsF) ? 0.0f : acc[i].bd2 * __builtin_amdgcn_rcpf(acc[i].bF3);
+            ym = fmaxf(ym, y[i]);
+        }
+        const float Y = wave_max_u(active ? ym : 0.0f);
+        const bool quick = fast && Y > 1e-30f;   // below, the ratios are not exact enough to rank by
+        if (quick && Y < (yq * yq) * (1.0f - 4.0f * kSel)) continue;
+        const float lim = Y * (1.0f - kSel);
         float best = -FLT_MAX;
         int bi = 0;
 #pragma unroll
-        for (int i = 0; i < CPL; ++i) {
-            float q = hex_acc_score(acc[i], f.epsD, f.epsF);
-            if (q > best) { best = q; bi = i; }
+        for (int i = 0; i < NQ; ++i) {
+            const bool in = active && (!quick || y[i] >= lim);
+            const bool cap = quick && acc[i].bd2 == f.acc0.bd2 && acc[i].bF3 == f.acc0.bF3;
+            float q = S0;
+            if (__ballot(in && !cap) != 0ull) {
+                const float qe = hex_acc_score(acc[i], f.epsD, f.epsF);
+                q = cap ? S0 : qe;
+            }
+            if (in && q > best) { best = q; bi = i; }
         }
-        if (!active) best = -FLT_MAX;
-        int cand = lane * NQ + i0 + bi;
-        block_argmax<W>(best, cand, rd.f, rd.i);
-        if (qcur < best) {
-            const int wi = cand % NQ, wj = (cand / NQ) % NQ, wk = cand / (NQ * NQ);
+        const float bm = wave_max_u(best);
+        if (qcur < bm) {
+            const int l = __builtin_ctzll(__ballot(best == bm));
+            const int wi = __builtin_amdgcn_readlane(bi, l), wj = l % NQ, wk = l / NQ;
             cx = grid_coord(a.aff, wi, NQ, gxm, gxM);
             cy = grid_coord(a.aff, wj, NQ, gym, gyM);
             cz = grid_coord(a.aff, wk, NQ, gzm, gzM);
-            qcur = best;
+            qcur = bm;
             moved = true;
         }
-        ds = ds * a.shrink;
     }
-    return moved;
-}
-
-template <int NQ, int W>
-__device__ void hex_vertex(const SearchArgs& a, int vid, bool emin, HexLds* s_hx, RedLds<W>& rd)
-{
-    const int tid = (W == 1) ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
-    const HexFrame f = hex_stage<W>(a, vid, emin, s_hx, rd);
-    if (hex_pinned(f)) return;   // uniform over the block: f is computed by every thread from the LDS
-    const float qcur = hex_score(f, s_hx, 0.0f, 0.0f, 0.0f);
-    float cx = f.x0x, cy = f.x0y, cz = f.x0z;
-    if (hex_levels<NQ, W>(a, f, s_hx, rd, qcur, cx, cy, cz) && tid == 0) {
-        a.xw[vid] = cx; a.yw[vid] = cy; a.zw[vid] = cz;
-    }
+    if (moved && lane == 0) { a.xw[vid] = cx; a.yw[vid] = cy; a.zw[vid] = cz; }
 }
 
 // ------------------------------------------------------------- flat tris
@@ -621,12 +827,15 @@ __global__ __launch_bounds__(64 * W, VSDMO_TET_MIN_WAVES) void k_search_tet(Sear
     __shared__ RedLds<W> rd;
     tet_vertex<NQ, W>(a, a.cStart + blockIdx.x, a.extentMin != 0, s_tc, rd);
 }
-template <int NQ, int W>
-__global__ __launch_bounds__(64 * W) void k_search_hex(SearchArgs a)
+#ifndef VSDMO_HEX_MIN_WAVES
+#define VSDMO_HEX_MIN_WAVES 4
+#endif
+template <int NQ>
+__global__ __launch_bounds__(64, VSDMO_HEX_MIN_WAVES) void k_search_hex(SearchArgs a, int ringCap)
 {
-    extern __shared__ HexLds s_hx[];
-    __shared__ RedLds<W> rd;
-    hex_vertex<NQ, W>(a, a.cStart + blockIdx.x, a.extentMin != 0, s_hx, rd);
+    extern __shared__ __align__(16) unsigned char s_hxv[];
+    hex_vertex<NQ>(a, a.cStart + blockIdx.x, a.extentMin != 0, reinterpret_cast<HexLds*>(s_hxv),
+                   hex_act(s_hxv, ringCap));
 }
 template <int NQ, int W>
 __global__ __launch_bounds__(64 * W) void k_search_flat(SearchArgs a)
@@ -1408,16 +1617,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 void k_search_hex_learned_def(SearchArgs a, LearnArgs la0, int ringCap, int nbList)
 {
     extern __shared__ __align__(16) unsigned char s_hxd[];
-    __shared__ RedLds<4> rd;
     const LearnArgs la = learn_resolve(la0);
     const int nbWin = (int)gridDim.x - nbList;
     if ((int)blockIdx.x >= nbWin) {
         const int lb = (int)blockIdx.x - nbWin;
         const int n = min(*la.cntIn, a.cEnd - a.cStart);
         if (lb == 0 && threadIdx.x == 0) atomicAdd(la.fallbacks, n);
-        for (int i = lb; i < n; i += nbList) {
-            hex_vertex<NQ, 4>(a, la.listIn[i], a.extentMin != 0, reinterpret_cast<HexLds*>(s_hxd), rd);
-            __syncthreads();
+        const int w = uniform((int)(threadIdx.x >> 6));   // one vertex per wave, in the wave's own LDS
+        unsigned char* lds = s_hxd + (size_t)w * hex_wave_lds(ringCap);
+        for (int i = lb + w * nbList; i < n; i += 4 * nbList) {
+            hex_vertex<NQ>(a, uniform(la.listIn[i]), a.extentMin != 0, reinterpret_cast<HexLds*>(lds),
+                           hex_act(lds, ringCap));
+            wave_lds_fence();   // the next vertex restages the ring
         }
         return;
     }
@@ -1441,25 +1652,25 @@ __global__ __launch_bounds__(64 * W) void k_search_list_tet(SearchArgs a, const 
         __syncthreads();   // the next vertex restages the LDS ring
     }
 }
-template <int NQ, int W>
-__global__ __launch_bounds__(64 * W) void k_search_list_hex(SearchArgs a, const int* __restrict__ list,
-                                                           const int* __restrict__ cnt, int* fallbacks)
+template <int NQ>
+__global__ __launch_bounds__(64) void k_search_list_hex(SearchArgs a, const int* __restrict__ list,
+                                                       const int* __restrict__ cnt, int* fallbacks, int ringCap)
 {
-    extern __shared__ HexLds s_hxf[];
-    __shared__ RedLds<W> rd;
+    extern __shared__ __align__(16) unsigned char s_hxf[];
     const int n = min(*cnt, a.cEnd - a.cStart);
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(fallbacks, n);
     for (int i = blockIdx.x; i < n; i += gridDim.x) {
-        hex_vertex<NQ, W>(a, list[i], a.extentMin != 0, s_hxf, rd);
-        __syncthreads();   // the next vertex restages the LDS ring
+        hex_vertex<NQ>(a, uniform(list[i]), a.extentMin != 0, reinterpret_cast<HexLds*>(s_hxf), hex_act(s_hxf, ringCap));
+        wave_lds_fence();   // the next vertex restages the ring
     }
 }
 template <int NQ, int W>
 static void list_nqw(int kind, const SearchArgs& a, const int* list, const int* cnt, int* fallbacks, int grid,
-                     size_t lds, hipStream_t s)
+                     int ringCap, hipStream_t s)
 {
+    const size_t lds = search_lds_bytes(kind, ringCap);
     if (kind == VSDMO_TET) launch_kernel(k_search_list_tet<NQ, W>, grid, 64 * W, lds, s, a, list, cnt, fallbacks);
-    else launch_kernel(k_search_list_hex<NQ, W>, grid, 64 * W, lds, s, a, list, cnt, fallbacks);
+    else launch_kernel(k_search_list_hex<NQ>, grid, 64, lds, s, a, list, cnt, fallbacks, ringCap);
 }
 
 template <int NQ, int LV, bool FUSED>
@@ -1563,17 +1774,16 @@ void launch_search_learned(int kind, int nq, const SearchArgs& a, const LearnNet
 #undef VSDMO_LEARN_CASE
     // second launch: the plain search of the fallbacks, W waves per vertex,
     // a quarter of the class's blocks (blocks loop when more fall back)
-    const size_t lds1 = (size_t)ringCap * per;
     const int g1 = std::max(1, std::min(nc, std::max(256, nc / 4)));
     switch (nq) {
-    case 2: list_nqw<2, 2>(kind, a, list, cnt, fallbacks, g1, lds1, s); break;
-    case 4: list_nqw<4, 4>(kind, a, list, cnt, fallbacks, g1, lds1, s); break;
-    case 6: list_nqw<6, 2>(kind, a, list, cnt, fallbacks, g1, lds1, s); break;
+    case 2: list_nqw<2, 2>(kind, a, list, cnt, fallbacks, g1, ringCap, s); break;
+    case 4: list_nqw<4, 4>(kind, a, list, cnt, fallbacks, g1, ringCap, s); break;
+    case 6: list_nqw<6, 2>(kind, a, list, cnt, fallbacks, g1, ringCap, s); break;
     case 8:
         // the fallback lists are short (a few per cent of the class): latency
         // bound, 4 waves per vertex (1, 2, 4 and 8 measured on the 40^3 tet
         // and 48^3 hex cubes)
-        list_nqw<8, 4>(kind, a, list, cnt, fallbacks, g1, lds1, s);
+        list_nqw<8, 4>(kind, a, list, cnt, fallbacks, g1, ringCap, s);
         break;
     default: break;
     }
@@ -1605,25 +1815,6 @@ __global__ __launch_bounds__(256, 5) void k_search_tet_split(SearchArgs a, int n
         tet_vertex<NQ, WT>(a, a.cStart + nHead + ((int)blockIdx.x - headBlocks), emin, s_tcs, rdt);
     }
 }
-template <int NQ, int WT>
-__global__ __launch_bounds__(256) void k_search_hex_split(SearchArgs a, int nHead, int ringCap)
-{
-    extern __shared__ HexLds s_hxs[];
-    __shared__ RedLds<1> rd1;
-    __shared__ RedLds<WT> rdt;
-    const bool emin = a.extentMin != 0;
-    const int headBlocks = (nHead + 3) >> 2;
-    if ((int)blockIdx.x < headBlocks) {
-        const int w = threadIdx.x >> 6;
-        const int i = 4 * (int)blockIdx.x + w;
-        if (i < nHead) hex_vertex<NQ, 1>(a, a.cStart + i, emin, s_hxs + (size_t)w * ringCap, rd1);
-        else __syncthreads();
-    } else {
-        static_assert(WT == 4, "the tail blocks use all 4 waves");
-        hex_vertex<NQ, WT>(a, a.cStart + nHead + ((int)blockIdx.x - headBlocks), emin, s_hxs, rdt);
-    }
-}
-
 // ------------------------------------------------------- batched sweep
 // Persistent kernel of one colour round of a batch of meshes: blocks take
 // work items from a queue (one atomic counter per round) until it is empty.
@@ -1637,7 +1828,7 @@ __global__ __launch_bounds__(256) void k_search_hex_split(SearchArgs a, int nHea
 // blocks so that they cost no atomics.
 template <int NQ, int W>
 __device__ __forceinline__ void batch_item(const SearchArgs& a, const int* rowHex, const int* valHex, int code,
-                                           float4* s_dyn, RedLds<W>& rd)
+                                           int hexCap, float4* s_dyn, RedLds<W>& rd)
 {
     const int vid = code & 0x3fffffff, type = (code >> 30) & 3;
     if (type == 0) tet_vertex<NQ, W>(a, vid, false, reinterpret_cast<TetC*>(s_dyn), rd);
@@ -1645,7 +1836,10 @@ __device__ __forceinline__ void batch_item(const SearchArgs& a, const int* rowHe
         SearchArgs ah = a;
         ah.ringRow = rowHex;
         ah.ringVal = valHex;
-        hex_vertex<NQ, W>(ah, vid, true, reinterpret_cast<HexLds*>(s_dyn), rd);
+        // one wave; the others of the block wait at the round's next barrier
+        if (threadIdx.x < 64)
+            hex_vertex<NQ>(ah, uniform(vid), true, reinterpret_cast<HexLds*>(s_dyn),
+                           hex_act(reinterpret_cast<unsigned char*>(s_dyn), hexCap));
     }
     else flat_vertex<NQ, W>(a, vid, reinterpret_cast<TriC*>(s_dyn), rd);
 }
@@ -1653,7 +1847,7 @@ __device__ __forceinline__ void batch_item(const SearchArgs& a, const int* rowHe
 template <int NQ, int W>
 __global__ __launch_bounds__(64 * W) void k_batch_round(SearchArgs a, const int* __restrict__ rowHex,
                                                        const int* __restrict__ valHex, const int* __restrict__ items,
-                                                       int lo, int mid, int hi, int* __restrict__ ctr)
+                                                       int lo, int mid, int hi, int* __restrict__ ctr, int hexCap)
 {
     extern __shared__ float4 s_dyn[];
     __shared__ RedLds<W> rd;
@@ -1664,11 +1858,11 @@ __global__ __launch_bounds__(64 * W) void k_batch_round(SearchArgs a, const int*
         __syncthreads();
         const int it = lo + s_item;
         if (it >= mid) break;
-        batch_item<NQ, W>(a, rowHex, valHex, items[it], s_dyn, rd);
+        batch_item<NQ, W>(a, rowHex, valHex, items[it], hexCap, s_dyn, rd);
     }
     for (int it = mid + (int)blockIdx.x; it < hi; it += (int)gridDim.x) {
         __syncthreads();
-        batch_item<NQ, W>(a, rowHex, valHex, items[it], s_dyn, rd);
+        batch_item<NQ, W>(a, rowHex, valHex, items[it], hexCap, s_dyn, rd);
     }
 }
 
@@ -1903,7 +2097,7 @@ template <int NQ, int W>
 static void launch_nqw(int kind, const SearchArgs& a, int nBlocks, size_t lds, hipStream_t s)
 {
     if (kind == VSDMO_TET) launch_kernel(k_search_tet<NQ, W>, nBlocks, 64 * W, lds, s, a);
-    else if (kind == VSDMO_HEX) launch_kernel(k_search_hex<NQ, W>, nBlocks, 64 * W, lds, s, a);
+    else if (kind == VSDMO_HEX) launch_kernel(k_search_hex<NQ>, nBlocks, 64, lds, s, a, (int)(lds / kHexLdsPer));
     else launch_kernel(k_search_flat<NQ, W>, nBlocks, 64 * W, lds, s, a);
 }
 template <int NQ>
@@ -1922,7 +2116,7 @@ template <int NQ, int W, int TYPE>
 __global__ __launch_bounds__(64 * W, TYPE == 0 ? VSDMO_TET_MIN_WAVES : 1) void k_batch_typed(SearchArgs a,
                                                                                         const int* __restrict__ rowHex,
                                                        const int* __restrict__ valHex, const int* __restrict__ items,
-                                                       int lo)
+                                                       int lo, int hexCap)
 {
     extern __shared__ float4 s_dyn[];
     __shared__ RedLds<W> rd;
@@ -1933,7 +2127,8 @@ __global__ __launch_bounds__(64 * W, TYPE == 0 ? VSDMO_TET_MIN_WAVES : 1) void k
         SearchArgs ah = a;
         ah.ringRow = rowHex;
         ah.ringVal = valHex;
-        hex_vertex<NQ, W>(ah, vid, true, reinterpret_cast<HexLds*>(s_dyn), rd);
+        hex_vertex<NQ>(ah, vid, true, reinterpret_cast<HexLds*>(s_dyn),
+                       hex_act(reinterpret_cast<unsigned char*>(s_dyn), hexCap));
     } else {
         flat_vertex<NQ, W>(a, vid, reinterpret_cast<TriC*>(s_dyn), rd);
     }
@@ -1944,9 +2139,9 @@ static void batch_typed_nqw(const SearchArgs& a, const int* rowHex, const int* v
                             int type, size_t lds, hipStream_t s)
 {
     const unsigned n = (unsigned)(hi - lo);
-    if (type == 0) k_batch_typed<NQ, W, 0><<<n, 64 * W, lds, s>>>(a, rowHex, valHex, items, lo);
-    else if (type == 1) k_batch_typed<NQ, W, 1><<<n, 64 * W, lds, s>>>(a, rowHex, valHex, items, lo);
-    else k_batch_typed<NQ, W, 2><<<n, 64 * W, lds, s>>>(a, rowHex, valHex, items, lo);
+    if (type == 0) k_batch_typed<NQ, W, 0><<<n, 64 * W, lds, s>>>(a, rowHex, valHex, items, lo, 0);
+    else if (type == 1) k_batch_typed<NQ, 1, 1><<<n, 64, lds, s>>>(a, rowHex, valHex, items, lo, (int)(lds / kHexLdsPer));
+    else k_batch_typed<NQ, W, 2><<<n, 64 * W, lds, s>>>(a, rowHex, valHex, items, lo, 0);
 }
 template <int NQ>
 static void batch_typed_nq(int w, const SearchArgs& a, const int* rowHex, const int* valHex, const int* items, int lo,
@@ -1968,11 +2163,12 @@ struct BatchLaunch {
     int grid;
     size_t lds;
     hipStream_t s;
+    int hexCap;
 };
 template <int NQ, int W>
 static void batch_nqw(const BatchLaunch& L)
 {
-    k_batch_round<NQ, W><<<L.grid, 64 * W, L.lds, L.s>>>(L.a, L.rowHex, L.valHex, L.items, L.lo, L.mid, L.hi, L.ctr);
+    k_batch_round<NQ, W><<<L.grid, 64 * W, L.lds, L.s>>>(L.a, L.rowHex, L.valHex, L.items, L.lo, L.mid, L.hi, L.ctr, L.hexCap);
 }
 template <int NQ, int W>
 static int batch_occ(size_t lds)
@@ -2002,22 +2198,18 @@ bool waves_supported(int nq, int w)
 }
 
 template <int NQ, int WT>
-static void split_nq(int kind, const SearchArgs& a, int nHead, int nTail, int ringCap, hipStream_t s)
+static void split_nq(const SearchArgs& a, int nHead, int nTail, int ringCap, hipStream_t s)
 {
     const int grid = (nHead + 3) / 4 + nTail;
     if (grid <= 0) return;
-    if (kind == VSDMO_TET)
-        launch_kernel(k_search_tet_split<NQ, WT>, grid, 256, sizeof(TetC) * 4 * (size_t)ringCap, s, a, nHead, ringCap);
-    else
-        launch_kernel(k_search_hex_split<NQ, WT>, grid, 256, sizeof(HexLds) * 4 * (size_t)ringCap, s, a, nHead, ringCap);
+    launch_kernel(k_search_tet_split<NQ, WT>, grid, 256, sizeof(TetC) * 4 * (size_t)ringCap, s, a, nHead, ringCap);
 }
 
 bool split_supported(int kind, int nq, int ringCap)
 {
-    if (kind != VSDMO_TET && kind != VSDMO_HEX) return false;
+    if (kind != VSDMO_TET) return false;   // hex searches run one wave per vertex
     if (nq != 4 && nq != 8) return false;   // the tail needs 4 waves per vertex (nq / 4 candidates per lane)
-    const size_t per = (kind == VSDMO_TET) ? sizeof(TetC) : sizeof(HexLds);
-    return per * 4 * (size_t)std::max(ringCap, 1) <= 65536;
+    return sizeof(TetC) * 4 * (size_t)std::max(ringCap, 1) <= 65536;
 }
 
 void launch_search_split(int kind, int nq, const SearchArgs& a, int tail, int ringCap, hipStream_t s)
@@ -2026,8 +2218,8 @@ void launch_search_split(int kind, int nq, const SearchArgs& a, int tail, int ri
     if (n <= 0) return;
     const int nTail = std::min(n, std::max(tail, 0));
     const int nHead = n - nTail;
-    if (nq == 4) split_nq<4, 4>(kind, a, nHead, nTail, ringCap, s);
-    else if (nq == 8) split_nq<8, 4>(kind, a, nHead, nTail, ringCap, s);
+    if (nq == 4) split_nq<4, 4>(a, nHead, nTail, ringCap, s);
+    else if (nq == 8) split_nq<8, 4>(a, nHead, nTail, ringCap, s);
 }
 
 int batch_round_blocks_per_cu(int nq, int w, size_t lds)
@@ -2041,10 +2233,10 @@ int batch_round_blocks_per_cu(int nq, int w, size_t lds)
 }
 
 void launch_batch_round(int nq, int w, const SearchArgs& a, const int* rowHex, const int* valHex, const int* items,
-                        int lo, int mid, int hi, int* ctr, int grid, size_t lds, hipStream_t s)
+                        int lo, int mid, int hi, int* ctr, int grid, size_t lds, int hexCap, hipStream_t s)
 {
     if (hi <= lo || grid <= 0) return;
-    BatchLaunch L{ a, rowHex, valHex, items, lo, mid, hi, ctr, grid, lds, s };
+    BatchLaunch L{ a, rowHex, valHex, items, lo, mid, hi, ctr, grid, lds, s, hexCap };
     switch (nq) {
     case 2: batch_nq<2>(w, L); break;
     case 4: batch_nq<4>(w, L); break;
@@ -2105,14 +2297,14 @@ void launch_batch_quality(const BatchQArgs& a, hipStream_t s)
 
 size_t batch_lds_bytes(int maxRingTet, int maxRingHex, int maxHETri)
 {
-    size_t b = std::max(sizeof(TetC) * (size_t)maxRingTet, sizeof(HexLds) * (size_t)maxRingHex);
+    size_t b = std::max(sizeof(TetC) * (size_t)maxRingTet, kHexLdsPer * (size_t)maxRingHex);
     b = std::max(b, sizeof(TriC) * (size_t)maxHETri);
     return std::max(b, (size_t)16);
 }
 
 size_t search_lds_bytes(int kind, int maxRing)
 {
-    size_t per = (kind == VSDMO_TET) ? sizeof(TetC) : (kind == VSDMO_HEX) ? sizeof(HexLds) : sizeof(TriC);
+    size_t per = (kind == VSDMO_TET) ? sizeof(TetC) : (kind == VSDMO_HEX) ? kHexLdsPer : sizeof(TriC);
     return per * (size_t)std::max(maxRing, 1);
 }
 
