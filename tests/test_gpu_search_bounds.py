@@ -1,5 +1,6 @@
 """The searches that leave out what a bound rules out give the full search's
-bits: hex levels score only the sub-tets that can decide a candidate
+bits: hex levels score only the sub-tets that can decide a candidate, tet
+levels only the candidates above the ring's tangent planes
 (csrc/dmo_kernels.hip).  Positions bit-exact against the oracle, which scores
 everything, on the forms where a bound or a selection could go wrong: exact
 and near ties (regular and barely jittered meshes), inverted and flat

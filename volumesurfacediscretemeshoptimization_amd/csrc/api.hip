@@ -574,18 +574,6 @@ vsdmo_status vsdmo_opt_create(vsdmo_mesh* m, int32_t criterion, float grid_scale
     });
 }
 
-// waves_per_vertex 0: one launch per class with one vertex per wave and the
-// last kSplitTail vertices at 4 waves each (tet / hex, nq 4 or 8)
-constexpr int kSplitTail = 1024;
-static void dispatch_search(vsdmo_opt* o, int kind, const SearchArgs& a, size_t lds, hipStream_t s)
-{
-    const int w = o->p.waves_per_vertex;
-    if (w == 0 && split_supported(kind, o->p.nq, o->m->maxRing))
-        launch_search_split(kind, o->p.nq, a, kSplitTail, o->m->maxRing, s);
-    else
-        launch_search(kind, o->p.nq, w == 0 ? 1 : w, a, lds, s);
-}
-
 // HIP events on every search launch while timing is on: the kernels' own
 // begin and end (KernelEvents; every timed launch goes through
 // launch_kernel).  The events are pooled and reused: creating them per
@@ -646,11 +634,11 @@ vsdmo_status vsdmo_opt_iterate(vsdmo_opt* o, int32_t n)
         a.ringRow = m->ringRow.p; a.ringVal = m->ringVal.p;
         a.heRow = m->heRow.p; a.heTarget = m->heTarget.p;
         a.gridScale = o->grid_scale; a.shrink = o->shrink; a.aff = o->aff;
+        a.reach = search_reach(o->grid_scale, o->shrink, o->p.depth);
         a.depth = o->p.depth; a.extentMin = o->extent_min;
         a.hexCorner8 = o->p.hex_metric == VSDMO_HEX_CORNER8;
         for (int it = 0; it < n; ++it) {
             if (m->elem == VSDMO_TET || m->elem == VSDMO_HEX) {
-                size_t lds = search_lds_bytes(m->elem, m->maxRing);
                 // the classes' fallback-list lengths start at zero (one fill per iteration)
                 const int nCls = (int)m->colOffInner.size() - 1;
                 const bool deferred = o->learn_mode != 0 && !o->rec && o->learn_fallback == VSDMO_FALLBACK_DEFERRED;
@@ -707,7 +695,7 @@ vsdmo_status vsdmo_opt_iterate(vsdmo_opt* o, int32_t n)
                         }
                         o->s_learned += nc;
                     } else {
-                        timed(o, [&]() { dispatch_search(o, m->elem, a, lds, m->stream); });
+                        timed(o, [&]() { launch_search(m->elem, o->p.nq, a, m->maxRing, m->stream); });
                     }
                     if (take > 0) {
                         launch_targets(m->x.p, m->y.p, m->z.p, a.cStart, a.cStart + take, ds->L.p, ds->v0.p,
@@ -756,10 +744,9 @@ vsdmo_status vsdmo_opt_iterate(vsdmo_opt* o, int32_t n)
                 surf_nn_launch(sa, m->stream);
                 surf_normals_launch(sa, m->stream);
             } else {
-                size_t lds = search_lds_bytes(VSDMO_TRI, m->maxHE);
                 for (size_t c = 0; c + 1 < m->colOffFree.size(); ++c) {
                     a.cStart = m->colOffFree[c]; a.cEnd = m->colOffFree[c + 1];
-                    timed(o, [&]() { dispatch_search(o, VSDMO_TRI, a, lds, m->stream); });
+                    timed(o, [&]() { launch_search(VSDMO_TRI, o->p.nq, a, m->maxHE, m->stream); });
                     o->s_surf += a.cEnd - a.cStart;
                 }
                 if (o->surface && o->last_min > 0.0f) {

@@ -139,6 +139,7 @@ SearchArgs search_args(vsdmo_batch* b)
     a.ringRow = b->rowTet.p; a.ringVal = b->ringTet.p;
     a.heRow = b->heRow.p; a.heTarget = b->heTarget.p;
     a.gridScale = b->p.grid_scale; a.shrink = b->shrink; a.aff = b->aff;
+    a.reach = search_reach(b->p.grid_scale, b->shrink, b->p.depth);
     a.depth = b->p.depth;
     a.hexCorner8 = b->p.hex_metric == VSDMO_HEX_CORNER8;
     return a;
@@ -185,7 +186,7 @@ void upload_items(vsdmo_batch* b)
 void size_grids(vsdmo_batch* b)
 {
     b->lds = batch_lds_bytes(b->maxRingTet, b->maxRingHex, b->maxHE);
-    int per = std::max(1, batch_round_blocks_per_cu(b->p.nq, b->p.waves_per_vertex, b->lds));
+    int per = std::max(1, batch_round_blocks_per_cu(b->p.nq, b->lds));
     b->grid.assign(b->roundOff.size() > 0 ? b->roundOff.size() - 1 : 0, 0);
     for (size_t r = 0; r + 1 < b->roundOff.size(); ++r) {
         int n = b->roundOff[r + 1] - b->roundOff[r];
@@ -290,20 +291,16 @@ void record_iteration(vsdmo_batch* b)
         if (!b->p.persistent) {
             // one block per item: a launch per element type, each with its
             // own body's registers and LDS
-            const int w = b->p.waves_per_vertex;
             if (!lt)
-                launch_batch_typed(b->p.nq, w, a, b->rowHex.p, b->ringHex.p, b->items.p, off, midT, 0,
-                                   batch_lds_bytes(b->maxRingTet, 0, 0), s);
+                launch_batch_typed(b->p.nq, a, b->rowHex.p, b->ringHex.p, b->items.p, off, midT, 0, b->maxRingTet, s);
             if (!lh)
-                launch_batch_typed(b->p.nq, w, a, b->rowHex.p, b->ringHex.p, b->items.p, midT, mid, 1,
-                                   batch_lds_bytes(0, b->maxRingHex, 0), s);
-            launch_batch_typed(b->p.nq, w, a, b->rowHex.p, b->ringHex.p, b->items.p, mid, hi, 2,
-                               batch_lds_bytes(0, 0, b->maxHE), s);
+                launch_batch_typed(b->p.nq, a, b->rowHex.p, b->ringHex.p, b->items.p, midT, mid, 1, b->maxRingHex, s);
+            launch_batch_typed(b->p.nq, a, b->rowHex.p, b->ringHex.p, b->items.p, mid, hi, 2, b->maxHE, s);
             continue;
         }
         auto plain = [&](int lo, int qend, int end) {
-            launch_batch_round(b->p.nq, b->p.waves_per_vertex, a, b->rowHex.p, b->ringHex.p, b->items.p, lo, qend, end,
-                               b->ctr.p + r, b->grid[r], b->lds, b->maxRingHex, s);
+            launch_batch_round(b->p.nq, a, b->rowHex.p, b->ringHex.p, b->items.p, lo, qend, end, b->ctr.p + r,
+                               b->grid[r], b->lds, std::max(b->maxRingTet, 1), std::max(b->maxRingHex, 1), s);
         };
         if (lh && !lt) {   // hexes learned, tets plain: the tets, then the triangles
             plain(off, midT, midT);

@@ -44,10 +44,20 @@ struct SearchArgs {
     const int* __restrict__ heTarget;
     int cStart, cEnd;                  // colour class [cStart, cEnd)
     float gridScale, shrink, aff;
+    float reach;                       // search_reach of the window and its levels
     int depth;
     int extentMin;
     int hexCorner8;                    // 1: hex metric over the 8 corner sub-tets (vsdmo_hex_metric)
 };
+
+// how far a search can move from its start, in units of the window's
+// half-extent: the sum of the levels' half-widths
+inline float search_reach(float gridScale, float shrink, int depth)
+{
+    double r = 0.0, d = gridScale;
+    for (int k = 0; k < depth; ++k, d *= shrink) r += d;
+    return (float)(r * (1.0 + 1e-6));
+}
 
 // element kinds of the quality kernels beyond vsdmo_elem: triangles of a
 // surface mesh on the surface path (unsigned 3D mean ratio)
@@ -159,24 +169,23 @@ struct BatchQArgs {
     int per;                   // elements per thread: chunks of <= 256 * per elements
 };
 
-size_t search_lds_bytes(int kind, int maxRing);
+size_t search_lds_bytes(int kind, int ringCap);
 bool waves_supported(int nq, int w);
-void launch_search(int kind, int nq, int w, const SearchArgs& a, size_t lds, hipStream_t s);
-// tet / hex class in one launch: one vertex per wave for all but the last
-// `tail` vertices, which get several waves each (waves_per_vertex = 0)
-bool split_supported(int kind, int nq, int ringCap);
-void launch_search_split(int kind, int nq, const SearchArgs& a, int tail, int ringCap, hipStream_t s);
-// one colour round of a batch, persistent: grid blocks take the tet / hex
-// items [lo, mid) from the atomic counter *ctr and stride over the flat
+// the plain searches of one colour class, one wave per vertex (flat triangle
+// classes of 4,096 and more: 4 vertices per wave); ringCap >= the largest
+// one-ring (tet / hex) or fan (flat)
+void launch_search(int kind, int nq, const SearchArgs& a, int ringCap, hipStream_t s);
+// one colour round of a batch, persistent: grid one-wave blocks take the tet /
+// hex items [lo, mid) from the atomic counter *ctr and stride over the flat
 // items [mid, hi) (the one-block-per-item schedule is launch_batch_typed)
-void launch_batch_round(int nq, int w, const SearchArgs& a, const int* rowHex, const int* valHex, const int* items,
-                        int lo, int mid, int hi, int* ctr, int grid, size_t lds, int hexCap, hipStream_t s);
-int batch_round_blocks_per_cu(int nq, int w, size_t lds);
+void launch_batch_round(int nq, const SearchArgs& a, const int* rowHex, const int* valHex, const int* items, int lo,
+                        int mid, int hi, int* ctr, int grid, size_t lds, int tetCap, int hexCap, hipStream_t s);
+int batch_round_blocks_per_cu(int nq, size_t lds);
 void launch_fill_int(int* p, int n, int v, hipStream_t s);
 // one block per item of items[lo, hi), all of element type `type` (0 tet,
 // 1 hex, 2 flat tri): that type's search body alone
-void launch_batch_typed(int nq, int w, const SearchArgs& a, const int* rowHex, const int* valHex, const int* items,
-                        int lo, int hi, int type, size_t lds, hipStream_t s);
+void launch_batch_typed(int nq, const SearchArgs& a, const int* rowHex, const int* valHex, const int* items, int lo,
+                        int hi, int type, int ringCap, hipStream_t s);
 // zero the n counters cnt + (*itDev & 1) * n (device-side iteration parity)
 void launch_parity_zero(int* cnt, int n, const int* itDev, hipStream_t s);
 // *p += v on the device (one thread)

@@ -1,12 +1,12 @@
 // dmo_kernels.hip -- DMO vertex-search and quality kernels for gfx950.
 //
-// One wave64 per vertex.  For the 3D searches the nq^3 candidates of a level
-// are split so that lane l = j + nq*k owns the nq candidates (i, j, k),
-// i = 0..nq-1, i.e. the contiguous candidate indices [nq*l, nq*l + nq): a
-// lowest-lane-then-lowest-i argmax is the reference's lowest-index tie rule.
-// The one-ring is staged in LDS as per-element constants in a vertex-local
-// frame; per element and lane the (y, z) part of det and L is formed once and
-// reused for the nq candidates along x.
+// One wave64 per vertex.  The one-ring is staged in LDS as per-element
+// constants in a vertex-local frame.  A level of the 3D searches has nq^3
+// candidates, index i + nq (j + nq k), the lowest index winning ties; bounds
+// leave out what cannot decide it (tet_vertex: candidates no better than the
+// current score; hex_vertex: sub-tets no candidate's minimum can be), and what
+// is left is scored in the canonical order, so every result is the full
+// search's, bit for bit.
 //
 // Reference kernels: k_optimizeHierarchicalInnerTet / Hex
 // (VSDMO/src/dmo/DMOTetImplCub.h:20-137, DMOHexImplCub.h:20-137) and
@@ -21,64 +21,35 @@
 
 namespace vsdmo {
 
-__device__ __forceinline__ float wave_max(float v)
-{
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v = fmaxf(v, __shfl_xor(v, m));
-    return v;
-}
-__device__ __forceinline__ float wave_min(float v)
-{
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v = fminf(v, __shfl_xor(v, m));
-    return v;
-}
-// argmax over the wave: larger score wins, equal scores -> smaller index
-__device__ __forceinline__ void wave_argmax(float& best, int& idx)
-{
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-        float ob = __shfl_xor(best, m);
-        int oi = __shfl_xor(idx, m);
-        bool take = (ob > best) || (ob == best && oi < idx);
-        best = take ? ob : best;
-        idx = take ? oi : idx;
-    }
-}
-
-// Reductions over the wave whose result is uniform (an SGPR): DPP moves inside
-// the rows of 16 lanes, two row broadcasts, lane 63 holds the result.  The
-// ds_bpermute of a shuffle costs an LDS round trip per step.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ float dpp_move(float v)
-{
-    const int i = __builtin_bit_cast(int, v);
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, CTRL, ROWS, 0xf, false));
-}
 __device__ __forceinline__ float lane_f(float v, int lane)
 {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
+// Reductions over the wave whose result is uniform (an SGPR): DPP operands
+// inside the rows of 16 lanes, two row broadcasts, lane 63 holds the result.  A
+// shuffle costs an LDS round trip per step, the compiler's DPP moves three
+// instructions (move, canonicalise, min); written out it is one.  A lane
+// without a source keeps its value; the s_nops are the two wait states between
+// a VALU write and a DPP read of the same register.
+#define VSDMO_WAVE_REDUCE(OP)                                                       \
+    asm("s_nop 1\n\t" OP " %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"    \
+        "s_nop 1\n\t" OP " %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf\n\t"    \
+        "s_nop 1\n\t" OP " %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf\n\t"    \
+        "s_nop 1\n\t" OP " %0, %0, %0 row_shr:8 row_mask:0xf bank_mask:0xf\n\t"    \
+        "s_nop 1\n\t" OP " %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t" \
+        "s_nop 1\n\t" OP " %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf"      \
+        : "+v"(v))
 __device__ __forceinline__ float wave_max_u(float v)
 {
-    v = fmaxf(v, dpp_move<0x111, 0xf>(v));   // row_shr 1, 2, 4, 8
-    v = fmaxf(v, dpp_move<0x112, 0xf>(v));
-    v = fmaxf(v, dpp_move<0x114, 0xf>(v));
-    v = fmaxf(v, dpp_move<0x118, 0xf>(v));
-    v = fmaxf(v, dpp_move<0x142, 0xa>(v));   // row_bcast 15 into rows 1, 3
-    v = fmaxf(v, dpp_move<0x143, 0xc>(v));   // row_bcast 31 into rows 2, 3
+    VSDMO_WAVE_REDUCE("v_max_f32_dpp");
     return lane_f(v, 63);
 }
 __device__ __forceinline__ float wave_min_u(float v)
 {
-    v = fminf(v, dpp_move<0x111, 0xf>(v));
-    v = fminf(v, dpp_move<0x112, 0xf>(v));
-    v = fminf(v, dpp_move<0x114, 0xf>(v));
-    v = fminf(v, dpp_move<0x118, 0xf>(v));
-    v = fminf(v, dpp_move<0x142, 0xa>(v));
-    v = fminf(v, dpp_move<0x143, 0xc>(v));
+    VSDMO_WAVE_REDUCE("v_min_f32_dpp");
     return lane_f(v, 63);
 }
+#undef VSDMO_WAVE_REDUCE
 // LDS written by some lanes of the wave, read by others of the same wave: its
 // LDS operations complete in order, the fence keeps the compiler's order
 __device__ __forceinline__ void wave_lds_fence()
@@ -88,294 +59,7 @@ __device__ __forceinline__ void wave_lds_fence()
 }
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// Block-level reductions for W waves per vertex (blockDim = 64*W).  With
-// W = 1 they are the wave shuffles alone; otherwise the per-wave results are
-// combined through LDS.  max/min and the (score, index) argmax are order
-// independent, so every W gives the same result.
-template <int W>
-__device__ __forceinline__ float block_max(float v, float* s)
-{
-    v = wave_max(v);
-    if constexpr (W > 1) {
-        const int w = threadIdx.x >> 6;
-        if ((threadIdx.x & 63) == 0) s[w] = v;
-        __syncthreads();
-        v = s[0];
-#pragma unroll
-        for (int k = 1; k < W; ++k) v = fmaxf(v, s[k]);
-        __syncthreads();
-    }
-    return v;
-}
-template <int W>
-__device__ __forceinline__ float block_min(float v, float* s)
-{
-    v = wave_min(v);
-    if constexpr (W > 1) {
-        const int w = threadIdx.x >> 6;
-        if ((threadIdx.x & 63) == 0) s[w] = v;
-        __syncthreads();
-        v = s[0];
-#pragma unroll
-        for (int k = 1; k < W; ++k) v = fminf(v, s[k]);
-        __syncthreads();
-    }
-    return v;
-}
-template <int W>
-__device__ __forceinline__ void block_argmax(float& best, int& idx, float* sf, int* si)
-{
-    wave_argmax(best, idx);
-    if constexpr (W > 1) {
-        const int w = threadIdx.x >> 6;
-        if ((threadIdx.x & 63) == 0) { sf[w] = best; si[w] = idx; }
-        __syncthreads();
-        best = sf[0];
-        idx = si[0];
-#pragma unroll
-        for (int k = 1; k < W; ++k) {
-            const float ob = sf[k];
-            const int oi = si[k];
-            if (ob > best || (ob == best && oi < idx)) { best = ob; idx = oi; }
-        }
-        __syncthreads();
-    }
-}
-
-// LDS scratch of the block reductions
-template <int W>
-struct RedLds { float f[W]; int i[W]; float e[4][W]; };
-
-// The staging reductions in one exchange: per-axis window half-extents (min
-// or max of the offsets) and the largest offset.  One barrier: rd.e is read
-// here and written again only by the next vertex's staging, after the
-// barrier that ends this one.
-template <int W>
-__device__ __forceinline__ void block_extents(bool emin, float& ex, float& ey, float& ez, float& mabs, RedLds<W>& rd)
-{
-    if (emin) { ex = wave_min(ex); ey = wave_min(ey); ez = wave_min(ez); }
-    else { ex = wave_max(ex); ey = wave_max(ey); ez = wave_max(ez); }
-    mabs = wave_max(mabs);
-    if constexpr (W > 1) {
-        const int w = threadIdx.x >> 6;
-        if ((threadIdx.x & 63) == 0) { rd.e[0][w] = ex; rd.e[1][w] = ey; rd.e[2][w] = ez; rd.e[3][w] = mabs; }
-        __syncthreads();
-        ex = rd.e[0][0]; ey = rd.e[1][0]; ez = rd.e[2][0]; mabs = rd.e[3][0];
-#pragma unroll
-        for (int k = 1; k < W; ++k) {
-            ex = emin ? fminf(ex, rd.e[0][k]) : fmaxf(ex, rd.e[0][k]);
-            ey = emin ? fminf(ey, rd.e[1][k]) : fmaxf(ey, rd.e[1][k]);
-            ez = emin ? fminf(ez, rd.e[2][k]) : fmaxf(ez, rd.e[2][k]);
-            mabs = fmaxf(mabs, rd.e[3][k]);
-        }
-    }
-}
-
-// ------------------------------------------------------------------ tets
-// The staged state of one vertex search: start position, window
-// half-extents, frame scale and ring size; the ring's constants are in LDS.
-struct TetFrame {
-    float x0x, x0y, x0z, ex, ey, ez, sg, is3;
-    int n;
-};
-
-// Stage vid's one-ring: per-axis window half-extent (max or min offset), the
-// frame scale and the constants of every ring element in LDS.  Every thread
-// of the block calls it; it ends with a barrier.
-template <int W>
-__device__ TetFrame tet_stage(const SearchArgs& a, int vid, bool emin, TetC* s_tc, RedLds<W>& rd)
-{
-    constexpr int T = 64 * W;
-    // W = 1 bodies also run one per wave inside wider blocks (k_search_split)
-    const int tid = (W == 1) ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
-    TetFrame f;
-    const int r0 = a.ringRow[vid];
-    f.n = a.ringRow[vid + 1] - r0;
-    f.x0x = a.x[vid]; f.x0y = a.y[vid]; f.x0z = a.z[vid];
-    float ex = emin ? FLT_MAX : -FLT_MAX, ey = ex, ez = ex, mabs = 0.0f;
-    auto extent = [&](float dxs, float dys, float dzs) {
-        const float dx = fabsf(dxs), dy = fabsf(dys), dz = fabsf(dzs);
-        ex = emin ? fminf(ex, dx) : fmaxf(ex, dx);
-        ey = emin ? fminf(ey, dy) : fmaxf(ey, dy);
-        ez = emin ? fminf(ez, dz) : fmaxf(ez, dz);
-        mabs = fmaxf(mabs, fmaxf(dx, fmaxf(dy, dz)));
-    };
-    // the thread's first element (all of them when the ring has at most T)
-    // keeps its corner offsets in registers for the constants, so the
-    // positions are read from memory once
-    const bool own0 = tid < f.n;
-    float d0[3][3];
-    if (own0) {
-        const int* h = a.ringVal + (size_t)(r0 + tid) * 3;
-#pragma unroll
-        for (int t = 0; t < 3; ++t) {
-            const int v = h[t];
-            d0[t][0] = a.x[v] - f.x0x; d0[t][1] = a.y[v] - f.x0y; d0[t][2] = a.z[v] - f.x0z;
-            extent(d0[t][0], d0[t][1], d0[t][2]);
-        }
-    }
-    for (int e = tid + T; e < f.n; e += T) {
-        const int* h = a.ringVal + (size_t)(r0 + e) * 3;
-#pragma unroll
-        for (int t = 0; t < 3; ++t) {
-            const int v = h[t];
-            extent(a.x[v] - f.x0x, a.y[v] - f.x0y, a.z[v] - f.x0z);
-        }
-    }
-    block_extents<W>(emin, ex, ey, ez, mabs, rd);
-    f.ex = ex; f.ey = ey; f.ez = ez;
-    f.sg = pow2_scale(mabs);
-    const float isg = 1.0f / f.sg;
-    f.is3 = ((1.0f * isg) * isg) * isg;
-    if (own0) {
-        f3 p[3];
-#pragma unroll
-        for (int t = 0; t < 3; ++t) p[t] = { d0[t][0] * f.sg, d0[t][1] * f.sg, d0[t][2] * f.sg };
-        s_tc[tid] = tet_consts(p[0], p[1], p[2]);
-    }
-    for (int e = tid + T; e < f.n; e += T) {
-        const int* h = a.ringVal + (size_t)(r0 + e) * 3;
-        f3 p[3];
-#pragma unroll
-        for (int t = 0; t < 3; ++t) {
-            int v = h[t];
-            p[t] = { (a.x[v] - f.x0x) * f.sg, (a.y[v] - f.x0y) * f.sg, (a.z[v] - f.x0z) * f.sg };
-        }
-        s_tc[e] = tet_consts(p[0], p[1], p[2]);
-    }
-    __syncthreads();
-    return f;
-}
-
-// ring score of one candidate p' (frame coordinates)
-__device__ __forceinline__ float tet_score(const TetFrame& f, const TetC* s_tc, float px, float py, float pz)
-{
-    const float Qyz = 3.0f * fmaf(pz, pz, py * py);
-    const float t3 = 3.0f * px;
-    TetAcc acc = tet_acc0();
-    for (int e = 0; e < f.n; ++e) {
-        const TetC c = s_tc[e];
-        float Tyz = fmaf(c.nny, py, fmaf(c.nnz, pz, c.D));
-        float Ryz = fmaf(c.m2sy, py, fmaf(c.m2sz, pz, c.K + Qyz));
-        tet_acc_add(acc, fmaf(c.nnx, px, Tyz), fmaf(px, t3 + c.m2sx, Ryz));
-    }
-    return tet_acc_score(acc, f.is3);
-}
-
-// The nested grid search from the start position (depth levels of NQ^3
-// candidates) with W waves.  Lane l = j + nq*k of wave w owns the candidates
-// (i, j, k) with i in [w*nq/W, (w+1)*nq/W); candidate index i + nq*l, so the
-// lowest index wins ties as in the reference.  The start score qcur is
-// accumulated in the first level's element loop (at p = 0, det = D and L =
-// K exactly: tet_score's terms, in ring order).  Returns whether the vertex
-// moved, and its position in (cx, cy, cz).
-template <int NQ, int W>
-__device__ bool tet_levels(const SearchArgs& a, const TetFrame& f, const TetC* s_tc, RedLds<W>& rd, float& cx,
-                           float& cy, float& cz)
-{
-    constexpr int CPL = NQ / W;
-    static_assert(NQ % W == 0, "nq must be a multiple of the waves per vertex");
-    const int tid = (W == 1) ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
-    const int lane = tid & 63, i0 = (tid >> 6) * CPL;
-    const int j = lane % NQ, k = lane / NQ;
-    const bool active = lane < NQ * NQ;
-    float ds = a.gridScale;
-    bool moved = false;
-    float qcur = 0.0f;
-    for (int d = 0; d < a.depth; ++d) {
-        const float gxM = cx + ds * f.ex, gxm = cx - ds * f.ex;
-        const float gyM = cy + ds * f.ey, gym = cy - ds * f.ey;
-        const float gzM = cz + ds * f.ez, gzm = cz - ds * f.ez;
-        const float py = (grid_coord(a.aff, j, NQ, gym, gyM) - f.x0y) * f.sg;
-        const float pz = (grid_coord(a.aff, k, NQ, gzm, gzM) - f.x0z) * f.sg;
-        float px[CPL], t3[CPL];
-#pragma unroll
-        for (int i = 0; i < CPL; ++i) {
-            px[i] = (grid_coord(a.aff, i0 + i, NQ, gxm, gxM) - f.x0x) * f.sg;
-            t3[i] = 3.0f * px[i];
-        }
-        const float Qyz = 3.0f * fmaf(pz, pz, py * py);
-        TetAcc acc[CPL];
-#pragma unroll
-        for (int i = 0; i < CPL; ++i) acc[i] = tet_acc0();
-        // two elements per iteration: their minima fold into v_min3 without
-        // canonicalising each accumulator per element (111 -> 97.5 VALU per
-        // element at 8 candidates per lane)
-        auto ring = [&](auto withQ0) {
-            constexpr bool WQ = decltype(withQ0)::value;
-            TetAcc acc0 = tet_acc0();
-#pragma unroll 2
-            for (int e = 0; e < f.n; ++e) {
-                const TetC c = s_tc[e];
-                const float Tyz = fmaf(c.nny, py, fmaf(c.nnz, pz, c.D));
-                const float Ryz = fmaf(c.m2sy, py, fmaf(c.m2sz, pz, c.K + Qyz));
-#pragma unroll
-                for (int i = 0; i < CPL; ++i)
-                    tet_acc_add(acc[i], fmaf(c.nnx, px[i], Tyz), fmaf(px[i], t3[i] + c.m2sx, Ryz));
-                if constexpr (WQ) tet_acc_add(acc0, c.D, c.K);
-            }
-            if constexpr (WQ) qcur = tet_acc_score(acc0, f.is3);
-        };
-        if (d == 0) ring(std::true_type{});
-        else ring(std::false_type{});
-        float best = -FLT_MAX;
-        int bi = 0;
-#pragma unroll
-        for (int i = 0; i < CPL; ++i) {
-            float q = tet_acc_score(acc[i], f.is3);
-            if (q > best) { best = q; bi = i; }
-        }
-        if (!active) best = -FLT_MAX;
-        int cand = lane * NQ + i0 + bi;
-        block_argmax<W>(best, cand, rd.f, rd.i);
-        if (qcur < best) {
-            const int wi = cand % NQ, wj = (cand / NQ) % NQ, wk = cand / (NQ * NQ);
-            cx = grid_coord(a.aff, wi, NQ, gxm, gxM);
-            cy = grid_coord(a.aff, wj, NQ, gym, gyM);
-            cz = grid_coord(a.aff, wk, NQ, gzm, gzM);
-            qcur = best;
-            moved = true;
-        }
-        ds = ds * a.shrink;
-    }
-    return moved;
-}
-
-// One vertex per block of W waves (or per wave, W = 1).
-template <int NQ, int W>
-__device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, TetC* s_tc, RedLds<W>& rd)
-{
-    const int tid = (W == 1) ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
-    const TetFrame f = tet_stage<W>(a, vid, emin, s_tc, rd);
-    float cx = f.x0x, cy = f.x0y, cz = f.x0z;
-    if (tet_levels<NQ, W>(a, f, s_tc, rd, cx, cy, cz) && tid == 0) {
-        a.xw[vid] = cx; a.yw[vid] = cy; a.zw[vid] = cz;
-    }
-}
-
-// ------------------------------------------------------------------ hexes
-struct HexLds { float cd[4], cF[4]; HexP hp[5]; };
-
-// LDS of a hex vertex search per ring element: the constants and the codes of
-// the element's sub-tets in the list of those a level scores
-constexpr size_t kHexLdsPer = sizeof(HexLds) + 5 * sizeof(int);
-// rounded up for a wave's slice of a block's LDS
-__host__ __device__ constexpr size_t hex_wave_lds(int ringCap) { return (kHexLdsPer * (size_t)ringCap + 15) / 16 * 16; }
-__device__ __forceinline__ int* hex_act(unsigned char* lds, int ringCap)
-{
-    return reinterpret_cast<int*>(lds + sizeof(HexLds) * (size_t)ringCap);
-}
-
-// staged state of a hex vertex search (as TetFrame), plus the accumulator of
-// the 4 sub-tets per ring element that do not contain the moving vertex
-struct HexFrame {
-    float x0x, x0y, x0z, ex, ey, ez, sg, epsD, epsF;
-    int n;
-    bool corner8;   // the principal-axes sub-tet (slot 4 of HexP) left out
-    bool inRange;   // hex_stage: every p-free pair is in sel_range
-    HexAcc acc0;
-};
-
+// ------------------------------------------------- the canonical selection
 // The canonical selection compares ratios det^2 / F^3 in FP32 products; it
 // picks by the true ratios wherever they differ by more than its rounding, as
 // long as no product leaves the normal range.  kSelF / kSelD bound F and det
@@ -412,6 +96,441 @@ __device__ __forceinline__ void select_lanes(float& bd2, float& bF3, bool hasAcc
         bF3 = take ? lF : bF3;
     }
 }
+
+// ------------------------------------------------------------------ tets
+// LDS of a tet vertex search: the ring's constants, the level's plane of each
+// element (4 floats: gradient, offset for cells; the offset for candidates in
+// an array of its own; both padded to tiles of 16), the cells a level keeps and
+// the candidates to score
+constexpr int kTetCells = 64, kTetBuf = 128, kTetFew = 3;
+__host__ __device__ constexpr int tet_rows(int ringCap) { return (ringCap + 15) / 16 * 16; }
+__host__ __device__ constexpr size_t tet_wave_lds(int ringCap)
+{
+    return sizeof(TetC) * (size_t)ringCap + 5 * sizeof(float) * (size_t)tet_rows(ringCap) +
+           (kTetCells + kTetBuf) * sizeof(int);
+}
+
+// the staged state of one vertex search
+struct TetFrame {
+    float x0x, x0y, x0z, ex, ey, ez, sg, is3;
+    int n;
+};
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+// or of the bits of 4 products: its sign bit says whether one is negative (a
+// fminf of a product costs a canonicalising v_max per operand besides)
+__device__ __forceinline__ int sign4(v4f v)
+{
+    const float a = v[0], b = v[1], c = v[2], d = v[3];
+    return __builtin_bit_cast(int, a) | __builtin_bit_cast(int, b) | __builtin_bit_cast(int, c) | __builtin_bit_cast(int, d);
+}
+// m[t]: per lane the or over 4 of 16 rows of column 16 t + lane % 16 (the lane's
+// group lane / 16 holds rows 4 (lane / 16) + 0..3).  Returns the or over all
+// rows of column `lane`: the swaps exchange halves, then odd and even groups,
+// so that group t collects column tile t.  Every lane must call it.
+__device__ __forceinline__ int or_columns(const int (&m)[4])
+{
+    auto swap32 = [](int a, int b) {
+        const auto r = __builtin_amdgcn_permlane32_swap((unsigned)a, (unsigned)b, false, false);
+        return (int)(r[0] | r[1]);
+    };
+    auto swap16 = [](int a, int b) {
+        const auto r = __builtin_amdgcn_permlane16_swap((unsigned)a, (unsigned)b, false, false);
+        return (int)(r[0] | r[1]);
+    };
+    return swap16(swap32(m[0], m[2]), swap32(m[1], m[3]));
+}
+
+// The nested grid search of a tet vertex, one wave.
+//
+// A candidate beats the current score q only if det > y L^1.5 for every ring
+// element, y = (q / kCTet)^1.5.  With L = 3 F, F = |p - g|^2 + K, the function f =
+// det - s F^1.5, s = 3^1.5 y, is concave (det is affine, F^1.5 convex), so it
+// stays below its tangent plane at the window's centre: a candidate below 0 on
+// some element's plane is no better.  One lane per element makes the level's
+// planes.  The 64 cells of 2 x 2 x 2 candidates (nq 8) are tried against them in
+// one small matrix product on the FP32 MFMA, (plane) x (cell centre, 1); a
+// plane's maximum over a cell is its value at the centre plus sum h |gradient|.
+// The kept cells' candidates are tried the same way, 8 cells at a time, and
+// what is left is scored in the canonical order, one candidate per lane over
+// the whole ring, or, up to kTetFew of them, one after the other with one
+// element per lane.  The best score (the lowest index on a tie) is the level's:
+// the full search's bits.  Scoring 512 candidates takes ~98 VALU operations per
+// element.  On 40^3 cubes 0 / 0-1 / 5-30 candidates of the three levels are
+// scored once the mesh has settled, 50-90 at the start.
+//
+// Margins: s carries -2^-9, the planes 2^-18 of the sum of their terms'
+// magnitudes over the search's reach P (a.reach in window units), K is lowered
+// by 2^-18 of L's terms, and a candidate's coordinates may be off by delta (1e-3
+// of the spacing and 2^-20 of the world coordinate); the canonical evaluation
+// rounds by a few 2^-24, its selection by ~2^-22 per comparison.  Vertices at q
+// < 0 (an inverted ring) look at the cells with positive planes first and at the
+// others only if no candidate there reaches 0.  Frames outside the planes'
+// range score every candidate.
+//
+// Bound by VALU issue (and the matrix unit, ~15 % of the time).  Scoring every
+// candidate, with 8 candidates per lane, took 9,200 VALU operations per vertex
+// and 81 us per class of the 40^3 cube (7,400 vertices); here 3,950 and 80 us
+// in the first iteration, 1,270 and 25 us in the 20th.  A gradient bound at
+// every cell's centre instead of the planes (23 operations per element and 64
+// cells) took 3,430 on average against 1,920; the planes as fused multiply-adds
+// over LDS broadcasts 2,240; ranking the kept candidates by det F^-1.5 on the
+// MFMA before scoring was slower than scoring them (8.9 against 6.9 ms per 20
+// iterations).
+template <int NQ>
+__device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, unsigned char* lds, int ringCap)
+{
+    const int lane = (int)(threadIdx.x & 63);
+    TetC* s_tc = reinterpret_cast<TetC*>(lds);
+    float* s_pl = reinterpret_cast<float*>(s_tc + ringCap);
+    float* s_pw = s_pl + 4 * tet_rows(ringCap);
+    int* s_cell = reinterpret_cast<int*>(s_pw + tet_rows(ringCap));
+    int* s_buf = s_cell + kTetCells;
+    TetFrame f;
+    const int r0 = uniform(a.ringRow[vid]);
+    f.n = uniform(a.ringRow[vid + 1]) - r0;
+    if (f.n <= 0) return;   // no element: nothing scores below the start
+    f.x0x = a.x[vid]; f.x0y = a.y[vid]; f.x0z = a.z[vid];
+    float ex = emin ? FLT_MAX : -FLT_MAX, ey = ex, ez = ex, mabs = 0.0f;
+    auto extent = [&](float dxs, float dys, float dzs) {
+        const float dx = fabsf(dxs), dy = fabsf(dys), dz = fabsf(dzs);
+        ex = emin ? fminf(ex, dx) : fmaxf(ex, dx);
+        ey = emin ? fminf(ey, dy) : fmaxf(ey, dy);
+        ez = emin ? fminf(ez, dz) : fmaxf(ez, dz);
+        mabs = fmaxf(mabs, fmaxf(dx, fmaxf(dy, dz)));
+    };
+    // the lane's first element keeps its corner offsets in registers for the
+    // constants, so the positions are read from memory once
+    const bool own0 = lane < f.n;
+    float d0[3][3];
+    if (own0) {
+        const int* h = a.ringVal + (size_t)(r0 + lane) * 3;
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const int v = h[t];
+            d0[t][0] = a.x[v] - f.x0x; d0[t][1] = a.y[v] - f.x0y; d0[t][2] = a.z[v] - f.x0z;
+            extent(d0[t][0], d0[t][1], d0[t][2]);
+        }
+    }
+    for (int e = lane + 64; e < f.n; e += 64) {
+        const int* h = a.ringVal + (size_t)(r0 + e) * 3;
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const int v = h[t];
+            extent(a.x[v] - f.x0x, a.y[v] - f.x0y, a.z[v] - f.x0z);
+        }
+    }
+    if (emin) { f.ex = wave_min_u(ex); f.ey = wave_min_u(ey); f.ez = wave_min_u(ez); }
+    else { f.ex = wave_max_u(ex); f.ey = wave_max_u(ey); f.ez = wave_max_u(ez); }
+    f.sg = pow2_scale(wave_max_u(mabs));
+    const float isg = 1.0f / f.sg;
+    f.is3 = ((1.0f * isg) * isg) * isg;
+    TetC c0{ 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f };
+    if (own0) {
+        f3 p[3];
+#pragma unroll
+        for (int t = 0; t < 3; ++t) p[t] = { d0[t][0] * f.sg, d0[t][1] * f.sg, d0[t][2] * f.sg };
+        c0 = tet_consts(p[0], p[1], p[2]);
+        s_tc[lane] = c0;
+    }
+    for (int e = lane + 64; e < f.n; e += 64) {
+        const int* h = a.ringVal + (size_t)(r0 + e) * 3;
+        f3 p[3];
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            int v = h[t];
+            p[t] = { (a.x[v] - f.x0x) * f.sg, (a.y[v] - f.x0y) * f.sg, (a.z[v] - f.x0z) * f.sg };
+        }
+        s_tc[e] = tet_consts(p[0], p[1], p[2]);
+    }
+    wave_lds_fence();
+
+    // the canonical score of one position from (det, L) of the ring's elements,
+    // one per lane (rings of at most 64); false where the lanes cannot tell
+    auto lanes_score = [&](float det, float L, float& q) -> bool {
+        const float dmin = wave_min_u(own0 ? det : FLT_MAX);
+        if (dmin < 0.0f) { q = (dmin * (1.0f / 6.0f)) * f.is3; return true; }
+        if (dmin == 0.0f) { q = 0.0f; return true; }
+        if (__ballot(own0 && !sel_range(det, L)) != 0ull) return false;
+        TetAcc acc = tet_acc0();
+        select_lanes(acc.bd2, acc.bL3, false, own0, det, L);
+        q = kCTet * cbrt_nr(acc.bd2 / acc.bL3);
+        return true;
+    };
+    // start score (p = 0: det = D, L = K exactly)
+    float qcur = 0.0f;
+    if (f.n > 64 || !lanes_score(c0.D, c0.K, qcur)) {
+        TetAcc acc = tet_acc0();
+        for (int e = 0; e < f.n; ++e) tet_acc_add(acc, s_tc[e].D, s_tc[e].K);
+        qcur = tet_acc_score(acc, f.is3);
+    }
+
+    constexpr int NB = NQ / 2, NC = NB * NB * NB;   // cells per axis, cells
+    constexpr unsigned long long kAllCells = NC == 64 ? ~0ull : (1ull << NC) - 1ull;
+    constexpr float kR = 0x1p-18f, kStep = 1.0f / (float)(NQ - 1);
+    // P bounds every candidate's frame coordinates
+    const float P = 2.03f * a.reach + 0x1p-17f * (fmaxf(fabsf(f.x0x), fmaxf(fabsf(f.x0y), fabsf(f.x0z))) * f.sg);
+    // the element's g and lowered K (F = |p - g|^2 + K)
+    struct Quad { float gx, gy, gz, K; };
+    auto quad = [&](const TetC& c) {
+        Quad q;
+        q.gx = c.m2sx * (-1.0f / 6.0f); q.gy = c.m2sy * (-1.0f / 6.0f); q.gz = c.m2sz * (-1.0f / 6.0f);
+        q.K = (c.K * (1.0f / 3.0f) - fmaf(q.gx, q.gx, fmaf(q.gy, q.gy, q.gz * q.gz))) -
+              kR * (c.K + P * (fabsf(c.m2sx) + fabsf(c.m2sy) + fabsf(c.m2sz) + 9.0f * P));
+        return q;
+    };
+    const Quad q0 = quad(c0);
+    const int comp = lane >> 4, col = lane & 15;   // the lane's row (x, y, z, 1) and column of the products' operands
+    const int nt = (f.n + 15) >> 4;
+    bool fast = false;
+    // cell `lane`, packed indices along x, y, z; column 16 t + col's place along
+    // the lane's axis in window half-widths (candidate i lies at 1 - 2 i / (nq -
+    // 1), a cell between candidates 2 b and 2 b + 1)
+    const int myCell = (lane % NB) | ((lane / NB) % NB) << 8 | (lane / (NB * NB)) << 16;
+    float cellU[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+    if constexpr (NC > 8) {
+        bool ok = P <= 32.0f && (!own0 || (q0.K >= kSelF && c0.K <= 4096.0f));
+        for (int e = lane + 64; e < f.n; e += 64) ok = ok && quad(s_tc[e]).K >= kSelF && s_tc[e].K <= 4096.0f;
+        fast = __ballot(!ok) == 0ull;
+        // rows past the ring bound nothing
+        if (lane < 16 * nt - f.n) {
+            const int e = f.n + lane;
+            *reinterpret_cast<float4*>(s_pl + 4 * e) = make_float4(0.0f, 0.0f, 0.0f, 1e30f);
+            s_pw[e] = 1e30f;
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int cell = 16 * t + col;
+            const int b = comp == 0 ? cell % NB : comp == 1 ? (cell / NB) % NB : cell / (NB * NB);
+            cellU[t] = 1.0f - kStep * (float)(4 * b + 1);
+        }
+    }
+    // the lane's plane operand of tile et, for cells and for candidates
+    const float* const opCell = s_pl + 4 * col + comp;
+    const float* const opCand = comp < 3 ? opCell : s_pw + col;
+    const int opStep = comp < 3 ? 64 : 16;
+
+    float cx = f.x0x, cy = f.x0y, cz = f.x0z, ds = a.gridScale;
+    bool moved = false;
+    for (int d = 0; d < a.depth; ++d, ds = ds * a.shrink) {
+        const float gxM = cx + ds * f.ex, gxm = cx - ds * f.ex;
+        const float gyM = cy + ds * f.ey, gym = cy - ds * f.ey;
+        const float gzM = cz + ds * f.ez, gzm = cz - ds * f.ez;
+        // det / L^1.5 of the current score, less the margin; 0: only the signs decide
+        float yq = 0.0f;
+        if (fast && qcur > 0.0f) {
+            const float t = qcur * (1.0f / kCTet);
+            yq = (t * __builtin_amdgcn_sqrtf(t)) * (1.0f - 0x1p-9f);
+            if (!(yq >= kSelY)) yq = 0.0f;
+        }
+        const float s = yq * 5.1961524f;   // 3^1.5: against det / F^1.5
+        unsigned long long mask = kAllCells, rest = 0ull;
+        float o = 0.0f, D = 0.0f;   // the window's centre and half-width along the lane's axis
+        if constexpr (NC > 8) if (fast) {
+            // the window in frame coordinates: centre, half-widths
+            const float ox = (cx - f.x0x) * f.sg, oy = (cy - f.x0y) * f.sg, oz = (cz - f.x0z) * f.sg;
+            const float Dx = (ds * f.ex) * f.sg, Dy = (ds * f.ey) * f.sg, Dz = (ds * f.ez) * f.sg;
+            const float dx = 1e-3f * kStep * Dx + 0x1p-20f * ((fabsf(cx) + ds * f.ex) * f.sg);
+            const float dy = 1e-3f * kStep * Dy + 0x1p-20f * ((fabsf(cy) + ds * f.ey) * f.sg);
+            const float dz = 1e-3f * kStep * Dz + 0x1p-20f * ((fabsf(cz) + ds * f.ez) * f.sg);
+            auto plane = [&](int e, const TetC& c, const Quad& q) {
+                const float wx = ox - q.gx, wy = oy - q.gy, wz = oz - q.gz;
+                const float F = fmaf(wx, wx, fmaf(wy, wy, fmaf(wz, wz, q.K)));
+                const float sr = s * __builtin_amdgcn_sqrtf(F), g = 3.0f * sr;
+                const float px = fmaf(-g, wx, c.nnx), py = fmaf(-g, wy, c.nny), pz = fmaf(-g, wz, c.nnz);
+                const float det = fmaf(c.nnx, ox, fmaf(c.nny, oy, fmaf(c.nnz, oz, c.D)));
+                const float ax = fabsf(px), ay = fabsf(py), az = fabsf(pz);
+                const float m = kR * (fabsf(c.D) + sr * F +
+                                      P * ((ax + ay + az) + (fabsf(c.nnx) + fabsf(c.nny) + fabsf(c.nnz))));
+                const float w = (fmaf(-sr, F, det) - fmaf(px, ox, fmaf(py, oy, pz * oz))) +
+                                (m + fmaf(ax, dx, fmaf(ay, dy, az * dz)));
+                *reinterpret_cast<float4*>(s_pl + 4 * e) =
+                    make_float4(px, py, pz, fmaf(ax, kStep * Dx, fmaf(ay, kStep * Dy, fmaf(az, kStep * Dz, w))));
+                s_pw[e] = w;
+            };
+            if (own0) plane(lane, c0, q0);
+            for (int e = lane + 64; e < f.n; e += 64) plane(e, s_tc[e], quad(s_tc[e]));
+            wave_lds_fence();
+            o = comp == 0 ? ox : comp == 1 ? oy : comp == 2 ? oz : 1.0f;
+            D = comp == 0 ? Dx : comp == 1 ? Dy : comp == 2 ? Dz : 0.0f;
+            int neg[4] = { 0, 0, 0, 0 };
+            for (int et = 0; et < nt; ++et) {
+                const float A = opCell[64 * et];
+#pragma unroll
+                for (int t = 0; t < (NC + 15) / 16; ++t) {
+                    neg[t] |= sign4(__builtin_amdgcn_mfma_f32_16x16x4f32(A, fmaf(D, cellU[t], o), v4f{ 0.0f, 0.0f, 0.0f, 0.0f }, 0, 0, 0));
+                }
+            }
+            mask = __ballot(or_columns(neg) >= 0) & kAllCells;
+            if (qcur < 0.0f) {
+                rest = kAllCells & ~mask;
+                if (mask == 0ull) { mask = rest; rest = 0ull; }
+            }
+        }
+        float best = -FLT_MAX;
+        int cand = 0;
+        auto better = [&](float q, int code) {   // uniform
+            if (q > best || (q == best && code < cand)) { best = q; cand = code; }
+        };
+        // the canonical scores of the first n (at most 64) buffered candidates,
+        // index i + nq (j + nq k)
+        auto score = [&](int n) {
+            const int code = s_buf[min(lane, n - 1)];   // lanes past n repeat the last one
+            if (n <= kTetFew && f.n <= 64) {
+                bool told = true;
+                for (int c = 0; c < n && told; ++c) {
+                    const int at = __builtin_amdgcn_readlane(code, c);
+                    const float px = (grid_coord(a.aff, at % NQ, NQ, gxm, gxM) - f.x0x) * f.sg;
+                    const float py = (grid_coord(a.aff, (at / NQ) % NQ, NQ, gym, gyM) - f.x0y) * f.sg;
+                    const float pz = (grid_coord(a.aff, at / (NQ * NQ), NQ, gzm, gzM) - f.x0z) * f.sg;
+                    const float Qyz = 3.0f * fmaf(pz, pz, py * py), t3 = 3.0f * px;
+                    const float Tyz = fmaf(c0.nny, py, fmaf(c0.nnz, pz, c0.D));
+                    const float Ryz = fmaf(c0.m2sy, py, fmaf(c0.m2sz, pz, c0.K + Qyz));
+                    float q = 0.0f;
+                    told = lanes_score(fmaf(c0.nnx, px, Tyz), fmaf(px, t3 + c0.m2sx, Ryz), q);
+                    if (told) better(q, at);
+                }
+                if (told) return;
+            }
+            // up to 16 (32) candidates: the four (two) lanes of a candidate take a
+            // quarter (half) of the ring each
+            const int split = !fast ? 1 : n <= 16 ? 4 : n <= 32 ? 2 : 1;
+            const int mine = split == 1 ? code : s_buf[min(lane & (split == 4 ? 15 : 31), n - 1)];
+            const int part = split == 1 ? 0 : split == 4 ? lane >> 4 : lane >> 5;
+            const float px = (grid_coord(a.aff, mine % NQ, NQ, gxm, gxM) - f.x0x) * f.sg;
+            const float py = (grid_coord(a.aff, (mine / NQ) % NQ, NQ, gym, gyM) - f.x0y) * f.sg;
+            const float pz = (grid_coord(a.aff, mine / (NQ * NQ), NQ, gzm, gzM) - f.x0z) * f.sg;
+            const float Qyz = 3.0f * fmaf(pz, pz, py * py), t3 = 3.0f * px;
+            TetAcc acc = tet_acc0();
+            auto ring = [&](int first, int len) {   // a part's last element may repeat: it changes nothing
+#pragma unroll 4
+                for (int e = 0; e < len; ++e) {
+                    const TetC t = s_tc[min(first + e, f.n - 1)];
+                    const float Tyz = fmaf(t.nny, py, fmaf(t.nnz, pz, t.D));
+                    const float Ryz = fmaf(t.m2sy, py, fmaf(t.m2sz, pz, t.K + Qyz));
+                    tet_acc_add(acc, fmaf(t.nnx, px, Tyz), fmaf(px, t3 + t.m2sx, Ryz));
+                }
+            };
+            const int len = (f.n + split - 1) / split;
+            ring(part * len, len);
+            if (split > 1) {
+                // the parts in ring order: the later one's pair where its ratio is
+                // clearly smaller, the earlier one's where it is clearly larger;
+                // where neither, or the determinants leave the selection's range,
+                // the wave scores the ring in one piece
+                bool told = true;
+                auto join = [&](int far) {
+                    const float od2 = __shfl_xor(acc.bd2, far), oL3 = __shfl_xor(acc.bL3, far), od = __shfl_xor(acc.dmin, far);
+                    const float u = od2 * acc.bL3, v = acc.bd2 * oL3;
+                    told = told && !(fabsf(u - v) <= 4.0f * kSel * fmaxf(u, v));
+                    acc.bd2 = u < v ? od2 : acc.bd2;
+                    acc.bL3 = u < v ? oL3 : acc.bL3;
+                    acc.dmin = fminf(acc.dmin, od);
+                };
+                if (split == 4) join(16);
+                join(32);
+                if (__ballot(!(told && acc.dmin >= kSelD) && !(acc.dmin < 0.0f)) != 0ull) {
+                    acc = tet_acc0();
+                    ring(0, f.n);
+                }
+            }
+            // no cube roots where no ratio reaches the current score's
+            if (yq > 0.0f &&
+                __ballot(acc.dmin > 0.0f && acc.bd2 * __builtin_amdgcn_rcpf(acc.bL3) >= yq * yq) == 0ull)
+                return;
+            const float q = tet_acc_score(acc, f.is3);
+            const float m = wave_max_u(q);
+            unsigned long long bal = __ballot(q == m);
+            int lo = 0x7fffffff;
+            while (bal) {
+                lo = min(lo, __builtin_amdgcn_readlane(mine, __builtin_ctzll(bal)));
+                bal &= bal - 1;
+            }
+            better(m, lo);
+        };
+        while (mask != 0ull) {
+            const int cnt = __popcll(mask);
+            if ((mask >> lane) & 1ull) s_cell[__popcll(mask & ((1ull << lane) - 1ull))] = myCell;
+            wave_lds_fence();
+            int nbuf = 0;
+            for (int c = 0; c < cnt; c += 8) {
+                // candidate `lane` of the chunk: cell lane / 8, corner lane % 8
+                const int cell = s_cell[min(c + (lane >> 3), cnt - 1)];
+                const int code = (2 * (cell & 255) + (lane & 1)) +
+                                 NQ * ((2 * ((cell >> 8) & 255) + ((lane >> 1) & 1)) +
+                                       NQ * (2 * (cell >> 16) + ((lane >> 2) & 1)));
+                bool keep = c + (lane >> 3) < cnt;
+                if constexpr (NC > 8) if (fast && qcur >= 0.0f) {
+                    // column 16 t + col: its coordinate along the lane's axis
+                    float B[4];
+                    int neg[4] = { 0, 0, 0, 0 };
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        const int cl = s_cell[min(c + 2 * t + (col >> 3), cnt - 1)];
+                        const int i = 2 * ((cl >> (8 * comp)) & 255) + ((lane >> comp) & 1);
+                        B[t] = fmaf(D, 1.0f - 2.0f * kStep * (float)i, o);
+                    }
+                    for (int et = 0; et < nt; ++et) {
+                        const float A = opCand[opStep * et];
+#pragma unroll
+                        for (int t = 0; t < 4; ++t)
+                            neg[t] |= sign4(__builtin_amdgcn_mfma_f32_16x16x4f32(A, B[t], v4f{ 0.0f, 0.0f, 0.0f, 0.0f }, 0, 0, 0));
+                    }
+                    const int v = or_columns(neg);   // every lane takes part
+                    keep = keep && v >= 0;
+                }
+                const unsigned long long bal = __ballot(keep);
+                if (keep) s_buf[nbuf + __popcll(bal & ((1ull << lane) - 1ull))] = code;
+                nbuf += __popcll(bal);
+                wave_lds_fence();
+                if (nbuf >= 64) {
+                    score(64);
+                    nbuf -= 64;
+                    const int mv = s_buf[64 + lane];
+                    wave_lds_fence();
+                    if (lane < nbuf) s_buf[lane] = mv;
+                    wave_lds_fence();
+                }
+            }
+            if (nbuf > 0) score(nbuf);
+            wave_lds_fence();   // the lists are rewritten
+            mask = 0ull;
+            if (!(best >= 0.0f)) { mask = rest; rest = 0ull; }
+        }
+        if (qcur < best) {
+            const int wi = cand % NQ, wj = (cand / NQ) % NQ, wk = cand / (NQ * NQ);
+            cx = grid_coord(a.aff, wi, NQ, gxm, gxM);
+            cy = grid_coord(a.aff, wj, NQ, gym, gyM);
+            cz = grid_coord(a.aff, wk, NQ, gzm, gzM);
+            qcur = best;
+            moved = true;
+        }
+    }
+    if (moved && lane == 0) { a.xw[vid] = cx; a.yw[vid] = cy; a.zw[vid] = cz; }
+}
+
+// ------------------------------------------------------------------ hexes
+struct HexLds { float cd[4], cF[4]; HexP hp[5]; };
+
+// LDS of a hex vertex search per ring element: the constants and the codes of
+// the element's sub-tets in the list of those a level scores
+constexpr size_t kHexLdsPer = sizeof(HexLds) + 5 * sizeof(int);
+// rounded up for a wave's slice of a block's LDS
+__host__ __device__ constexpr size_t hex_wave_lds(int ringCap) { return (kHexLdsPer * (size_t)ringCap + 15) / 16 * 16; }
+__device__ __forceinline__ int* hex_act(unsigned char* lds, int ringCap)
+{
+    return reinterpret_cast<int*>(lds + sizeof(HexLds) * (size_t)ringCap);
+}
+
+// staged state of a hex vertex search (as TetFrame), plus the accumulator of
+// the 4 sub-tets per ring element that do not contain the moving vertex
+struct HexFrame {
+    float x0x, x0y, x0z, ex, ey, ez, sg, epsD, epsF;
+    int n;
+    bool corner8;   // the principal-axes sub-tet (slot 4 of HexP) left out
+    bool inRange;   // hex_stage: every p-free pair is in sel_range
+    HexAcc acc0;
+};
 
 // One-wave staging of vid's ring: constants in LDS, the p-free accumulator.
 __device__ HexFrame hex_stage(const SearchArgs& a, int vid, bool emin, HexLds* s_hx)
@@ -604,8 +723,9 @@ __device__ __forceinline__ void hex_add_cpl(HexAcc* acc, const HexP& h, const fl
 // better: the level is decided without scoring.  Rings or frames outside the
 // bounds' range score every sub-tet.
 //
-// Bound by VALU issue and, now, by the staging: 15,000 -> ~2,700 VALU
-// instructions per vertex.
+// Bound by VALU issue: 15,000 -> 2,300 VALU operations per vertex, 214 -> 50 us
+// per class of the 48^3 cube (13.8k vertices); about half of it is the staging
+// of the ring, 8 of 64 lanes wide.
 template <int NQ>
 __device__ void hex_vertex(const SearchArgs& a, int vid, bool emin, HexLds* s_hx, int* s_act)
 {
@@ -737,36 +857,34 @@ __device__ void hex_vertex(const SearchArgs& a, int vid, bool emin, HexLds* s_hx
 // Lane l of wave 0 holds the reference thread t = l/2's candidate B (l even)
 // or A (l odd): A = (t/nq, t%nq), B = (t/nq + nq/2, t%nq).  The lowest lane
 // among the maxima is the reference's winner (lowest thread; B on an exact
-// tie).  Further waves (W > 1) only help stage the ring.
-template <int NQ, int W>
-__device__ void flat_vertex(const SearchArgs& a, int vid, TriC* s_tr, RedLds<W>& rd)
+// tie).
+template <int NQ>
+__device__ void flat_vertex(const SearchArgs& a, int vid, TriC* s_tr)
 {
-    constexpr int T = 64 * W;
-    // W = 1 bodies also run one per wave inside wider blocks (k_search_split)
-    const int tid = (W == 1) ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
-    const int h0 = a.heRow[vid];
-    const int n = a.heRow[vid + 1] - h0;
+    const int tid = (int)(threadIdx.x & 63);
+    const int h0 = uniform(a.heRow[vid]);
+    const int n = uniform(a.heRow[vid + 1]) - h0;
     const float x0x = a.x[vid], x0y = a.y[vid];
 
     float ex = -FLT_MAX, ey = -FLT_MAX, mabs = 0.0f;
-    for (int e = tid; e < n; e += T) {
+    for (int e = tid; e < n; e += 64) {
         int v = a.heTarget[h0 + e];
         float dx = fabsf(a.x[v] - x0x), dy = fabsf(a.y[v] - x0y);
         ex = fmaxf(ex, dx);
         ey = fmaxf(ey, dy);
         mabs = fmaxf(mabs, fmaxf(dx, dy));
     }
-    float ez = 0.0f;
-    block_extents<W>(false, ex, ey, ez, mabs, rd);
-    const float sg = pow2_scale(mabs);
+    ex = wave_max_u(ex);
+    ey = wave_max_u(ey);
+    const float sg = pow2_scale(wave_max_u(mabs));
     const float isg = 1.0f / sg;
     const float is2 = (1.0f * isg) * isg;
-    for (int e = tid; e < n; e += T) {
+    for (int e = tid; e < n; e += 64) {
         int va = a.heTarget[h0 + e];
         int vb = a.heTarget[h0 + (e + 1 == n ? 0 : e + 1)];
         s_tr[e] = tri_consts((a.x[va] - x0x) * sg, (a.y[va] - x0y) * sg, (a.x[vb] - x0x) * sg, (a.y[vb] - x0y) * sg);
     }
-    __syncthreads();
+    wave_lds_fence();
 
     auto score = [&](float px, float py) {
         const float Q2 = 2.0f * (py * py);
@@ -786,19 +904,19 @@ __device__ void flat_vertex(const SearchArgs& a, int vid, TriC* s_tr, RedLds<W>&
     const int t = tid >> 1;
     const bool isA = (tid & 1) != 0;
     const int ci = t / NQ + (isA ? 0 : NQ / 2), cj = t % NQ;
-    const bool active = tid < 64 && t < NQ * NQ / 2;
+    const bool active = t < NQ * NQ / 2;
     float cx = x0x, cy = x0y;
     float ds = a.gridScale;
     float qlast = -FLT_MAX;
     for (int d = 0; d < a.depth; ++d) {
         const float gxM = cx + ds * ex, gxm = cx - ds * ex;
         const float gyM = cy + ds * ey, gym = cy - ds * ey;
-        float best = active ? score((grid_coord(a.aff, ci, NQ, gxm, gxM) - x0x) * sg,
-                                    (grid_coord(a.aff, cj, NQ, gym, gyM) - x0y) * sg)
-                            : -FLT_MAX;
-        int wl = tid;
-        block_argmax<W>(best, wl, rd.f, rd.i);
+        const float q = active ? score((grid_coord(a.aff, ci, NQ, gxm, gxM) - x0x) * sg,
+                                       (grid_coord(a.aff, cj, NQ, gym, gyM) - x0y) * sg)
+                               : -FLT_MAX;
+        const float best = wave_max_u(q);
         if (qcur < best) {
+            const int wl = __builtin_ctzll(__ballot(q == best));
             const int wt = wl >> 1;
             const int wi = wt / NQ + ((wl & 1) ? 0 : NQ / 2), wj = wt % NQ;
             cx = grid_coord(a.aff, wi, NQ, gxm, gxM);
@@ -811,22 +929,21 @@ __device__ void flat_vertex(const SearchArgs& a, int vid, TriC* s_tr, RedLds<W>&
     if (qold < qlast && tid == 0) { a.xw[vid] = cx; a.yw[vid] = cy; }
 }
 
-// one vertex per block, vertices [cStart, cEnd) of one colour class.  The
-// tet search asks for at least 5 waves per SIMD (launch bounds' second
-// argument; 89 VGPRs, no spill): a colour class of the 40^3 cube (~7.4k
-// vertices) runs in ~1.45 rounds of the 256 CUs' 5 x 4 wave slots.  6 or 7
-// waves per SIMD spill (7 / 18 registers) with the element loop taking two
-// elements per iteration.
+// one vertex per wave and block, vertices [cStart, cEnd) of one colour class.
+// The tet search asks for 6 waves per SIMD (79 VGPRs, no spill): 40^3 cube, 20
+// iterations, 6.53 ms against 6.64 at 5, 6.66 at 7 and 6.84 at 8 (both spill)
 #ifndef VSDMO_TET_MIN_WAVES
-#define VSDMO_TET_MIN_WAVES 5
+#define VSDMO_TET_MIN_WAVES 6
 #endif
-template <int NQ, int W>
-__global__ __launch_bounds__(64 * W, VSDMO_TET_MIN_WAVES) void k_search_tet(SearchArgs a)
+template <int NQ>
+__global__ __launch_bounds__(64, VSDMO_TET_MIN_WAVES) void k_search_tet(SearchArgs a, int ringCap)
 {
-    extern __shared__ TetC s_tc[];
-    __shared__ RedLds<W> rd;
-    tet_vertex<NQ, W>(a, a.cStart + blockIdx.x, a.extentMin != 0, s_tc, rd);
+    extern __shared__ __align__(16) unsigned char s_tcv[];
+    tet_vertex<NQ>(a, a.cStart + blockIdx.x, a.extentMin != 0, s_tcv, ringCap);
 }
+// the hex search asks for 4 waves per SIMD (128 VGPRs, no spill): 48^3 cube,
+// 10 iterations, 5.1 ms against 5.5 ms at 3 (129 VGPRs) and 5.1-5.2 ms at 5
+// and 6 (spills); 31^3 with the surface free 4.9, 4.8, 5.3 and 5.3 ms
 #ifndef VSDMO_HEX_MIN_WAVES
 #define VSDMO_HEX_MIN_WAVES 4
 #endif
@@ -837,12 +954,11 @@ __global__ __launch_bounds__(64, VSDMO_HEX_MIN_WAVES) void k_search_hex(SearchAr
     hex_vertex<NQ>(a, a.cStart + blockIdx.x, a.extentMin != 0, reinterpret_cast<HexLds*>(s_hxv),
                    hex_act(s_hxv, ringCap));
 }
-template <int NQ, int W>
-__global__ __launch_bounds__(64 * W) void k_search_flat(SearchArgs a)
+template <int NQ>
+__global__ __launch_bounds__(64) void k_search_flat(SearchArgs a)
 {
     extern __shared__ TriC s_tr[];
-    __shared__ RedLds<W> rd;
-    flat_vertex<NQ, W>(a, a.cStart + blockIdx.x, s_tr, rd);
+    flat_vertex<NQ>(a, a.cStart + blockIdx.x, s_tr);
 }
 
 KernelEvents*& kernel_events()
@@ -1108,10 +1224,9 @@ __global__ __launch_bounds__(256) void k_batch_flat8x4(SearchArgs a, const int* 
 // launch spreads over more CUs with one vertex per wave; measured on the 64^2
 // grid's ~960-vertex classes, 0.112 against 0.123 ms per iteration)
 constexpr int kFlat4MinVertices = 256 * kFlatGroups;
-static bool flat8x4_ok(int nq, size_t ldsPerVertex, int nVertices)
+static bool flat8x4_ok(int nq, int ringCap, int nVertices)
 {
-    return nq == 8 && ldsPerVertex >= sizeof(TriC) && kFlatGroups * ldsPerVertex <= 65536 &&
-           nVertices >= kFlat4MinVertices;
+    return nq == 8 && kFlatGroups * sizeof(TriC) * (size_t)ringCap <= 65536 && nVertices >= kFlat4MinVertices;
 }
 
 
@@ -1595,16 +1710,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 void k_search_tet_learned_def(SearchArgs a, LearnArgs la0, int ringCap, int nbList)
 {
     extern __shared__ __align__(16) unsigned char s_tcd[];
-    __shared__ RedLds<4> rd;
     const LearnArgs la = learn_resolve(la0);
     const int nbWin = (int)gridDim.x - nbList;
     if ((int)blockIdx.x >= nbWin) {
         const int lb = (int)blockIdx.x - nbWin;
         const int n = min(*la.cntIn, a.cEnd - a.cStart);
         if (lb == 0 && threadIdx.x == 0) atomicAdd(la.fallbacks, n);
-        for (int i = lb; i < n; i += nbList) {
-            tet_vertex<NQ, 4>(a, la.listIn[i], a.extentMin != 0, reinterpret_cast<TetC*>(s_tcd), rd);
-            __syncthreads();   // the next vertex restages the LDS ring
+        const int w = uniform((int)(threadIdx.x >> 6));   // one vertex per wave, in the wave's own LDS
+        unsigned char* lds = s_tcd + (size_t)w * tet_wave_lds(ringCap);
+        for (int i = lb + w * nbList; i < n; i += 4 * nbList) {
+            tet_vertex<NQ>(a, uniform(la.listIn[i]), a.extentMin != 0, lds, ringCap);
+            wave_lds_fence();   // the next vertex restages the ring
         }
         return;
     }
@@ -1639,17 +1755,16 @@ void k_search_hex_learned_def(SearchArgs a, LearnArgs la0, int ringCap, int nbLi
 // one vertex per block of W waves at a time, blocks striding over the list
 // (the grid is sized for a typical fallback share, the length is only known
 // on the device)
-template <int NQ, int W>
-__global__ __launch_bounds__(64 * W) void k_search_list_tet(SearchArgs a, const int* __restrict__ list,
-                                                           const int* __restrict__ cnt, int* fallbacks)
+template <int NQ>
+__global__ __launch_bounds__(64) void k_search_list_tet(SearchArgs a, const int* __restrict__ list,
+                                                       const int* __restrict__ cnt, int* fallbacks, int ringCap)
 {
-    extern __shared__ TetC s_tcf[];
-    __shared__ RedLds<W> rd;
+    extern __shared__ __align__(16) unsigned char s_tcf[];
     const int n = min(*cnt, a.cEnd - a.cStart);
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(fallbacks, n);
     for (int i = blockIdx.x; i < n; i += gridDim.x) {
-        tet_vertex<NQ, W>(a, list[i], a.extentMin != 0, s_tcf, rd);
-        __syncthreads();   // the next vertex restages the LDS ring
+        tet_vertex<NQ>(a, uniform(list[i]), a.extentMin != 0, s_tcf, ringCap);
+        wave_lds_fence();   // the next vertex restages the ring
     }
 }
 template <int NQ>
@@ -1664,12 +1779,12 @@ __global__ __launch_bounds__(64) void k_search_list_hex(SearchArgs a, const int*
         wave_lds_fence();   // the next vertex restages the ring
     }
 }
-template <int NQ, int W>
-static void list_nqw(int kind, const SearchArgs& a, const int* list, const int* cnt, int* fallbacks, int grid,
+template <int NQ>
+static void list_nq(int kind, const SearchArgs& a, const int* list, const int* cnt, int* fallbacks, int grid,
                      int ringCap, hipStream_t s)
 {
     const size_t lds = search_lds_bytes(kind, ringCap);
-    if (kind == VSDMO_TET) launch_kernel(k_search_list_tet<NQ, W>, grid, 64 * W, lds, s, a, list, cnt, fallbacks);
+    if (kind == VSDMO_TET) launch_kernel(k_search_list_tet<NQ>, grid, 64, lds, s, a, list, cnt, fallbacks, ringCap);
     else launch_kernel(k_search_list_hex<NQ>, grid, 64, lds, s, a, list, cnt, fallbacks, ringCap);
 }
 
@@ -1746,7 +1861,8 @@ void launch_search_learned(int kind, int nq, const SearchArgs& a, const LearnNet
         la.itDev = def->itDev; la.listStride = def->listStride; la.cntStride = def->cntStride;
         const int nbList = std::max(1, std::min(nc, std::max(64, nc / 8)));
         const int nb = (nc + kMlpRows - 1) / kMlpRows;
-        const size_t lds = fused ? fused_lds(kind, ringCap) : (size_t)kMlpRows * ringCap * per;
+        const size_t wave = kind == VSDMO_TET ? tet_wave_lds(ringCap) : hex_wave_lds(ringCap);
+        const size_t lds = std::max(fused ? fused_lds(kind, ringCap) : (size_t)kMlpRows * ringCap * per, 4 * wave);
         switch (nq) {   // the full searches use 4 waves: nq 4 and 8 (learned_deferred_ok)
         case 4: fused ? learned_def_nq<4, true>(kind, a, la, ringCap, nbList, nb, lds, s)
                       : learned_def_nq<4, false>(kind, a, la, ringCap, nbList, nb, lds, s); break;
@@ -1772,49 +1888,18 @@ void launch_search_learned(int kind, int nq, const SearchArgs& a, const LearnNet
     default: break;
     }
 #undef VSDMO_LEARN_CASE
-    // second launch: the plain search of the fallbacks, W waves per vertex,
-    // a quarter of the class's blocks (blocks loop when more fall back)
+    // second launch: the plain search of the fallbacks, a wave per vertex, a
+    // quarter of the class's vertices at a time (blocks loop when more fall back)
     const int g1 = std::max(1, std::min(nc, std::max(256, nc / 4)));
     switch (nq) {
-    case 2: list_nqw<2, 2>(kind, a, list, cnt, fallbacks, g1, ringCap, s); break;
-    case 4: list_nqw<4, 4>(kind, a, list, cnt, fallbacks, g1, ringCap, s); break;
-    case 6: list_nqw<6, 2>(kind, a, list, cnt, fallbacks, g1, ringCap, s); break;
-    case 8:
-        // the fallback lists are short (a few per cent of the class): latency
-        // bound, 4 waves per vertex (1, 2, 4 and 8 measured on the 40^3 tet
-        // and 48^3 hex cubes)
-        list_nqw<8, 4>(kind, a, list, cnt, fallbacks, g1, ringCap, s);
-        break;
+    case 2: list_nq<2>(kind, a, list, cnt, fallbacks, g1, ringCap, s); break;
+    case 4: list_nq<4>(kind, a, list, cnt, fallbacks, g1, ringCap, s); break;
+    case 6: list_nq<6>(kind, a, list, cnt, fallbacks, g1, ringCap, s); break;
+    case 8: list_nq<8>(kind, a, list, cnt, fallbacks, g1, ringCap, s); break;
     default: break;
     }
 }
 
-// ------------------------------------------------------- split launches
-// One colour class in one launch of 256-thread blocks: the first nHead
-// vertices one per wave (the W = 1 body, its ring staged in the wave's own
-// quarter of the LDS), the remaining ones one per block with 4 (or 2) waves
-// per vertex.  The end of a launch, where few waves are left on the GPU,
-// then drains in finer grains.  Every body gives the same result, so the
-// split changes no bits.  All 4 waves of a block pass the same barriers: a
-// head wave without a vertex passes the single barrier of a W = 1 search.
-template <int NQ, int WT>
-__global__ __launch_bounds__(256, 5) void k_search_tet_split(SearchArgs a, int nHead, int ringCap)
-{
-    extern __shared__ TetC s_tcs[];
-    __shared__ RedLds<1> rd1;
-    __shared__ RedLds<WT> rdt;
-    const bool emin = a.extentMin != 0;
-    const int headBlocks = (nHead + 3) >> 2;
-    if ((int)blockIdx.x < headBlocks) {
-        const int w = threadIdx.x >> 6;
-        const int i = 4 * (int)blockIdx.x + w;
-        if (i < nHead) tet_vertex<NQ, 1>(a, a.cStart + i, emin, s_tcs + (size_t)w * ringCap, rd1);
-        else __syncthreads();   // the one barrier of a W = 1 search
-    } else {
-        static_assert(WT == 4, "the tail blocks use all 4 waves");
-        tet_vertex<NQ, WT>(a, a.cStart + nHead + ((int)blockIdx.x - headBlocks), emin, s_tcs, rdt);
-    }
-}
 // ------------------------------------------------------- batched sweep
 // Persistent kernel of one colour round of a batch of meshes: blocks take
 // work items from a queue (one atomic counter per round) until it is empty.
@@ -1826,43 +1911,38 @@ __global__ __launch_bounds__(256, 5) void k_search_tet_split(SearchArgs a, int n
 // round's counter (their cost varies with the ring); items [mid, hi) are flat
 // triangle searches, ~100x cheaper and uniform, statically strided over the
 // blocks so that they cost no atomics.
-template <int NQ, int W>
+template <int NQ>
 __device__ __forceinline__ void batch_item(const SearchArgs& a, const int* rowHex, const int* valHex, int code,
-                                           int hexCap, float4* s_dyn, RedLds<W>& rd)
+                                           int tetCap, int hexCap, unsigned char* lds)
 {
-    const int vid = code & 0x3fffffff, type = (code >> 30) & 3;
-    if (type == 0) tet_vertex<NQ, W>(a, vid, false, reinterpret_cast<TetC*>(s_dyn), rd);
+    const int vid = uniform(code & 0x3fffffff), type = uniform((code >> 30) & 3);
+    if (type == 0) tet_vertex<NQ>(a, vid, false, lds, tetCap);
     else if (type == 1) {
         SearchArgs ah = a;
         ah.ringRow = rowHex;
         ah.ringVal = valHex;
-        // one wave; the others of the block wait at the round's next barrier
-        if (threadIdx.x < 64)
-            hex_vertex<NQ>(ah, uniform(vid), true, reinterpret_cast<HexLds*>(s_dyn),
-                           hex_act(reinterpret_cast<unsigned char*>(s_dyn), hexCap));
+        hex_vertex<NQ>(ah, vid, true, reinterpret_cast<HexLds*>(lds), hex_act(lds, hexCap));
     }
-    else flat_vertex<NQ, W>(a, vid, reinterpret_cast<TriC*>(s_dyn), rd);
+    else flat_vertex<NQ>(a, vid, reinterpret_cast<TriC*>(lds));
 }
 
-template <int NQ, int W>
-__global__ __launch_bounds__(64 * W) void k_batch_round(SearchArgs a, const int* __restrict__ rowHex,
-                                                       const int* __restrict__ valHex, const int* __restrict__ items,
-                                                       int lo, int mid, int hi, int* __restrict__ ctr, int hexCap)
+template <int NQ>
+__global__ __launch_bounds__(64) void k_batch_round(SearchArgs a, const int* __restrict__ rowHex,
+                                                   const int* __restrict__ valHex, const int* __restrict__ items,
+                                                   int lo, int mid, int hi, int* __restrict__ ctr, int tetCap, int hexCap)
 {
-    extern __shared__ float4 s_dyn[];
-    __shared__ RedLds<W> rd;
-    __shared__ int s_item;
+    extern __shared__ __align__(16) unsigned char s_dyn[];
     for (;;) {
-        __syncthreads();   // previous item's LDS reads are done
-        if (threadIdx.x == 0) s_item = atomicAdd(ctr, 1);
-        __syncthreads();
-        const int it = lo + s_item;
+        int at = 0;
+        if (threadIdx.x == 0) at = atomicAdd(ctr, 1);
+        const int it = lo + uniform(at);
         if (it >= mid) break;
-        batch_item<NQ, W>(a, rowHex, valHex, items[it], hexCap, s_dyn, rd);
+        batch_item<NQ>(a, rowHex, valHex, items[it], tetCap, hexCap, s_dyn);
+        wave_lds_fence();   // the next item restages the LDS
     }
     for (int it = mid + (int)blockIdx.x; it < hi; it += (int)gridDim.x) {
-        __syncthreads();
-        batch_item<NQ, W>(a, rowHex, valHex, items[it], hexCap, s_dyn, rd);
+        batch_item<NQ>(a, rowHex, valHex, items[it], tetCap, hexCap, s_dyn);
+        wave_lds_fence();
     }
 }
 
@@ -2093,103 +2173,55 @@ __global__ void k_histogram(const float* __restrict__ q, int n, int ncols, int* 
 }
 
 // ------------------------------------------------------------- launchers
-template <int NQ, int W>
-static void launch_nqw(int kind, const SearchArgs& a, int nBlocks, size_t lds, hipStream_t s)
-{
-    if (kind == VSDMO_TET) launch_kernel(k_search_tet<NQ, W>, nBlocks, 64 * W, lds, s, a);
-    else if (kind == VSDMO_HEX) launch_kernel(k_search_hex<NQ>, nBlocks, 64, lds, s, a, (int)(lds / kHexLdsPer));
-    else launch_kernel(k_search_flat<NQ, W>, nBlocks, 64 * W, lds, s, a);
-}
 template <int NQ>
-static void launch_nq(int kind, int w, const SearchArgs& a, int nBlocks, size_t lds, hipStream_t s)
+static void launch_nq(int kind, const SearchArgs& a, int nBlocks, int ringCap, hipStream_t s)
 {
-    if (w == 2 && NQ % 2 == 0) launch_nqw<NQ, (NQ % 2 == 0 ? 2 : 1)>(kind, a, nBlocks, lds, s);
-    else if (w == 4 && NQ % 4 == 0) launch_nqw<NQ, (NQ % 4 == 0 ? 4 : 1)>(kind, a, nBlocks, lds, s);
-    else launch_nqw<NQ, 1>(kind, a, nBlocks, lds, s);
+    const size_t lds = search_lds_bytes(kind, ringCap);
+    if (kind == VSDMO_TET) launch_kernel(k_search_tet<NQ>, nBlocks, 64, lds, s, a, ringCap);
+    else if (kind == VSDMO_HEX) launch_kernel(k_search_hex<NQ>, nBlocks, 64, lds, s, a, ringCap);
+    else launch_kernel(k_search_flat<NQ>, nBlocks, 64, lds, s, a);
 }
 // Non-persistent variant of a round: one block per item, scheduled by the
 // hardware dispatcher (no queue, no atomics), one launch per element type
 // (0 tet, 1 hex, 2 flat tri) with the search body of that type alone, so
 // that each keeps the registers and LDS of its own body.  The tet body asks
 // for the plain tet search's occupancy (VSDMO_TET_MIN_WAVES waves per SIMD).
-template <int NQ, int W, int TYPE>
-__global__ __launch_bounds__(64 * W, TYPE == 0 ? VSDMO_TET_MIN_WAVES : 1) void k_batch_typed(SearchArgs a,
-                                                                                        const int* __restrict__ rowHex,
-                                                       const int* __restrict__ valHex, const int* __restrict__ items,
-                                                       int lo, int hexCap)
+template <int NQ, int TYPE>
+__global__ __launch_bounds__(64, TYPE == 0 ? VSDMO_TET_MIN_WAVES : TYPE == 1 ? VSDMO_HEX_MIN_WAVES : 1)
+void k_batch_typed(SearchArgs a, const int* __restrict__ rowHex, const int* __restrict__ valHex,
+                   const int* __restrict__ items, int lo, int ringCap)
 {
-    extern __shared__ float4 s_dyn[];
-    __shared__ RedLds<W> rd;
+    extern __shared__ __align__(16) unsigned char s_typ[];
     const int vid = items[lo + blockIdx.x] & 0x3fffffff;
     if constexpr (TYPE == 0) {
-        tet_vertex<NQ, W>(a, vid, false, reinterpret_cast<TetC*>(s_dyn), rd);
+        tet_vertex<NQ>(a, vid, false, s_typ, ringCap);
     } else if constexpr (TYPE == 1) {
         SearchArgs ah = a;
         ah.ringRow = rowHex;
         ah.ringVal = valHex;
-        hex_vertex<NQ>(ah, vid, true, reinterpret_cast<HexLds*>(s_dyn),
-                       hex_act(reinterpret_cast<unsigned char*>(s_dyn), hexCap));
+        hex_vertex<NQ>(ah, vid, true, reinterpret_cast<HexLds*>(s_typ), hex_act(s_typ, ringCap));
     } else {
-        flat_vertex<NQ, W>(a, vid, reinterpret_cast<TriC*>(s_dyn), rd);
+        flat_vertex<NQ>(a, vid, reinterpret_cast<TriC*>(s_typ));
     }
 }
 
-template <int NQ, int W>
-static void batch_typed_nqw(const SearchArgs& a, const int* rowHex, const int* valHex, const int* items, int lo, int hi,
-                            int type, size_t lds, hipStream_t s)
+template <int NQ>
+static void batch_typed_nq(const SearchArgs& a, const int* rowHex, const int* valHex, const int* items, int lo, int hi,
+                           int type, int ringCap, hipStream_t s)
 {
     const unsigned n = (unsigned)(hi - lo);
-    if (type == 0) k_batch_typed<NQ, W, 0><<<n, 64 * W, lds, s>>>(a, rowHex, valHex, items, lo, 0);
-    else if (type == 1) k_batch_typed<NQ, 1, 1><<<n, 64, lds, s>>>(a, rowHex, valHex, items, lo, (int)(lds / kHexLdsPer));
-    else k_batch_typed<NQ, W, 2><<<n, 64 * W, lds, s>>>(a, rowHex, valHex, items, lo, 0);
-}
-template <int NQ>
-static void batch_typed_nq(int w, const SearchArgs& a, const int* rowHex, const int* valHex, const int* items, int lo,
-                           int hi, int type, size_t lds, hipStream_t s)
-{
-    if (w == 2 && NQ % 2 == 0) batch_typed_nqw<NQ, (NQ % 2 == 0 ? 2 : 1)>(a, rowHex, valHex, items, lo, hi, type, lds, s);
-    else if (w == 4 && NQ % 4 == 0)
-        batch_typed_nqw<NQ, (NQ % 4 == 0 ? 4 : 1)>(a, rowHex, valHex, items, lo, hi, type, lds, s);
-    else batch_typed_nqw<NQ, 1>(a, rowHex, valHex, items, lo, hi, type, lds, s);
+    const size_t lds = search_lds_bytes(type == 0 ? VSDMO_TET : type == 1 ? VSDMO_HEX : VSDMO_TRI, ringCap);
+    if (type == 0) k_batch_typed<NQ, 0><<<n, 64, lds, s>>>(a, rowHex, valHex, items, lo, ringCap);
+    else if (type == 1) k_batch_typed<NQ, 1><<<n, 64, lds, s>>>(a, rowHex, valHex, items, lo, ringCap);
+    else k_batch_typed<NQ, 2><<<n, 64, lds, s>>>(a, rowHex, valHex, items, lo, ringCap);
 }
 
-struct BatchLaunch {
-    SearchArgs a;
-    const int* rowHex;
-    const int* valHex;
-    const int* items;
-    int lo, mid, hi;
-    int* ctr;
-    int grid;
-    size_t lds;
-    hipStream_t s;
-    int hexCap;
-};
-template <int NQ, int W>
-static void batch_nqw(const BatchLaunch& L)
-{
-    k_batch_round<NQ, W><<<L.grid, 64 * W, L.lds, L.s>>>(L.a, L.rowHex, L.valHex, L.items, L.lo, L.mid, L.hi, L.ctr, L.hexCap);
-}
-template <int NQ, int W>
-static int batch_occ(size_t lds)
+template <int NQ>
+static int batch_occ_nq(size_t lds)
 {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_batch_round<NQ, W>, 64 * W, lds) != hipSuccess) nb = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_batch_round<NQ>, 64, lds) != hipSuccess) nb = 1;
     return nb;
-}
-template <int NQ>
-static void batch_nq(int w, const BatchLaunch& L)
-{
-    if (w == 2 && NQ % 2 == 0) batch_nqw<NQ, (NQ % 2 == 0 ? 2 : 1)>(L);
-    else if (w == 4 && NQ % 4 == 0) batch_nqw<NQ, (NQ % 4 == 0 ? 4 : 1)>(L);
-    else batch_nqw<NQ, 1>(L);
-}
-template <int NQ>
-static int batch_occ_nq(int w, size_t lds)
-{
-    if (w == 2 && NQ % 2 == 0) return batch_occ<NQ, (NQ % 2 == 0 ? 2 : 1)>(lds);
-    if (w == 4 && NQ % 4 == 0) return batch_occ<NQ, (NQ % 4 == 0 ? 4 : 1)>(lds);
-    return batch_occ<NQ, 1>(lds);
 }
 
 bool waves_supported(int nq, int w)
@@ -2197,69 +2229,47 @@ bool waves_supported(int nq, int w)
     return w == 0 || w == 1 || (w == 2 && nq % 2 == 0) || (w == 4 && nq % 4 == 0);
 }
 
-template <int NQ, int WT>
-static void split_nq(const SearchArgs& a, int nHead, int nTail, int ringCap, hipStream_t s)
-{
-    const int grid = (nHead + 3) / 4 + nTail;
-    if (grid <= 0) return;
-    launch_kernel(k_search_tet_split<NQ, WT>, grid, 256, sizeof(TetC) * 4 * (size_t)ringCap, s, a, nHead, ringCap);
-}
-
-bool split_supported(int kind, int nq, int ringCap)
-{
-    if (kind != VSDMO_TET) return false;   // hex searches run one wave per vertex
-    if (nq != 4 && nq != 8) return false;   // the tail needs 4 waves per vertex (nq / 4 candidates per lane)
-    return sizeof(TetC) * 4 * (size_t)std::max(ringCap, 1) <= 65536;
-}
-
-void launch_search_split(int kind, int nq, const SearchArgs& a, int tail, int ringCap, hipStream_t s)
-{
-    const int n = a.cEnd - a.cStart;
-    if (n <= 0) return;
-    const int nTail = std::min(n, std::max(tail, 0));
-    const int nHead = n - nTail;
-    if (nq == 4) split_nq<4, 4>(a, nHead, nTail, ringCap, s);
-    else if (nq == 8) split_nq<8, 4>(a, nHead, nTail, ringCap, s);
-}
-
-int batch_round_blocks_per_cu(int nq, int w, size_t lds)
+int batch_round_blocks_per_cu(int nq, size_t lds)
 {
     switch (nq) {
-    case 2: return batch_occ_nq<2>(w, lds);
-    case 4: return batch_occ_nq<4>(w, lds);
-    case 6: return batch_occ_nq<6>(w, lds);
-    default: return batch_occ_nq<8>(w, lds);
+    case 2: return batch_occ_nq<2>(lds);
+    case 4: return batch_occ_nq<4>(lds);
+    case 6: return batch_occ_nq<6>(lds);
+    default: return batch_occ_nq<8>(lds);
     }
 }
 
-void launch_batch_round(int nq, int w, const SearchArgs& a, const int* rowHex, const int* valHex, const int* items,
-                        int lo, int mid, int hi, int* ctr, int grid, size_t lds, int hexCap, hipStream_t s)
+void launch_batch_round(int nq, const SearchArgs& a, const int* rowHex, const int* valHex, const int* items, int lo,
+                        int mid, int hi, int* ctr, int grid, size_t lds, int tetCap, int hexCap, hipStream_t s)
 {
     if (hi <= lo || grid <= 0) return;
-    BatchLaunch L{ a, rowHex, valHex, items, lo, mid, hi, ctr, grid, lds, s, hexCap };
+#define VSDMO_ROUND_CASE(Q)                                                                                        \
+    case Q: k_batch_round<Q><<<grid, 64, lds, s>>>(a, rowHex, valHex, items, lo, mid, hi, ctr, tetCap, hexCap); break;
     switch (nq) {
-    case 2: batch_nq<2>(w, L); break;
-    case 4: batch_nq<4>(w, L); break;
-    case 6: batch_nq<6>(w, L); break;
-    case 8: batch_nq<8>(w, L); break;
+        VSDMO_ROUND_CASE(2)
+        VSDMO_ROUND_CASE(4)
+        VSDMO_ROUND_CASE(6)
+        VSDMO_ROUND_CASE(8)
     default: break;
     }
+#undef VSDMO_ROUND_CASE
 }
 
-void launch_batch_typed(int nq, int w, const SearchArgs& a, const int* rowHex, const int* valHex, const int* items,
-                        int lo, int hi, int type, size_t lds, hipStream_t s)
+void launch_batch_typed(int nq, const SearchArgs& a, const int* rowHex, const int* valHex, const int* items, int lo,
+                        int hi, int type, int ringCap, hipStream_t s)
 {
     if (hi <= lo) return;
-    if (type == 2 && w == 1 && flat8x4_ok(nq, lds, hi - lo)) {
+    ringCap = std::max(ringCap, 1);
+    if (type == 2 && flat8x4_ok(nq, ringCap, hi - lo)) {
         const int groups = (hi - lo + kFlatGroups - 1) / kFlatGroups;
-        k_batch_flat8x4<<<groups, 256, kFlatGroups * lds, s>>>(a, items, lo, hi, (int)(lds / sizeof(TriC)));
+        k_batch_flat8x4<<<groups, 256, kFlatGroups * sizeof(TriC) * (size_t)ringCap, s>>>(a, items, lo, hi, ringCap);
         return;
     }
     switch (nq) {
-    case 2: batch_typed_nq<2>(w, a, rowHex, valHex, items, lo, hi, type, lds, s); break;
-    case 4: batch_typed_nq<4>(w, a, rowHex, valHex, items, lo, hi, type, lds, s); break;
-    case 6: batch_typed_nq<6>(w, a, rowHex, valHex, items, lo, hi, type, lds, s); break;
-    case 8: batch_typed_nq<8>(w, a, rowHex, valHex, items, lo, hi, type, lds, s); break;
+    case 2: batch_typed_nq<2>(a, rowHex, valHex, items, lo, hi, type, ringCap, s); break;
+    case 4: batch_typed_nq<4>(a, rowHex, valHex, items, lo, hi, type, ringCap, s); break;
+    case 6: batch_typed_nq<6>(a, rowHex, valHex, items, lo, hi, type, ringCap, s); break;
+    case 8: batch_typed_nq<8>(a, rowHex, valHex, items, lo, hi, type, ringCap, s); break;
     default: break;
     }
 }
@@ -2295,33 +2305,34 @@ void launch_batch_quality(const BatchQArgs& a, hipStream_t s)
     k_batch_history_next<<<1, 64, 0, s>>>(a.hctr);
 }
 
+size_t search_lds_bytes(int kind, int ringCap)
+{
+    ringCap = std::max(ringCap, 1);
+    if (kind == VSDMO_TET) return tet_wave_lds(ringCap);
+    return (kind == VSDMO_HEX ? kHexLdsPer : sizeof(TriC)) * (size_t)ringCap;
+}
+
 size_t batch_lds_bytes(int maxRingTet, int maxRingHex, int maxHETri)
 {
-    size_t b = std::max(sizeof(TetC) * (size_t)maxRingTet, kHexLdsPer * (size_t)maxRingHex);
-    b = std::max(b, sizeof(TriC) * (size_t)maxHETri);
-    return std::max(b, (size_t)16);
+    return std::max(search_lds_bytes(VSDMO_TET, maxRingTet),
+                    std::max(search_lds_bytes(VSDMO_HEX, maxRingHex), search_lds_bytes(VSDMO_TRI, maxHETri)));
 }
 
-size_t search_lds_bytes(int kind, int maxRing)
-{
-    size_t per = (kind == VSDMO_TET) ? sizeof(TetC) : (kind == VSDMO_HEX) ? kHexLdsPer : sizeof(TriC);
-    return per * (size_t)std::max(maxRing, 1);
-}
-
-void launch_search(int kind, int nq, int w, const SearchArgs& a, size_t lds, hipStream_t s)
+void launch_search(int kind, int nq, const SearchArgs& a, int ringCap, hipStream_t s)
 {
     int nBlocks = a.cEnd - a.cStart;
     if (nBlocks <= 0) return;
-    if (kind == VSDMO_TRI && w == 1 && flat8x4_ok(nq, lds, nBlocks)) {
+    ringCap = std::max(ringCap, 1);
+    if (kind == VSDMO_TRI && flat8x4_ok(nq, ringCap, nBlocks)) {
         const int groups = (nBlocks + kFlatGroups - 1) / kFlatGroups;
-        launch_kernel(k_search_flat8x4, groups, 256, kFlatGroups * lds, s, a, (int)(lds / sizeof(TriC)));
+        launch_kernel(k_search_flat8x4, groups, 256, kFlatGroups * sizeof(TriC) * (size_t)ringCap, s, a, ringCap);
         return;
     }
     switch (nq) {
-    case 2: launch_nq<2>(kind, w, a, nBlocks, lds, s); break;
-    case 4: launch_nq<4>(kind, w, a, nBlocks, lds, s); break;
-    case 6: launch_nq<6>(kind, w, a, nBlocks, lds, s); break;
-    case 8: launch_nq<8>(kind, w, a, nBlocks, lds, s); break;
+    case 2: launch_nq<2>(kind, a, nBlocks, ringCap, s); break;
+    case 4: launch_nq<4>(kind, a, nBlocks, ringCap, s); break;
+    case 6: launch_nq<6>(kind, a, nBlocks, ringCap, s); break;
+    case 8: launch_nq<8>(kind, a, nBlocks, ringCap, s); break;
     default: break;
     }
 }
