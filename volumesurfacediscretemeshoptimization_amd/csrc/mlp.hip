@@ -1,17 +1,19 @@
-// mlp.hip -- the learned vertex proposal: BF16 MFMA GEMMs with fused
-// epilogues, the 96-128-128-3 GELU MLP (forward, backward, Adam), its
-// training set and the one-ring feature encoding.
+// mlp.hip -- the learned vertex proposal: the 96-128-128-3 GELU MLP (forward,
+// backward, Adam) on BF16 MFMA tiles, its training set and the one-ring
+// feature encoding.
 //
 // There is no learned component in the reference.  The network predicts the
 // displacement DMO gives a vertex (dmo/DMOTetImplCub.h:20-137,
 // DMOHexImplCub.h:20-137) from its one-ring; the optimiser then searches a
 // small window around the prediction and falls back to the full search.
 //
-// GEMMs: one wave per 16x16 output tile, __builtin_amdgcn_mfma_f32_16x16x32_bf16
-// over K in chunks of 32 (lane l: A row l%16 and B column l%16, k = 8*(l/16)
-// + 0..7; D column l%16, rows 4*(l/16) + 0..3), operands read through
-// arbitrary (row, column) strides so that the transposed products of the
-// backward pass need no copies.
+// A training step is two launches: k_mlp_rows takes 16 rows per block through
+// the forward and the backward pass in LDS and leaves the activations and
+// their gradients feature-major, and k_mlp_grads forms the weight gradients
+// (one wave per 16x16 tile, its chain over the rows in order), the bias
+// gradients and the Adam update from them.  Tiles are
+// __builtin_amdgcn_mfma_f32_16x16x32_bf16 (lane l: A row l%16 and B column
+// l%16, k = 8*(l/16) + 0..7; D column l%16, rows 4*(l/16) + 0..3).
 #include <float.h>
 #include <math.h>
 
@@ -30,148 +32,380 @@ __device__ __forceinline__ float gelu_d(float z)
     return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
 }
 
-enum { EPI_F32 = 0, EPI_GELU = 1, EPI_DGELU = 2 };
-
-struct GemmArgs {
-    int M, N, K;
-    const uint16_t* A;
-    long long sam, sak;      // A[m][k] = A[m*sam + k*sak]
-    const uint16_t* B;
-    long long sbk, sbn;      // B[k][n] = B[k*sbk + n*sbn]
-    const float* bias;       // [N] or null
-    int mode;
-    float* Cf;               // EPI_F32: acc (+bias); EPI_GELU: Z = acc + bias
-    long long ldcf;
-    uint16_t* Cb;            // EPI_GELU: bf16(gelu(Z)); EPI_DGELU: bf16(acc * gelu'(Zin))
-    long long ldcb;
-    const float* Zin;
-    long long ldz;
+// Forward and backward of 16 rows per block of 4 waves.  Wave w owns the
+// columns [32w, 32w + 32) of every 128-wide layer, forward and backward, so the
+// pre-activations it needs for gelu' stay in its registers; A operands come
+// from LDS, weight operands as 16-byte rows from global memory (W2 of the
+// backward product from its transposed copy).  Outputs are feature-major
+// ([feature][ld], ld = rows padded to 32): a lane's 4 rows of a column are 8
+// contiguous bytes, and the weight-gradient tiles read 16 bytes along the rows.
+// Rows past n are zero in X and dY.  Bound by the latency of its five layers'
+// chain; 13.3 us at 4,096 rows (256 blocks, one per CU).
+struct RowsArgs {
+    const float* Xf;         // n x 96 rows, rounded to BF16 here, or
+    const uint16_t* Xb;      // BF16 rows and targets perm[0..n) of a dataset
+    const float* T;
+    const int* perm;
+    int n, ld;
+    const uint16_t* wb;
+    const uint16_t* w2t;     // W2 transposed
+    const float* w;
+    uint16_t *XT, *H1T, *H2T, *dZ1T, *dZ2T, *dYT;
+    float* dYf;              // 3 x ld
+    double* rowLoss;         // squared error of each row
 };
 
-__global__ __launch_bounds__(256) void k_gemm(GemmArgs g)
+struct RowsLds {
+    MlpLds f;
+    __align__(16) uint16_t dZ2[kMlpRows * kLdh];
+    uint16_t dY[kMlpRows][4];
+};
+
+// 4 BF16 values of consecutive rows
+__device__ __forceinline__ void store4(uint16_t* p, const uint16_t (&v)[4])
 {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int tilesN = (g.N + 15) >> 4, tilesM = (g.M + 15) >> 4;
-    const int tile = blockIdx.x * 4 + wave;
-    if (tile >= tilesM * tilesN) return;   // whole wave; the kernel has no block barrier
-    const int mt = tile / tilesN, nt = tile - mt * tilesN;
-    const int row = mt * 16 + (lane & 15);
-    const int col = nt * 16 + (lane & 15);
-    const int kq = (lane >> 4) * 8;
-    f32x4 acc = { 0.0f, 0.0f, 0.0f, 0.0f };
-    for (int k0 = 0; k0 < g.K; k0 += 32) {
-        bf16x8 a, b;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int k = k0 + kq + j;
-            uint16_t av = (row < g.M && k < g.K) ? g.A[(long long)row * g.sam + (long long)k * g.sak] : (uint16_t)0;
-            uint16_t bv = (col < g.N && k < g.K) ? g.B[(long long)k * g.sbk + (long long)col * g.sbn] : (uint16_t)0;
-            a[j] = __builtin_bit_cast(__bf16, av);
-            b[j] = __builtin_bit_cast(__bf16, bv);
-        }
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-    }
-    const int n = nt * 16 + (lane & 15);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int m = mt * 16 + 4 * (lane >> 4) + r;
-        if (m >= g.M || n >= g.N) continue;
-        float v = acc[r];
-        if (g.mode == EPI_F32) {
-            if (g.bias) v += g.bias[n];
-            g.Cf[(long long)m * g.ldcf + n] = v;
-        } else if (g.mode == EPI_GELU) {
-            v += g.bias[n];
-            g.Cf[(long long)m * g.ldcf + n] = v;
-            g.Cb[(long long)m * g.ldcb + n] = f2bf(gelu(v));
-        } else {
-            g.Cb[(long long)m * g.ldcb + n] = f2bf(v * gelu_d(g.Zin[(long long)m * g.ldz + n]));
-        }
-    }
+    *reinterpret_cast<uint2*>(p) = make_uint2((uint32_t)v[0] | (uint32_t)v[1] << 16, (uint32_t)v[2] | (uint32_t)v[3] << 16);
 }
 
-static void gemm(const GemmArgs& g, hipStream_t s)
+__global__ __launch_bounds__(256) void k_mlp_rows(RowsArgs a)
 {
-    const int tiles = ((g.M + 15) / 16) * ((g.N + 15) / 16);
-    if (tiles <= 0 || g.K <= 0) return;
-    k_gemm<<<(tiles + 3) / 4, 256, 0, s>>>(g);
-}
-
-// mean squared error over n rows of 3: loss partial per block (FP64, fixed
-// tree), dY = 2 (Y - T) / n in FP32 and BF16
-__global__ void k_mse(const float* __restrict__ Y, const float* __restrict__ T, int n, float* __restrict__ dYf,
-                      uint16_t* __restrict__ dY16, double* __restrict__ part)
-{
-    __shared__ double s[256];
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    double l = 0.0;
-    if (i < n) {
-        for (int c = 0; c < 3; ++c) {
-            float d = Y[3 * i + c] - T[3 * i + c];
-            l += (double)d * (double)d;
-            float gy = 2.0f * d / (float)n;
-            dYf[3 * i + c] = gy;
-            dY16[3 * i + c] = f2bf(gy);
+    __shared__ RowsLds sm;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int r16 = lane & 15, kq = (lane >> 4) * 8, rq = (lane >> 4) * 4;
+    const int row0 = blockIdx.x * kMlpRows;
+    const MlpW m = mlp_load_w16(a.wb, a.w);
+    if (tid < kMlpRows * (kIn / 8)) {   // 8 features per thread
+        const int r = tid / (kIn / 8), c = (tid - r * (kIn / 8)) * 8;
+        union { uint16_t h[8]; uint4 q; } x;
+        x.q = make_uint4(0, 0, 0, 0);
+        if (row0 + r < a.n) {
+            if (a.Xb) {
+                x.q = *reinterpret_cast<const uint4*>(a.Xb + (size_t)a.perm[row0 + r] * kIn + c);
+            } else {
+                const float* src = a.Xf + (size_t)(row0 + r) * kIn + c;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) x.h[j] = f2bf(src[j]);
+            }
         }
+        *reinterpret_cast<uint4*>(sm.f.X + r * kLdx + c) = x.q;
     }
-    s[threadIdx.x] = l;
+    // layers 2 and 3 and the backward products' operands
+    bf16x8 b2[kHid / 32][2], bt[kHid / 32][2], b3[kHid / 32], b3t[2];
+    const bf16x8 zero8 = __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0));
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int col = (2 * wave + t) * 16 + r16;
+#pragma unroll
+        for (int i = 0; i < kHid / 32; ++i) {
+            b2[i][t] = *reinterpret_cast<const bf16x8*>(a.wb + kOW2 + (size_t)col * kHid + 32 * i + kq);
+            bt[i][t] = *reinterpret_cast<const bf16x8*>(a.w2t + (size_t)col * kHid + 32 * i + kq);
+        }
+        b3t[t] = zero8;   // W3[k][col], k < 3: the first 16 lanes' first three
+        if (lane < 16)
+#pragma unroll
+            for (int k = 0; k < kOut; ++k) b3t[t][k] = __builtin_bit_cast(__bf16, a.wb[kOW3 + k * kHid + col]);
+    }
+    float bias3 = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kHid / 32; ++i) b3[i] = zero8;
+    if (wave == 0 && r16 < kOut) {
+#pragma unroll
+        for (int i = 0; i < kHid / 32; ++i)
+            b3[i] = *reinterpret_cast<const bf16x8*>(a.wb + kOW3 + (size_t)r16 * kHid + 32 * i + kq);
+        bias3 = a.w[kOB3 + r16];
+    }
     __syncthreads();
-    for (int k = 128; k > 0; k >>= 1) {
-        if ((int)threadIdx.x < k) s[threadIdx.x] += s[threadIdx.x + k];
-        __syncthreads();
+    for (int q = tid; q < kIn * 4; q += 256) {
+        const int c = q >> 2, r = (q & 3) * 4;
+        const uint16_t v[4] = { sm.f.X[r * kLdx + c], sm.f.X[(r + 1) * kLdx + c], sm.f.X[(r + 2) * kLdx + c],
+                                sm.f.X[(r + 3) * kLdx + c] };
+        store4(a.XT + (size_t)c * a.ld + row0 + r, v);
     }
-    if (threadIdx.x == 0) part[blockIdx.x] = s[0];
+    float z1[2][4], z2[2][4];
+    // layer 1
+    {
+        f32x4 acc[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[t] = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+        for (int i = 0; i < kIn / 32; ++i) {
+            const bf16x8 av = *reinterpret_cast<const bf16x8*>(sm.f.X + r16 * kLdx + 32 * i + kq);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, m.b1[i][t], acc[t], 0, 0, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int col = (2 * wave + t) * 16 + r16;
+            uint16_t h[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                z1[t][r] = acc[t][r] + m.bias1[t];
+                h[r] = f2bf(gelu(z1[t][r]));
+                sm.f.H1[(rq + r) * kLdh + col] = h[r];
+            }
+            store4(a.H1T + (size_t)col * a.ld + row0 + rq, h);
+        }
+    }
+    __syncthreads();
+    // layer 2
+    {
+        f32x4 acc[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[t] = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+        for (int i = 0; i < kHid / 32; ++i) {
+            const bf16x8 av = *reinterpret_cast<const bf16x8*>(sm.f.H1 + r16 * kLdh + 32 * i + kq);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, b2[i][t], acc[t], 0, 0, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int col = (2 * wave + t) * 16 + r16;
+            uint16_t h[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                z2[t][r] = acc[t][r] + m.bias2[t];
+                h[r] = f2bf(gelu(z2[t][r]));
+                sm.f.H2[(rq + r) * kLdh + col] = h[r];
+            }
+            store4(a.H2T + (size_t)col * a.ld + row0 + rq, h);
+        }
+    }
+    __syncthreads();
+    // layer 3, the squared error and its gradient dY = 2 (Y - T) / n
+    if (wave == 0) {
+        f32x4 acc = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+        for (int i = 0; i < kHid / 32; ++i) {
+            const bf16x8 av = *reinterpret_cast<const bf16x8*>(sm.f.H2 + r16 * kLdh + 32 * i + kq);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, b3[i], acc, 0, 0, 0);
+        }
+        if (r16 < kOut) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sm.f.Y[rq + r][r16] = acc[r] + bias3;
+        }
+    }
+    __syncthreads();
+    if (tid < kMlpRows) {
+        const int row = row0 + tid;
+        const bool live = row < a.n;
+        const size_t src = live ? (size_t)(a.Xb ? a.perm[row] : row) : 0;
+        double l = 0.0;
+#pragma unroll
+        for (int c = 0; c < kOut; ++c) {
+            float gy = 0.0f;
+            if (live) {
+                const float d = sm.f.Y[tid][c] - a.T[3 * src + c];
+                l += (double)d * (double)d;
+                gy = 2.0f * d / (float)a.n;
+            }
+            a.dYf[(size_t)c * a.ld + row] = gy;
+            const uint16_t h = f2bf(gy);
+            a.dYT[(size_t)c * a.ld + row] = h;
+            sm.dY[tid][c] = h;
+        }
+        a.rowLoss[row] = l;
+    }
+    __syncthreads();
+    // dZ2 = (dY W3) gelu'(Z2)
+    {
+        bf16x8 av = zero8;
+        if (lane < 16)
+#pragma unroll
+            for (int k = 0; k < kOut; ++k) av[k] = __builtin_bit_cast(__bf16, sm.dY[r16][k]);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int col = (2 * wave + t) * 16 + r16;
+            const f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, b3t[t], f32x4{ 0.0f, 0.0f, 0.0f, 0.0f }, 0, 0, 0);
+            uint16_t h[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                h[r] = f2bf(acc[r] * gelu_d(z2[t][r]));
+                sm.dZ2[(rq + r) * kLdh + col] = h[r];
+            }
+            store4(a.dZ2T + (size_t)col * a.ld + row0 + rq, h);
+        }
+    }
+    __syncthreads();
+    // dZ1 = (dZ2 W2) gelu'(Z1)
+    {
+        f32x4 acc[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[t] = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+        for (int i = 0; i < kHid / 32; ++i) {
+            const bf16x8 av = *reinterpret_cast<const bf16x8*>(sm.dZ2 + r16 * kLdh + 32 * i + kq);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bt[i][t], acc[t], 0, 0, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int col = (2 * wave + t) * 16 + r16;
+            uint16_t h[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) h[r] = f2bf(acc[t][r] * gelu_d(z1[t][r]));
+            store4(a.dZ1T + (size_t)col * a.ld + row0 + rq, h);
+        }
+    }
 }
 
-// loss = sum(part) / n, added to *acc (one thread, fixed order)
-__global__ void k_loss_final(const double* __restrict__ part, int nb, int n, double* __restrict__ acc)
+struct GradsArgs {
+    const uint16_t *XT, *H1T, *H2T, *dZ1T, *dZ2T, *dYT;
+    const float* dYf;
+    const double* rowLoss;
+    int n, ld;
+    double* part;            // squared error of every 256 rows
+    float* g;                // packed gradients, or (null) the Adam update of
+    float *w, *m1, *m2;
+    uint16_t *wb, *w2t;
+    float lr, c1, c2;
+};
+
+// the gradient gi of parameter i: stored, or Adam (beta 0.9 / 0.999, eps 1e-8)
+__device__ __forceinline__ void take_grad(const GradsArgs& a, int i, float gi)
+{
+    if (a.g) { a.g[i] = gi; return; }
+    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+    float m = b1 * a.m1[i] + (1.0f - b1) * gi;
+    float v = b2 * a.m2[i] + (1.0f - b2) * gi * gi;
+    a.m1[i] = m;
+    a.m2[i] = v;
+    float mh = m / a.c1, vh = v / a.c2;
+    float wi = a.w[i] - a.lr * mh / (sqrtf(vh) + eps);
+    a.w[i] = wi;
+    const uint16_t h = f2bf(wi);
+    a.wb[i] = h;
+    if (i >= kOW2 && i < kOB2) a.w2t[((i - kOW2) & (kHid - 1)) * kHid + ((i - kOW2) >> 7)] = h;
+}
+
+// the weight-gradient tiles of dW2, dW1 and dW3
+constexpr int kTiles2 = (kHid / 16) * (kHid / 16), kTiles1 = (kHid / 16) * (kIn / 16), kTiles3 = kHid / 16;
+constexpr int kTiles = kTiles2 + kTiles1 + kTiles3, kCols = 2 * kHid + kOut;
+
+// dW = dZ^T H and the bias gradients of one step, one wave per block: the
+// first kTiles blocks one 16x16 tile each, accumulated over the rows in order
+// (32 per MFMA, the next kAhead x 32 rows' operands in flight; the same sums as
+// a product per layer), the next kCols blocks a column sum each (256 strided
+// FP64 sums, then a fixed tree), the others the squared error of 256 rows each.
+// Bound by the loads' latency: 12.7 us at 4,096 rows (8, 12, 16 and 24 steps in
+// flight measure the same; the column sums with 2-byte loads 23 us).  The two
+// launches replace 16 per step (a product per layer and direction with strided
+// 2-byte operand loads), 370 us at 4,096 rows.
+__global__ __launch_bounds__(64) void k_mlp_grads(GradsArgs a)
+{
+    const int lane = threadIdx.x;
+    int b = blockIdx.x;
+    if (b < kTiles) {
+        const int r16 = lane & 15, kq = (lane >> 4) * 8;
+        const uint16_t *A, *B;
+        int off, ldg, mt, nt, rows = kHid;
+        if (b < kTiles2) {
+            A = a.dZ2T; B = a.H1T; off = kOW2; ldg = kHid;
+            mt = b / (kHid / 16); nt = b % (kHid / 16);
+        } else if (b < kTiles2 + kTiles1) {
+            b -= kTiles2;
+            A = a.dZ1T; B = a.XT; off = kOW1; ldg = kIn;
+            mt = b / (kIn / 16); nt = b % (kIn / 16);
+        } else {
+            A = a.dYT; B = a.H2T; off = kOW3; ldg = kHid; rows = kOut;
+            mt = 0; nt = b - kTiles2 - kTiles1;
+        }
+        const bool has = mt * 16 + r16 < rows;
+        const uint16_t* pa = A + (size_t)(has ? mt * 16 + r16 : 0) * a.ld + kq;
+        const uint16_t* pb = B + (size_t)(nt * 16 + r16) * a.ld + kq;
+        f32x4 acc = { 0.0f, 0.0f, 0.0f, 0.0f };
+        constexpr int kAhead = 8;
+        const int steps = a.ld / 32;
+        const bf16x8 zero8 = __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0));
+        bf16x8 va[2][kAhead], vb[2][kAhead];
+        auto load = [&](int s0, bf16x8 (&x)[kAhead], bf16x8 (&y)[kAhead]) {
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const int s = s0 + u < steps ? s0 + u : steps - 1;
+                x[u] = *reinterpret_cast<const bf16x8*>(pa + 32 * s);
+                y[u] = *reinterpret_cast<const bf16x8*>(pb + 32 * s);
+            }
+        };
+        auto mul = [&](int s0, const bf16x8 (&x)[kAhead], const bf16x8 (&y)[kAhead]) {
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u)
+                if (s0 + u < steps) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(has ? x[u] : zero8, y[u], acc, 0, 0, 0);
+        };
+        load(0, va[0], vb[0]);
+        for (int s = 0; s < steps; s += 2 * kAhead) {
+            load(s + kAhead, va[1], vb[1]);
+            mul(s, va[0], vb[0]);
+            load(s + 2 * kAhead, va[0], vb[0]);
+            mul(s + kAhead, va[1], vb[1]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int mrow = mt * 16 + 4 * (lane >> 4) + r;
+            if (mrow < rows) take_grad(a, off + mrow * ldg + nt * 16 + r16, acc[r]);
+        }
+        return;
+    }
+    __shared__ double s[256];
+    b -= kTiles;
+    auto tree = [&]() {
+        __syncthreads();
+        for (int k = 128; k > 0; k >>= 1) {
+            for (int t = lane; t < k; t += 64) s[t] += s[t + k];
+            __syncthreads();
+        }
+    };
+    if (b < kCols) {
+        // sum t takes rows t, t + 256, ...; lane l < 32 holds sums 8l..8l+7, so
+        // that its loads are 16 bytes (rows past n are zero)
+        if (lane < 32) {
+            double acc[8] = { 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0 };
+            if (b < 2 * kHid) {
+                const uint16_t* col = (b < kHid ? a.dZ1T + (size_t)b * a.ld : a.dZ2T + (size_t)(b - kHid) * a.ld);
+#pragma unroll 8
+                for (int r = 8 * lane; r < a.ld; r += 256) {
+                    union { uint4 q; uint16_t h[8]; } v;
+                    v.q = *reinterpret_cast<const uint4*>(col + r);
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) acc[j] += (double)bf2f(v.h[j]);
+                }
+            } else {
+                const float* col = a.dYf + (size_t)(b - 2 * kHid) * a.ld;
+#pragma unroll 4
+                for (int r = 8 * lane; r < a.ld; r += 256) {
+                    const float4 u = *reinterpret_cast<const float4*>(col + r), v = *reinterpret_cast<const float4*>(col + r + 4);
+                    acc[0] += (double)u.x; acc[1] += (double)u.y; acc[2] += (double)u.z; acc[3] += (double)u.w;
+                    acc[4] += (double)v.x; acc[5] += (double)v.y; acc[6] += (double)v.z; acc[7] += (double)v.w;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) s[8 * lane + j] = acc[j];
+        }
+        tree();
+        if (lane == 0)
+            take_grad(a, b < kHid ? kOB1 + b : b < 2 * kHid ? kOB2 + b - kHid : kOB3 + b - 2 * kHid, (float)s[0]);
+        return;
+    }
+    b -= kCols;
+    for (int t = lane; t < 256; t += 64) {
+        const int r = b * 256 + t;
+        s[t] = r < a.n ? a.rowLoss[r] : 0.0;
+    }
+    tree();
+    if (lane == 0) a.part[b] = s[0];
+}
+
+// mean loss of `steps` batches of n rows, from the nb partial sums of each
+// (one thread, fixed order)
+__global__ void k_loss_final(const double* __restrict__ part, int nb, int n, int steps, double* __restrict__ out)
 {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double s = 0.0;
-    for (int i = 0; i < nb; ++i) s += part[i];
-    *acc += s / (double)n;
-}
-
-// column sums (bias gradients): one block of 256 per column, strided FP64
-// partial sums then a fixed tree, so the order depends only on `rows`
-template <class T>
-__device__ __forceinline__ double as_f64(T v);
-template <>
-__device__ __forceinline__ double as_f64<float>(float v) { return (double)v; }
-template <>
-__device__ __forceinline__ double as_f64<uint16_t>(uint16_t v) { return (double)bf2f(v); }
-
-template <class T>
-__global__ __launch_bounds__(256) void k_colsum(const T* __restrict__ a, int rows, int cols, float* __restrict__ out)
-{
-    __shared__ double s[256];
-    const int c = blockIdx.x;
     double acc = 0.0;
-    for (int r = threadIdx.x; r < rows; r += 256) acc += as_f64<T>(a[(long long)r * cols + c]);
-    s[threadIdx.x] = acc;
-    __syncthreads();
-    for (int k = 128; k > 0; k >>= 1) {
-        if ((int)threadIdx.x < k) s[threadIdx.x] += s[threadIdx.x + k];
-        __syncthreads();
+    for (int st = 0; st < steps; ++st) {
+        double s = 0.0;
+        for (int i = 0; i < nb; ++i) s += part[(size_t)st * nb + i];
+        acc += s / (double)n;
     }
-    if (threadIdx.x == 0) out[c] = (float)s[0];
-}
-
-__global__ void k_adam(float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m1,
-                       float* __restrict__ m2, uint16_t* __restrict__ wb, int n, float lr, float c1, float c2)
-{
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    float gi = g[i];
-    float a = b1 * m1[i] + (1.0f - b1) * gi;
-    float b = b2 * m2[i] + (1.0f - b2) * gi * gi;
-    m1[i] = a;
-    m2[i] = b;
-    float mh = a / c1, vh = b / c2;
-    float wi = w[i] - lr * mh / (sqrtf(vh) + eps);
-    w[i] = wi;
-    wb[i] = f2bf(wi);
+    *out = acc;
 }
 
 __global__ void k_to_bf16(const float* __restrict__ a, long long n, uint16_t* __restrict__ b)
@@ -180,16 +414,11 @@ __global__ void k_to_bf16(const float* __restrict__ a, long long n, uint16_t* __
     if (i < n) b[i] = f2bf(a[i]);
 }
 
-// batch gather through a permutation
-__global__ void k_gather_rows(const uint16_t* __restrict__ X, const float* __restrict__ T, const int* __restrict__ perm,
-                              int n, uint16_t* __restrict__ Xo, float* __restrict__ To)
+// BF16 copy of W2, transposed
+__global__ void k_w2_transposed(const uint16_t* __restrict__ wb, uint16_t* __restrict__ w2t)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n * kIn) return;
-    int r = i / kIn, c = i - r * kIn;
-    long long src = perm[r];
-    Xo[i] = X[src * kIn + c];
-    if (c < 3) To[3 * r + c] = T[src * 3 + c];
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < kHid * kHid) w2t[(i & (kHid - 1)) * kHid + (i >> 7)] = wb[kOW2 + i];
 }
 
 // one-ring features of vertex v into o[0..95] (bf16); returns L
@@ -241,7 +470,7 @@ struct InferArgs {
     const float* z;
     const int* nbr;
     int lo, n;
-    const uint16_t* Xin;   // optional precomputed features (n x 96)
+    const float* Xin;      // optional precomputed features (n x 96, rounded to BF16 here)
     const uint16_t* wb;
     const float* w;
     float* Y;
@@ -259,7 +488,7 @@ __global__ __launch_bounds__(256) void k_mlp_infer(InferArgs a)
     if (a.Xin) {
         for (int i = tid; i < kMlpRows * kIn; i += 256) {
             int r = i / kIn, c = i - r * kIn;
-            sm.X[r * kLdx + c] = (row0 + r < a.n) ? a.Xin[(size_t)(row0 + r) * kIn + c] : (uint16_t)0;
+            sm.X[r * kLdx + c] = (row0 + r < a.n) ? f2bf(a.Xin[(size_t)(row0 + r) * kIn + c]) : (uint16_t)0;
         }
     } else {
         const int r = tid >> 4;
@@ -276,7 +505,7 @@ __global__ __launch_bounds__(256) void k_mlp_infer(InferArgs a)
 }
 
 void launch_mlp_infer(vsdmo_mlp* m, const float* x, const float* y, const float* z, const int* nbr, int lo, int hi,
-                      const uint16_t* Xin, float* Y, float* L, hipStream_t s)
+                      const float* Xin, float* Y, float* L, hipStream_t s)
 {
     const int n = hi - lo;
     if (n <= 0) return;
@@ -340,87 +569,49 @@ void build_neighbour_table(vsdmo_mesh& m)
 void mlp_reserve(vsdmo_mlp* m, int n)
 {
     if (n <= m->cap) return;
-    int c = std::max(n, 2 * m->cap);
-    m->X.alloc((size_t)c * kIn);
-    m->H1.alloc((size_t)c * kHid);
-    m->H2.alloc((size_t)c * kHid);
-    m->dZ1.alloc((size_t)c * kHid);
-    m->dZ2.alloc((size_t)c * kHid);
-    m->dY16.alloc((size_t)c * kOut);
-    m->Z1.alloc((size_t)c * kHid);
-    m->Z2.alloc((size_t)c * kHid);
-    m->Y.alloc((size_t)c * kOut);
-    m->T.alloc((size_t)c * kOut);
-    m->part.alloc((size_t)c * kOut);   // dY in FP32
-    m->lossd.alloc((size_t)(c + 255) / 256 + 1);
-    m->cap = c;
+    const size_t c = (size_t)(std::max(n, 2 * m->cap) + 31) / 32 * 32;
+    m->XT.alloc(c * kIn);
+    m->H1T.alloc(c * kHid);
+    m->H2T.alloc(c * kHid);
+    m->dZ1T.alloc(c * kHid);
+    m->dZ2T.alloc(c * kHid);
+    m->dYT.alloc(c * kOut);
+    m->dYf.alloc(c * kOut);
+    m->rowLoss.alloc(c);
+    m->cap = (int)c;
 }
 
-static GemmArgs gargs(int M, int N, int K, const uint16_t* A, long long sam, long long sak, const uint16_t* B,
-                      long long sbk, long long sbn)
-{
-    GemmArgs g{};
-    g.M = M; g.N = N; g.K = K;
-    g.A = A; g.sam = sam; g.sak = sak;
-    g.B = B; g.sbk = sbk; g.sbn = sbn;
-    return g;
-}
+// n rows of features and targets: FP32 rows, or rows perm[0..n) of a dataset
+struct MlpBatch {
+    const float* Xf = nullptr;
+    const uint16_t* Xb = nullptr;
+    const float* T = nullptr;
+    const int* perm = nullptr;
+    int n = 0;
+};
 
-// forward of n rows (X bf16 device) -> Y (device, FP32); keeps Z1, H1, Z2, H2
-void mlp_forward_dev(vsdmo_mlp* m, const uint16_t* X, int n, float* Y, hipStream_t s)
+// forward, backward and the weight gradients of a batch; the squared error of
+// every 256 rows in part; gradients in m->g, or (adam) the update of step
+// m->step with rate lr
+static void mlp_step(vsdmo_mlp* m, const MlpBatch& x, double* part, bool adam, float lr, hipStream_t s)
 {
-    const uint16_t* wb = m->wb.p;
-    const float* w = m->w.p;
-    // Z1 = X W1^T + b1, H1 = gelu(Z1)
-    GemmArgs g = gargs(n, kHid, kIn, X, kIn, 1, wb + kOW1, 1, kIn);
-    g.bias = w + kOB1; g.mode = EPI_GELU; g.Cf = m->Z1.p; g.ldcf = kHid; g.Cb = m->H1.p; g.ldcb = kHid;
-    gemm(g, s);
-    g = gargs(n, kHid, kHid, m->H1.p, kHid, 1, wb + kOW2, 1, kHid);
-    g.bias = w + kOB2; g.mode = EPI_GELU; g.Cf = m->Z2.p; g.ldcf = kHid; g.Cb = m->H2.p; g.ldcb = kHid;
-    gemm(g, s);
-    g = gargs(n, kOut, kHid, m->H2.p, kHid, 1, wb + kOW3, 1, kHid);
-    g.bias = w + kOB3; g.mode = EPI_F32; g.Cf = Y; g.ldcf = kOut;
-    gemm(g, s);
-}
-
-// loss and gradients of n rows (X, T in the work buffers); adds the mean
-// loss to *lossAcc
-static void mlp_backward_dev(vsdmo_mlp* m, int n, double* lossAcc, hipStream_t s)
-{
-    const uint16_t* wb = m->wb.p;
-    float* gr = m->g.p;
-    mlp_forward_dev(m, m->X.p, n, m->Y.p, s);
-    const int nb = (n + 255) / 256;
-    k_mse<<<nb, 256, 0, s>>>(m->Y.p, m->T.p, n, m->part.p, m->dY16.p, m->lossd.p);
-    k_loss_final<<<1, 64, 0, s>>>(m->lossd.p, nb, n, lossAcc);
-    // dW3 = dY^T H2 ; db3 = colsum dY
-    GemmArgs g = gargs(kOut, kHid, n, m->dY16.p, 1, kOut, m->H2.p, kHid, 1);
-    g.mode = EPI_F32; g.Cf = gr + kOW3; g.ldcf = kHid;
-    gemm(g, s);
-    k_colsum<float><<<kOut, 256, 0, s>>>(m->part.p, n, kOut, gr + kOB3);
-    // dZ2 = (dY W3) * gelu'(Z2)
-    g = gargs(n, kHid, kOut, m->dY16.p, kOut, 1, wb + kOW3, kHid, 1);
-    g.mode = EPI_DGELU; g.Cb = m->dZ2.p; g.ldcb = kHid; g.Zin = m->Z2.p; g.ldz = kHid;
-    gemm(g, s);
-    // dW2 = dZ2^T H1 ; db2
-    g = gargs(kHid, kHid, n, m->dZ2.p, 1, kHid, m->H1.p, kHid, 1);
-    g.mode = EPI_F32; g.Cf = gr + kOW2; g.ldcf = kHid;
-    gemm(g, s);
-    k_colsum<uint16_t><<<kHid, 256, 0, s>>>(m->dZ2.p, n, kHid, gr + kOB2);
-    // dZ1 = (dZ2 W2) * gelu'(Z1)
-    g = gargs(n, kHid, kHid, m->dZ2.p, kHid, 1, wb + kOW2, kHid, 1);
-    g.mode = EPI_DGELU; g.Cb = m->dZ1.p; g.ldcb = kHid; g.Zin = m->Z1.p; g.ldz = kHid;
-    gemm(g, s);
-    // dW1 = dZ1^T X ; db1
-    g = gargs(kHid, kIn, n, m->dZ1.p, 1, kHid, m->X.p, kIn, 1);
-    g.mode = EPI_F32; g.Cf = gr + kOW1; g.ldcf = kIn;
-    gemm(g, s);
-    k_colsum<uint16_t><<<kHid, 256, 0, s>>>(m->dZ1.p, n, kHid, gr + kOB1);
+    const int ld = (x.n + 31) / 32 * 32;
+    k_mlp_rows<<<ld / kMlpRows, 256, 0, s>>>(RowsArgs{ x.Xf, x.Xb, x.T, x.perm, x.n, ld, m->wb.p, m->w2t.p, m->w.p, m->XT.p,
+                                                      m->H1T.p, m->H2T.p, m->dZ1T.p, m->dZ2T.p, m->dYT.p, m->dYf.p,
+                                                      m->rowLoss.p });
+    GradsArgs g{ m->XT.p, m->H1T.p, m->H2T.p, m->dZ1T.p, m->dZ2T.p, m->dYT.p, m->dYf.p, m->rowLoss.p, x.n, ld, part,
+                 adam ? nullptr : m->g.p, m->w.p, m->m1.p, m->m2.p, m->wb.p, m->w2t.p, lr, 1.0f, 1.0f };
+    if (adam) {
+        g.c1 = 1.0f - std::pow(0.9f, (float)m->step);
+        g.c2 = 1.0f - std::pow(0.999f, (float)m->step);
+    }
+    k_mlp_grads<<<kTiles + kCols + (x.n + 255) / 256, 64, 0, s>>>(g);
 }
 
 static void refresh_bf16(vsdmo_mlp* m, hipStream_t s)
 {
     k_to_bf16<<<(kNParams + 255) / 256, 256, 0, s>>>(m->w.p, kNParams, m->wb.p);
+    k_w2_transposed<<<kHid * kHid / 256, 256, 0, s>>>(m->wb.p, m->w2t.p);
 }
 
 static vsdmo_status fail_m(vsdmo_status st, const std::string& msg)
@@ -441,6 +632,13 @@ static vsdmo_status guarded_m(F&& f)
     } catch (const std::bad_alloc&) {
         return fail_m(VSDMO_HIP_ERROR, "host allocation failed");
     }
+}
+
+// the FP32 rows and targets of the host calls
+static void reserve_rows(vsdmo_mlp* m, int n)
+{
+    if (m->Xf.n < (size_t)n * kIn) m->Xf.alloc((size_t)n * kIn);
+    if (m->T.n < (size_t)n * kOut) m->T.alloc((size_t)n * kOut);
 }
 
 static uint64_t smix(uint64_t& s)
@@ -482,6 +680,7 @@ vsdmo_status vsdmo_mlp_create(uint64_t seed, vsdmo_mlp** out)
             fill(kOW3, kOut * kHid, kHid); fill(kOB3, kOut, kHid);
             m->w.alloc(kNParams); m->g.alloc(kNParams); m->m1.alloc(kNParams); m->m2.alloc(kNParams);
             m->wb.alloc(kNParams);
+            m->w2t.alloc((size_t)kHid * kHid);
             m->w.upload(w.data(), kNParams, m->stream);
             std::vector<float> zero(kNParams, 0.0f);
             m->m1.upload(zero.data(), kNParams, m->stream);
@@ -541,12 +740,10 @@ vsdmo_status vsdmo_mlp_forward(vsdmo_mlp* m, const float* X, int32_t n, float* Y
     return guarded_m([&]() -> vsdmo_status {
         if (!m || !X || !Y || n < 0) return fail_m(VSDMO_INVALID_ARG, "bad argument");
         if (n == 0) return VSDMO_OK;
-        mlp_reserve(m, n);
-        std::vector<uint16_t> xb((size_t)n * kIn);
-        for (size_t i = 0; i < xb.size(); ++i) xb[i] = f2bf(X[i]);
-        m->X.upload(xb.data(), xb.size(), m->stream);
-        launch_mlp_infer(m, nullptr, nullptr, nullptr, nullptr, 0, n, m->X.p, m->Y.p, nullptr, m->stream);
-        m->Y.download(Y, (size_t)n * kOut, m->stream);
+        reserve_rows(m, n);
+        m->Xf.upload(X, (size_t)n * kIn, m->stream);
+        launch_mlp_infer(m, nullptr, nullptr, nullptr, nullptr, 0, n, m->Xf.p, m->T.p, nullptr, m->stream);
+        m->T.download(Y, (size_t)n * kOut, m->stream);
         VSDMO_HIP(hipStreamSynchronize(m->stream));
         return VSDMO_OK;
     });
@@ -557,17 +754,19 @@ vsdmo_status vsdmo_mlp_gradients(vsdmo_mlp* m, const float* X, const float* T, i
     return guarded_m([&]() -> vsdmo_status {
         if (!m || !X || !T || n <= 0) return fail_m(VSDMO_INVALID_ARG, "bad argument");
         mlp_reserve(m, n);
-        std::vector<uint16_t> xb((size_t)n * kIn);
-        for (size_t i = 0; i < xb.size(); ++i) xb[i] = f2bf(X[i]);
-        m->X.upload(xb.data(), xb.size(), m->stream);
+        reserve_rows(m, n);
+        m->Xf.upload(X, (size_t)n * kIn, m->stream);
         m->T.upload(T, (size_t)n * kOut, m->stream);
-        DevBuf<double> acc(1);
-        double z = 0.0;
-        acc.upload(&z, 1, m->stream);
-        mlp_backward_dev(m, n, acc.p, m->stream);
+        const int nb = (n + 255) / 256;
+        DevBuf<double> part((size_t)nb + 1);   // partial sums, then the loss
+        MlpBatch x;
+        x.Xf = m->Xf.p; x.T = m->T.p; x.n = n;
+        mlp_step(m, x, part.p, false, 0.0f, m->stream);
+        k_loss_final<<<1, 64, 0, m->stream>>>(part.p, nb, n, 1, part.p + nb);
+        VSDMO_HIP(hipGetLastError());
         if (grad) m->g.download(grad, kNParams, m->stream);
         double l = 0.0;
-        acc.download(&l, 1, m->stream);
+        VSDMO_HIP(hipMemcpyAsync(&l, part.p + nb, sizeof(double), hipMemcpyDeviceToHost, m->stream));
         VSDMO_HIP(hipStreamSynchronize(m->stream));
         if (loss) *loss = l;
         return VSDMO_OK;
@@ -586,31 +785,44 @@ vsdmo_status vsdmo_mlp_train(vsdmo_mlp* m, vsdmo_dataset* ds, int32_t epochs, in
         hipStream_t s = m->stream;
         VSDMO_HIP(hipStreamSynchronize(ds->stream));
         mlp_reserve(m, batch);
+        if (epochs == 0) return VSDMO_OK;
         m->perm.alloc((size_t)N);
-        std::vector<int> perm((size_t)N);
-        DevBuf<double> acc(1);
-        uint64_t rs = seed;
         const long long steps = N / batch;   // the ragged tail of each shuffled epoch is dropped
+        const int nb = (batch + 255) / 256;
+        DevBuf<double> part((size_t)steps * nb), loss((size_t)epochs);
+        // the host shuffles an epoch while the GPU runs the one before: two
+        // permutations in turn, each free again once its upload is done
+        std::vector<int> perm[2] = { std::vector<int>((size_t)N), std::vector<int>((size_t)N) };
+        struct Events {
+            hipEvent_t e[2] = { nullptr, nullptr };
+            ~Events() { for (hipEvent_t x : e) if (x) (void)hipEventDestroy(x); }
+        } up;
+        struct Drain {   // an early exit must not free what the stream still reads
+            hipStream_t s;
+            ~Drain() { (void)hipStreamSynchronize(s); }
+        } drain{ s };
+        for (hipEvent_t& e : up.e) VSDMO_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        uint64_t rs = seed;
         for (int ep = 0; ep < epochs; ++ep) {
-            for (long long i = 0; i < N; ++i) perm[i] = (int)i;
-            for (long long i = N - 1; i > 0; --i) std::swap(perm[i], perm[(long long)(smix(rs) % (uint64_t)(i + 1))]);
-            m->perm.upload(perm.data(), (size_t)N, s);
-            double z = 0.0;
-            acc.upload(&z, 1, s);
+            std::vector<int>& p = perm[ep & 1];
+            if (ep >= 2) VSDMO_HIP(hipEventSynchronize(up.e[ep & 1]));
+            for (long long i = 0; i < N; ++i) p[i] = (int)i;
+            for (long long i = N - 1; i > 0; --i) std::swap(p[i], p[(long long)(smix(rs) % (uint64_t)(i + 1))]);
+            m->perm.upload(p.data(), (size_t)N, s);
+            VSDMO_HIP(hipEventRecord(up.e[ep & 1], s));
             for (long long st = 0; st < steps; ++st) {
-                k_gather_rows<<<(batch * kIn + 255) / 256, 256, 0, s>>>(ds->X.p, ds->T.p, m->perm.p + st * batch, batch,
-                                                                      m->X.p, m->T.p);
-                mlp_backward_dev(m, batch, acc.p, s);
+                MlpBatch x;
+                x.Xb = ds->X.p; x.T = ds->T.p; x.perm = m->perm.p + st * batch; x.n = batch;
                 m->step++;
-                const float c1 = 1.0f - std::pow(0.9f, (float)m->step), c2 = 1.0f - std::pow(0.999f, (float)m->step);
-                k_adam<<<(kNParams + 255) / 256, 256, 0, s>>>(m->w.p, m->g.p, m->m1.p, m->m2.p, m->wb.p, kNParams, lr,
-                                                            c1, c2);
+                mlp_step(m, x, part.p + st * nb, true, lr, s);
             }
-            double l = 0.0;
-            acc.download(&l, 1, s);
-            VSDMO_HIP(hipStreamSynchronize(s));
-            if (epoch_loss) epoch_loss[ep] = l / (double)steps;
+            k_loss_final<<<1, 64, 0, s>>>(part.p, nb, batch, (int)steps, loss.p + ep);
         }
+        std::vector<double> l((size_t)epochs);
+        loss.download(l.data(), (size_t)epochs, s);
+        VSDMO_HIP(hipStreamSynchronize(s));
+        if (epoch_loss)
+            for (int ep = 0; ep < epochs; ++ep) epoch_loss[ep] = l[ep] / (double)steps;
         VSDMO_HIP(hipGetLastError());
         return VSDMO_OK;
     });

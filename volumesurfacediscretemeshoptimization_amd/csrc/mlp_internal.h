@@ -302,18 +302,19 @@ struct vsdmo_mlp {
     int step = 0;
     int cap = 0;                         // batch capacity of the work buffers
     int n_users = 0;                     // optimisers and batches with this network as their proposal
-    vsdmo::DevBuf<uint16_t> X, H1, H2, dY16, dZ1, dZ2;
-    vsdmo::DevBuf<float> Z1, Z2, Y, T, part;
-    vsdmo::DevBuf<double> lossd;
+    vsdmo::DevBuf<uint16_t> w2t;         // bf16 copy of W2, transposed
+    // work buffers of a batch, feature-major (k_mlp_rows)
+    vsdmo::DevBuf<uint16_t> XT, H1T, H2T, dZ1T, dZ2T, dYT;
+    vsdmo::DevBuf<float> dYf;
+    vsdmo::DevBuf<double> rowLoss;
+    vsdmo::DevBuf<float> Xf, T;          // rows and targets (or outputs) of the host calls
     vsdmo::DevBuf<int> perm;
 };
 
 namespace vsdmo {
-// forward of n rows of bf16 features X (device) into Y (device, n x 3)
-void mlp_forward_dev(vsdmo_mlp* m, const uint16_t* X, int n, float* Y, hipStream_t s);
 void mlp_reserve(vsdmo_mlp* m, int n);
 // fused inference (features + 3 layers) of vertices [lo, hi) or of rows of
 // Xin (n = hi - lo); Y (n x 3) and, when computing features, L (n)
 void launch_mlp_infer(vsdmo_mlp* m, const float* x, const float* y, const float* z, const int* nbr, int lo, int hi,
-                      const uint16_t* Xin, float* Y, float* L, hipStream_t s);
+                      const float* Xin, float* Y, float* L, hipStream_t s);
 }  // namespace vsdmo
