@@ -79,16 +79,16 @@ static void destroy_mesh(vsdmo_mesh* m)
 
 using namespace vsdmo;
 
-// 16 bytes of pinned host memory for the per-iteration quality readback
+// pinned host memory of the per-iteration quality
 struct PinnedQ {
-    double* p = nullptr;
+    QualityOut* p = nullptr;
     PinnedQ() = default;
     PinnedQ(const PinnedQ&) = delete;
     PinnedQ& operator=(const PinnedQ&) = delete;
     ~PinnedQ() { if (p) (void)hipHostFree(p); }
     void alloc()
     {
-        if (!p) VSDMO_HIP(hipHostMalloc(reinterpret_cast<void**>(&p), 2 * sizeof(double), hipHostMallocDefault));
+        if (!p) VSDMO_HIP(hipHostMalloc(reinterpret_cast<void**>(&p), sizeof(QualityOut), hipHostMallocDefault));
     }
 };
 
@@ -109,8 +109,8 @@ struct vsdmo_opt {
     int64_t launches = 0;
     DevBuf<float> q, pmin;
     DevBuf<double> psum;
-    DevBuf<double> qout;   // [0]: minimum (float in bytes 0-3, surface error bits in 4-7), [1]: FP64 sum
-    PinnedQ hq;            // their host copy
+    DevBuf<int> qflags;    // [0]: surface error bits, then the quality kernel's tickets
+    PinnedQ hq;            // minimum, error bits and FP64 sum, written by the quality kernel
     std::vector<hipEvent_t> ev;   // pool of events, [0, ev_used) in use by the timed launches
     size_t ev_used = 0;
     std::vector<std::pair<size_t, size_t>> ev_pairs;   // (begin, end) event of every timed launch
@@ -411,17 +411,12 @@ static void opt_quality(vsdmo_opt* o)
     vsdmo_mesh* m = o->m;
     QualityArgs qa{ m->x.p, m->y.p, m->z.p, m->cells.p, m->nE, m->npe, o->qelem, o->q.p,
                     o->p.hex_metric == VSDMO_HEX_CORNER8 };
-    launch_quality(qa, o->pmin.p, o->psum.p, reinterpret_cast<float*>(o->qout.p), o->qout.p + 1, m->stream);
+    launch_quality(qa, o->pmin.p, o->psum.p, o->qflags.p + kTicketStride, o->qflags.p, o->hq.p, m->stream);
     VSDMO_HIP(hipGetLastError());
-    // one 16-byte copy into pinned memory (no staging, one synchronisation)
-    VSDMO_HIP(hipMemcpyAsync(o->hq.p, o->qout.p, 2 * sizeof(double), hipMemcpyDeviceToHost, m->stream));
     VSDMO_HIP(hipStreamSynchronize(m->stream));
-    float mn = 0.0f;
-    int err = 0;
-    std::memcpy(&mn, o->hq.p, sizeof(float));
-    std::memcpy(&err, reinterpret_cast<const char*>(o->hq.p) + sizeof(float), sizeof(int));
-    o->last_min = mn;
-    o->last_sum = o->hq.p[1];
+    const int err = o->hq.p->err;
+    o->last_min = o->hq.p->min;
+    o->last_sum = o->hq.p->sum;
     if (err & kSurfErrUnsectored)
         throw StatusError{ VSDMO_TOPOLOGY, "a feature vertex has surface neighbours after its last feature "
                                            "neighbour (open fan): they belong to no feature sector" };
@@ -468,7 +463,7 @@ static SurfArgs surf_args(vsdmo_opt* o)
     a.gridScale = o->grid_scale; a.shrink = o->shrink; a.aff = o->aff; a.depth = o->p.depth;
     a.hexCorner8 = o->p.hex_metric == VSDMO_HEX_CORNER8;
     a.ring2 = o->p.surface_ring == 2;
-    a.err = reinterpret_cast<int*>(o->qout.p) + 1;
+    a.err = o->qflags.p;
     return a;
 }
 
@@ -559,8 +554,8 @@ vsdmo_status vsdmo_opt_create(vsdmo_mesh* m, int32_t criterion, float grid_scale
             int nb = (m->nE + 255) / 256;
             o->q.alloc(m->nE);
             o->pmin.alloc(nb); o->psum.alloc(nb);
-            o->qout.alloc(2);
-            VSDMO_HIP(hipMemsetAsync(o->qout.p, 0, 2 * sizeof(double), m->stream));
+            o->qflags.alloc(kTicketStride + kTicketInts);
+            launch_fill_int(o->qflags.p, kTicketStride + kTicketInts, 0, m->stream);
             o->hq.alloc();
             if (!p.fixed_boundary || surfMesh) surface_init(o);
             opt_quality(o);
@@ -708,9 +703,9 @@ vsdmo_status vsdmo_opt_iterate(vsdmo_opt* o, int32_t n)
                     SurfArgs sa = surf_args(o);
                     size_t slds = surf_lds_bytes(m->elem, m->maxRing);
                     const int tet = (m->elem == VSDMO_TET);
+                    if (m->colOffFree.size() > 1) snapshot_launch(sa, m->stream);
                     for (size_t c = 0; c + 1 < m->colOffFree.size(); ++c) {
                         int lo = m->colOffFree[c], hi = m->colOffFree[c + 1];
-                        snapshot_launch(sa, m->stream);
                         surf_search2d_launch(sa, lo, hi, o->p.nq, tet, slds, m->stream);
                         o->s_surf += hi - lo;
                     }
@@ -725,24 +720,20 @@ vsdmo_status vsdmo_opt_iterate(vsdmo_opt* o, int32_t n)
                 // surface mesh on the surface path (DMOTri.cu:128-170, DMOQuad.cu:128-170):
                 // free 2D passes, feature 1D passes, NN walk, normals; no quality gate
                 SurfArgs sa = surf_args(o);
+                snapshot_launch(sa, m->stream);
                 for (size_t c = 0; c + 1 < m->colOffFree.size(); ++c) {
                     int lo = m->colOffFree[c], hi = m->colOffFree[c + 1];
-                    snapshot_launch(sa, m->stream);
                     timed(o, [&]() { surf_fan2d_launch(sa, lo, hi, o->p.nq, m->stream); });
                     o->s_surf += hi - lo;
                 }
                 if (!o->p.fixed_boundary) {
                     for (size_t c = 0; c + 1 < m->colOffFeature.size(); ++c) {
                         int lo = m->colOffFeature[c], hi = m->colOffFeature[c + 1];
-                        if (m->elem == VSDMO_QUAD) {   // quad fan diagonals read the pass snapshot
-                            snapshot_launch(sa, m->stream);
-                        }
                         timed(o, [&]() { surf_fan1d_launch(sa, lo, hi, o->p.nq, m->stream); });
                         for (int v = lo; v < hi; ++v) o->s_feat += o->opt1d_host[v];
                     }
                 }
-                surf_nn_launch(sa, m->stream);
-                surf_normals_launch(sa, m->stream);
+                surf_nn_normals_launch(sa, m->stream);
             } else {
                 for (size_t c = 0; c + 1 < m->colOffFree.size(); ++c) {
                     a.cStart = m->colOffFree[c]; a.cEnd = m->colOffFree[c + 1];

@@ -81,9 +81,14 @@ struct SurfArgs {
     float* xw;
     float* yw;
     float* zw;
-    const float* sx;        // positions snapshot at the start of a surface colour pass
+    // snapshot of the surface positions at the start of the iteration's surface
+    // passes: the start-of-pass positions of the class being searched, whose
+    // vertices have not moved before their own pass; any other vertex is read
+    // from x / y / z, which no pass changes but its own
+    const float* sx;
     const float* sy;
     const float* sz;
+    int cLo, cHi;           // the class being searched (set by the launchers)
     const int* ringRow;
     const int* ringVal;
     const int* heRow;
@@ -135,11 +140,12 @@ void surf_search1d_launch(const SurfArgs& a, int cStart, int cEnd, int nq, int t
 void surf_flat1d_launch(const SurfArgs& a, int cStart, int cEnd, int nq, hipStream_t s);
 void surf_points_launch(const SurfArgs& a, int vid, int nu, int nv, int mode, int sid, float* out, hipStream_t s);
 // surface meshes (tri / quad, chosen by a.fpe): free-vertex 2D and
-// feature-vertex 1D searches of one colour class, normals from the current
-// positions, Laplace smoothing of one colour class
+// feature-vertex 1D searches of one colour class, Laplace smoothing of one
+// colour class
 void surf_fan2d_launch(const SurfArgs& a, int cStart, int cEnd, int nq, hipStream_t s);
 void surf_fan1d_launch(const SurfArgs& a, int cStart, int cEnd, int nq, hipStream_t s);
-void surf_normals_launch(const SurfArgs& a, hipStream_t s);
+// the nearest-neighbour walk and the face and vertex normals, from the current positions
+void surf_nn_normals_launch(const SurfArgs& a, hipStream_t s);
 // snapshot of the surface positions into a.sx / a.sy / a.sz
 void snapshot_launch(const SurfArgs& a, hipStream_t s);
 void laplace_launch(float* x, float* y, float* z, const int* heRow, const int* heTarget, int lo, int hi, hipStream_t s);
@@ -245,7 +251,19 @@ bool learned_deferred_ok(int kind, int nq, int ringCap);
 bool learned_fused_ok(int kind, int ringCap);
 void launch_batch_quality(const BatchQArgs& a, hipStream_t s);
 size_t batch_lds_bytes(int maxRingTet, int maxRingHex, int maxHETri);
-void launch_quality(const QualityArgs& a, float* pmin, double* psum, float* omin, double* osum, hipStream_t s);
+// pinned host memory that the quality kernel writes
+struct QualityOut {
+    float min;
+    int err;      // surface error bits (kSurfErr*)
+    double sum;
+};
+// arrival counters of the quality kernel's blocks: one over the groups, then
+// one per group, each on a cache line of its own
+constexpr int kTicketGroups = 32, kTicketStride = 32;
+constexpr int kTicketInts = (kTicketGroups + 1) * kTicketStride;
+// ticket: kTicketInts zeros on entry and on completion; out: pinned host memory
+void launch_quality(const QualityArgs& a, float* pmin, double* psum, int* ticket, const int* err, QualityOut* out,
+                    hipStream_t s);
 void launch_histogram(const float* q, int n, int ncols, int* bins, hipStream_t s);
 
 }  // namespace vsdmo

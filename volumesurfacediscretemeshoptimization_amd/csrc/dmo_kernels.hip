@@ -2057,12 +2057,38 @@ __device__ __forceinline__ void block_minsum256(float& m, double& s)
     s = (ws[0] + ws[1]) + (ws[2] + ws[3]);
 }
 
-// the qualities of the block's 256 * per elements (per per thread, strided
-// by 256), written to q, and their min and FP64 sum in a fixed order
-// (per-block partials for k_reduce_final)
-__global__ __launch_bounds__(256) void k_elem_quality(QualityArgs a, float* __restrict__ pmin,
-                                                      double* __restrict__ psum, int per)
+// true in the one thread that arrives last of all blocks, each of which has
+// one thread call it after its agent-scope stores.  Those are complete at the
+// point of coherence once they have left the wave's memory counter, so no
+// release of the whole L2 is needed.
+__device__ __forceinline__ bool last_block(int* ticket, int b, int nb)
 {
+    __builtin_amdgcn_s_waitcnt(0);
+    asm volatile("" ::: "memory");
+    const int g = b % kTicketGroups, ng = nb < kTicketGroups ? nb : kTicketGroups;
+    const int members = nb / kTicketGroups + (g < nb % kTicketGroups);
+    if (__hip_atomic_fetch_add(ticket + (g + 1) * kTicketStride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+        != members - 1) return false;
+    return __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == ng - 1;
+}
+
+// the qualities of the block's 256 * per elements (per per thread, strided by
+// 256), written to q, and their min and FP64 sum in a fixed order.  The block
+// that takes the last ticket reduces the blocks' partials (strided, then a
+// fixed tree: the order of the additions depends only on the block count) and
+// writes {min, surface error bits, sum} straight into pinned host memory: one
+// launch, where a second reduction kernel (3-5 us with its gap) and a 16-byte
+// copy (2-5 us) followed.  Partials and tickets go through the device's point of
+// coherence (agent-scope stores and loads), as the blocks run on all XCDs.
+// The tickets are counted in groups, then over the groups: with one counter
+// and a release of the L2 by every block, 750 blocks (384k elements) took
+// 9 us more per iteration than the two launches; in groups they take 1-2 us less.
+__global__ __launch_bounds__(256) void k_elem_quality(QualityArgs a, float* pmin, double* psum, int* ticket,
+                                                      const int* err, QualityOut* out, int per)
+{
+    __shared__ float smin[256];
+    __shared__ double ssum[256];
+    __shared__ int s_last;
     float v = FLT_MAX;
     double sv = 0.0;
     for (int k = 0; k < per; ++k) {
@@ -2075,7 +2101,36 @@ __global__ __launch_bounds__(256) void k_elem_quality(QualityArgs a, float* __re
         }
     }
     block_minsum256(v, sv);
-    if (threadIdx.x == 0) { pmin[blockIdx.x] = v; psum[blockIdx.x] = sv; }
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(pmin + blockIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(psum + blockIdx.x, sv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = last_block(ticket, (int)blockIdx.x, (int)gridDim.x);
+    }
+    __syncthreads();
+    if (!s_last) return;
+    float m = FLT_MAX;
+    double s = 0.0;
+    for (int i = threadIdx.x; i < (int)gridDim.x; i += 256) {
+        m = fminf(m, __hip_atomic_load(pmin + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        s = s + __hip_atomic_load(psum + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    smin[threadIdx.x] = m;
+    ssum[threadIdx.x] = s;
+    __syncthreads();
+    for (int k = 128; k > 0; k >>= 1) {
+        if ((int)threadIdx.x < k) {
+            smin[threadIdx.x] = fminf(smin[threadIdx.x], smin[threadIdx.x + k]);
+            ssum[threadIdx.x] = ssum[threadIdx.x] + ssum[threadIdx.x + k];
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        out->min = smin[0];
+        out->err = *err;
+        out->sum = ssum[0];
+    }
+    // for the next launch
+    if (threadIdx.x <= kTicketGroups) ticket[threadIdx.x * kTicketStride] = 0;
 }
 
 // batch qualities: one block of 256 per chunk of at most 256 * a.per
@@ -2137,29 +2192,6 @@ __global__ void k_batch_mesh_reduce(BatchQArgs a)
 __global__ void k_batch_history_next(int* hctr)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) *hctr = *hctr + 1;
-}
-
-// one block of 256 threads: strided partial sums then a fixed tree (the order
-// of additions depends only on n, so the FP64 sum is reproducible)
-__global__ void k_reduce_final(const float* __restrict__ pmin, const double* __restrict__ psum, int n,
-                               float* __restrict__ omin, double* __restrict__ osum)
-{
-    __shared__ float smin[256];
-    __shared__ double ssum[256];
-    float m = FLT_MAX;
-    double s = 0.0;
-    for (int i = threadIdx.x; i < n; i += 256) { m = fminf(m, pmin[i]); s = s + psum[i]; }
-    smin[threadIdx.x] = m;
-    ssum[threadIdx.x] = s;
-    __syncthreads();
-    for (int k = 128; k > 0; k >>= 1) {
-        if (threadIdx.x < k) {
-            smin[threadIdx.x] = fminf(smin[threadIdx.x], smin[threadIdx.x + k]);
-            ssum[threadIdx.x] = ssum[threadIdx.x] + ssum[threadIdx.x + k];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) { *omin = smin[0]; *osum = ssum[0]; }
 }
 
 __global__ void k_histogram(const float* __restrict__ q, int n, int ncols, int* __restrict__ bins)
@@ -2337,12 +2369,12 @@ void launch_search(int kind, int nq, const SearchArgs& a, int ringCap, hipStream
     }
 }
 
-void launch_quality(const QualityArgs& a, float* pmin, double* psum, float* omin, double* osum, hipStream_t s)
+void launch_quality(const QualityArgs& a, float* pmin, double* psum, int* ticket, const int* err, QualityOut* out,
+                    hipStream_t s)
 {
     const int per = quality_per_thread(a.nE);
     const int nb = (a.nE + 256 * per - 1) / (256 * per);
-    k_elem_quality<<<nb, 256, 0, s>>>(a, pmin, psum, per);
-    k_reduce_final<<<1, 256, 0, s>>>(pmin, psum, nb, omin, osum);
+    k_elem_quality<<<nb, 256, 0, s>>>(a, pmin, psum, ticket, err, out, per);
 }
 
 void launch_histogram(const float* q, int n, int ncols, int* bins, hipStream_t s)

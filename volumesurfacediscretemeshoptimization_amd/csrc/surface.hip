@@ -121,14 +121,17 @@ __device__ void fit_quadric(LSurf& s, const w3* pts, int np)
 }
 
 // ------------------------------------------------------------- init kernels
-__global__ void k_surf_face_normals(SurfArgs a)
+__device__ __forceinline__ void face_normal(const SurfArgs& a, int f)
 {
-    int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= a.nFaces) return;
     const int* F = a.faces + (size_t)f * a.fpe;
     w3 p0 = WP(a.x, a.y, a.z, F[0]), p1 = WP(a.x, a.y, a.z, F[1]), p2 = WP(a.x, a.y, a.z, F[a.fpe == 3 ? 2 : 3]);
     w3 n = wnormalize(wcross(wsub(p1, p0), wsub(p2, p0)));
     a.fnorm[3 * f] = n.x; a.fnorm[3 * f + 1] = n.y; a.fnorm[3 * f + 2] = n.z;
+}
+__global__ void k_surf_face_normals(SurfArgs a)
+{
+    const int f = blockIdx.x * blockDim.x + threadIdx.x;
+    if (f < a.nFaces) face_normal(a, f);
 }
 
 __global__ void k_surf_vertex_init(SurfArgs a)
@@ -307,10 +310,8 @@ __global__ void k_sector_fit(SurfArgs a, const int* secN, const int* secCnt, int
 
 // nearest-neighbour walk over the initial surface positions within the
 // vertex's feature class (k_updateNearestNeighbor)
-__global__ void k_update_nn(SurfArgs a)
+__device__ void update_nn(const SurfArgs& a, int v)
 {
-    int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= a.nS) return;
     w3 p = WP(a.x, a.y, a.z, v);
     int vh = a.nn[v];
     w3 d0 = wsub(p, W(a.pinit + 3 * vh));
@@ -330,6 +331,11 @@ __global__ void k_update_nn(SurfArgs a)
     } while (vnew != vh);
     a.nn[v] = vnew;
 }
+__global__ void k_update_nn(SurfArgs a)
+{
+    const int v = blockIdx.x * blockDim.x + threadIdx.x;
+    if (v < a.nS) update_nn(a, v);
+}
 
 // ------------------------------------------------------------- projection
 // localSurfaceEstimationWithFeature: evaluate the nearest neighbour's quadric
@@ -340,6 +346,13 @@ __global__ void k_update_nn(SurfArgs a)
 // nearest neighbours' initial positions and the sector choice -- is the same
 // for all candidates of a search, so the searches stage it once in LDS
 // (Proj2 / Proj1) and blend from there.
+
+// position of surface vertex t at the start of the running colour pass
+__device__ __forceinline__ w3 pass_start(const SurfArgs& a, int t)
+{
+    const bool own = t >= a.cLo && t < a.cHi;   // its class is being searched
+    return WP(own ? a.sx : a.x, own ? a.sy : a.y, own ? a.sz : a.z, t);
+}
 
 // the surface a one-ring neighbour projects onto: the fit of its nearest
 // neighbour nn, or for a feature nn the sector fit of the halfedge of nn whose
@@ -352,7 +365,7 @@ __device__ LSurf neighbour_fit(const SurfArgs& a, int nn, w3 vidPos)
     float md = 3.40282347e+38f;
     int arg = 0, idx = 0;
     for (int h = a.heRow[nn]; h < a.heRow[nn + 1]; ++h, ++idx) {
-        w3 t = wsub(WP(a.sx, a.sy, a.sz, a.heTarget[h]), vidPos);
+        w3 t = wsub(pass_start(a, a.heTarget[h]), vidPos);
         float dd = wdot(t, t);
         if (dd < md) { md = dd; arg = idx; }
     }
@@ -903,11 +916,10 @@ __global__ __launch_bounds__(64) void k_search_feat1d(SurfArgs a, int cStart, in
 // for quads the diagonal d_i, the target of the halfedge after vid -> r_i in
 // its face); closed (r_n = r_0) unless open.  Returns false (uniformly) when
 // the vertex has no fan element.  dist: the largest distance from vid to the
-// r_i (and d_i).  The d_i come from the pass snapshot: on a surface boundary
+// r_i (and d_i).  The d_i are start-of-pass positions: on a surface boundary
 // the "diagonal" of the boundary halfedge is the boundary neighbour of the
 // next boundary vertex, which can be in the colour class being updated;
-// every other fan vertex shares an element with vid, so the snapshot holds
-// its current position.
+// every other fan vertex shares an element with vid, so it does not move.
 template <bool QUAD>
 __device__ bool stage_fan(const SurfArgs& a, int vid, bool open, w3* pts, FanScore<QUAD>& sc, float& dist)
 {
@@ -924,7 +936,7 @@ __device__ bool stage_fan(const SurfArgs& a, int vid, bool open, w3* pts, FanSco
         mx = wnorm(wsub(r, x0));
         if (QUAD) {
             const int nx = a.heNext[h];
-            const w3 dg = WP(a.sx, a.sy, a.sz, a.heTarget[nx >= 0 ? nx : h]);
+            const w3 dg = pass_start(a, a.heTarget[nx >= 0 ? nx : h]);
             pts[K * lane + 1] = dg;
             mx = fmaxf(mx, wnorm(wsub(dg, x0)));
         }
@@ -967,6 +979,20 @@ __global__ __launch_bounds__(64) void k_search_fan1d(SurfArgs a, int cStart, int
     surf1d_search(a, vid, WP(a.x, a.y, a.z, vid), dist, nq, sc);
 }
 
+// after a surface mesh's passes: the nearest-neighbour walk (the first nbS
+// blocks) and the face normals, both from the final positions
+__global__ __launch_bounds__(256) void k_nn_face_normals(SurfArgs a, int nbS)
+{
+    const int b = (int)blockIdx.x, t = (int)threadIdx.x;
+    if (b < nbS) {
+        const int v = b * 256 + t;
+        if (v < a.nS) update_nn(a, v);
+    } else {
+        const int f = (b - nbS) * 256 + t;
+        if (f < a.nFaces) face_normal(a, f);
+    }
+}
+
 // vertex normals from the current face normals (k_calcVertexNormals)
 __global__ void k_surf_vertex_normals(SurfArgs a)
 {
@@ -979,7 +1005,7 @@ __global__ void k_surf_vertex_normals(SurfArgs a)
     a.vnorm[3 * v] = n.x; a.vnorm[3 * v + 1] = n.y; a.vnorm[3 * v + 2] = n.z;
 }
 
-// positions snapshot at the start of a colour pass (one launch for x, y, z)
+// positions snapshot before the surface passes (one launch for x, y, z)
 __global__ void k_snapshot(const float* x, const float* y, const float* z, float* sx, float* sy, float* sz, int n)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1099,9 +1125,15 @@ void surf_nn_launch(const SurfArgs& a, hipStream_t s)
 {
     k_update_nn<<<nb256(a.nS), 256, 0, s>>>(a);
 }
+static SurfArgs of_class(const SurfArgs& a, int cStart, int cEnd)
+{
+    SurfArgs c = a;
+    c.cLo = cStart; c.cHi = cEnd;
+    return c;
+}
 void surf_search2d_launch(const SurfArgs& a, int cStart, int cEnd, int nq, int tet, size_t lds, hipStream_t s)
 {
-    if (cEnd > cStart) k_search_surf2d<<<cEnd - cStart, 64, lds, s>>>(a, cStart, nq, tet);
+    if (cEnd > cStart) k_search_surf2d<<<cEnd - cStart, 64, lds, s>>>(of_class(a, cStart, cEnd), cStart, nq, tet);
 }
 void surf_search1d_launch(const SurfArgs& a, int cStart, int cEnd, int nq, int tet, size_t lds, hipStream_t s)
 {
@@ -1119,18 +1151,21 @@ void surf_flat1d_launch(const SurfArgs& a, int cStart, int cEnd, int nq, hipStre
 void surf_fan2d_launch(const SurfArgs& a, int cStart, int cEnd, int nq, hipStream_t s)
 {
     if (cEnd <= cStart) return;
-    if (a.fpe == 4) launch_kernel(k_search_fan2d<true>, cEnd - cStart, 64, 0, s, a, cStart, nq);
-    else launch_kernel(k_search_fan2d<false>, cEnd - cStart, 64, 0, s, a, cStart, nq);
+    const SurfArgs c = of_class(a, cStart, cEnd);
+    if (a.fpe == 4) launch_kernel(k_search_fan2d<true>, cEnd - cStart, 64, 0, s, c, cStart, nq);
+    else launch_kernel(k_search_fan2d<false>, cEnd - cStart, 64, 0, s, c, cStart, nq);
 }
 void surf_fan1d_launch(const SurfArgs& a, int cStart, int cEnd, int nq, hipStream_t s)
 {
     if (cEnd <= cStart) return;
-    if (a.fpe == 4) launch_kernel(k_search_fan1d<true>, cEnd - cStart, 64, 0, s, a, cStart, nq);
-    else launch_kernel(k_search_fan1d<false>, cEnd - cStart, 64, 0, s, a, cStart, nq);
+    const SurfArgs c = of_class(a, cStart, cEnd);
+    if (a.fpe == 4) launch_kernel(k_search_fan1d<true>, cEnd - cStart, 64, 0, s, c, cStart, nq);
+    else launch_kernel(k_search_fan1d<false>, cEnd - cStart, 64, 0, s, c, cStart, nq);
 }
-void surf_normals_launch(const SurfArgs& a, hipStream_t s)
+void surf_nn_normals_launch(const SurfArgs& a, hipStream_t s)
 {
-    k_surf_face_normals<<<nb256(a.nFaces), 256, 0, s>>>(a);
+    const int nbS = nb256(a.nS);
+    k_nn_face_normals<<<nbS + nb256(a.nFaces), 256, 0, s>>>(a, nbS);
     k_surf_vertex_normals<<<nb256(a.nS), 256, 0, s>>>(a);
 }
 void snapshot_launch(const SurfArgs& a, hipStream_t s)
