@@ -21,35 +21,6 @@
 
 namespace vsdmo {
 
-__device__ __forceinline__ float lane_f(float v, int lane)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
-}
-// Reductions over the wave whose result is uniform (an SGPR): DPP operands
-// inside the rows of 16 lanes, two row broadcasts, lane 63 holds the result.  A
-// shuffle costs an LDS round trip per step, the compiler's DPP moves three
-// instructions (move, canonicalise, min); written out it is one.  A lane
-// without a source keeps its value; the s_nops are the two wait states between
-// a VALU write and a DPP read of the same register.
-#define VSDMO_WAVE_REDUCE(OP)                                                       \
-    asm("s_nop 1\n\t" OP " %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"    \
-        "s_nop 1\n\t" OP " %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf\n\t"    \
-        "s_nop 1\n\t" OP " %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf\n\t"    \
-        "s_nop 1\n\t" OP " %0, %0, %0 row_shr:8 row_mask:0xf bank_mask:0xf\n\t"    \
-        "s_nop 1\n\t" OP " %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t" \
-        "s_nop 1\n\t" OP " %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf"      \
-        : "+v"(v))
-__device__ __forceinline__ float wave_max_u(float v)
-{
-    VSDMO_WAVE_REDUCE("v_max_f32_dpp");
-    return lane_f(v, 63);
-}
-__device__ __forceinline__ float wave_min_u(float v)
-{
-    VSDMO_WAVE_REDUCE("v_min_f32_dpp");
-    return lane_f(v, 63);
-}
-#undef VSDMO_WAVE_REDUCE
 // LDS written by some lanes of the wave, read by others of the same wave: its
 // LDS operations complete in order, the fence keeps the compiler's order
 __device__ __forceinline__ void wave_lds_fence()
@@ -57,7 +28,6 @@ __device__ __forceinline__ void wave_lds_fence()
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
 }
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // ------------------------------------------------- the canonical selection
 // The canonical selection compares ratios det^2 / F^3 in FP32 products; it

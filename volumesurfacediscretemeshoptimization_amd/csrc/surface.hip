@@ -456,19 +456,19 @@ __device__ w3 blend1(const Src& s, float u)
 }
 
 // staged (LDS) sources
-struct Proj2 {
+struct alignas(16) Proj2 {
     LSurf L;
-    w3 q0;
-    int n;
-    w3 qn[kMaxNeigh];
     LSurf LN[kMaxNeigh];
+    float4 q[kMaxNeigh + 1];   // q0, then qn; w unused
+    int n;
 };
 struct Proj2Src {
     const Proj2* c;
+    __device__ w3 q(int i) const { const float4 t = c->q[i]; return { t.x, t.y, t.z }; }
     __device__ LSurf L() const { return c->L; }
-    __device__ w3 q0() const { return c->q0; }
+    __device__ w3 q0() const { return q(0); }
     __device__ int nh() const { return c->n; }
-    __device__ w3 qn(int i) const { return c->qn[i]; }
+    __device__ w3 qn(int i) const { return q(i + 1); }
     __device__ LSurf LN(int i) const { return c->LN[i]; }
 };
 struct Proj1 {
@@ -500,15 +500,74 @@ __device__ void stage_proj2(const SurfArgs& a, int vid, w3 vidPos, Proj2* c)
     if (lane == 0) {
         const int n0 = a.nn[vid];
         c->L = reinterpret_cast<const LSurf*>(a.ls)[n0];
-        c->q0 = W(a.pinit + 3 * n0);
+        const w3 q = W(a.pinit + 3 * n0);
+        c->q[0] = { q.x, q.y, q.z, 0.0f };
         c->n = nh;
     }
     if (lane < nh) {
         const int nn = a.nn[a.heTarget[h0 + lane]];
-        c->qn[lane] = W(a.pinit + 3 * nn);
+        const w3 q = W(a.pinit + 3 * nn);
+        c->q[lane + 1] = { q.x, q.y, q.z, 0.0f };
         c->LN[lane] = neighbour_fit(a, nn, vidPos);
     }
     __syncthreads();
+}
+
+// blend2 of the staged data, the same operations on the same values with two
+// savings: 1 / x by recip_rn, and each of the first kBlendRegs weights computed
+// once and kept for the second loop.  A position whose weights leave
+// recip_rn's range (or NaN) takes blend2 itself.  The searches are bound by
+// the issue of vector instructions: a triangle fan's vertex took 4,420, it
+// takes 2,630 with this and FanScore's ratios (sphere of 55k vertices, one
+// colour: 65.6 -> 41.0 us; quads of a 181^2 field 48.1 -> 35.3; the 2D passes
+// of a 13^3 tet cube 16.2 -> 13.9).  The empty asm keeps the compiler from
+// loading all neighbours' fits ahead of the levels (215 registers, and spills
+// under any bound: 113 us); as it is it takes 52.
+constexpr int kBlendRegs = 8;
+__device__ __forceinline__ w3 blend2_staged(const Proj2* c, float u, float v)
+{
+    const Proj2Src s{ c };
+    const int nh = uniform(c->n);
+    asm volatile("" ::: "memory");
+    const LSurf L = c->L;
+    const w3 pw = l2w(L, u, v, poly(L, u, v));
+    const auto weight = [&](int i) {
+        const w3 d = wsub(s.q(i), pw);
+        return recip_rn(wdot(d, d) + kSEps);
+    };
+    asm volatile("" ::: "memory");
+    const float w0 = weight(0);
+    float isum = w0, wmin = w0, w[kBlendRegs];
+#pragma unroll
+    for (int i = 0; i < kBlendRegs; ++i) {
+        if (i >= nh) break;
+        w[i] = weight(i + 1);
+        isum += w[i];
+        wmin = fminf(wmin, w[i]);
+    }
+    for (int i = kBlendRegs; i < nh; ++i) {
+        const float t = weight(i + 1);
+        isum += t;
+        wmin = fminf(wmin, t);
+    }
+    // every x below 2^100 (a NaN or an infinity among them makes isum NaN)
+    if (!(wmin > 0x1p-100f && isum < 0x1p100f)) return blend2(s, u, v);
+    const float ii = recip_rn(isum);
+    w3 sum = wadd(w3{ 0.0f, 0.0f, 0.0f }, wmul(ii, wmul(w0, pw)));
+    const auto term = [&](int i, float wi) {
+        const LSurf LN = c->LN[i];
+        const w3 q = wsub(pw, LN.p0);
+        const float lu = wdot(q, LN.e[0]), lv = wdot(q, LN.e[1]);
+        return wmul(ii, wmul(wi, l2w(LN, lu, lv, poly(LN, lu, lv))));
+    };
+#pragma unroll
+    for (int i = 0; i < kBlendRegs; ++i) {
+        if (i >= nh) break;
+        if (i % 2 == 0) asm volatile("" ::: "memory");
+        sum = wadd(sum, term(i, w[i]));
+    }
+    for (int i = kBlendRegs; i < nh; ++i) sum = wadd(sum, term(i, weight(i + 1)));
+    return sum;
 }
 
 // feature neighbours of vid that have exactly two feature neighbours
@@ -685,18 +744,6 @@ __device__ float ring_score(const RingFrame& f, bool tet, const void* lds, const
     return hex_acc_score(acc, f.epsD, f.epsF);
 }
 
-__device__ __forceinline__ void wave_argmax_s(float& best, int& idx)
-{
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-        float ob = __shfl_xor(best, m);
-        int oi = __shfl_xor(idx, m);
-        bool take = (ob > best) || (ob == best && oi < idx);
-        best = take ? ob : best;
-        idx = take ? oi : idx;
-    }
-}
-
 // ------------------------------------------------------------- search bodies
 // Scorers: score(p) is what the search maximises (one candidate per lane);
 // start(p0, qs, qref) gives the start position's score and the reference the
@@ -709,6 +756,8 @@ struct VolScore {
     const void* lds;
     HexAcc hacc;
     __device__ float score(w3 p) const { return ring_score(f, tet, lds, hacc, p); }
+    static constexpr int kLanes = 1;
+    __device__ float score_lanes(w3 p) const { return score(p); }
     // start score (maximised from) and the reference the last level must beat
     __device__ void start(w3 p, float& qs, float& qref) const { qs = score(p); qref = qs; }
 };
@@ -717,11 +766,20 @@ struct VolScore {
 // 30-50): triangles (p, r_k, r_k+1), quads (p, r_k, d_k, r_k+1); score()
 // signs each element by the nearest neighbour's vertex normal n, final_ref()
 // uses the unsigned metric
+template <int CTRL>
+__device__ __forceinline__ float lane_swap(float v)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
 template <bool QUAD>
 struct FanScore {
     const w3* pts;
+    // per element, what no candidate changes: triangles (r_k+1, |e2|^2);
+    // quads (e1, |e1|^2), (e2, |e2|^2), (r_k+1, -)
+    const float4* cst;
     int ne;
     w3 n;
+    bool unitN;   // |n| within 1 %, or 0
     __device__ float elem(w3 p, int k, bool oriented) const
     {
         const f3 nn = { n.x, n.y, n.z };
@@ -746,11 +804,93 @@ struct FanScore {
             mr_tri3_both(q, f3{ a.x, a.y, a.z }, f3{ b.x, b.y, b.z }, nn, qs, qu);
         }
     }
+    // the minimum over the fan.  The elements' qualities are first compared by
+    // ratios that need no square root, unit normal or division of their own
+    // (of exactly the values that the metric would use), and the metric's last
+    // steps are done once, for the smallest: rounding is monotonic, so its
+    // value is the minimum of the rounded ones.  Where an element's sign, the
+    // smallest element or the range of a value is not certain, the lane
+    // evaluates every element instead.  The metric spent 110 instructions on a
+    // triangle, 36 of them in the unit normal's divisions and 25 in the root
+    // and the quotient; this takes 42.
     __device__ float score(w3 p) const
     {
+        float r1 = 0x1p126f, r2 = 0x1p126f, sA = 0.0f, sB = 0.0f, sl = 1.0f;
+        bool unsure = !unitN, fail = false;
+        const w3 f = pts[0];
+        w3 e0 = wsub(f, p);
+        float d0 = wdot(e0, e0);
+        for (int k = 0; k < ne; ++k) {
+            float key, l, A, Bq = 0.0f;
+            if (QUAD) {
+                const float4 c1 = cst[3 * k], c2 = cst[3 * k + 1], c3 = cst[3 * k + 2];
+                const w3 e1 = { c1.x, c1.y, c1.z }, e2 = { c2.x, c2.y, c2.z };
+                const w3 g = wsub(w3{ c3.x, c3.y, c3.z }, p);   // -e3
+                const float d3 = wdot(g, g);
+                l = ((d0 + c1.w) + c2.w) + d3;
+                // e1 x -e0 and e3 x -e2
+                const w3 N1 = wcross(e0, e1), N2 = wcross(g, e2);
+                A = wdot(N1, N1);
+                Bq = wdot(N2, N2);
+                const float t1 = fdot(N1), t2 = fdot(N2);
+                // n . unit(N) against 0.7, both sides squared
+                const float lo = 0.49f * (1.0f - 0x1p-16f), hi = 0.49f * (1.0f + 0x1p-16f);
+                const bool f1 = t1 < 0.0f || t1 * t1 < lo * A, f2 = t2 < 0.0f || t2 * t2 < lo * Bq;
+                const bool ok1 = t1 > 0.0f && t1 * t1 > hi * A, ok2 = t2 > 0.0f && t2 * t2 > hi * Bq;
+                const bool inA = A > 0x1p-96f && A < 0x1p100f, inB = Bq > 0x1p-96f && Bq < 0x1p100f;
+                fail = fail || (inA && f1) || (inB && f2);
+                unsure = unsure || !(inA && inB && ok1 && ok2);
+                key = (__builtin_amdgcn_sqrtf(A) + __builtin_amdgcn_sqrtf(Bq)) * __builtin_amdgcn_rcpf(l);
+                unsure = unsure || !(key > 0x1p-60f);
+                e0 = g;
+                d0 = d3;
+            } else {
+                const float4 c = cst[k];
+                const w3 e1 = wsub(w3{ c.x, c.y, c.z }, p);
+                const float d1 = wdot(e1, e1);
+                l = (d0 + d1) + c.w;
+                const w3 N = wcross(e0, e1);
+                A = wdot(N, N);
+                const float t = fdot(N);
+                // both signs of n . unit(N) and of the rounded t agree beyond
+                // 8 ulp of |N| |n|
+                unsure = unsure || !(t * t > 0x1p-36f * A && A > 0x1p-96f);
+                key = A * __builtin_amdgcn_rcpf(l * l);
+                unsure = unsure || !(key > 0x1p-60f);
+                key = __builtin_copysignf(key, t);
+                e0 = e1;
+                d0 = d1;
+            }
+            r2 = __builtin_amdgcn_fmed3f(r1, r2, key);
+            const bool take = key < r1;
+            r1 = take ? key : r1;
+            sA = take ? A : sA;
+            if (QUAD) sB = take ? Bq : sB;
+            sl = take ? l : sl;
+        }
+        if (QUAD && unitN && fail) return -1.0f;
+        // the metric's roundings and the ratios' own stay below 2^-20 of the key
+        unsure = unsure || !(r2 - r1 > 0x1p-18f * (fabsf(r1) + fabsf(r2)));
+        if (!unsure) {
+            if (QUAD) return (2.0f * (sqrt_rn(sA) + sqrt_rn(sB))) / sl;
+            return (kTwoSqrt3 * __builtin_copysignf(sqrt_rn(sA), r1)) / sl;
+        }
         float q = FLT_MAX;
         for (int k = 0; k < ne; ++k) q = fminf(q, elem(p, k, true));
         return q;
+    }
+    __device__ __forceinline__ float fdot(w3 N) const { return fmaf(N.z, n.z, fmaf(N.y, n.y, N.x * n.x)); }
+    // the same minimum for a position that eight lanes hold, an element per
+    // lane: a 1D search has 8 candidates and left 56 lanes idle (sphere of 55k
+    // vertices, one colour: 16.6 -> 10.4 us)
+    static constexpr int kLanes = 8;
+    __device__ float score_lanes(w3 p) const
+    {
+        float q = FLT_MAX;
+        for (int k = threadIdx.x % kLanes; k < ne; k += kLanes) q = fminf(q, elem(p, k, true));
+        q = fminf(q, lane_swap<0xB1>(q));    // lane ^ 1
+        q = fminf(q, lane_swap<0x4E>(q));    // lane ^ 2
+        return fminf(q, lane_swap<0x141>(q));   // 7 - lane within each eight
     }
     // lane k < ne evaluates fan element k signed and unsigned; two wave
     // min-reductions (fminf is exact, so the order does not matter)
@@ -790,6 +930,8 @@ struct FlatScore {
         }
         return tri_acc_score(acc, is2);
     }
+    static constexpr int kLanes = 1;
+    __device__ float score_lanes(w3 p) const { return score(p); }
     __device__ void start(w3 p, float& qs, float& qref) const { qs = score(p); qref = qs; }
 };
 
@@ -803,7 +945,6 @@ __device__ void surf2d_search(const SurfArgs& a, int vid, w3 vidPos, float dist,
     const int lane = threadIdx.x;
     __shared__ Proj2 s_proj;
     stage_proj2(a, vid, vidPos, &s_proj);
-    const Proj2Src ps{ &s_proj };
     const LSurf L = s_proj.L;
     w3 cur = vidPos;
     const w3 cvec = wsub(cur, L.p0);
@@ -824,15 +965,16 @@ __device__ void surf2d_search(const SurfArgs& a, int vid, w3 vidPos, float dist,
         if (active) {
             u = cu + a.aff * ((float)ci * uMin + (float)(nq - 1 - ci) * uMax);
             v = cv + a.aff * ((float)cj * uMin + (float)(nq - 1 - cj) * uMax);
-            pc = blend2(ps, u, v);
+            pc = blend2_staged(&s_proj, u, v);
             best = sc.score(pc);
         }
-        int wl = lane;
-        wave_argmax_s(best, wl);
+        const float own = best;
+        best = wave_max_u(own);
         if (qcur < best) {
             // the winner's projected point (the projection of (bu, bv))
-            cu = __shfl(u, wl); cv = __shfl(v, wl);
-            cur = { __shfl(pc.x, wl), __shfl(pc.y, wl), __shfl(pc.z, wl) };
+            const int wl = __builtin_ctzll(__ballot(own == best));
+            cu = lane_f(u, wl); cv = lane_f(v, wl);
+            cur = { lane_f(pc.x, wl), lane_f(pc.y, wl), lane_f(pc.z, wl) };
             qcur = best;
         }
         qlast = best;
@@ -841,8 +983,8 @@ __device__ void surf2d_search(const SurfArgs& a, int vid, w3 vidPos, float dist,
     if (qold < qlast && lane == 0) { a.xw[vid] = cur.x; a.yw[vid] = cur.y; a.zw[vid] = cur.z; }
 }
 
-// 1D search along the feature curve: lane i < nq holds candidate i; the
-// curve projection blends the fits of the curve neighbours
+// 1D search along the feature curve: lanes S::kLanes * i and on hold candidate
+// i < nq; the curve projection blends the fits of the curve neighbours
 template <class S>
 __device__ void surf1d_search(const SurfArgs& a, int vid, w3 vidPos, float dist, int nq, const S& sc)
 {
@@ -857,22 +999,24 @@ __device__ void surf1d_search(const SurfArgs& a, int vid, w3 vidPos, float dist,
     float qcur, qold;
     sc.start(cur, qcur, qold);
     float qlast = -FLT_MAX;
-    const bool active = lane < nq;
+    const int ci = lane / S::kLanes;
+    const bool active = ci < nq;
     float ds = a.gridScale;
     for (int d = 0; d < a.depth; ++d) {
         const float uMax = ds * dist, uMin = -(ds * dist);
         float best = -FLT_MAX, u = 0.0f;
         w3 pc = { 0.0f, 0.0f, 0.0f };
         if (active) {
-            u = cu + a.aff * ((float)lane * uMin + (float)(nq - 1 - lane) * uMax);
+            u = cu + a.aff * ((float)ci * uMin + (float)(nq - 1 - ci) * uMax);
             pc = blend1(ps, u);
-            best = sc.score(pc);
+            best = sc.score_lanes(pc);
         }
-        int wl = lane;
-        wave_argmax_s(best, wl);
+        const float own = best;
+        best = wave_max_u(own);
         if (qcur < best) {
-            cu = __shfl(u, wl);
-            cur = { __shfl(pc.x, wl), __shfl(pc.y, wl), __shfl(pc.z, wl) };
+            const int wl = __builtin_ctzll(__ballot(own == best));
+            cu = lane_f(u, wl);
+            cur = { lane_f(pc.x, wl), lane_f(pc.y, wl), lane_f(pc.z, wl) };
             qcur = best;
         }
         qlast = best;
@@ -921,13 +1065,19 @@ __global__ __launch_bounds__(64) void k_search_feat1d(SurfArgs a, int cStart, in
 // next boundary vertex, which can be in the colour class being updated;
 // every other fan vertex shares an element with vid, so it does not move.
 template <bool QUAD>
-__device__ bool stage_fan(const SurfArgs& a, int vid, bool open, w3* pts, FanScore<QUAD>& sc, float& dist)
+struct FanLds {
+    float4 cst[(QUAD ? 3 : 1) * kMaxNeigh];
+    w3 pts[(QUAD ? 2 : 1) * kMaxNeigh + 1];
+};
+template <bool QUAD>
+__device__ bool stage_fan(const SurfArgs& a, int vid, bool open, FanLds<QUAD>& lds, FanScore<QUAD>& sc, float& dist)
 {
     const int lane = threadIdx.x;
     const int h0 = a.heRow[vid], n = a.heRow[vid + 1] - h0;
     if (n <= 0 || n > kMaxNeigh) return false;
     const w3 x0 = WP(a.x, a.y, a.z, vid);
     const int K = QUAD ? 2 : 1;
+    w3* pts = lds.pts;
     float mx = -FLT_MAX;
     if (lane < n) {
         const int h = h0 + lane;
@@ -942,13 +1092,28 @@ __device__ bool stage_fan(const SurfArgs& a, int vid, bool open, w3* pts, FanSco
         }
     }
     if (lane == 0 && !open) pts[K * n] = WP(a.x, a.y, a.z, a.heTarget[h0]);
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) mx = fmaxf(mx, __shfl_xor(mx, m));
     __syncthreads();
     sc.pts = pts;
+    sc.cst = lds.cst;
     sc.ne = open ? n - 1 : n;
     sc.n = W(a.vnorm + 3 * a.nn[vid]);
-    dist = mx;
+    const float nn = wdot(sc.n, sc.n);
+    sc.unitN = nn < 1.02f && (nn > 0.98f || nn == 0.0f);
+    dist = wave_max_u(mx);
+    if (lane < sc.ne) {
+        const w3 r = pts[K * (lane + 1)], a0 = pts[K * lane];
+        if (QUAD) {
+            const w3 dg = pts[2 * lane + 1];
+            const w3 e1 = wsub(dg, a0), e2 = wsub(r, dg);
+            lds.cst[3 * lane] = { e1.x, e1.y, e1.z, wdot(e1, e1) };
+            lds.cst[3 * lane + 1] = { e2.x, e2.y, e2.z, wdot(e2, e2) };
+            lds.cst[3 * lane + 2] = { r.x, r.y, r.z, 0.0f };
+        } else {
+            const w3 e2 = wsub(r, a0);
+            lds.cst[lane] = { r.x, r.y, r.z, wdot(e2, e2) };
+        }
+    }
+    __syncthreads();
     return sc.ne > 0;
 }
 
@@ -957,7 +1122,7 @@ __device__ bool stage_fan(const SurfArgs& a, int vid, bool open, w3* pts, FanSco
 template <bool QUAD>
 __global__ __launch_bounds__(64) void k_search_fan2d(SurfArgs a, int cStart, int nq)
 {
-    __shared__ w3 s_fan[2 * kMaxNeigh + 1];
+    __shared__ FanLds<QUAD> s_fan;
     const int vid = cStart + blockIdx.x;
     FanScore<QUAD> sc;
     float dist;
@@ -970,7 +1135,7 @@ __global__ __launch_bounds__(64) void k_search_fan2d(SurfArgs a, int cStart, int
 template <bool QUAD>
 __global__ __launch_bounds__(64) void k_search_fan1d(SurfArgs a, int cStart, int nq)
 {
-    __shared__ w3 s_fan[2 * kMaxNeigh + 1];
+    __shared__ FanLds<QUAD> s_fan;
     const int vid = cStart + blockIdx.x;
     if (!a.opt1d[vid]) return;   // uniform over the block
     FanScore<QUAD> sc;

@@ -65,6 +65,58 @@ __host__ __device__ inline float pow2_scale(float m)
     return bitsf((254u - e) << 23);
 }
 
+// ---------------------------------------------------------------- wave
+__device__ __forceinline__ float lane_f(float v, int lane)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+}
+// Reductions over the wave whose result is uniform (an SGPR): DPP operands
+// inside the rows of 16 lanes, two row broadcasts, lane 63 holds the result.  A
+// shuffle costs an LDS round trip per step, the compiler's DPP moves three
+// instructions (move, canonicalise, min); written out it is one.  A lane
+// without a source keeps its value; the s_nops are the two wait states between
+// a VALU write and a DPP read of the same register.
+#define VSDMO_WAVE_REDUCE(OP)                                                       \
+    asm("s_nop 1\n\t" OP " %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"    \
+        "s_nop 1\n\t" OP " %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf\n\t"    \
+        "s_nop 1\n\t" OP " %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf\n\t"    \
+        "s_nop 1\n\t" OP " %0, %0, %0 row_shr:8 row_mask:0xf bank_mask:0xf\n\t"    \
+        "s_nop 1\n\t" OP " %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t" \
+        "s_nop 1\n\t" OP " %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf"      \
+        : "+v"(v))
+__device__ __forceinline__ float wave_max_u(float v)
+{
+    VSDMO_WAVE_REDUCE("v_max_f32_dpp");
+    return lane_f(v, 63);
+}
+__device__ __forceinline__ float wave_min_u(float v)
+{
+    VSDMO_WAVE_REDUCE("v_min_f32_dpp");
+    return lane_f(v, 63);
+}
+#undef VSDMO_WAVE_REDUCE
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// ------------------------------------------- correctly rounded, fewer steps
+// 1 / x for x in [2^-126, 2^126): the hardware's reciprocal and one Newton
+// step in fused arithmetic (Markstein, IBM J. Res. Dev. 34, 1990), 3
+// instructions where the division takes 11.  Equal to 1.0f / x for every
+// mantissa at exponents across the range.
+__device__ __forceinline__ float recip_rn(float x)
+{
+    const float y = __builtin_amdgcn_rcpf(x);
+    return fmaf(fmaf(-x, y, 1.0f), y, y);
+}
+// sqrt(x) for x in [2^-96, 2^128): g = x * rsqrt(x), one step on the exact
+// residual x - g^2.  Equal to sqrtf(x) for every mantissa at exponents across
+// the range, both parities.
+__device__ __forceinline__ float sqrt_rn(float x)
+{
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float g = x * y;
+    return fmaf(fmaf(-g, g, x), 0.5f * y, g);
+}
+
 struct f3 { float x, y, z; };
 __device__ __forceinline__ f3 sub3(f3 a, f3 b) { return { a.x - b.x, a.y - b.y, a.z - b.z }; }
 __device__ __forceinline__ f3 add3(f3 a, f3 b) { return { a.x + b.x, a.y + b.y, a.z + b.z }; }
