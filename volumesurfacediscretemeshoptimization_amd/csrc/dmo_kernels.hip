@@ -21,14 +21,6 @@
 
 namespace vsdmo {
 
-// LDS written by some lanes of the wave, read by others of the same wave: its
-// LDS operations complete in order, the fence keeps the compiler's order
-__device__ __forceinline__ void wave_lds_fence()
-{
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // ------------------------------------------------- the canonical selection
 // The canonical selection compares ratios det^2 / F^3 in FP32 products; it
 // picks by the true ratios wherever they differ by more than its rounding, as

@@ -16,6 +16,7 @@
 #include <numeric>
 
 #include "vsdmo_internal.h"
+#include "vsdmo_numerics.h"
 
 namespace vsdmo {
 
@@ -134,6 +135,14 @@ static void scan_levels(const int* in, int* out, int n, int* sums, hipStream_t s
     k_scan_add<<<nblk(n), TB, 0, s>>>(out, sums, n);
 }
 
+// exclusive scan of n ints (out may alias in), the total left on the device
+void exclusive_scan_nototal(const int* in, int* out, int n, hipStream_t s)
+{
+    if (n <= 0) return;
+    scan_levels(in, out, n, build_slots(scan_sums_need(n)).sums, s);
+    VSDMO_HIP(hipGetLastError());
+}
+
 // exclusive scan of n ints (out may alias in); returns the total
 int exclusive_scan(const int* in, int* out, int n, hipStream_t s)
 {
@@ -147,45 +156,65 @@ int exclusive_scan(const int* in, int* out, int n, hipStream_t s)
 }
 
 // ------------------------------------------------------ counting-sort CSR
-__global__ void k_count_keys(const int* __restrict__ key, int n, int* __restrict__ cnt)
+// cnt[key]++, and the item's place among its key's (in any order): the counts'
+// scan plus that place is a slot of its own, without a second round of atomics
+__global__ void k_count_keys(const int* __restrict__ key, int n, int* __restrict__ cnt, int* __restrict__ place)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) atomicAdd(&cnt[key[i]], 1);
+    if (i < n) place[i] = atomicAdd(&cnt[key[i]], 1);
 }
 
-__global__ void k_scatter_keys(const int* __restrict__ key, int n, int* __restrict__ cursor, int* __restrict__ items)
+__global__ void k_scatter_keys(const int* __restrict__ key, const int* __restrict__ place, int n,
+                               const int* __restrict__ row, int* __restrict__ items)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) items[atomicAdd(&cursor[key[i]], 1)] = i;
+    if (i < n) items[row[key[i]] + place[i]] = i;
 }
 
-// sort each row's item indices ascending (restores the stable order)
-__global__ void k_sort_rows(const int* __restrict__ row, int nrows, int* __restrict__ items)
+__device__ __forceinline__ int lane_i(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+
+// sort each row's item indices ascending (restores the stable order): a wave
+// per row of up to 64 items, one on each lane, whose position is the number of
+// smaller ones.  (A thread per row sorted by insertion in memory, one load
+// after the other: 77 us for the 69k rows of 24 of a 40^3 tet cube, against
+// 18.)  Longer rows are sorted by insertion.
+__global__ __launch_bounds__(TB) void k_sort_rows(const int* __restrict__ row, int nrows, int* __restrict__ items)
 {
-    int r = blockIdx.x * blockDim.x + threadIdx.x;
+    const int r = blockIdx.x * (TB / 64) + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (r >= nrows) return;
-    int s = row[r], t = row[r + 1];
-    for (int i = s + 1; i < t; ++i) {
-        int x = items[i], j = i - 1;
-        while (j >= s && items[j] > x) { items[j + 1] = items[j]; --j; }
-        items[j + 1] = x;
+    const int s = uniform(row[r]), n = uniform(row[r + 1]) - s;
+    if (n <= 64) {
+        const int x = lane < n ? items[s + lane] : 0;
+        int rank = 0;
+        for (int j = 0; j < n; ++j) rank += lane_i(x, j) < x ? 1 : 0;
+        if (lane < n) items[s + rank] = x;
+    } else if (lane == 0) {
+        for (int i = s + 1; i < s + n; ++i) {
+            int x = items[i], j = i - 1;
+            while (j >= s && items[j] > x) { items[j + 1] = items[j]; --j; }
+            items[j + 1] = x;
+        }
     }
 }
 
-// stable CSR of items 0..n-1 grouped by key in [0,nk): row[nk+1], items[n]
-void stable_csr(const int* key, int n, int nk, DevBuf<int>& row, DevBuf<int>& items, hipStream_t s)
+// CSR of items 0..n-1 grouped by key in [0,nk): row[nk+1], items[n]; within a
+// row ascending if sorted, else in any order
+void group_csr(const int* key, int n, int nk, DevBuf<int>& row, DevBuf<int>& items, bool sorted, hipStream_t s)
 {
     row.alloc((size_t)nk + 1);
     items.alloc((size_t)std::max(n, 1));
+    DevBuf<int> place((size_t)std::max(n, 1));
     VSDMO_HIP(hipMemsetAsync(row.p, 0, sizeof(int) * ((size_t)nk + 1), s));
-    if (n > 0) k_count_keys<<<nblk(n), TB, 0, s>>>(key, n, row.p);
-    exclusive_scan(row.p, row.p, nk + 1, s);
-    DevBuf<int> cursor(nk > 0 ? nk : 1);
-    if (nk > 0) VSDMO_HIP(hipMemcpyAsync(cursor.p, row.p, sizeof(int) * nk, hipMemcpyDeviceToDevice, s));
-    if (n > 0) k_scatter_keys<<<nblk(n), TB, 0, s>>>(key, n, cursor.p, items.p);
-    if (nk > 0) k_sort_rows<<<nblk(nk), TB, 0, s>>>(row.p, nk, items.p);
+    if (n > 0) k_count_keys<<<nblk(n), TB, 0, s>>>(key, n, row.p, place.p);
+    exclusive_scan_nototal(row.p, row.p, nk + 1, s);
+    if (n > 0) k_scatter_keys<<<nblk(n), TB, 0, s>>>(key, place.p, n, row.p, items.p);
+    if (sorted && nk > 0) k_sort_rows<<<nblk((long long)nk * 64), TB, 0, s>>>(row.p, nk, items.p);
     VSDMO_HIP(hipGetLastError());
     VSDMO_HIP(hipStreamSynchronize(s));
+}
+void stable_csr(const int* key, int n, int nk, DevBuf<int>& row, DevBuf<int>& items, hipStream_t s)
+{
+    group_csr(key, n, nk, row, items, true, s);
 }
 
 // ------------------------------------------------------------ boundary faces
@@ -211,40 +240,81 @@ __global__ void k_emit_faces(const int* __restrict__ cells, int nE, int tet, int
     }
 }
 
-__device__ __forceinline__ bool face_less(const int* fk, int a, int b, int k)
+// a face's order in its bucket (same first vertex): (v1, v2[, v3], emit index);
+// v3 is 0 for triangles
+struct FaceKey { int v1, v2, v3, idx; };
+__device__ __forceinline__ FaceKey face_key(const int* fk, int item, int k)
 {
-    for (int i = 1; i < k; ++i) {
-        int x = fk[(size_t)a * 4 + i], y = fk[(size_t)b * 4 + i];
-        if (x != y) return x < y;
-    }
-    return a < b;
+    const int* a = fk + (size_t)item * 4;
+    return { a[1], a[2], k == 4 ? a[3] : 0, item };
+}
+__device__ __forceinline__ bool face_less(FaceKey a, FaceKey b)
+{
+    if (a.v1 != b.v1) return a.v1 < b.v1;
+    if (a.v2 != b.v2) return a.v2 < b.v2;
+    if (a.v3 != b.v3) return a.v3 < b.v3;
+    return a.idx < b.idx;
+}
+// b cancels a: (a,c,b) for (a,b,c) with b<c, (a,d,c,b) for (a,b,c,d) with b<d
+__device__ __forceinline__ bool face_cancels(FaceKey a, FaceKey b, int k)
+{
+    return k == 3 ? a.v1 < a.v2 && b.v1 == a.v2 && b.v2 == a.v1
+                  : a.v1 < a.v3 && b.v1 == a.v3 && b.v2 == a.v2 && b.v3 == a.v1;
 }
 
-// per bucket (same first vertex): sort by (v1, v2[, v3], emit index), then
-// cancel each (a,b,c) with b<c (quads (a,b,c,d) with b<d) against the first
-// (a,c,b) (quads (a,d,c,b)) after it (reference k_markDuplicateTris/Quads)
-__global__ void k_bucket_faces(const int* __restrict__ row, int nb, int* __restrict__ items,
-                               const int* __restrict__ fk, int k, uint8_t* __restrict__ dead)
+// per bucket (same first vertex): sort by (v1, v2[, v3], emit index) into
+// sorted, then cancel each face against the first of the opposite orientation
+// after it (reference k_markDuplicateTris/Quads).  Those of the opposite
+// orientation share one key beyond the emit index and sort after the face, so
+// the first is the one of the smallest emit index.  A wave per bucket, a face
+// on each lane: its position is the number of smaller ones, its match is found
+// in the same pass.  (A thread per bucket sorted by insertion, every comparison
+// a chain of loads: 323 us for the 69k buckets of 22 of a 40^3 tet cube,
+// against 98.)  Buckets of more than 64 faces read the others' keys from
+// memory, 64 faces at a time.
+__global__ __launch_bounds__(TB) void k_bucket_faces(const int* __restrict__ row, int nb,
+                                                     const int* __restrict__ items, const int* __restrict__ fk, int k,
+                                                     int* __restrict__ sorted, uint8_t* __restrict__ dead)
 {
-    int b = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ int s_dead[TB];
+    const int b = blockIdx.x * (TB / 64) + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (b >= nb) return;
-    int s = row[b], t = row[b + 1];
-    for (int i = s + 1; i < t; ++i) {
-        int x = items[i], j = i - 1;
-        while (j >= s && face_less(fk, x, items[j], k)) { items[j + 1] = items[j]; --j; }
-        items[j + 1] = x;
-    }
-    for (int i = s; i < t; ++i) dead[i] = 0;
-    for (int i = s; i < t; ++i) {
-        const int* a = fk + (size_t)items[i] * 4;
-        bool search = (k == 3) ? (a[1] < a[2]) : (a[1] < a[3]);
-        if (!search) continue;
-        for (int j = i + 1; j < t; ++j) {
-            const int* c = fk + (size_t)items[j] * 4;
-            bool match = (k == 3) ? (c[1] == a[2] && c[2] == a[1])
-                                  : (c[1] == a[3] && c[2] == a[2] && c[3] == a[1]);
-            if (match) { dead[i] = 1; dead[j] = 1; break; }
+    const int s = uniform(row[b]), n = uniform(row[b + 1]) - s;
+    if (n <= 64) {
+        int* const deadOf = s_dead + (threadIdx.x & ~63);
+        deadOf[lane] = 0;
+        const bool have = lane < n;
+        const FaceKey x = have ? face_key(fk, items[s + lane], k) : FaceKey{ 0, 0, 0, 0 };
+        int rank = 0, match = INT_MAX, at = 0;
+        for (int j = 0; j < n; ++j) {
+            const FaceKey y = { lane_i(x.v1, j), lane_i(x.v2, j), lane_i(x.v3, j), lane_i(x.idx, j) };
+            rank += face_less(y, x) ? 1 : 0;
+            if (face_cancels(x, y, k) && y.idx < match) { match = y.idx; at = j; }
         }
+        wave_lds_fence();
+        if (have && match != INT_MAX) { deadOf[lane] = 1; deadOf[at] = 1; }
+        wave_lds_fence();
+        if (have) { sorted[s + rank] = x.idx; dead[s + rank] = (uint8_t)deadOf[lane]; }
+        return;
+    }
+    for (int i = lane; i < n; i += 64) {
+        const FaceKey x = face_key(fk, items[s + i], k);
+        int rank = 0;
+        bool off = false;   // cancels a later face, or is the first to cancel an earlier one
+        for (int j = 0; j < n; ++j) {
+            const FaceKey y = face_key(fk, items[s + j], k);
+            rank += face_less(y, x) ? 1 : 0;
+            if (face_cancels(x, y, k)) off = true;
+            if (!off && face_cancels(y, x, k)) {
+                off = true;
+                for (int l = 0; l < n && off; ++l) {
+                    const FaceKey z = face_key(fk, items[s + l], k);
+                    off = !(face_cancels(y, z, k) && z.idx < x.idx);
+                }
+            }
+        }
+        sorted[s + rank] = x.idx;
+        dead[s + rank] = off ? 1 : 0;
     }
 }
 
@@ -449,67 +519,146 @@ __global__ void k_lower_fill(Incidence inc, int lo, int hi, const int* __restric
 }
 
 // The greedy first-fit colouring of k_color_greedy_round in one launch: each
-// vertex polls the colours of its lower neighbours until all are set, then
-// takes the smallest colour none of them uses.  A colour depends only on the
-// final colours of the lower neighbours, so the result is the sequential
-// greedy colouring.  A vertex waits only for lower vertices: those of its own
-// wave (the wave loops until all its lanes are done, so the lowest waiting
-// lane always finds its neighbours set) and those of lower workgroups, which
-// are dispatched before it.  The wait is bounded all the same: a vertex that
-// has polled spinLimit times stops uncoloured and raises *gaveUp, and the
-// round kernel completes the colouring with the same colours.  Colours are
-// loaded and stored at device scope, so that a poll sees a store made on
-// another XCD.
+// vertex waits for the colours of its lower neighbours, then takes the
+// smallest colour none of them uses.  A colour depends only on the final
+// colours of the lower neighbours, so the result is the sequential greedy
+// colouring.  A vertex waits only for lower vertices: those of its own wave
+// (the wave loops until all its lanes are done, so the lowest waiting lane
+// always finds its neighbours set), those of lower waves of its workgroup, and
+// those of lower workgroups, which are dispatched before it.  The wait is
+// bounded all the same: a vertex that has polled spinLimit times stops
+// uncoloured and raises *gaveUp, and the round kernel completes the colouring
+// with the same colours.
+// The chains of waiting vertices bound it (a mesh numbered along its rows
+// chains every vertex to the one before).  So a colour passes from lane to
+// lane within a wave, through LDS within the workgroup (256 vertices), and
+// only from workgroup to workgroup through memory, at device scope, ~2 us a
+// step, where every step used to take that way: 59k inner vertices of a 40^3
+// tet cube 884 us, 230 us now.
 __global__ __launch_bounds__(256) void k_color_greedy_sweep(const int* __restrict__ row, const int* __restrict__ val,
                                                            int n, int* __restrict__ col, int spinLimit,
                                                            int* __restrict__ gaveUp)
 {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ int s_col[256];   // colours of the workgroup's vertices, -1 until set
+    const int t = threadIdx.x, lane = t & 63, wave = uniform(t >> 6);
+    const int b0 = blockIdx.x * 256, v = b0 + t;
+    s_col[t] = -1;
+    __syncthreads();
+    const auto lds_colour = [&](int i) { return __hip_atomic_load(s_col + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+    const auto mem_colour = [&](int u) { return __hip_atomic_load(col + u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
     bool todo = v < n;
-    const int r1 = todo ? row[v + 1] : 0;
-    int k = todo ? row[v] : 0;        // lower neighbours [row[v], k) are coloured and in mask
-    uint64_t mask = 0;
-    bool big = false;
+    const int r0 = todo ? row[v] : 0, r1 = todo ? row[v + 1] : 0;
+    constexpr int B = 8;    // list entries read together (their latencies overlap)
+    constexpr int S = 12;   // lower neighbours in lower workgroups polled together
+    int k = r0, id[S] = {}; // entries [r0, k) are read; id[]: those polled
+    int pend = 0;           // the ids not yet coloured
+    uint64_t mask = 0;      // colours of the lower neighbours seen so far
+    bool big = false;       // one of them is 64 or more
+    uint64_t own = 0, low[3] = { 0, 0, 0 };   // waiting for: lanes of this wave, of the workgroup's lower waves
+    uint64_t passed = 0;                      // lanes of this wave whose colour has been passed on
     int polls = 0;
-    constexpr int B = 8;   // list entries loaded together (their latencies overlap)
+    const auto seen = [&](int c) { if (c < 64) mask |= 1ull << c; else big = true; };
     while (__ballot(todo) != 0) {
-        if (todo) {
-            bool blocked = false;
-            while (k < r1 && !blocked) {
-                int id[B], cu[B];
-                // entries past the list re-read its last one (k < r1), so every
-                // load is unconditional and in bounds; their values are ignored
+        // lower workgroups: up to S distinct ids, read ahead of the wait (the
+        // list, which names a neighbour once per shared element, takes several
+        // loads one after the other) and polled together
+        while (todo && (pend != 0 || k < r1)) {
+            if (pend == 0) {
+                int cnt = 0;
+                while (k < r1 && cnt < S) {
+                    int e[B], used = 0;
+                    // entries past the list re-read its last one (k < r1), so every
+                    // load is unconditional and in bounds; their values are ignored
 #pragma unroll
-                for (int j = 0; j < B; ++j) id[j] = val[min(k + j, r1 - 1)];
+                    for (int j = 0; j < B; ++j) e[j] = val[min(k + j, r1 - 1)];
 #pragma unroll
-                for (int j = 0; j < B; ++j) cu[j] = __hip_atomic_load(col + id[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                int done = 0;   // entries taken in order before the first uncoloured one
+                    for (int j = 0; j < B; ++j) {
+                        if (k + j >= r1 || cnt == S) continue;
+                        ++used;
+                        const int i = e[j] - b0;
+                        if (i < 0) {
+                            bool known = false;
 #pragma unroll
-                for (int j = 0; j < B; ++j) {
-                    if (blocked || k + j >= r1) continue;
-                    if (cu[j] < 0) { blocked = true; continue; }
-                    if (cu[j] < 64) mask |= 1ull << cu[j]; else big = true;
-                    ++done;
+                            for (int q = 0; q < S; ++q) known = known || (q < cnt && id[q] == e[j]);
+                            if (known) continue;
+#pragma unroll
+                            for (int q = 0; q < S; ++q) id[q] = q == cnt ? e[j] : id[q];
+                            ++cnt;
+                            continue;
+                        }
+                        const uint64_t bit = 1ull << (i & 63);
+                        if ((i >> 6) == wave) own |= bit;
+                        else if ((i >> 6) == 0) low[0] |= bit;
+                        else if ((i >> 6) == 1) low[1] |= bit;
+                        else low[2] |= bit;
+                    }
+                    k += used;
                 }
-                k += done;
+                pend = (1 << cnt) - 1;
+#pragma unroll
+                for (int q = 0; q < S; ++q) id[q] = q < cnt ? id[q] : v;   // loads stay in bounds
             }
-            if (k == r1) {
-                int cc = (~mask == 0ull) ? 64 : __builtin_ctzll(~mask);
+            if (pend != 0) {
+                int cu[S];
+#pragma unroll
+                for (int q = 0; q < S; ++q) cu[q] = mem_colour(id[q]);
+#pragma unroll
+                for (int q = 0; q < S; ++q)
+                    if ((pend >> q & 1) && cu[q] >= 0) { seen(cu[q]); pend &= ~(1 << q); }
+                if (pend != 0) break;
+            }
+        }
+        // the workgroup's lower waves
+#pragma unroll
+        for (int w = 0; w < 3; ++w) {
+            uint64_t rest = todo ? low[w] : 0;
+            while (rest) {
+                const int i = __builtin_ctzll(rest);
+                rest &= rest - 1;
+                const int c = lds_colour(w * 64 + i);
+                if (c < 0) break;
+                seen(c);
+                low[w] &= ~(1ull << i);
+            }
+        }
+        // lanes of this wave that passed their colour on before this lane read
+        // its list that far
+        for (uint64_t rest = todo ? own & passed : 0; rest; rest &= rest - 1) seen(lds_colour(wave * 64 + __builtin_ctzll(rest)));
+        own &= ~passed;
+        // this wave: lanes that are ready take their colour and pass it on, until none is
+        for (;;) {
+            const bool ready = todo && pend == 0 && k == r1 && (low[0] | low[1] | low[2] | own) == 0;
+            uint64_t done = __ballot(ready);
+            if (done == 0) break;
+            passed |= done;
+            int cc = 0;
+            if (ready) {
+                cc = (~mask == 0ull) ? 64 : __builtin_ctzll(~mask);
                 if (big && cc == 64) {
                     // more than 64 colours around v: linear mex search
                     for (;; ++cc) {
                         bool used = false;
-                        for (int j = row[v]; j < r1 && !used; ++j)
-                            used = __hip_atomic_load(col + val[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == cc;
+                        for (int j = r0; j < r1 && !used; ++j)
+                            used = (val[j] >= b0 ? lds_colour(val[j] - b0) : mem_colour(val[j])) == cc;
                         if (!used) break;
                     }
                 }
+                __hip_atomic_store(s_col + t, cc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 __hip_atomic_store(col + v, cc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 todo = false;
-            } else if (++polls >= spinLimit) {
-                __hip_atomic_store(gaveUp, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                todo = false;
             }
+            while (done) {
+                const int l = __builtin_ctzll(done);
+                done &= done - 1;
+                const int c = lane_i(cc, l);
+                if (own >> l & 1) { seen(c); own &= ~(1ull << l); }
+            }
+        }
+        // a poll of memory counts as 16 of LDS, which are that much shorter
+        polls += pend != 0 ? 16 : 1;
+        if (todo && (polls >> 4) >= spinLimit) {
+            __hip_atomic_store(gaveUp, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            todo = false;
         }
         __builtin_amdgcn_s_sleep(1);
     }
@@ -682,7 +831,7 @@ std::vector<int> colour_and_sort(vsdmo_mesh& m, Renumber& rn, const int* incRow,
         DevBuf<int> lval((size_t)std::max(tot, 1));
         k_lower_fill<<<nblk(n), TB, 0, s>>>(inc, lo, hi, lrow.p, lval.p);
         VSDMO_HIP(hipMemsetAsync(gave.p, 0, sizeof(int), s));
-        k_color_greedy_sweep<<<nblk(n), TB, 0, s>>>(lrow.p, lval.p, n, col.p, polls, gave.p);
+        k_color_greedy_sweep<<<nblk(n), TB, 0, s>>>(lrow.p, lval.p, n, col.p, std::min(polls, 1 << 26), gave.p);
         VSDMO_HIP(hipGetLastError());
         h_left = read_int(gave.p, s);
     }
@@ -794,11 +943,11 @@ void build_volume(vsdmo_mesh& m, const vsdmo_mesh_params& prm)
     {
         int nf = tet ? 4 : 6, k = tet ? 3 : 4;
         int n = nE * nf;
-        DevBuf<int> fk((size_t)n * 4), v0(n), row, items, pos(n), alive(n);
+        DevBuf<int> fk((size_t)n * 4), v0(n), row, any, items(n), pos(n), alive(n);
         DevBuf<uint8_t> dead(n);
         k_emit_faces<<<nblk(nE), TB, 0, s>>>(m.cells.p, nE, tet, fk.p, v0.p);
-        stable_csr(v0.p, n, nV, row, items, s);
-        k_bucket_faces<<<nblk(nV), TB, 0, s>>>(row.p, nV, items.p, fk.p, k, dead.p);
+        group_csr(v0.p, n, nV, row, any, false, s);
+        k_bucket_faces<<<nblk((long long)nV * 64), TB, 0, s>>>(row.p, nV, any.p, fk.p, k, items.p, dead.p);
         k_alive<<<nblk(n), TB, 0, s>>>(dead.p, n, alive.p);
         int nb = exclusive_scan(alive.p, pos.p, n, s);
         m.fpe = k;

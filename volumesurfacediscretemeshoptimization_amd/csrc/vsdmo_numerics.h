@@ -95,6 +95,13 @@ __device__ __forceinline__ float wave_min_u(float v)
     return lane_f(v, 63);
 }
 #undef VSDMO_WAVE_REDUCE
+// LDS written by some lanes of the wave, read by others of the same wave: its
+// LDS operations complete in order, the fence keeps the compiler's order
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // ------------------------------------------- correctly rounded, fewer steps
