@@ -17,6 +17,8 @@
 #include "vsdmo_internal.h"
 
 namespace vsdmo {
+// positions from xyz (nV x 3, host), colours 0, identity numbering; true if every z is 0
+bool init_mesh(vsdmo_mesh& m, const float* xyz);
 void build_volume(vsdmo_mesh& m, const vsdmo_mesh_params& prm);
 void build_surface_mesh(vsdmo_mesh& m, const vsdmo_mesh_params& prm);
 void check_classes(const vsdmo_mesh& m, const std::vector<int>& off);
@@ -66,6 +68,37 @@ static vsdmo_status copy_dev(const DevBuf<T>& b, size_t n, T* out, hipStream_t s
         VSDMO_HIP(hipStreamSynchronize(s));
         return VSDMO_OK;
     });
+}
+
+// every index in [0, nV)
+static bool indices_in_range(const int32_t* cells, long long n, int32_t nV)
+{
+    uint32_t top = 0;
+    for (long long i = 0; i < n; ++i) top = std::max(top, (uint32_t)cells[i]);
+    return top < (uint32_t)nV;
+}
+
+// the first element with a repeated vertex, -1 if there is none: groups of
+// elements without a branch per pair, the group that has one again by element
+template <int NPE>
+static long long first_repeat(const int32_t* cells, long long nCells)
+{
+    const auto repeats = [&](long long e) {
+        const int32_t* c = cells + e * NPE;
+        int r = 0;
+        for (int a = 0; a < NPE; ++a)
+            for (int b = a + 1; b < NPE; ++b) r |= c[a] == c[b];
+        return r;
+    };
+    constexpr long long G = 512;
+    for (long long e0 = 0; e0 < nCells; e0 += G) {
+        const long long e1 = std::min(e0 + G, nCells);
+        int any = 0;
+        for (long long e = e0; e < e1; ++e) any |= repeats(e);
+        for (long long e = e0; any && e < e1; ++e)
+            if (repeats(e)) return e;
+    }
+    return -1;
 }
 
 static void destroy_mesh(vsdmo_mesh* m)
@@ -185,13 +218,10 @@ vsdmo_status vsdmo_mesh_create(vsdmo_elem type, const float* xyz, int32_t nV, co
         const bool surfaceMesh = (type == VSDMO_TRI || type == VSDMO_QUAD);
         long long nci = (long long)nCells * npe;
         if (nci > (long long)0x7fffffff / 2) return fail(VSDMO_INVALID_ARG, "mesh too large for int32 indexing");
-        for (long long i = 0; i < nci; ++i)
-            if (cells[i] < 0 || cells[i] >= nV) return fail(VSDMO_INVALID_ARG, "element vertex index out of range");
-        for (long long e = 0; e < nCells; ++e)
-            for (int a = 0; a < npe; ++a)
-                for (int b = a + 1; b < npe; ++b)
-                    if (cells[e * npe + a] == cells[e * npe + b])
-                        return fail(VSDMO_INVALID_ARG, "element with repeated vertex " + std::to_string(e));
+        if (!indices_in_range(cells, nci, nV)) return fail(VSDMO_INVALID_ARG, "element vertex index out of range");
+        const long long rep = npe == 3 ? first_repeat<3>(cells, nCells)
+                            : npe == 4 ? first_repeat<4>(cells, nCells) : first_repeat<8>(cells, nCells);
+        if (rep >= 0) return fail(VSDMO_INVALID_ARG, "element with repeated vertex " + std::to_string(rep));
         vsdmo_mesh_params prm;
         vsdmo_mesh_params_default(&prm);
         if (params) prm = *params;
@@ -204,26 +234,12 @@ vsdmo_status vsdmo_mesh_create(vsdmo_elem type, const float* xyz, int32_t nV, co
             m->elem = type; m->npe = npe; m->nV = nV; m->nE = nCells;
             VSDMO_HIP(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
             hipStream_t s = m->stream;
-            std::vector<float> hx(nV), hy(nV), hz(nV);
-            int flat = 1;
-            for (int i = 0; i < nV; ++i) {
-                hx[i] = xyz[3 * i]; hy[i] = xyz[3 * i + 1]; hz[i] = xyz[3 * i + 2];
-                if (hz[i] != 0.0f) flat = 0;
-            }
-            m->flat = surfaceMesh ? flat : 0;
             m->x.alloc(nV); m->y.alloc(nV); m->z.alloc(nV);
-            m->x.upload(hx.data(), nV, s); m->y.upload(hy.data(), nV, s); m->z.upload(hz.data(), nV, s);
             m->cells.alloc(nci);
             m->cells.upload(cells, nci, s);
             m->colorOf.alloc(nV);
-            VSDMO_HIP(hipMemsetAsync(m->colorOf.p, 0, sizeof(int) * nV, s));
             m->newOfOld.alloc(nV);
-            {
-                std::vector<int> id(nV);
-                for (int i = 0; i < nV; ++i) id[i] = i;
-                m->newOfOld.upload(id.data(), nV, s);
-                VSDMO_HIP(hipStreamSynchronize(s));
-            }
+            m->flat = init_mesh(*m, xyz) && surfaceMesh;
             if (surfaceMesh) build_surface_mesh(*m, prm);
             else build_volume(*m, prm);
             m->new_of_old = m->newOfOld.to_host(s);

@@ -96,14 +96,15 @@ static BuildSlots& build_slots(size_t sumsNeed = 0)
     return b;
 }
 
-// one int of device memory, read back through the pinned slot
-int read_int(const int* d, hipStream_t s)
+// n <= kSlots ints of device memory, read back through the pinned slots
+const int* read_ints(const int* d, int n, hipStream_t s)
 {
     BuildSlots& b = build_slots();
-    VSDMO_HIP(hipMemcpyAsync(b.host, d, sizeof(int), hipMemcpyDeviceToHost, s));
+    VSDMO_HIP(hipMemcpyAsync(b.host, d, n * sizeof(int), hipMemcpyDeviceToHost, s));
     VSDMO_HIP(hipStreamSynchronize(s));
-    return b.host[0];
+    return b.host;
 }
+int read_int(const int* d, hipStream_t s) { return read_ints(d, 1, s)[0]; }
 
 __global__ void k_copy_int(const int* __restrict__ src, int* __restrict__ dst) { *dst = *src; }
 __global__ void k_scan_total(const int* __restrict__ out, int n, const int* __restrict__ last, int* __restrict__ total)
@@ -199,22 +200,22 @@ __global__ __launch_bounds__(TB) void k_sort_rows(const int* __restrict__ row, i
 
 // CSR of items 0..n-1 grouped by key in [0,nk): row[nk+1], items[n]; within a
 // row ascending if sorted, else in any order
-void group_csr(const int* key, int n, int nk, DevBuf<int>& row, DevBuf<int>& items, bool sorted, hipStream_t s)
+void group_csr(BuildArena& ar, const int* key, int n, int nk, DevBuf<int>& row, DevBuf<int>& items, bool sorted,
+               hipStream_t s)
 {
     row.alloc((size_t)nk + 1);
     items.alloc((size_t)std::max(n, 1));
-    DevBuf<int> place((size_t)std::max(n, 1));
+    DevBuf<int> place(ar, (size_t)std::max(n, 1));
     VSDMO_HIP(hipMemsetAsync(row.p, 0, sizeof(int) * ((size_t)nk + 1), s));
     if (n > 0) k_count_keys<<<nblk(n), TB, 0, s>>>(key, n, row.p, place.p);
     exclusive_scan_nototal(row.p, row.p, nk + 1, s);
     if (n > 0) k_scatter_keys<<<nblk(n), TB, 0, s>>>(key, place.p, n, row.p, items.p);
     if (sorted && nk > 0) k_sort_rows<<<nblk((long long)nk * 64), TB, 0, s>>>(row.p, nk, items.p);
     VSDMO_HIP(hipGetLastError());
-    VSDMO_HIP(hipStreamSynchronize(s));
 }
-void stable_csr(const int* key, int n, int nk, DevBuf<int>& row, DevBuf<int>& items, hipStream_t s)
+void stable_csr(BuildArena& ar, const int* key, int n, int nk, DevBuf<int>& row, DevBuf<int>& items, hipStream_t s)
 {
-    group_csr(key, n, nk, row, items, true, s);
+    group_csr(ar, key, n, nk, row, items, true, s);
 }
 
 // ------------------------------------------------------------ boundary faces
@@ -354,71 +355,79 @@ __global__ void k_partition_ids(const int* __restrict__ flag, const int* __restr
     newid[v] = first ? before : nFirst + (v - before);
 }
 
-__global__ void k_permute_f(const int* __restrict__ newid, int n, const float* __restrict__ a, float* __restrict__ b)
+// One renumbering in one launch: positions and the optional per-vertex arrays
+// go to their spare copies, element and face ids are remapped in place, the
+// composed renumbering and its inverse updated.  (Ten launches of 2-6 us, a
+// gap before each.)
+struct RenumberArgs {
+    const int* newid;
+    int nV, n8;                       // vertices; of them with u8 data (the first n8)
+    long long nc, nf;
+    const float* x; const float* y; const float* z;
+    float* tx; float* ty; float* tz;
+    int* cells; int* faces;
+    int* newOfOld; int* oldOfCur;
+    const uint8_t* a8[2]; uint8_t* t8[2];
+    const int* a32; int* t32;
+};
+__global__ void k_renumber(RenumberArgs r)
 {
-    int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v < n) b[newid[v]] = a[v];
-}
-__global__ void k_permute_i(const int* __restrict__ newid, int n, const int* __restrict__ a, int* __restrict__ b)
-{
-    int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v < n) b[newid[v]] = a[v];
-}
-__global__ void k_permute_u8(const int* __restrict__ newid, int n, const uint8_t* __restrict__ a, uint8_t* __restrict__ b)
-{
-    int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v < n) b[newid[v]] = a[v];
-}
-__global__ void k_remap(int* __restrict__ ids, long long n, const int* __restrict__ newid)
-{
-    long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) ids[i] = newid[ids[i]];
-}
-__global__ void k_invert(const int* __restrict__ newOfOld, int n, int* __restrict__ oldOfNew)
-{
-    int o = blockIdx.x * blockDim.x + threadIdx.x;
-    if (o < n) oldOfNew[newOfOld[o]] = o;
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < r.nc) r.cells[i] = r.newid[r.cells[i]];
+    if (i < r.nf) r.faces[i] = r.newid[r.faces[i]];
+    if (i >= r.nV) return;
+    const int w = r.newid[i];
+    r.tx[w] = r.x[i]; r.ty[w] = r.y[i]; r.tz[w] = r.z[i];
+    if (r.a32) r.t32[w] = r.a32[i];
+    if (i < r.n8) { r.t8[0][w] = r.a8[0][i]; r.t8[1][w] = r.a8[1][i]; }
+    const int o = r.newid[r.newOfOld[i]];
+    r.newOfOld[i] = o;
+    r.oldOfCur[o] = (int)i;
 }
 
 // Applies newid (a permutation of all nV current ids) to positions, elements,
 // faces, the composed renumbering and optional per-vertex arrays.
 struct Renumber {
     vsdmo_mesh& m;
+    BuildArena& ar;
     DevBuf<int> oldOfCur;   // current id -> input id
-    explicit Renumber(vsdmo_mesh& mesh) : m(mesh) {}
-
-    void apply(const int* newid, std::vector<DevBuf<uint8_t>*> u8 = {}, std::vector<DevBuf<int>*> i32 = {})
+    // the arrays that the mesh's change places with
+    DevBuf<float> tx, ty, tz;
+    DevBuf<uint8_t> t8[2];
+    DevBuf<int> t32;
+    Renumber(vsdmo_mesh& mesh, BuildArena& arena) : m(mesh), ar(arena), oldOfCur(arena, mesh.nV)
     {
-        hipStream_t s = m.stream;
-        int n = m.nV;
-        DevBuf<float> t(n);
-        k_permute_f<<<nblk(n), TB, 0, s>>>(newid, n, m.x.p, t.p);
-        std::swap(m.x, t);
-        k_permute_f<<<nblk(n), TB, 0, s>>>(newid, n, m.y.p, t.p);
-        std::swap(m.y, t);
-        k_permute_f<<<nblk(n), TB, 0, s>>>(newid, n, m.z.p, t.p);
-        std::swap(m.z, t);
-        long long nc = (long long)m.nE * m.npe;
-        k_remap<<<nblk(nc), TB, 0, s>>>(m.cells.p, nc, newid);
-        long long nf = (long long)m.nFaces * m.fpe;
-        if (nf > 0 && m.faces.p != m.cells.p) k_remap<<<nblk(nf), TB, 0, s>>>(m.faces.p, nf, newid);
-        k_remap<<<nblk(n), TB, 0, s>>>(m.newOfOld.p, n, newid);
-        for (auto* b : u8) {
-            DevBuf<uint8_t> tb(b->n);
-            int nn = (int)b->n;
-            k_permute_u8<<<nblk(nn), TB, 0, s>>>(newid, nn, b->p, tb.p);
-            std::swap(*b, tb);
+        tx.alloc(m.nV); ty.alloc(m.nV); tz.alloc(m.nV); t32.alloc(m.nV);
+    }
+
+    void apply(const int* newid, bool flags = false, bool colours = false)
+    {
+        RenumberArgs r{};
+        r.newid = newid;
+        r.nV = m.nV;
+        r.nc = (long long)m.nE * m.npe;
+        r.nf = (m.faces.p != m.cells.p) ? (long long)m.nFaces * m.fpe : 0;
+        r.x = m.x.p; r.y = m.y.p; r.z = m.z.p;
+        r.tx = tx.p; r.ty = ty.p; r.tz = tz.p;
+        r.cells = m.cells.p; r.faces = m.faces.p;
+        r.newOfOld = m.newOfOld.p; r.oldOfCur = oldOfCur.p;
+        if (flags) {
+            DevBuf<uint8_t>* a[2] = { &m.isB1D, &m.isFeature };
+            r.n8 = (int)m.isB1D.n;
+            for (int i = 0; i < 2; ++i) {
+                if (t8[i].n != a[i]->n) t8[i].alloc(a[i]->n);
+                r.a8[i] = a[i]->p; r.t8[i] = t8[i].p;
+            }
         }
-        for (auto* b : i32) {
-            DevBuf<int> tb(b->n);
-            int nn = (int)b->n;
-            k_permute_i<<<nblk(nn), TB, 0, s>>>(newid, nn, b->p, tb.p);
-            std::swap(*b, tb);
-        }
-        oldOfCur.alloc(n);
-        k_invert<<<nblk(n), TB, 0, s>>>(m.newOfOld.p, n, oldOfCur.p);
+        if (colours) { r.a32 = m.colorOf.p; r.t32 = t32.p; }
+        const long long n = std::max({ (long long)m.nV, r.nc, r.nf });
+        k_renumber<<<nblk(n), TB, 0, m.stream>>>(r);
         VSDMO_HIP(hipGetLastError());
-        VSDMO_HIP(hipStreamSynchronize(s));
+        std::swap(m.x, tx);
+        std::swap(m.y, ty);
+        std::swap(m.z, tz);
+        if (flags) { std::swap(m.isB1D, t8[0]); std::swap(m.isFeature, t8[1]); }
+        if (colours) std::swap(m.colorOf, t32);
     }
 };
 
@@ -730,12 +739,14 @@ __global__ __launch_bounds__(TB) void k_colour_place(const int* __restrict__ col
     newid[lo + i] = lo + pos[(size_t)c * nb + blockIdx.x] + r;
 }
 
-// first position of each colour: off[c] = pos[c * nb]
-__global__ void k_colour_offsets(const int* __restrict__ pos, int nb, int nc, int* __restrict__ off)
+// first vertex of each colour, off[c] = lo + pos[c * nb], and the end of the last
+__global__ void k_colour_offsets(const int* __restrict__ pos, int nb, int nc, int lo, int n, int* __restrict__ off)
 {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < nc) off[c] = pos[(size_t)c * nb];
+    if (c <= nc) off[c] = lo + (c < nc ? pos[(size_t)c * nb] : n);
 }
+
+__global__ void k_fill_int(int* p, int v) { *p = v; }
 
 __global__ void k_iota(int* __restrict__ a, int n)
 {
@@ -778,22 +789,42 @@ __global__ void k_check_classes(const int* __restrict__ cells, int nE, int npe, 
     }
 }
 
+// the partitions' verdicts, read together with the last of the build's values
+struct ClassChecks {
+    DevBuf<int> bad;   // per partition: the lowest class with two vertices of one element, INT_MAX if none
+    std::vector<std::vector<int>> off;
+    explicit ClassChecks(BuildArena& ar) : bad(ar, kMax) {}
+    static constexpr int kMax = 3;
+    void add(const vsdmo_mesh& m, const int* doff, const std::vector<int>& o)
+    {
+        const int i = (int)off.size(), nc = (int)o.size() - 1;
+        off.push_back(o);
+        k_fill_int<<<1, 1, 0, m.stream>>>(bad.p + i, INT_MAX);
+        if (nc > 0 && m.nE > 0) k_check_classes<<<nblk(m.nE), TB, 0, m.stream>>>(m.cells.p, m.nE, m.npe, doff, nc, bad.p + i);
+        VSDMO_HIP(hipGetLastError());
+    }
+    void verify(hipStream_t s) const
+    {
+        if (off.empty()) return;
+        const int* h = read_ints(bad.p, (int)off.size(), s);
+        for (size_t i = 0; i < off.size(); ++i)
+            if (h[i] != INT_MAX)
+                throw StatusError{ VSDMO_TOPOLOGY, "colour class " + std::to_string(h[i]) + " (vertices " +
+                                                       std::to_string(off[i][h[i]]) + ".." +
+                                                       std::to_string(off[i][h[i] + 1] - 1) +
+                                                       ") holds two vertices of one element" };
+    }
+};
+
+// a partition given by the caller
 void check_classes(const vsdmo_mesh& m, const std::vector<int>& off)
 {
-    const int nc = (int)off.size() - 1;
-    if (nc <= 0 || m.nE == 0) return;
-    hipStream_t s = m.stream;
-    DevBuf<int> doff(off.size()), bad(1);
-    doff.upload(off.data(), off.size(), s);
-    const int none = INT_MAX;
-    bad.upload(&none, 1, s);
-    k_check_classes<<<nblk(m.nE), TB, 0, s>>>(m.cells.p, m.nE, m.npe, doff.p, nc, bad.p);
-    VSDMO_HIP(hipGetLastError());
-    const int h = read_int(bad.p, s);
-    if (h != none)
-        throw StatusError{ VSDMO_TOPOLOGY, "colour class " + std::to_string(h) + " (vertices " +
-                                               std::to_string(off[h]) + ".." + std::to_string(off[h + 1] - 1) +
-                                               ") holds two vertices of one element" };
+    BuildArena ar(sizeof(int) * off.size() + 4096, m.stream);
+    DevBuf<int> doff(ar, off.size());
+    ClassChecks checks(ar);
+    doff.upload(off.data(), off.size(), m.stream);
+    checks.add(m, doff.p, off);
+    checks.verify(m.stream);
 }
 
 // colour [lo,hi) of the current numbering and sort it stably by colour.
@@ -803,9 +834,10 @@ void check_classes(const vsdmo_mesh& m, const std::vector<int>& off)
 // the meshes here need a few hundred)
 constexpr int kSweepPolls = 1 << 16;
 
-std::vector<int> colour_and_sort(vsdmo_mesh& m, Renumber& rn, const int* incRow, const int* incVal, int lo, int hi,
-                                 const vsdmo_mesh_params& prm, std::vector<DevBuf<uint8_t>*> u8)
+std::vector<int> colour_and_sort(vsdmo_mesh& m, Renumber& rn, ClassChecks& checks, const int* incRow,
+                                 const int* incVal, int lo, int hi, const vsdmo_mesh_params& prm, bool flags)
 {
+    BuildArena& ar = rn.ar;
     hipStream_t s = m.stream;
     int n = hi - lo;
     if (n <= 0) return { lo };
@@ -818,23 +850,31 @@ std::vector<int> colour_and_sort(vsdmo_mesh& m, Renumber& rn, const int* incRow,
     // vertex coloured and changes nothing, so the colours are those of one
     // check per round, with 1/kRoundsPerCheck of the syncs
     constexpr int kRoundsPerCheck = 16;
-    DevBuf<int> col(n), left(kRoundsPerCheck);
+    DevBuf<int> col(ar, n), left(ar, kRoundsPerCheck), flag(ar, 2);   // flag: polls ran out, largest colour
     VSDMO_HIP(hipMemsetAsync(col.p, 0xff, sizeof(int) * n, s));
-    int h_left = 1;
+    VSDMO_HIP(hipMemsetAsync(flag.p, 0, 2 * sizeof(int), s));
+    int h_left = 1, nc = 0;
+    const auto colours = [&]() {
+        k_max_reduce<<<nblk(n), TB, 0, s>>>(col.p, n, flag.p + 1);
+        VSDMO_HIP(hipGetLastError());
+        const int* h = read_ints(flag.p, 2, s);
+        h_left = h[0];
+        nc = h[1] + 1;
+    };
     if (mode != VSDMO_COLOR_JPL) {
         // greedy: one sweep over lower-neighbour lists; the rounds below only
         // run if a vertex ran out of polls
-        DevBuf<int> lrow((size_t)n + 1), gave(1);
+        DevBuf<int> lrow(ar, (size_t)n + 1);
         k_lower_count<<<nblk(n), TB, 0, s>>>(inc, lo, hi, lrow.p);
         VSDMO_HIP(hipMemsetAsync(lrow.p + n, 0, sizeof(int), s));
         const int tot = exclusive_scan(lrow.p, lrow.p, n + 1, s);
-        DevBuf<int> lval((size_t)std::max(tot, 1));
+        DevBuf<int> lval(ar, (size_t)std::max(tot, 1));
         k_lower_fill<<<nblk(n), TB, 0, s>>>(inc, lo, hi, lrow.p, lval.p);
-        VSDMO_HIP(hipMemsetAsync(gave.p, 0, sizeof(int), s));
-        k_color_greedy_sweep<<<nblk(n), TB, 0, s>>>(lrow.p, lval.p, n, col.p, std::min(polls, 1 << 26), gave.p);
+        k_color_greedy_sweep<<<nblk(n), TB, 0, s>>>(lrow.p, lval.p, n, col.p, std::min(polls, 1 << 26), flag.p);
         VSDMO_HIP(hipGetLastError());
-        h_left = read_int(gave.p, s);
+        colours();
     }
+    const bool rounds = h_left != 0;
     for (int round = 0; h_left != 0;) {
         if (round > n + 1) throw StatusError{ VSDMO_TOPOLOGY, "colouring did not converge" };
         VSDMO_HIP(hipMemsetAsync(left.p, 0, sizeof(int) * kRoundsPerCheck, s));
@@ -847,31 +887,24 @@ std::vector<int> colour_and_sort(vsdmo_mesh& m, Renumber& rn, const int* incRow,
         VSDMO_HIP(hipGetLastError());
         h_left = read_int(left.p + kRoundsPerCheck - 1, s);
     }
-    DevBuf<int> mx(1);
-    VSDMO_HIP(hipMemsetAsync(mx.p, 0, sizeof(int), s));
-    k_max_reduce<<<nblk(n), TB, 0, s>>>(col.p, n, mx.p);
-    const int nc = read_int(mx.p, s) + 1;
+    if (rounds) colours();
     if (nc > kMaxSortColours) throw StatusError{ VSDMO_NOT_SUPPORTED, "more than 16384 colours" };
     // stable counting sort by colour: per block of TB vertices the count of
     // each colour, scanned colour-major, gives each (colour, block) its first
     // position; a vertex adds the same-coloured vertices before it in its block
     const int nb = nblk(n);
-    DevBuf<int> newid(m.nV), pos((size_t)nc * nb), doff(nc);
+    DevBuf<int> newid(ar, m.nV), pos(ar, (size_t)nc * nb), doff(ar, (size_t)nc + 1);
     k_iota<<<nblk(m.nV), TB, 0, s>>>(newid.p, m.nV);
     k_colour_hist<<<nb, TB, sizeof(int) * nc, s>>>(col.p, n, nc, nb, pos.p);
-    exclusive_scan(pos.p, pos.p, nc * nb, s);
+    exclusive_scan_nototal(pos.p, pos.p, nc * nb, s);
     k_colour_place<<<nb, TB, 0, s>>>(col.p, n, nb, pos.p, lo, newid.p);
-    k_colour_offsets<<<nblk(nc), TB, 0, s>>>(pos.p, nb, nc, doff.p);
+    k_colour_offsets<<<nblk(nc + 1), TB, 0, s>>>(pos.p, nb, nc, lo, n, doff.p);
     std::vector<int> off(nc + 1, 0);
-    doff.download(off.data(), nc, s);
-    VSDMO_HIP(hipStreamSynchronize(s));
-    off[nc] = n;
-    VSDMO_HIP(hipGetLastError());
+    doff.download(off.data(), nc + 1, s);
     k_fill_range<<<nblk(n), TB, 0, s>>>(m.colorOf.p, lo, n, col.p);
-    std::vector<DevBuf<int>*> i32 = { &m.colorOf };
-    rn.apply(newid.p, u8, i32);
-    for (int& o : off) o += lo;
-    check_classes(m, off);
+    rn.apply(newid.p, flags, true);
+    VSDMO_HIP(hipStreamSynchronize(s));
+    checks.add(m, doff.p, off);
     return off;
 }
 
@@ -881,10 +914,13 @@ __constant__ int c_halfhex[8][7] = { { 1, 2, 3, 4, 5, 6, 7 }, { 5, 6, 2, 0, 4, 7
                                      { 7, 4, 0, 2, 6, 5, 1 }, { 0, 3, 7, 5, 1, 2, 6 }, { 4, 7, 6, 1, 0, 3, 2 },
                                      { 5, 4, 7, 2, 1, 0, 3 }, { 6, 5, 4, 3, 2, 1, 0 } };
 
-__global__ void k_ring_counts(const int* __restrict__ incRow, const int* __restrict__ oldOfCur, int n, int* __restrict__ cnt)
+// ring sizes, in cnt[n] and (with a zero at its end, for the scan) in row[n + 1]
+__global__ void k_ring_counts(const int* __restrict__ incRow, const int* __restrict__ oldOfCur, int n,
+                              int* __restrict__ cnt, int* __restrict__ row)
 {
     int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v < n) { int o = oldOfCur[v]; cnt[v] = incRow[o + 1] - incRow[o]; }
+    if (v < n) { int o = oldOfCur[v]; cnt[v] = row[v] = incRow[o + 1] - incRow[o]; }
+    if (v == n) row[v] = 0;
 }
 
 __global__ void k_ring_fill(const int* __restrict__ incRow, const int* __restrict__ incVal, const int* __restrict__ oldOfCur,
@@ -919,9 +955,37 @@ struct SurfaceInputs {
     const int* incRow;   // incidence over input ids (colouring adjacency)
     const int* incVal;
 };
-void build_surface(vsdmo_mesh& m, Renumber& rn, const SurfaceInputs& si, const vsdmo_mesh_params& prm);
+void build_surface(vsdmo_mesh& m, Renumber& rn, ClassChecks& checks, const SurfaceInputs& si,
+                   const vsdmo_mesh_params& prm);
 
 // ------------------------------------------------------------------ build
+__global__ void k_mesh_init(const float* __restrict__ xyz, int nV, float* __restrict__ x, float* __restrict__ y,
+                            float* __restrict__ z, int* __restrict__ colorOf, int* __restrict__ newOfOld,
+                            int* __restrict__ notFlat)
+{
+    const int v = blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= nV) return;
+    x[v] = xyz[3 * (size_t)v];
+    y[v] = xyz[3 * (size_t)v + 1];
+    const float pz = xyz[3 * (size_t)v + 2];
+    z[v] = pz;
+    if (pz != 0.0f) *notFlat = 1;
+    colorOf[v] = 0;
+    newOfOld[v] = v;
+}
+
+bool init_mesh(vsdmo_mesh& m, const float* xyz)
+{
+    hipStream_t s = m.stream;
+    DevBuf<float> in((size_t)m.nV * 3);
+    DevBuf<int> notFlat(1);
+    in.upload(xyz, (size_t)m.nV * 3, s);
+    VSDMO_HIP(hipMemsetAsync(notFlat.p, 0, sizeof(int), s));
+    k_mesh_init<<<nblk(m.nV), TB, 0, s>>>(in.p, m.nV, m.x.p, m.y.p, m.z.p, m.colorOf.p, m.newOfOld.p, notFlat.p);
+    VSDMO_HIP(hipGetLastError());
+    return read_int(notFlat.p, s) == 0;
+}
+
 void build_volume(vsdmo_mesh& m, const vsdmo_mesh_params& prm)
 {
     hipStream_t s = m.stream;
@@ -929,38 +993,44 @@ void build_volume(vsdmo_mesh& m, const vsdmo_mesh_params& prm)
     const int npe = m.npe, nV = m.nV, nE = m.nE;
     const long long nci = (long long)nE * npe;
 
+    const int nf = tet ? 4 : 6, k = tet ? 3 : 4, n = nE * nf;
+    // the largest at one time: the incidence, and the faces' arrays (8 ints a face)
+    BuildArena ar(sizeof(int) * ((size_t)nci + 9 * (size_t)n + 8 * (size_t)nV) + (1 << 20), s);
+
     // incidence in input ids: vertex -> (element, corner), ordered by element
-    DevBuf<int> incRow, incVal;
+    DevBuf<int> incRow(ar), incVal(ar, nci);
     {
-        DevBuf<int> key(nci), items;
+        DevBuf<int> key(ar, nci), items(ar);
         k_incidence_keys<<<nblk(nci), TB, 0, s>>>(m.cells.p, nci, key.p);
-        stable_csr(key.p, (int)nci, nV, incRow, items, s);
-        incVal.alloc(nci);
+        stable_csr(ar, key.p, (int)nci, nV, incRow, items, s);
         k_incidence_vals<<<nblk(nci), TB, 0, s>>>(items.p, nci, npe, incVal.p);
     }
 
     // boundary faces
     {
-        int nf = tet ? 4 : 6, k = tet ? 3 : 4;
-        int n = nE * nf;
-        DevBuf<int> fk((size_t)n * 4), v0(n), row, any, items(n), pos(n), alive(n);
-        DevBuf<uint8_t> dead(n);
+        DevBuf<int> fk(ar, (size_t)n * 4), v0(ar, n), row(ar), any(ar);
+        DevBuf<uint8_t> dead(ar, n);
         k_emit_faces<<<nblk(nE), TB, 0, s>>>(m.cells.p, nE, tet, fk.p, v0.p);
-        group_csr(v0.p, n, nV, row, any, false, s);
+        group_csr(ar, v0.p, n, nV, row, any, false, s);
+        DevBuf<int> items(ar, n);
         k_bucket_faces<<<nblk((long long)nV * 64), TB, 0, s>>>(row.p, nV, any.p, fk.p, k, items.p, dead.p);
-        k_alive<<<nblk(n), TB, 0, s>>>(dead.p, n, alive.p);
-        int nb = exclusive_scan(alive.p, pos.p, n, s);
+        // the keys and the unsorted order are no longer needed
+        int* const alive = v0.p;
+        int* const pos = any.p;
+        k_alive<<<nblk(n), TB, 0, s>>>(dead.p, n, alive);
+        int nb = exclusive_scan(alive, pos, n, s);
         m.fpe = k;
         m.nFaces = nb;
         m.faces.alloc((size_t)std::max(nb, 1) * k);
-        k_compact_faces<<<nblk(n), TB, 0, s>>>(items.p, dead.p, pos.p, n, fk.p, k, m.faces.p);
+        k_compact_faces<<<nblk(n), TB, 0, s>>>(items.p, dead.p, pos, n, fk.p, k, m.faces.p);
         VSDMO_HIP(hipGetLastError());
     }
 
-    Renumber rn(m);
+    Renumber rn(m, ar);
+    ClassChecks checks(ar);
     // [surface | inner], stable
     {
-        DevBuf<int> flag(nV), scan(nV), newid(nV);
+        DevBuf<int> flag(ar, nV), scan(ar, nV), newid(ar, nV);
         VSDMO_HIP(hipMemsetAsync(flag.p, 0, sizeof(int) * nV, s));
         long long nfi = (long long)m.nFaces * m.fpe;
         if (nfi > 0) k_mark_vertices<<<nblk(nfi), TB, 0, s>>>(m.faces.p, (int)nfi, flag.p);
@@ -971,28 +1041,27 @@ void build_volume(vsdmo_mesh& m, const vsdmo_mesh_params& prm)
         m.nInner = nV - nS;
     }
     // inner colouring and colour sort
-    m.colOffInner = colour_and_sort(m, rn, incRow.p, incVal.p, m.nSurf, nV, prm, {});
+    m.colOffInner = colour_and_sort(m, rn, checks, incRow.p, incVal.p, m.nSurf, nV, prm, false);
 
     // surface: features, [free | feature], colouring, halfedges
     SurfaceInputs si{ incRow.p, incVal.p };
-    build_surface(m, rn, si, prm);
+    build_surface(m, rn, checks, si, prm);
 
     // one-ring CSR in the final numbering
     {
-        DevBuf<int> cnt(nV);
-        k_ring_counts<<<nblk(nV), TB, 0, s>>>(incRow.p, rn.oldOfCur.p, nV, cnt.p);
+        DevBuf<int> cnt(ar, nV);
         m.ringRow.alloc((size_t)nV + 1);
-        VSDMO_HIP(hipMemcpyAsync(m.ringRow.p, cnt.p, sizeof(int) * nV, hipMemcpyDeviceToDevice, s));
-        VSDMO_HIP(hipMemsetAsync(m.ringRow.p + nV, 0, sizeof(int), s));
-        int tot = exclusive_scan(m.ringRow.p, m.ringRow.p, nV + 1, s);
+        k_ring_counts<<<nblk((long long)nV + 1), TB, 0, s>>>(incRow.p, rn.oldOfCur.p, nV, cnt.p, m.ringRow.p);
+        exclusive_scan_nototal(m.ringRow.p, m.ringRow.p, nV + 1, s);
         int st = tet ? 3 : 7;
-        m.ringVal.alloc((size_t)std::max(tot, 1) * st);
+        m.ringVal.alloc((size_t)nci * st);   // an entry per element and corner
         k_ring_fill<<<nblk(nV), TB, 0, s>>>(incRow.p, incVal.p, rn.oldOfCur.p, m.ringRow.p, m.cells.p, nV, tet, m.ringVal.p);
-        DevBuf<int> mx(1);
+        DevBuf<int> mx(ar, 1);
         VSDMO_HIP(hipMemsetAsync(mx.p, 0, sizeof(int), s));
         k_max_reduce<<<nblk(nV), TB, 0, s>>>(cnt.p, nV, mx.p);
         VSDMO_HIP(hipGetLastError());
         m.maxRing = read_int(mx.p, s);
+        checks.verify(s);
     }
 }
 
@@ -1002,12 +1071,13 @@ void build_surface_mesh(vsdmo_mesh& m, const vsdmo_mesh_params& prm)
     hipStream_t s = m.stream;
     const int npe = m.npe, nV = m.nV, nE = m.nE;
     const long long nci = (long long)nE * npe;
-    DevBuf<int> incRow, incVal;
+    // the largest at one time: the incidence and the halfedges' arrays
+    BuildArena ar(sizeof(int) * (18 * (size_t)nci + 8 * (size_t)nV) + (1 << 20), s);
+    DevBuf<int> incRow(ar), incVal(ar, nci);
     {
-        DevBuf<int> key(nci), items;
+        DevBuf<int> key(ar, nci), items(ar);
         k_incidence_keys<<<nblk(nci), TB, 0, s>>>(m.cells.p, nci, key.p);
-        stable_csr(key.p, (int)nci, nV, incRow, items, s);
-        incVal.alloc(nci);
+        stable_csr(ar, key.p, (int)nci, nV, incRow, items, s);
         k_incidence_vals<<<nblk(nci), TB, 0, s>>>(items.p, nci, npe, incVal.p);
     }
     m.nSurf = nV;
@@ -1017,17 +1087,18 @@ void build_surface_mesh(vsdmo_mesh& m, const vsdmo_mesh_params& prm)
     m.nFaces = nE;
     m.faces.alloc((size_t)nE * npe);
     VSDMO_HIP(hipMemcpyAsync(m.faces.p, m.cells.p, sizeof(int) * nci, hipMemcpyDeviceToDevice, s));
-    Renumber rn(m);
+    Renumber rn(m, ar);
+    ClassChecks checks(ar);
     {
-        DevBuf<int> id(nV);
+        DevBuf<int> id(ar, nV);
         k_iota<<<nblk(nV), TB, 0, s>>>(id.p, nV);
         rn.apply(id.p);
     }
     SurfaceInputs si{ incRow.p, incVal.p };
-    build_surface(m, rn, si, prm);
+    build_surface(m, rn, checks, si, prm);
     m.ringRow.alloc((size_t)nV + 1);
     VSDMO_HIP(hipMemsetAsync(m.ringRow.p, 0, sizeof(int) * ((size_t)nV + 1), s));
-    VSDMO_HIP(hipStreamSynchronize(s));
+    checks.verify(s);
 }
 
 }  // namespace vsdmo
@@ -1261,9 +1332,11 @@ __global__ void k_row_sizes(const int* __restrict__ row, int n, int* __restrict_
     if (v < n) atomicMax(mx, row[v + 1] - row[v]);
 }
 
-void build_surface(vsdmo_mesh& m, Renumber& rn, const SurfaceInputs& si, const vsdmo_mesh_params& prm)
+void build_surface(vsdmo_mesh& m, Renumber& rn, ClassChecks& checks, const SurfaceInputs& si,
+                   const vsdmo_mesh_params& prm)
 {
     hipStream_t s = m.stream;
+    BuildArena& ar = rn.ar;
     const int nS = m.nSurf, nF = m.nFaces, k = m.fpe;
     const int nV = m.nV;
     m.isB1D.alloc(std::max(nS, 1));
@@ -1283,11 +1356,11 @@ void build_surface(vsdmo_mesh& m, Renumber& rn, const SurfaceInputs& si, const v
     const float cthr = (float)std::cos((double)ang * 3.14159265358979323846 / 180.0);
     // features on the current numbering
     {
-        DevBuf<float> fn((size_t)nF * 3);
+        DevBuf<float> fn(ar, (size_t)nF * 3);
         k_face_normals<<<nblk(nF), TB, 0, s>>>(m.x.p, m.y.p, m.z.p, m.faces.p, nF, k, fn.p);
-        DevBuf<int> key(nRaw), row, items, opp(nRaw);
+        DevBuf<int> key(ar, nRaw), row(ar), items(ar), opp(ar, nRaw);
         k_he_src<<<nblk(nRaw), TB, 0, s>>>(m.faces.p, nRaw, key.p);
-        stable_csr(key.p, nRaw, nS, row, items, s);
+        stable_csr(ar, key.p, nRaw, nS, row, items, s);
         k_he_opp_raw<<<nblk(nS), TB, 0, s>>>(row.p, items.p, nS, m.faces.p, k, opp.p);
         k_features<<<nblk(nS), TB, 0, s>>>(row.p, items.p, opp.p, nS, m.faces.p, k, fn.p, m.flat, cthr,
                                            m.isB1D.p, m.isFeature.p);
@@ -1295,39 +1368,42 @@ void build_surface(vsdmo_mesh& m, Renumber& rn, const SurfaceInputs& si, const v
     }
     // [free | feature], stable
     {
-        DevBuf<int> flag(nS), scan(nS), newid(nV);
+        DevBuf<int> flag(ar, nS), scan(ar, nS), newid(ar, nV);
         k_u8_to_int<<<nblk(nS), TB, 0, s>>>(m.isFeature.p, nS, flag.p);
         int nFeat = exclusive_scan(flag.p, scan.p, nS, s);
         int nFree = nS - nFeat;
         k_partition_surface<<<nblk(nV), TB, 0, s>>>(flag.p, scan.p, nS, nV, nFree, newid.p);
-        rn.apply(newid.p, { &m.isB1D, &m.isFeature });
+        rn.apply(newid.p, true);
         m.nFree = nFree;
         m.nFeature = nFeat;
     }
-    m.colOffFree = colour_and_sort(m, rn, si.incRow, si.incVal, 0, m.nFree, prm, { &m.isB1D, &m.isFeature });
-    m.colOffFeature = colour_and_sort(m, rn, si.incRow, si.incVal, m.nFree, nS, prm, { &m.isB1D, &m.isFeature });
+    m.colOffFree = colour_and_sort(m, rn, checks, si.incRow, si.incVal, 0, m.nFree, prm, true);
+    m.colOffFeature = colour_and_sort(m, rn, checks, si.incRow, si.incVal, m.nFree, nS, prm, true);
     // halfedges on the final numbering
     {
-        DevBuf<int> key(nRaw), row, items, opp(nRaw), noopp(nRaw), dpos(nRaw);
+        DevBuf<int> key(ar, nRaw), row(ar), items(ar), opp(ar, nRaw), noopp(ar, nRaw), dpos(ar, nRaw);
         k_he_src<<<nblk(nRaw), TB, 0, s>>>(m.faces.p, nRaw, key.p);
-        stable_csr(key.p, nRaw, nS, row, items, s);
+        stable_csr(ar, key.p, nRaw, nS, row, items, s);
         k_he_opp_raw<<<nblk(nS), TB, 0, s>>>(row.p, items.p, nS, m.faces.p, k, opp.p);
         k_noopp<<<nblk(nRaw), TB, 0, s>>>(opp.p, nRaw, noopp.p);
         int nd = exclusive_scan(noopp.p, dpos.p, nRaw, s);
         int tot = nRaw + nd;
-        DevBuf<int> mKey(tot), mTgt(tot), mFace(tot);
+        DevBuf<int> mKey(ar, tot), mTgt(ar, tot), mFace(ar, tot);
         k_he_merge<<<nblk(nS), TB, 0, s>>>(row.p, items.p, opp.p, dpos.p, nS, nRaw, m.faces.p, k, mKey.p, mTgt.p, mFace.p);
-        DevBuf<int> items2;
-        stable_csr(mKey.p, tot, nS, m.heRow, items2, s);
-        DevBuf<int> sTgt(tot), sFace(tot), sOpp(tot), order(tot), err(1);
+        DevBuf<int> items2(ar);
+        stable_csr(ar, mKey.p, tot, nS, m.heRow, items2, s);
+        DevBuf<int> sTgt(ar, tot), sFace(ar, tot), sOpp(ar, tot), order(ar, tot), err(ar, 2);   // err: fan walk, longest row
         k_gather2<<<nblk(tot), TB, 0, s>>>(items2.p, tot, mTgt.p, mFace.p, sTgt.p, sFace.p);
         k_opp_sorted<<<nblk(nS), TB, 0, s>>>(m.heRow.p, nS, sTgt.p, sOpp.p);
-        VSDMO_HIP(hipMemsetAsync(err.p, 0, sizeof(int), s));
+        VSDMO_HIP(hipMemsetAsync(err.p, 0, 2 * sizeof(int), s));
         VSDMO_HIP(hipMemsetAsync(order.p, 0, sizeof(int) * tot, s));
         k_ccw<<<nblk(nS), TB, 0, s>>>(m.heRow.p, nS, sTgt.p, sFace.p, sOpp.p, m.isB1D.p, m.isFeature.p, m.faces.p, k,
                                       order.p, err.p);
+        k_row_sizes<<<nblk(nS), TB, 0, s>>>(m.heRow.p, nS, err.p + 1);
         {
-            const int herr = read_int(err.p, s);
+            const int* h = read_ints(err.p, 2, s);
+            const int herr = h[0];
+            m.maxHE = h[1];
             if (herr)
                 throw StatusError{ VSDMO_TOPOLOGY, "surface halfedge fan walk failed (non-manifold surface?) code " +
                                                        std::to_string(herr) };
@@ -1335,11 +1411,7 @@ void build_surface(vsdmo_mesh& m, Renumber& rn, const SurfaceInputs& si, const v
         m.heTarget.alloc(tot); m.heFace.alloc(tot); m.heOpp.alloc(tot); m.heNext.alloc(tot);
         k_gather2<<<nblk(tot), TB, 0, s>>>(order.p, tot, sTgt.p, sFace.p, m.heTarget.p, m.heFace.p);
         k_opp_next<<<nblk(nS), TB, 0, s>>>(m.heRow.p, nS, m.heTarget.p, m.heFace.p, m.heOpp.p, m.heNext.p);
-        DevBuf<int> mx(1);
-        VSDMO_HIP(hipMemsetAsync(mx.p, 0, sizeof(int), s));
-        k_row_sizes<<<nblk(nS), TB, 0, s>>>(m.heRow.p, nS, mx.p);
         VSDMO_HIP(hipGetLastError());
-        m.maxHE = read_int(mx.p, s);
         m.nHE = tot;
     }
 }

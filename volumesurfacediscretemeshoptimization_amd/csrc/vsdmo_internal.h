@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+#include <cstddef>
 #include <string>
 #include <vector>
 
@@ -31,18 +33,91 @@ struct StatusError {
     std::string msg;
 };
 
+// Device scratch of one mesh build, on one stream: a few large allocations
+// handed out in pieces, first fit.  hipMalloc of 4 MB and more takes ~300 us,
+// and a hipFree waits for the device; a build takes some 90 pieces.  A piece
+// that is put back is handed out again without a wait, as everything that uses
+// it is on the one stream.  The destructor waits for the stream and frees all.
+class BuildArena {
+public:
+    BuildArena(size_t bytes, hipStream_t s) : stream_(s) { grow(bytes); }
+    BuildArena(const BuildArena&) = delete;
+    BuildArena& operator=(const BuildArena&) = delete;
+    ~BuildArena()
+    {
+        (void)hipStreamSynchronize(stream_);
+        for (char* c : chunks_) (void)hipFree(c);
+    }
+    void* get(size_t bytes)
+    {
+        bytes = (bytes + 255) & ~size_t(255);
+        for (int attempt = 0;; ++attempt) {
+            for (size_t i = 0; i < pieces_.size(); ++i) {
+                if (pieces_[i].used || pieces_[i].n < bytes) continue;
+                const Piece rest{ pieces_[i].p + bytes, pieces_[i].n - bytes, false };
+                pieces_[i].n = bytes;
+                pieces_[i].used = true;
+                char* const p = pieces_[i].p;
+                if (rest.n) pieces_.insert(pieces_.begin() + (std::ptrdiff_t)i + 1, rest);
+                return p;
+            }
+            grow(bytes);
+        }
+    }
+    void put(void* q) noexcept
+    {
+        for (size_t i = 0; i < pieces_.size(); ++i) {
+            if (pieces_[i].p != q) continue;
+            pieces_[i].used = false;
+            join(i);
+            if (i > 0) join(i - 1);
+            return;
+        }
+    }
+
+private:
+    struct Piece { char* p; size_t n; bool used; };
+    void grow(size_t bytes)
+    {
+        bytes = std::max(bytes, size_t(1) << 20);
+        void* c = nullptr;
+        VSDMO_HIP(hipMalloc(&c, bytes));
+        try {
+            chunks_.push_back(static_cast<char*>(c));
+        } catch (...) {
+            (void)hipFree(c);
+            throw;
+        }
+        pieces_.push_back({ static_cast<char*>(c), bytes, false });
+    }
+    // piece i with its successor, if both are free and contiguous
+    void join(size_t i) noexcept
+    {
+        if (i + 1 >= pieces_.size() || pieces_[i].used || pieces_[i + 1].used) return;
+        if (pieces_[i].p + pieces_[i].n != pieces_[i + 1].p) return;
+        pieces_[i].n += pieces_[i + 1].n;
+        pieces_.erase(pieces_.begin() + (std::ptrdiff_t)i + 1);
+    }
+    hipStream_t stream_;
+    std::vector<char*> chunks_;
+    std::vector<Piece> pieces_;   // each chunk's in address order
+};
+
+// device array, its own allocation or (arena) a piece of a build's scratch
 template <class T>
 struct DevBuf {
     T* p = nullptr;
     size_t n = 0;
+    BuildArena* arena = nullptr;
     DevBuf() = default;
     explicit DevBuf(size_t count) { alloc(count); }
+    explicit DevBuf(BuildArena& a, size_t count = 0) : arena(&a) { alloc(count); }
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
-    DevBuf(DevBuf&& o) noexcept : p(o.p), n(o.n) { o.p = nullptr; o.n = 0; }
+    DevBuf(DevBuf&& o) noexcept : p(o.p), n(o.n), arena(o.arena) { o.p = nullptr; o.n = 0; }
     DevBuf& operator=(DevBuf&& o) noexcept
     {
-        if (this != &o) { release(); p = o.p; n = o.n; o.p = nullptr; o.n = 0; }
+        if (this != &o) { release(); p = o.p; n = o.n; arena = o.arena; o.p = nullptr; o.n = 0; }
         return *this;
     }
     ~DevBuf() { release(); }
@@ -50,11 +125,14 @@ struct DevBuf {
     {
         release();
         n = count;
-        if (count) VSDMO_HIP(hipMalloc(&p, count * sizeof(T)));
+        if (!count) return;
+        if (arena) p = static_cast<T*>(arena->get(count * sizeof(T)));
+        else VSDMO_HIP(hipMalloc(&p, count * sizeof(T)));
     }
     void release()
     {
-        if (p) (void)hipFree(p);
+        if (p && arena) arena->put(p);
+        else if (p) (void)hipFree(p);
         p = nullptr;
         n = 0;
     }
