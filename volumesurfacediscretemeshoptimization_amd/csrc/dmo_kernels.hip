@@ -682,8 +682,11 @@ __device__ __forceinline__ void hex_add_cpl(HexAcc* acc, const HexP& h, const fl
 // 40 sub-tets are left (the windows are scaled by the smallest one-ring offset
 // and the p-free sub-tets cap the minimum).  With none left every candidate
 // scores exactly the cap, and with U clearly below the current score none is
-// better: the level is decided without scoring.  Rings or frames outside the
-// bounds' range score every sub-tet.
+// better: the level is decided without scoring.  Where the bounds as a whole
+// are out of range (a sub-tet may be inverted or flat in the window), the p-free
+// minimum alone still rules out the sub-tets that are clearly above it: every
+// candidate's selection starts from it.  Rings whose p-free sub-tets are out of
+// range score every sub-tet.
 //
 // Bound by VALU issue: 15,000 -> 2,300 VALU operations per vertex, 214 -> 50 us
 // per class of the 48^3 cube (13.8k vertices); about half of it is the staging
@@ -731,14 +734,16 @@ __device__ void hex_vertex(const SearchArgs& a, int vid, bool emin, HexLds* s_hx
         const bool fast = f.inRange && __ballot(!sel) == 0ull && U >= kSelY;
         const float tq = qcur * (1.0f / 3.0f), yq = tq * __builtin_amdgcn_sqrtf(tq);   // qcur's det / F^1.5
         if (fast && U * (1.0f + kSel) < yq * (1.0f - kSel)) continue;   // no candidate reaches qcur
+        const float lim0 = (fast ? U : capY) * (1.0f + 2.0f * kSel);
+        const bool drops = fast || (f.inRange && capY >= kSelY);
         int nAct = 0;
         for (int t0 = 0; t0 < nSub; t0 += 64) {
             const int t = t0 + lane;
             const int e = sub_elem(t, f.corner8), s = t - e * ns;
             bool keep = t < nSub;
-            if (keep && fast) {
+            if (keep && drops) {
                 const HexBound b = t0 == 0 ? b0 : bound(t);
-                keep = !(b.clear && b.lb * (1.0f - kSel) > U * (1.0f + 2.0f * kSel));
+                keep = !(b.clear && b.sel && b.lb * (1.0f - kSel) > lim0);
             }
             const unsigned long long bal = __ballot(keep);
             if (keep)
@@ -1022,6 +1027,26 @@ constexpr int kLV = 4;
 // ~9x against a second window of the first's size, 1/6.7 and 1/5 measured
 // the same, 1/2 and 1/1 slower; a power of two keeps the scaling exact)
 constexpr float kMode3Window = 0.25f;
+
+// over the 16 lanes of the DPP row, in all of them.  The rows of a wave may be
+// in different branches, the lanes of one may not.
+#define VSDMO_ROW_REDUCE(OP)                                       \
+    asm("s_nop 1\n\t" OP " %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t" \
+        "s_nop 1\n\t" OP " %0, %0, %0 row_ror:4 row_mask:0xf bank_mask:0xf\n\t" \
+        "s_nop 1\n\t" OP " %0, %0, %0 row_ror:2 row_mask:0xf bank_mask:0xf\n\t" \
+        "s_nop 1\n\t" OP " %0, %0, %0 row_ror:1 row_mask:0xf bank_mask:0xf"      \
+        : "+v"(v))
+__device__ __forceinline__ float row_max(float v)
+{
+    VSDMO_ROW_REDUCE("v_max_f32_dpp");
+    return v;
+}
+__device__ __forceinline__ float row_min(float v)
+{
+    VSDMO_ROW_REDUCE("v_min_f32_dpp");
+    return v;
+}
+#undef VSDMO_ROW_REDUCE
 
 template <int G>
 __device__ __forceinline__ float group_max(float v)
@@ -1470,14 +1495,19 @@ __device__ void tet_window(const SearchArgs& a, const LearnArgs& la, int ringCap
     if (need && la.epoch) la.epoch[vid] = la.it;
 }
 
-// C8: the eight-corner hex metric (a.hexCorner8) as a template argument: a
-// runtime branch around the principal-axes slot held its LDS reads back in
-// this loop (36.5 -> 38.1 us per 48^3 class)
+// As tet_window for hexes, with hex_vertex's bounds in front of every level.
+// Every level scored the 40 sub-tets of a regular ring for all 64 candidates;
+// with the bounds a few are left (15.2 -> 9.5 M VALU operations per 48^3 class,
+// 35.8 -> 29.0 us).  A branch per lane (the sub-tet's alpha, a short circuit)
+// costs more here than what it skips: selects as arithmetic, 44 -> 37 us; the
+// last waves set the time, hence the early ends for pinned and inverted rings.
+// C8: the eight-corner hex metric (a.hexCorner8) as a template argument.
 template <int NQ, int LV, int WPB, bool FUSED, bool C8>
 __device__ void hex_window(const SearchArgs& a, const LearnArgs& la, int ringCap, int blk, unsigned char* s_hxl)
 {
     constexpr int NL = 4, G = 64 / LV, CPL = NL * NL * NL / G;
     constexpr int VPB = WPB * LV;
+    static_assert(G == 16 && CPL == NL, "a lane group is a DPP row, a lane a line of candidates along x");
     static_assert(!FUSED || VPB == kMlpRows, "one network tile per block");
     const int s = threadIdx.x % G, gb = threadIdx.x / G;
     const int nc = a.cEnd - a.cStart, ci0 = VPB * blk;
@@ -1557,70 +1587,181 @@ __device__ void hex_window(const SearchArgs& a, const LearnArgs& la, int ringCap
         hx[e] = L;
     }
     __syncthreads();
-    f.acc0 = hex_acc0();
-    for (int e = 0; e < f.n; ++e)
+    // the selection over the group's pairs pair(0..n-1), continued from acc (as
+    // select_lanes, whose conditions are checked here: else in order)
+    const int gbase = (int)(threadIdx.x & 63) & ~(G - 1);
+    const auto group_bits = [&](bool b) { return (unsigned)(__ballot(b) >> gbase) & 0xffffu; };
+    const auto select = [&](HexAcc& acc, bool hasAcc, bool accInRange, int n, auto pair) {
+        bool ok = accInRange && n > 0 && n <= 4 * G;
+        float y[4], dm = FLT_MAX, fm = FLT_MAX, ym = FLT_MAX;
 #pragma unroll
-        for (int sIdx = 0; sIdx < 4; ++sIdx) hex_acc_add(f.acc0, hx[e].cd[sIdx], hx[e].cF[sIdx]);
+        for (int q = 0; q < 4; ++q) {
+            y[q] = FLT_MAX;
+            if (s + q * G < n) {
+                const float2 v = pair(s + q * G);
+                ok = ok & sel_range(v.x, v.y);
+                dm = fminf(dm, v.x);
+                fm = fminf(fm, v.y);
+                y[q] = (v.x * v.x) * __builtin_amdgcn_rcpf((v.y * v.y) * v.y);
+                ym = fminf(ym, y[q]);
+            }
+        }
+        ok = group_bits(!ok) == 0;
+        if (n <= 4 * G) {
+            acc.dmin = fminf(acc.dmin, row_min(dm));
+            acc.fmin = fminf(acc.fmin, row_min(fm));
+            if (acc.dmin < f.epsD || acc.fmin < f.epsF) return false;   // scores 0, whatever is selected
+        }
+        if (!ok) {
+            for (int t = 0; t < n; ++t) { const float2 v = pair(t); hex_acc_add(acc, v.x, v.y); }
+            return false;
+        }
+        const float ya = hasAcc ? acc.bd2 * __builtin_amdgcn_rcpf(acc.bF3) : FLT_MAX;
+        const float lim = fminf(row_min(ym), ya) * (1.0f + 2.0f * kSel);
+        unsigned long long band = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) band |= (unsigned long long)group_bits(y[q] <= lim) << (16 * q);
+        if (!(ya <= lim)) { acc.bd2 = 1.0f; acc.bF3 = 0.0f; }   // replaced by the band's first
+        for (; band; band &= band - 1) {
+            const float2 v = pair(__builtin_ctzll(band));
+            const float d2 = v.x * v.x, F3 = (v.y * v.y) * v.y;
+            const bool take = d2 * acc.bF3 < acc.bd2 * F3;
+            acc.bd2 = take ? d2 : acc.bd2;
+            acc.bF3 = take ? F3 : acc.bF3;
+        }
+        return true;
+    };
+    constexpr int ns = C8 ? 4 : 5;
+    const int nSub = ns * f.n;
+    const auto sub = [&](int t) -> const HexP& {
+        const int e = sub_elem(t, C8);
+        return hx[e].hp[t - e * ns];
+    };
+    const auto alpha3 = [&](int t) { return (0x12 >> (t - sub_elem(t, C8) * ns) & 1) != 0; };   // slots 1 and 4
+    f.acc0 = hex_acc0();
+    f.inRange = select(f.acc0, false, true, 4 * f.n, [&](int t) { return make_float2(hx[t >> 2].cd[t & 3], hx[t >> 2].cF[t & 3]); });
+    // q0: the start position's score (at p = 0: det = D, |J|^2 = K exactly)
+    float q0;
+    {
+        HexAcc acc = f.acc0;
+        select(acc, true, f.inRange, nSub, [&](int t) { const HexP& h = sub(t); return make_float2(h.D, h.K); });
+        q0 = hex_acc_score(acc, f.epsD, f.epsF);
+    }
+    const float S0 = hex_acc_score(f.acc0, f.epsD, f.epsF);   // the score of a candidate that selects none
+    const float capY = f.inRange ? __builtin_amdgcn_sqrtf(f.acc0.bd2 * __builtin_amdgcn_rcpf(f.acc0.bF3)) : FLT_MAX;
+    const bool bounded = f.inRange && nSub <= 4 * G;
+    const bool pinned = hex_pinned(f);   // every candidate scores 0
 
     float cx = f.x0x, cy = f.x0y, cz = f.x0z;
     if (learn_uses_net(la.mode)) { cx = f.x0x + pl * py0; cy = f.x0y + pl * py1; cz = f.x0z + pl * py2; }
-    // q0, the start position's score, is accumulated beside the candidates
-    // of the first level (at p = 0: det = D, |J|^2 = K exactly, the terms
-    // hex_score adds, in the same order)
-    float q0 = 0.0f, qbest = 0.0f;
-    bool haveQ0 = false;
+    float qbest = q0;
     bool moved = false, tie = false;
     const float affL = 1.0f / (float)(NL - 1);
-    const int lj = s % NL, lk = (s / NL) % NL, i0 = (s / (NL * NL)) * CPL;
+    const int lj = s % NL, lk = s / NL;
+    // depthL levels of the 4x4x4 window around (cx, cy, cz), by the bounds of
+    // hex_vertex: up to 4 sub-tets on each lane of the group, and only those
+    // that can decide a candidate are scored (per candidate in ring order, the
+    // same bits).  The branches are uniform over the vertex's lane group.
     auto levels = [&](float scale) {
         float ds = (la.frac * scale) * a.gridScale;
-        for (int d = 0; d < la.depthL; ++d) {
+        for (int d = 0; d < la.depthL && !pinned; ++d, ds = ds * (2.0f / (float)(NL - 1))) {
             const float gxM = cx + ds * f.ex, gxm = cx - ds * f.ex;
             const float gyM = cy + ds * f.ey, gym = cy - ds * f.ey;
             const float gzM = cz + ds * f.ez, gzm = cz - ds * f.ez;
-            const float py = (grid_coord(affL, lj, NL, gym, gyM) - f.x0y) * f.sg;
-            const float pz = (grid_coord(affL, lk, NL, gzm, gzM) - f.x0z) * f.sg;
-            float px[CPL], t3[CPL];
-    #pragma unroll
-            for (int i = 0; i < CPL; ++i) {
-                px[i] = (grid_coord(affL, i0 + i, NL, gxm, gxM) - f.x0x) * f.sg;
-                t3[i] = 3.0f * px[i];
-            }
-            const float Q1 = fmaf(pz, pz, py * py), Q3 = 3.0f * Q1;
-            HexAcc acc[CPL];
-    #pragma unroll
-            for (int i = 0; i < CPL; ++i) acc[i] = f.acc0;
-            // the first level run also accumulates q0 (later levels and mode
-            // 3's window skip it)
-            auto ring = [&](auto withQ0) {
-                constexpr bool WQ = decltype(withQ0)::value;
-                HexAcc accO = f.acc0;
-                for (int e = 0; e < f.n; ++e) {
-    #pragma unroll
-                    for (int sIdx = 0; sIdx < (C8 ? 4 : 5); ++sIdx) {
-                        const HexP h = hx[e].hp[sIdx];
-                        const bool a3 = (sIdx == 1 || sIdx == 4);
-                        const float Tyz = fmaf(h.gy, py, fmaf(h.gz, pz, h.D));
-                        const float Ryz = fmaf(h.sy, py, fmaf(h.sz, pz, h.K + (a3 ? Q3 : Q1)));
-    #pragma unroll
-                        for (int i = 0; i < CPL; ++i)
-                            hex_acc_add(acc[i], fmaf(h.gx, px[i], Tyz), fmaf(px[i], (a3 ? t3[i] : px[i]) + h.sx, Ryz));
-                        if constexpr (WQ) hex_acc_add(accO, h.D, h.K);
+            const float tq = qbest * (1.0f / 3.0f), yq = tq * __builtin_amdgcn_sqrtf(tq);   // qbest's det / F^1.5
+            bool fast = false;
+            unsigned long long act = ~0ull;
+            if (bounded) {
+                const float wx = (cx - f.x0x) * f.sg, wy = (cy - f.x0y) * f.sg, wz = (cz - f.x0z) * f.sg;
+                const float Hx = 1.001f * (ds * f.ex) * f.sg + 0x1p-20f * (fabsf(cx) + ds * f.ex) * f.sg;
+                const float Hy = 1.001f * (ds * f.ey) * f.sg + 0x1p-20f * (fabsf(cy) + ds * f.ey) * f.sg;
+                const float Hz = 1.001f * (ds * f.ez) * f.sg + 0x1p-20f * (fabsf(cz) + ds * f.ez) * f.sg;
+                float u = FLT_MAX, lb[4];   // lb: -FLT_MAX where the sub-tet has to be scored
+                bool sel = true;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    lb[q] = -FLT_MAX;
+                    const int t = s + q * G;
+                    if (t < nSub) {
+                        const HexBound b = hex_bound(sub(t), alpha3(t), wx, wy, wz, Hx, Hy, Hz, f.epsD, f.epsF);
+                        u = fminf(u, b.ub);
+                        sel = sel & b.sel;
+                        lb[q] = b.clear && b.sel ? b.lb : -FLT_MAX;
                     }
                 }
-                if constexpr (WQ) { q0 = hex_acc_score(accO, f.epsD, f.epsF); qbest = q0; haveQ0 = true; }
-            };
-            if (!haveQ0) ring(std::true_type{});
-            else ring(std::false_type{});
-            float best = -FLT_MAX;
-            int bi = 0;
-    #pragma unroll
-            for (int i = 0; i < CPL; ++i) {
-                float q = hex_acc_score(acc[i], f.epsD, f.epsF);
-                if (q > best) { best = q; bi = i; }
+                const float U = fminf(row_min(u), capY);
+                if (U < 0.0f) continue;   // every candidate scores 0
+                fast = group_bits(!sel) == 0 && U >= kSelY;
+                if (fast && U * (1.0f + kSel) < yq * (1.0f - kSel)) continue;   // no candidate reaches qbest
+                const float lim0 = (fast ? U : capY >= kSelY ? capY : FLT_MAX) * (1.0f + 2.0f * kSel);
+                act = 0;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const bool drop = lb[q] * (1.0f - kSel) > lim0;
+                    act |= (unsigned long long)group_bits(s + q * G < nSub && !drop) << (16 * q);
+                }
             }
-            int cand = i0 + bi + NL * (s % (NL * NL));
-            group_argmax<G>(best, cand);
+            float best = S0;   // with nothing to score every candidate scores S0: the first
+            int cand = 0;
+            if (act != 0) {
+                const float py = (grid_coord(affL, lj, NL, gym, gyM) - f.x0y) * f.sg;
+                const float pz = (grid_coord(affL, lk, NL, gzm, gzM) - f.x0z) * f.sg;
+                float px[CPL];
+#pragma unroll
+                for (int i = 0; i < CPL; ++i) px[i] = (grid_coord(affL, i, NL, gxm, gxM) - f.x0x) * f.sg;
+                const float Q1 = fmaf(pz, pz, py * py);
+                HexAcc acc[CPL];
+#pragma unroll
+                for (int i = 0; i < CPL; ++i) acc[i] = f.acc0;
+                const auto alpha = [&](int t) { return alpha3(t) ? 3.0f : 1.0f; };   // 1 * x is x, to the bit
+                const auto add = [&](const HexP h, float al) {
+                    const float Tyz = fmaf(h.gy, py, fmaf(h.gz, pz, h.D));
+                    const float Ryz = fmaf(h.sy, py, fmaf(h.sz, pz, h.K + al * Q1));
+#pragma unroll
+                    for (int i = 0; i < CPL; ++i)
+                        hex_acc_add(acc[i], fmaf(h.gx, px[i], Tyz), fmaf(px[i], al * px[i] + h.sx, Ryz));
+                };
+                if (bounded) {
+                    HexP h = sub(__builtin_ctzll(act));
+                    float al = alpha(__builtin_ctzll(act));
+                    for (unsigned long long m = act & (act - 1);; m &= m - 1) {   // the next one's loads ahead
+                        const int t = __builtin_ctzll(m | 1ull << 63);
+                        const HexP hn = sub(m ? t : 0);
+                        const float an = alpha(m ? t : 0);
+                        add(h, al);
+                        if (!m) break;
+                        h = hn;
+                        al = an;
+                    }
+                } else {
+                    for (int t = 0; t < nSub; ++t) add(sub(t), alpha(t));
+                }
+                // scores: only of candidates whose ratio is within rounding of the best one's
+                float y[CPL], ym = 0.0f;
+#pragma unroll
+                for (int i = 0; i < CPL; ++i) {
+                    y[i] = (acc[i].dmin < f.epsD || acc[i].fmin < f.epsF) ? 0.0f : acc[i].bd2 * __builtin_amdgcn_rcpf(acc[i].bF3);
+                    ym = fmaxf(ym, y[i]);
+                }
+                const float Y = row_max(ym);
+                const bool quick = fast && Y > 1e-30f;   // below, the ratios are not exact enough to rank by
+                if (quick && Y < (yq * yq) * (1.0f - 4.0f * kSel)) continue;
+                const float lim = Y * (1.0f - kSel);
+                best = -FLT_MAX;
+                int bi = 0;
+#pragma unroll
+                for (int i = 0; i < CPL; ++i) {
+                    const bool in = !quick || y[i] >= lim;
+                    float q = S0;
+                    if (in && !(quick && acc[i].bd2 == f.acc0.bd2 && acc[i].bF3 == f.acc0.bF3))
+                        q = hex_acc_score(acc[i], f.epsD, f.epsF);
+                    if (in && q > best) { best = q; bi = i; }
+                }
+                const float own = best;
+                best = row_max(own);
+                const int l = __builtin_ctz(group_bits(own == best) | 0x10000u) & (G - 1);
+                cand = __shfl(bi, gbase + l) + NL * l;
+            }
             tie = tie || (best == q0 && q0 > 0.0f);
             if (qbest < best) {
                 cx = grid_coord(affL, cand % NL, NL, gxm, gxM);
@@ -1629,7 +1770,6 @@ __device__ void hex_window(const SearchArgs& a, const LearnArgs& la, int ringCap
                 qbest = best;
                 moved = true;
             }
-            ds = ds * (2.0f / (float)(NL - 1));
         }
     };
     levels(1.0f);
@@ -1701,6 +1841,10 @@ void k_search_hex_learned_def(SearchArgs a, LearnArgs la0, int ringCap, int nbLi
         const int lb = (int)blockIdx.x - nbWin;
         const int n = min(*la.cntIn, a.cEnd - a.cStart);
         if (lb == 0 && threadIdx.x == 0) atomicAdd(la.fallbacks, n);
+        // a full search alone takes as long as the windows' four rounds beside it:
+        // it goes first (last wave of a class at 23 us instead of 31; the tet
+        // kernel's shorter searches gained nothing by it)
+        __builtin_amdgcn_s_setprio(3);
         const int w = uniform((int)(threadIdx.x >> 6));   // one vertex per wave, in the wave's own LDS
         unsigned char* lds = s_hxd + (size_t)w * hex_wave_lds(ringCap);
         for (int i = lb + w * nbList; i < n; i += 4 * nbList) {
