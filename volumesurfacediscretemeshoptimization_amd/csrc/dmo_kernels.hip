@@ -1029,7 +1029,9 @@ constexpr int kLV = 4;
 constexpr float kMode3Window = 0.25f;
 
 // over the 16 lanes of the DPP row, in all of them.  The rows of a wave may be
-// in different branches, the lanes of one may not.
+// in different branches, the lanes of one may not.  (Shuffles, an LDS round trip
+// for each of 4 steps and each value, made the learned 40^3 tet iterations 2 %
+// longer.)
 #define VSDMO_ROW_REDUCE(OP)                                       \
     asm("s_nop 1\n\t" OP " %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t" \
         "s_nop 1\n\t" OP " %0, %0, %0 row_ror:4 row_mask:0xf bank_mask:0xf\n\t" \
@@ -1048,32 +1050,14 @@ __device__ __forceinline__ float row_min(float v)
 }
 #undef VSDMO_ROW_REDUCE
 
-template <int G>
-__device__ __forceinline__ float group_max(float v)
+// the place in its row of 16 of the first lane that b holds for (some lane's)
+__device__ __forceinline__ int row_first(bool b)
 {
-#pragma unroll
-    for (int m = G / 2; m >= 1; m >>= 1) v = fmaxf(v, __shfl_xor(v, m));
-    return v;
+    const unsigned m = (unsigned)(__ballot(b) >> ((int)(threadIdx.x & 63) & ~15)) & 0xffffu;
+    return __builtin_ctz(m | 0x10000u) & 15;
 }
-template <int G>
-__device__ __forceinline__ float group_min(float v)
-{
-#pragma unroll
-    for (int m = G / 2; m >= 1; m >>= 1) v = fminf(v, __shfl_xor(v, m));
-    return v;
-}
-template <int G>
-__device__ __forceinline__ void group_argmax(float& best, int& idx)
-{
-#pragma unroll
-    for (int m = G / 2; m >= 1; m >>= 1) {
-        float ob = __shfl_xor(best, m);
-        int oi = __shfl_xor(idx, m);
-        bool take = (ob > best) || (ob == best && oi < idx);
-        best = take ? ob : best;
-        idx = take ? oi : idx;
-    }
-}
+// a lane's value of the row, the same lane in all of them
+__device__ __forceinline__ int row_lane(int v, int l) { return __shfl(v, l, 16); }
 
 // The flat search of flat_vertex at nq = 8 for 4 vertices per wave.  The 64
 // candidate slots of a vertex are the lanes of the one-wave layout (thread
@@ -1102,9 +1086,9 @@ __device__ void flat_group8(const SearchArgs& a, int vid, TriC* s_tr)
         ey = fmaxf(ey, dy);
         mabs = fmaxf(mabs, fmaxf(dx, dy));
     }
-    ex = group_max<G>(ex);
-    ey = group_max<G>(ey);
-    mabs = group_max<G>(mabs);
+    ex = row_max(ex);
+    ey = row_max(ey);
+    mabs = row_max(mabs);
     const float sg = pow2_scale(mabs);
     const float isg = 1.0f / sg;
     const float is2 = (1.0f * isg) * isg;
@@ -1170,8 +1154,9 @@ __device__ void flat_group8(const SearchArgs& a, int vid, TriC* s_tr)
             const float q = tri_acc_score(acc[i], is2);
             if (q > best) { best = q; bi = i; }
         }
-        int wl = 4 * s + bi;
-        group_argmax<G>(best, wl);
+        const float own = best;
+        best = row_max(own);
+        const int l = row_first(own == best), wl = 4 * l + row_lane(bi, l);
         if (qcur < best) {
             const int wt = wl >> 1;
             const int wi = wt / NQ + ((wl & 1) ? 0 : NQ / 2), wj = wt % NQ;
@@ -1280,6 +1265,7 @@ __device__ void tet_window(const SearchArgs& a, const LearnArgs& la, int ringCap
 {
     constexpr int NL = 4, G = 64 / LV, CPL = NL * NL * NL / G;   // lanes per vertex, candidates per lane
     constexpr int VPB = WPB * LV;
+    static_assert(G == 16 && CPL == NL, "a lane group is a DPP row, a lane a line of candidates along x");
     static_assert(!FUSED || VPB == kMlpRows, "one network tile per block");
     const int s = threadIdx.x % G, gb = threadIdx.x / G;
     const int nc = a.cEnd - a.cStart, ci0 = VPB * blk;
@@ -1377,9 +1363,9 @@ __device__ void tet_window(const SearchArgs& a, const LearnArgs& la, int ringCap
             extent(dx, dy, dz);
         }
     }
-    if (emin) { ex = group_min<G>(ex); ey = group_min<G>(ey); ez = group_min<G>(ez); }
-    else { ex = group_max<G>(ex); ey = group_max<G>(ey); ez = group_max<G>(ez); }
-    mabs = group_max<G>(mabs);
+    if (emin) { ex = row_min(ex); ey = row_min(ey); ez = row_min(ez); }
+    else { ex = row_max(ex); ey = row_max(ey); ez = row_max(ez); }
+    mabs = row_max(mabs);
     f.ex = ex; f.ey = ey; f.ez = ez;
     f.sg = pow2_scale(mabs);
     const float isg = 1.0f / f.sg;
@@ -1421,7 +1407,7 @@ __device__ void tet_window(const SearchArgs& a, const LearnArgs& la, int ringCap
     bool haveQ0 = false;
     bool moved = false, tie = false;
     const float affL = 1.0f / (float)(NL - 1);
-    const int lj = s % NL, lk = (s / NL) % NL, i0 = (s / (NL * NL)) * CPL;
+    const int lj = s % NL, lk = s / NL;
     // depthL levels of the 4x4x4 window around (cx, cy, cz); the branch
     // conditions are uniform over the vertex's lane group
     auto levels = [&](float scale) {
@@ -1435,7 +1421,7 @@ __device__ void tet_window(const SearchArgs& a, const LearnArgs& la, int ringCap
             float px[CPL], t3[CPL];
     #pragma unroll
             for (int i = 0; i < CPL; ++i) {
-                px[i] = (grid_coord(affL, i0 + i, NL, gxm, gxM) - f.x0x) * f.sg;
+                px[i] = (grid_coord(affL, i, NL, gxm, gxM) - f.x0x) * f.sg;
                 t3[i] = 3.0f * px[i];
             }
             const float Qyz = 3.0f * fmaf(pz, pz, py * py);
@@ -1469,8 +1455,9 @@ __device__ void tet_window(const SearchArgs& a, const LearnArgs& la, int ringCap
                 float q = tet_acc_score(acc[i], f.is3);
                 if (q > best) { best = q; bi = i; }
             }
-            int cand = i0 + bi + NL * (s % (NL * NL));
-            group_argmax<G>(best, cand);
+            const float own = best;
+            best = row_max(own);
+            const int l = row_first(own == best), cand = row_lane(bi, l) + NL * l;
             tie = tie || (best == q0 && q0 > 0.0f);
             if (qbest < best) {
                 cx = grid_coord(affL, cand % NL, NL, gxm, gxM);
@@ -1566,10 +1553,10 @@ __device__ void hex_window(const SearchArgs& a, const LearnArgs& la, int ringCap
                 mabs = fmaxf(mabs, fmaxf(dx, fmaxf(dy, dz)));
             }
         }
-        if (emin) { ex = group_min<G>(ex); ey = group_min<G>(ey); ez = group_min<G>(ez); }
-        else { ex = group_max<G>(ex); ey = group_max<G>(ey); ez = group_max<G>(ez); }
+        if (emin) { ex = row_min(ex); ey = row_min(ey); ez = row_min(ez); }
+        else { ex = row_max(ex); ey = row_max(ey); ez = row_max(ez); }
         f.ex = ex; f.ey = ey; f.ez = ez;
-        f.sg = pow2_scale(group_max<G>(mabs));
+        f.sg = pow2_scale(row_max(mabs));
     }
     const float s2 = f.sg * f.sg, s3 = s2 * f.sg;
     f.epsD = kHexEps * s3; f.epsF = kHexEps * s2;
@@ -1759,8 +1746,8 @@ __device__ void hex_window(const SearchArgs& a, const LearnArgs& la, int ringCap
                 }
                 const float own = best;
                 best = row_max(own);
-                const int l = __builtin_ctz(group_bits(own == best) | 0x10000u) & (G - 1);
-                cand = __shfl(bi, gbase + l) + NL * l;
+                const int l = row_first(own == best);
+                cand = row_lane(bi, l) + NL * l;
             }
             tie = tie || (best == q0 && q0 > 0.0f);
             if (qbest < best) {
