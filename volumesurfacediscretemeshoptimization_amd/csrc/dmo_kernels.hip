@@ -21,44 +21,6 @@
 
 namespace vsdmo {
 
-// ------------------------------------------------- the canonical selection
-// The canonical selection compares ratios det^2 / F^3 in FP32 products; it
-// picks by the true ratios wherever they differ by more than its rounding, as
-// long as no product leaves the normal range.  kSelF / kSelD bound F and det
-// from below for that (det^2 F^3 >= 2^-108), kSel is the relative distance
-// (on det / F^1.5) beyond which a ratio counts as clearly larger: 2^-10,
-// against the selection's ~2^-22 per comparison.
-constexpr float kSelF = 0x1p-13f, kSelD = 0x1p-24f, kSelY = 0x1p-15f, kSel = 0x1p-10f;
-constexpr float kSelMax = 0x1p16f;   // and from above: no product overflows
-__device__ __forceinline__ bool sel_range(float det, float F)
-{
-    return det >= kSelD && det <= kSelMax && F >= kSelF && F <= kSelMax;   // false for NaN
-}
-
-// The running selection over up to 64 (det, F) pairs held one per lane (lane
-// order = selection order; have: the lane holds one), continued from acc:
-// the pair with the smallest ratio, found by one reduction.  Where several
-// lie within kSel of it, those alone are taken in order: a clearly larger one
-// never ends up selected, whatever its place.  Every lane calls it; at least
-// one holds a pair, and all pairs are in sel_range (as is acc's when it has one).
-__device__ __forceinline__ void select_lanes(float& bd2, float& bF3, bool hasAcc, bool have, float det, float F)
-{
-    const float d2 = det * det, F3 = (F * F) * F;
-    const float y = have ? d2 * __builtin_amdgcn_rcpf(F3) : FLT_MAX;
-    const float ya = hasAcc ? bd2 * __builtin_amdgcn_rcpf(bF3) : FLT_MAX;
-    const float lim = fminf(wave_min_u(y), ya) * (1.0f + 2.0f * kSel);
-    unsigned long long band = __ballot(have && y <= lim);
-    if (!(ya <= lim)) { bd2 = 1.0f; bF3 = 0.0f; }   // replaced by the band's first
-    while (band) {
-        const int l = __builtin_ctzll(band);
-        band &= band - 1;
-        const float ld = lane_f(d2, l), lF = lane_f(F3, l);
-        const bool take = ld * bF3 < bd2 * lF;
-        bd2 = take ? ld : bd2;
-        bF3 = take ? lF : bF3;
-    }
-}
-
 // ------------------------------------------------------------------ tets
 // LDS of a tet vertex search: the ring's constants, the level's plane of each
 // element (4 floats: gradient, offset for cells; the offset for candidates in
@@ -207,18 +169,7 @@ __device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, unsigned cha
     }
     wave_lds_fence();
 
-    // the canonical score of one position from (det, L) of the ring's elements,
-    // one per lane (rings of at most 64); false where the lanes cannot tell
-    auto lanes_score = [&](float det, float L, float& q) -> bool {
-        const float dmin = wave_min_u(own0 ? det : FLT_MAX);
-        if (dmin < 0.0f) { q = (dmin * (1.0f / 6.0f)) * f.is3; return true; }
-        if (dmin == 0.0f) { q = 0.0f; return true; }
-        if (__ballot(own0 && !sel_range(det, L)) != 0ull) return false;
-        TetAcc acc = tet_acc0();
-        select_lanes(acc.bd2, acc.bL3, false, own0, det, L);
-        q = kCTet * cbrt_nr(acc.bd2 / acc.bL3);
-        return true;
-    };
+    auto lanes_score = [&](float det, float L, float& q) { return tet_lanes_score(own0, det, L, f.is3, q); };
     // start score (p = 0: det = D, L = K exactly)
     float qcur = 0.0f;
     if (f.n > 64 || !lanes_score(c0.D, c0.K, qcur)) {
@@ -490,7 +441,7 @@ struct HexFrame {
     float x0x, x0y, x0z, ex, ey, ez, sg, epsD, epsF;
     int n;
     bool corner8;   // the principal-axes sub-tet (slot 4 of HexP) left out
-    bool inRange;   // hex_stage: every p-free pair is in sel_range
+    bool inRange;   // hex_free_lanes: every p-free pair is in sel_range
     HexAcc acc0;
 };
 
@@ -558,26 +509,8 @@ __device__ HexFrame hex_stage(const SearchArgs& a, int vid, bool emin, HexLds* s
         s_hx[e] = L;
     }
     wave_lds_fence();
-    // p-free sub-tets of the whole ring, in ring order: one pair per lane
-    // where the ring has at most 16 hexes
     f.acc0 = hex_acc0();
-    f.inRange = false;
-    if (f.n > 0 && 4 * f.n <= 64) {
-        const bool have = lane < 4 * f.n;
-        const int e = have ? lane >> 2 : 0;
-        const float det = s_hx[e].cd[lane & 3], F = s_hx[e].cF[lane & 3];
-        f.inRange = __ballot(have && !sel_range(det, F)) == 0ull;
-        if (f.inRange) {
-            f.acc0.dmin = wave_min_u(have ? det : FLT_MAX);
-            f.acc0.fmin = wave_min_u(have ? F : FLT_MAX);
-            select_lanes(f.acc0.bd2, f.acc0.bF3, false, have, det, F);
-        }
-    }
-    if (!f.inRange) {
-        for (int e = 0; e < f.n; ++e)
-#pragma unroll
-            for (int sIdx = 0; sIdx < 4; ++sIdx) hex_acc_add(f.acc0, s_hx[e].cd[sIdx], s_hx[e].cF[sIdx]);
-    }
+    f.inRange = hex_free_lanes(s_hx, f.n, f.acc0);
     return f;
 }
 
@@ -590,34 +523,6 @@ __device__ HexFrame hex_stage(const SearchArgs& a, int vid, bool emin, HexLds* s
 __device__ __forceinline__ bool hex_pinned(const HexFrame& f)
 {
     return f.acc0.dmin < f.epsD || f.acc0.fmin < f.epsF;
-}
-
-// ring element of the p-dependent sub-tet t (5 or 4 per element; t < 2^14)
-__device__ __forceinline__ int sub_elem(int t, bool corner8)
-{
-    return corner8 ? t >> 2 : (int)(((unsigned)t * 52429u) >> 18);
-}
-
-// the p-dependent sub-tets of the ring at the start position (p = 0: det = D,
-// |J|^2 = K exactly), in ring order
-__device__ __forceinline__ float hex_start_score(const HexFrame& f, const HexLds* s_hx)
-{
-    const int lane = (int)(threadIdx.x & 63), ns = f.corner8 ? 4 : 5;
-    HexAcc acc = f.acc0;
-    if (f.inRange && ns * f.n <= 64) {
-        const bool have = lane < ns * f.n;
-        const int e = have ? sub_elem(lane, f.corner8) : 0, s = have ? lane - e * ns : 0;
-        const float det = s_hx[e].hp[s].D, F = s_hx[e].hp[s].K;
-        if (__ballot(have && !sel_range(det, F)) == 0ull) {
-            acc.dmin = fminf(acc.dmin, wave_min_u(have ? det : FLT_MAX));
-            acc.fmin = fminf(acc.fmin, wave_min_u(have ? F : FLT_MAX));
-            select_lanes(acc.bd2, acc.bF3, true, have, det, F);
-            return hex_acc_score(acc, f.epsD, f.epsF);
-        }
-    }
-    for (int e = 0; e < f.n; ++e)
-        for (int s = 0; s < ns; ++s) hex_acc_add(acc, s_hx[e].hp[s].D, s_hx[e].hp[s].K);
-    return hex_acc_score(acc, f.epsD, f.epsF);
 }
 
 // What a level can say about one p-dependent sub-tet over its whole window (a
@@ -698,7 +603,7 @@ __device__ void hex_vertex(const SearchArgs& a, int vid, bool emin, HexLds* s_hx
     const HexFrame f = hex_stage(a, vid, emin, s_hx);
     if (hex_pinned(f)) return;   // uniform: every lane holds the same frame
     const int ns = f.corner8 ? 4 : 5, nSub = ns * f.n;
-    float qcur = hex_start_score(f, s_hx);
+    float qcur = hex_start_lanes(s_hx, f.n, f.corner8, f.acc0, f.inRange, f.epsD, f.epsF);
     const float S0 = hex_acc_score(f.acc0, f.epsD, f.epsF);   // the score of a candidate that selects none
     // the cap's det / F^1.5
     const float capY = f.inRange ? __builtin_amdgcn_sqrtf(f.acc0.bd2 * __builtin_amdgcn_rcpf(f.acc0.bF3)) : FLT_MAX;

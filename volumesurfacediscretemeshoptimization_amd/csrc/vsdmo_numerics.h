@@ -334,6 +334,113 @@ __device__ __forceinline__ float hex_acc_score(const HexAcc& a, float epsD, floa
     return 3.0f * cbrt_nr(a.bd2 / a.bF3);
 }
 
+// ------------------------------------------------- the canonical selection
+// The canonical selection compares ratios det^2 / F^3 in FP32 products; it
+// picks by the true ratios wherever they differ by more than its rounding, as
+// long as no product leaves the normal range.  kSelF / kSelD bound F and det
+// from below for that (det^2 F^3 >= 2^-108), kSel is the relative distance
+// (on det / F^1.5) beyond which a ratio counts as clearly larger: 2^-10,
+// against the selection's ~2^-22 per comparison.
+constexpr float kSelF = 0x1p-13f, kSelD = 0x1p-24f, kSelY = 0x1p-15f, kSel = 0x1p-10f;
+constexpr float kSelMax = 0x1p16f;   // and from above: no product overflows
+__device__ __forceinline__ bool sel_range(float det, float F)
+{
+    return det >= kSelD && det <= kSelMax && F >= kSelF && F <= kSelMax;   // false for NaN
+}
+
+// The running selection over up to 64 (det, F) pairs held one per lane (lane
+// order = selection order; have: the lane holds one), continued from acc:
+// the pair with the smallest ratio, found by one reduction.  Where several
+// lie within kSel of it, those alone are taken in order: a clearly larger one
+// never ends up selected, whatever its place.  Every lane calls it; at least
+// one holds a pair, and all pairs are in sel_range (as is acc's when it has one).
+__device__ __forceinline__ void select_lanes(float& bd2, float& bF3, bool hasAcc, bool have, float det, float F)
+{
+    const float d2 = det * det, F3 = (F * F) * F;
+    const float y = have ? d2 * __builtin_amdgcn_rcpf(F3) : 3.40282347e+38f;
+    const float ya = hasAcc ? bd2 * __builtin_amdgcn_rcpf(bF3) : 3.40282347e+38f;
+    const float lim = fminf(wave_min_u(y), ya) * (1.0f + 2.0f * kSel);
+    unsigned long long band = __ballot(have && y <= lim);
+    if (!(ya <= lim)) { bd2 = 1.0f; bF3 = 0.0f; }   // replaced by the band's first
+    while (band) {
+        const int l = __builtin_ctzll(band);
+        band &= band - 1;
+        const float ld = lane_f(d2, l), lF = lane_f(F3, l);
+        const bool take = ld * bF3 < bd2 * lF;
+        bd2 = take ? ld : bd2;
+        bF3 = take ? lF : bF3;
+    }
+}
+
+// ring element of the p-dependent sub-tet t (5 or 4 per element; t < 2^14)
+__device__ __forceinline__ int sub_elem(int t, bool corner8)
+{
+    return corner8 ? t >> 2 : (int)(((unsigned)t * 52429u) >> 18);
+}
+
+// The ring's selections with a pair per lane of the wave (every lane calls
+// them; L: a ring element's constants, cd, cF, hp in LDS).
+//
+// the p-free sub-tets of up to 16 hexes, in ring order, added to the empty acc;
+// true if they are all in sel_range (otherwise they are added one by one)
+template <class L>
+__device__ __forceinline__ bool hex_free_lanes(const L* hx, int n, HexAcc& acc)
+{
+    const int lane = (int)(threadIdx.x & 63);
+    if (n > 0 && 4 * n <= 64) {
+        const bool have = lane < 4 * n;
+        const int e = have ? lane >> 2 : 0;
+        const float det = hx[e].cd[lane & 3], F = hx[e].cF[lane & 3];
+        if (__ballot(have && !sel_range(det, F)) == 0ull) {
+            acc.dmin = wave_min_u(have ? det : 3.40282347e+38f);
+            acc.fmin = wave_min_u(have ? F : 3.40282347e+38f);
+            select_lanes(acc.bd2, acc.bF3, false, have, det, F);
+            return true;
+        }
+    }
+    for (int e = 0; e < n; ++e)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) hex_acc_add(acc, hx[e].cd[s], hx[e].cF[s]);
+    return false;
+}
+// the score of the start position: the p-dependent sub-tets at p = 0 (det = D,
+// |J|^2 = K exactly), in ring order, continued from acc (accInRange: as
+// hex_free_lanes returned it)
+template <class L>
+__device__ __forceinline__ float hex_start_lanes(const L* hx, int n, bool corner8, HexAcc acc, bool accInRange,
+                                                 float epsD, float epsF)
+{
+    const int lane = (int)(threadIdx.x & 63), ns = corner8 ? 4 : 5;
+    if (accInRange && ns * n <= 64) {
+        const bool have = lane < ns * n;
+        const int e = have ? sub_elem(lane, corner8) : 0, s = have ? lane - e * ns : 0;
+        const float det = hx[e].hp[s].D, F = hx[e].hp[s].K;
+        if (__ballot(have && !sel_range(det, F)) == 0ull) {
+            acc.dmin = fminf(acc.dmin, wave_min_u(have ? det : 3.40282347e+38f));
+            acc.fmin = fminf(acc.fmin, wave_min_u(have ? F : 3.40282347e+38f));
+            select_lanes(acc.bd2, acc.bF3, true, have, det, F);
+            return hex_acc_score(acc, epsD, epsF);
+        }
+    }
+    for (int e = 0; e < n; ++e)
+        for (int s = 0; s < ns; ++s) hex_acc_add(acc, hx[e].hp[s].D, hx[e].hp[s].K);
+    return hex_acc_score(acc, epsD, epsF);
+}
+// the canonical tet score from (det, L) of the ring's elements, one per lane
+// (have: the lane holds one; rings of at most 64); false where the lanes
+// cannot tell
+__device__ __forceinline__ bool tet_lanes_score(bool have, float det, float L, float is3, float& q)
+{
+    const float dmin = wave_min_u(have ? det : 3.40282347e+38f);
+    if (dmin < 0.0f) { q = (dmin * (1.0f / 6.0f)) * is3; return true; }
+    if (dmin == 0.0f) { q = 0.0f; return true; }
+    if (__ballot(have && !sel_range(det, L)) != 0ull) return false;
+    TetAcc acc = tet_acc0();
+    select_lanes(acc.bd2, acc.bL3, false, have, det, L);
+    q = kCTet * cbrt_nr(acc.bd2 / acc.bL3);
+    return true;
+}
+
 // ---------------------------------------------------------------- tri 2D
 // Ring element (a, b) of a fan: cross(p) = (a-p)x(b-a) = C + gx px + gy py,
 // L(p) = 2|p|^2 + S.p + K with d = b - a, C = ax*dy - ay*dx, g = (-dy, dx),
