@@ -819,7 +819,7 @@ struct ClassChecks {
 // a partition given by the caller
 void check_classes(const vsdmo_mesh& m, const std::vector<int>& off)
 {
-    BuildArena ar(sizeof(int) * off.size() + 4096, m.stream);
+    BuildArena ar(0, m.stream);
     DevBuf<int> doff(ar, off.size());
     ClassChecks checks(ar);
     doff.upload(off.data(), off.size(), m.stream);
@@ -995,7 +995,7 @@ void build_volume(vsdmo_mesh& m, const vsdmo_mesh_params& prm)
 
     const int nf = tet ? 4 : 6, k = tet ? 3 : 4, n = nE * nf;
     // the largest at one time: the incidence, and the faces' arrays (8 ints a face)
-    BuildArena ar(sizeof(int) * ((size_t)nci + 9 * (size_t)n + 8 * (size_t)nV) + (1 << 20), s);
+    BuildArena ar(sizeof(int) * ((size_t)nci + 9 * (size_t)n + 8 * (size_t)nV), s);
 
     // incidence in input ids: vertex -> (element, corner), ordered by element
     DevBuf<int> incRow(ar), incVal(ar, nci);
@@ -1072,7 +1072,7 @@ void build_surface_mesh(vsdmo_mesh& m, const vsdmo_mesh_params& prm)
     const int npe = m.npe, nV = m.nV, nE = m.nE;
     const long long nci = (long long)nE * npe;
     // the largest at one time: the incidence and the halfedges' arrays
-    BuildArena ar(sizeof(int) * (18 * (size_t)nci + 8 * (size_t)nV) + (1 << 20), s);
+    BuildArena ar(sizeof(int) * (18 * (size_t)nci + 8 * (size_t)nV), s);
     DevBuf<int> incRow(ar), incVal(ar, nci);
     {
         DevBuf<int> key(ar, nci), items(ar);

@@ -33,14 +33,19 @@ struct StatusError {
     std::string msg;
 };
 
-// Device scratch of one mesh build, on one stream: a few large allocations
-// handed out in pieces, first fit.  hipMalloc of 4 MB and more takes ~300 us,
-// and a hipFree waits for the device; a build takes some 90 pieces.  A piece
-// that is put back is handed out again without a wait, as everything that uses
-// it is on the one stream.  The destructor waits for the stream and frees all.
+// Device scratch of one mesh build, on one stream: a few allocations handed
+// out in pieces, first fit.  hipMalloc of 4 MB and more takes ~300 us, of 2 MB
+// ~50 us, up to 1 MB ~0.5 us (hipFree alike), and a hipFree waits for the
+// device; a build takes some 90 pieces.  So a build that needs more than 4 MB
+// takes it at once, a smaller one as it goes, in chunks of 1 MB.  A piece that
+// is put back is handed out again without a wait, as everything that uses it is
+// on the one stream.  The destructor waits for the stream and frees all.
 class BuildArena {
 public:
-    BuildArena(size_t bytes, hipStream_t s) : stream_(s) { grow(bytes); }
+    BuildArena(size_t bytes, hipStream_t s) : stream_(s)
+    {
+        if (bytes > (size_t(4) << 20)) grow(bytes);
+    }
     BuildArena(const BuildArena&) = delete;
     BuildArena& operator=(const BuildArena&) = delete;
     ~BuildArena()
@@ -51,7 +56,7 @@ public:
     void* get(size_t bytes)
     {
         bytes = (bytes + 255) & ~size_t(255);
-        for (int attempt = 0;; ++attempt) {
+        for (;;) {
             for (size_t i = 0; i < pieces_.size(); ++i) {
                 if (pieces_[i].used || pieces_[i].n < bytes) continue;
                 const Piece rest{ pieces_[i].p + bytes, pieces_[i].n - bytes, false };
