@@ -428,6 +428,142 @@ __device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, unsigned cha
     if (moved && lane == 0) { a.xw[vid] = cx; a.yw[vid] = cy; a.zw[vid] = cz; }
 }
 
+// The same search on the 4 waves of a block, every candidate scored: lane l = j
+// + nq k of wave w owns the candidates (i, j, k), i = w nq / 4 and on.  It takes
+// twice the operations of tet_vertex, four times as many lanes at once, and
+// none of tet_vertex's chain of filters and lists: for launches that leave most
+// of the chip idle, where a vertex's chain sets the time (kTetWideMax).
+// lds: tet_wide_lds bytes.
+struct TetBest { float q; int cand; };
+__host__ __device__ constexpr size_t tet_wide_lds(int ringCap)
+{
+    return sizeof(TetC) * (size_t)ringCap + 8 * sizeof(TetBest);
+}
+template <int NQ>
+__device__ void tet_vertex_wide(const SearchArgs& a, int vid, unsigned char* lds, int ringCap)
+{
+    constexpr int W = 4, CPL = NQ / W;
+    static_assert(NQ % W == 0 && NQ * NQ <= 64, "nq 4 or 8");
+    const int lane = (int)(threadIdx.x & 63), wave = uniform((int)(threadIdx.x >> 6));
+    const bool emin = a.extentMin != 0;
+    TetC* s_tc = reinterpret_cast<TetC*>(lds);
+    TetBest* s_best = reinterpret_cast<TetBest*>(s_tc + ringCap);   // [level parity][wave]
+    TetFrame f;
+    const int r0 = uniform(a.ringRow[vid]);
+    f.n = uniform(a.ringRow[vid + 1]) - r0;
+    if (f.n <= 0) return;
+    f.x0x = a.x[vid]; f.x0y = a.y[vid]; f.x0z = a.z[vid];
+    // every wave reads the whole ring (its frame needs no barrier), the first
+    // one writes the constants
+    float ex = emin ? FLT_MAX : -FLT_MAX, ey = ex, ez = ex, mabs = 0.0f;
+    const bool own0 = lane < f.n;
+    f3 d0[3];
+    for (int e = lane; e < f.n; e += 64) {
+        const int* h = a.ringVal + (size_t)(r0 + e) * 3;
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const int v = h[t];
+            const f3 o = { a.x[v] - f.x0x, a.y[v] - f.x0y, a.z[v] - f.x0z };
+            if (e == lane) d0[t] = o;
+            const float dx = fabsf(o.x), dy = fabsf(o.y), dz = fabsf(o.z);
+            ex = emin ? fminf(ex, dx) : fmaxf(ex, dx);
+            ey = emin ? fminf(ey, dy) : fmaxf(ey, dy);
+            ez = emin ? fminf(ez, dz) : fmaxf(ez, dz);
+            mabs = fmaxf(mabs, fmaxf(dx, fmaxf(dy, dz)));
+        }
+    }
+    if (emin) { f.ex = wave_min_u(ex); f.ey = wave_min_u(ey); f.ez = wave_min_u(ez); }
+    else { f.ex = wave_max_u(ex); f.ey = wave_max_u(ey); f.ez = wave_max_u(ez); }
+    f.sg = pow2_scale(wave_max_u(mabs));
+    const float isg = 1.0f / f.sg;
+    f.is3 = ((1.0f * isg) * isg) * isg;
+    TetC c0{ 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f };
+    if (own0) {
+        c0 = tet_consts(scl3(d0[0], f.sg), scl3(d0[1], f.sg), scl3(d0[2], f.sg));
+        if (wave == 0) s_tc[lane] = c0;
+    }
+    if (wave == 0)
+        for (int e = lane + 64; e < f.n; e += 64) {
+            const int* h = a.ringVal + (size_t)(r0 + e) * 3;
+            f3 p[3];
+            for (int t = 0; t < 3; ++t) {
+                const int v = h[t];
+                p[t] = { (a.x[v] - f.x0x) * f.sg, (a.y[v] - f.x0y) * f.sg, (a.z[v] - f.x0z) * f.sg };
+            }
+            s_tc[e] = tet_consts(p[0], p[1], p[2]);
+        }
+    __syncthreads();
+    float qcur = 0.0f;
+    if (f.n > 64 || !tet_lanes_score(own0, c0.D, c0.K, f.is3, qcur)) {
+        TetAcc acc = tet_acc0();
+        for (int e = 0; e < f.n; ++e) tet_acc_add(acc, s_tc[e].D, s_tc[e].K);
+        qcur = tet_acc_score(acc, f.is3);
+    }
+    float cx = f.x0x, cy = f.x0y, cz = f.x0z, ds = a.gridScale;
+    const int j = lane % NQ, k = lane / NQ;
+    const bool active = lane < NQ * NQ;
+    bool moved = false;
+    for (int d = 0; d < a.depth; ++d, ds = ds * a.shrink) {
+        const float gxM = cx + ds * f.ex, gxm = cx - ds * f.ex;
+        const float gyM = cy + ds * f.ey, gym = cy - ds * f.ey;
+        const float gzM = cz + ds * f.ez, gzm = cz - ds * f.ez;
+        const float py = (grid_coord(a.aff, j, NQ, gym, gyM) - f.x0y) * f.sg;
+        const float pz = (grid_coord(a.aff, k, NQ, gzm, gzM) - f.x0z) * f.sg;
+        const float Qyz = 3.0f * fmaf(pz, pz, py * py);
+        float px[CPL], t3[CPL];
+        TetAcc acc[CPL];
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) {
+            px[i] = (grid_coord(a.aff, wave * CPL + i, NQ, gxm, gxM) - f.x0x) * f.sg;
+            t3[i] = 3.0f * px[i];
+            acc[i] = tet_acc0();
+        }
+#pragma unroll 4
+        for (int e = 0; e < f.n; ++e) {
+            const TetC c = s_tc[e];
+            const float Tyz = fmaf(c.nny, py, fmaf(c.nnz, pz, c.D));
+            const float Ryz = fmaf(c.m2sy, py, fmaf(c.m2sz, pz, c.K + Qyz));
+#pragma unroll
+            for (int i = 0; i < CPL; ++i)
+                tet_acc_add(acc[i], fmaf(c.nnx, px[i], Tyz), fmaf(px[i], t3[i] + c.m2sx, Ryz));
+        }
+        float own = -FLT_MAX;
+        int bi = 0;
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) {
+            const float q = tet_acc_score(acc[i], f.is3);
+            if (active && q > own) { own = q; bi = i; }
+        }
+        const float m = wave_max_u(own);
+        const int l = __builtin_ctzll(__ballot(own == m));
+        if (lane == l) s_best[(d & 1) * W + wave] = { m, wave * CPL + bi + NQ * l };
+        __syncthreads();   // one a level: the next one's values go to the other half
+        float best = -FLT_MAX;
+        int cand = 0;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            const TetBest b = s_best[(d & 1) * W + w];
+            if (b.q > best || (b.q == best && b.cand < cand)) { best = b.q; cand = b.cand; }
+        }
+        if (qcur < best) {
+            cx = grid_coord(a.aff, cand % NQ, NQ, gxm, gxM);
+            cy = grid_coord(a.aff, (cand / NQ) % NQ, NQ, gym, gyM);
+            cz = grid_coord(a.aff, cand / (NQ * NQ), NQ, gzm, gzM);
+            qcur = best;
+            moved = true;
+        }
+    }
+    if (moved && threadIdx.x == 0) { a.xw[vid] = cx; a.yw[vid] = cy; a.zw[vid] = cz; }
+    __syncthreads();   // the next vertex restages the ring
+}
+// vertices up to which a launch takes tet_vertex_wide: by themselves, 4 waves
+// per SIMD (plain tet cubes, 6 iterations, one wave per vertex against wide: 13^3
+// with classes of ~170 vertices 1.24 / 0.92 ms, 20^3 with 500-900 1.45 / 1.30,
+// 24^3 with up to 1,600 1.65 / 1.61; with the line at 2,048 24^3 takes 1.74), and
+// beside a class's windows (40^3, mode 1: at 256 1.75 ms, at 512 1.77, at 1,024
+// 1.84, never 1.87)
+constexpr int kTetWideMax = 1024, kTetWideDef = 256;
+
 // ------------------------------------------------------------------ hexes
 struct HexLds { float cd[4], cF[4]; HexP hp[5]; };
 
@@ -818,6 +954,12 @@ __global__ __launch_bounds__(64, VSDMO_TET_MIN_WAVES) void k_search_tet(SearchAr
 {
     extern __shared__ __align__(16) unsigned char s_tcv[];
     tet_vertex<NQ>(a, a.cStart + blockIdx.x, a.extentMin != 0, s_tcv, ringCap);
+}
+template <int NQ>
+__global__ __launch_bounds__(256) void k_search_tet_wide(SearchArgs a, int ringCap)
+{
+    extern __shared__ __align__(16) unsigned char s_twv[];
+    tet_vertex_wide<NQ>(a, a.cStart + blockIdx.x, s_twv, ringCap);
 }
 // the hex search asks for 4 waves per SIMD (128 VGPRs, no spill): 48^3 cube,
 // 10 iterations, 5.1 ms against 5.5 ms at 3 (129 VGPRs) and 5.1-5.2 ms at 5
@@ -1716,6 +1858,11 @@ void k_search_tet_learned_def(SearchArgs a, LearnArgs la0, int ringCap, int nbLi
         const int lb = (int)blockIdx.x - nbWin;
         const int n = min(*la.cntIn, a.cEnd - a.cStart);
         if (lb == 0 && threadIdx.x == 0) atomicAdd(la.fallbacks, n);
+        __builtin_amdgcn_s_setprio(3);   // as in the hex kernel below
+        if (n <= kTetWideDef) {
+            for (int i = lb; i < n; i += nbList) tet_vertex_wide<NQ>(a, uniform(la.listIn[i]), s_tcd, ringCap);
+            return;
+        }
         const int w = uniform((int)(threadIdx.x >> 6));   // one vertex per wave, in the wave's own LDS
         unsigned char* lds = s_tcd + (size_t)w * tet_wave_lds(ringCap);
         for (int i = lb + w * nbList; i < n; i += 4 * nbList) {
@@ -1759,15 +1906,25 @@ void k_search_hex_learned_def(SearchArgs a, LearnArgs la0, int ringCap, int nbLi
 // one vertex per block of W waves at a time, blocks striding over the list
 // (the grid is sized for a typical fallback share, the length is only known
 // on the device)
-template <int NQ>
-__global__ __launch_bounds__(64) void k_search_list_tet(SearchArgs a, const int* __restrict__ list,
-                                                       const int* __restrict__ cnt, int* fallbacks, int ringCap)
+// WIDE: blocks of 4 waves, which take a vertex together while the list is
+// short, a vertex each otherwise
+template <int NQ, bool WIDE>
+__global__ __launch_bounds__(WIDE ? 256 : 64) void k_search_list_tet(SearchArgs a, const int* __restrict__ list,
+                                                                    const int* __restrict__ cnt, int* fallbacks,
+                                                                    int ringCap)
 {
     extern __shared__ __align__(16) unsigned char s_tcf[];
     const int n = min(*cnt, a.cEnd - a.cStart);
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(fallbacks, n);
-    for (int i = blockIdx.x; i < n; i += gridDim.x) {
-        tet_vertex<NQ>(a, uniform(list[i]), a.extentMin != 0, s_tcf, ringCap);
+    if constexpr (WIDE) {
+        if (n <= kTetWideMax) {
+            for (int i = blockIdx.x; i < n; i += gridDim.x) tet_vertex_wide<NQ>(a, uniform(list[i]), s_tcf, ringCap);
+            return;
+        }
+    }
+    const int w = uniform((int)(threadIdx.x >> 6));
+    for (int i = blockIdx.x + w * gridDim.x; i < n; i += (WIDE ? 4 : 1) * gridDim.x) {
+        tet_vertex<NQ>(a, uniform(list[i]), a.extentMin != 0, s_tcf + (size_t)w * tet_wave_lds(ringCap), ringCap);
         wave_lds_fence();   // the next vertex restages the ring
     }
 }
@@ -1788,7 +1945,13 @@ static void list_nq(int kind, const SearchArgs& a, const int* list, const int* c
                      int ringCap, hipStream_t s)
 {
     const size_t lds = search_lds_bytes(kind, ringCap);
-    if (kind == VSDMO_TET) launch_kernel(k_search_list_tet<NQ>, grid, 64, lds, s, a, list, cnt, fallbacks, ringCap);
+    if constexpr (NQ % 4 == 0) {
+        if (kind == VSDMO_TET && 4 * lds <= 64 * 1024) {   // a vertex per wave fits a block's LDS
+            launch_kernel(k_search_list_tet<NQ, true>, grid, 256, 4 * lds, s, a, list, cnt, fallbacks, ringCap);
+            return;
+        }
+    }
+    if (kind == VSDMO_TET) launch_kernel(k_search_list_tet<NQ, false>, grid, 64, lds, s, a, list, cnt, fallbacks, ringCap);
     else launch_kernel(k_search_list_hex<NQ>, grid, 64, lds, s, a, list, cnt, fallbacks, ringCap);
 }
 
@@ -2213,6 +2376,12 @@ template <int NQ>
 static void launch_nq(int kind, const SearchArgs& a, int nBlocks, int ringCap, hipStream_t s)
 {
     const size_t lds = search_lds_bytes(kind, ringCap);
+    if constexpr (NQ % 4 == 0) {
+        if (kind == VSDMO_TET && nBlocks <= kTetWideMax) {
+            launch_kernel(k_search_tet_wide<NQ>, nBlocks, 256, tet_wide_lds(ringCap), s, a, ringCap);
+            return;
+        }
+    }
     if (kind == VSDMO_TET) launch_kernel(k_search_tet<NQ>, nBlocks, 64, lds, s, a, ringCap);
     else if (kind == VSDMO_HEX) launch_kernel(k_search_hex<NQ>, nBlocks, 64, lds, s, a, ringCap);
     else launch_kernel(k_search_flat<NQ>, nBlocks, 64, lds, s, a);
