@@ -6,6 +6,7 @@ rings, scales and both nq that have the wide form."""
 import numpy as np
 import pytest
 
+from test_gpu_learned_oracle import oracle_learned
 from volumesurfacediscretemeshoptimization_amd import DMOMeshTetFactory, DMOTetClass, synth
 
 pytestmark = pytest.mark.gpu
@@ -31,3 +32,25 @@ def test_classes_on_both_sides(oracle, nq, jitter, scale):
     finally:
         opt.close()
         g.close()
+
+
+def test_lists_beside_windows(oracle):
+    """deferred fallback lists of classes on both sides of 4,096 vertices, up
+    to which a short list takes 4 waves per vertex"""
+    xyz, cells = synth.tet_cube(34, seed=35, jitter=0.3)
+    ref, fb = oracle_learned(oracle, "tet", xyz, cells, None, 2, 1, 0.25, "deferred", 3)
+    m = DMOMeshTetFactory.create(xyz, cells)
+    sizes = np.diff(m.color_offsets("inner"))
+    assert sizes.min() < 4096 < sizes.max()
+    o = DMOTetClass(m, n_iter=3, fixed_boundary=True, quality_guard=False)
+    try:
+        o.set_proposal(None, mode=2, depth=1, window_frac=0.25, fallback="deferred")
+        for it in range(3):
+            o.iterate(1)
+            gp = m.positions(original_order=False)
+            bad = (gp.view(np.uint32) != ref[it].view(np.uint32)).any(axis=1)
+            assert not bad.any(), (it, int(bad.sum()), np.nonzero(bad)[0][:5])
+        assert o.stats()["fallbacks"] == fb > 0
+    finally:
+        o.close()
+        m.close()

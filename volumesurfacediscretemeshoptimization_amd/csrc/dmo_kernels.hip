@@ -561,8 +561,13 @@ __device__ void tet_vertex_wide(const SearchArgs& a, int vid, unsigned char* lds
 // with classes of ~170 vertices 1.24 / 0.92 ms, 20^3 with 500-900 1.45 / 1.30,
 // 24^3 with up to 1,600 1.65 / 1.61; with the line at 2,048 24^3 takes 1.74), and
 // beside a class's windows (40^3, mode 1: at 256 1.75 ms, at 512 1.77, at 1,024
-// 1.84, never 1.87)
-constexpr int kTetWideMax = 1024, kTetWideDef = 256;
+// 1.84, never 1.87).  Beside the windows of a class of more than 4,096 vertices a
+// short list is over before they are, in one wave per vertex and without the raised
+// priority: four waves and the priority only hold the windows up (40^3, mode 3,
+// ~100 vertices deferred of classes of ~7,400, one-mesh batch: 0.206 ms an iteration
+// wide, 0.203 in one wave at raised priority, 0.201 in one wave without; 16^3 to
+// 40^3 in mode 1 are the same within 2 %)
+constexpr int kTetWideMax = 1024, kTetWideDef = 256, kTetWideClass = 4096;
 
 // ------------------------------------------------------------------ hexes
 struct HexLds { float cd[4], cF[4]; HexP hp[5]; };
@@ -1858,8 +1863,9 @@ void k_search_tet_learned_def(SearchArgs a, LearnArgs la0, int ringCap, int nbLi
         const int lb = (int)blockIdx.x - nbWin;
         const int n = min(*la.cntIn, a.cEnd - a.cStart);
         if (lb == 0 && threadIdx.x == 0) atomicAdd(la.fallbacks, n);
-        __builtin_amdgcn_s_setprio(3);   // as in the hex kernel below
-        if (n <= kTetWideDef) {
+        const bool small = a.cEnd - a.cStart <= kTetWideClass;
+        if (small || n > kTetWideDef) __builtin_amdgcn_s_setprio(3);   // as in the hex kernel below
+        if (small && n <= kTetWideDef) {
             for (int i = lb; i < n; i += nbList) tet_vertex_wide<NQ>(a, uniform(la.listIn[i]), s_tcd, ringCap);
             return;
         }
@@ -1887,8 +1893,7 @@ void k_search_hex_learned_def(SearchArgs a, LearnArgs la0, int ringCap, int nbLi
         const int n = min(*la.cntIn, a.cEnd - a.cStart);
         if (lb == 0 && threadIdx.x == 0) atomicAdd(la.fallbacks, n);
         // a full search alone takes as long as the windows' four rounds beside it:
-        // it goes first (last wave of a class at 23 us instead of 31; the tet
-        // kernel's shorter searches gained nothing by it)
+        // it goes first (last wave of a class at 23 us instead of 31)
         __builtin_amdgcn_s_setprio(3);
         const int w = uniform((int)(threadIdx.x >> 6));   // one vertex per wave, in the wave's own LDS
         unsigned char* lds = s_hxd + (size_t)w * hex_wave_lds(ringCap);
