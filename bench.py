@@ -49,7 +49,8 @@ LEARN_MODE = {"tet": 3, "hex": 1}
 # first-level window, reported beside the tuned window
 SPEC_WINDOW = (1, 0.25)
 PEAK_FP32_TFLOPS = 157.3
-# Work of one tet / hex vertex update in canonical FP32 operations: the
+# Work of one tet / hex vertex update in canonical FP32 operations, of the
+# full search (the kernels leave out what their bounds rule out): the
 # candidates of a full search (3 levels x 512) and the start position, times
 # the one-ring size (24 tets / 8 hexes on the structured cubes), times the
 # operations the canonical evaluation executes per (candidate, ring element)
@@ -83,25 +84,25 @@ SURF_FLOP = {"tri": 3 * 64 * (57 + 69 * 6 + 59 * 6), "quad": 3 * 64 * (57 + 69 *
 # for the search's own instruction mix (bench.py --calibrate's selection-step
 # probe, 3.81 wave-instructions per CU per ns), from the counter passes of
 # profiles/learned_vs_plain_tet40_hex48.md
-VALU_ISSUE_FRAC = {"k_search_tet": 0.81, "k_search_hex": 0.93, "k_search_tet_learned_def": 0.37,
-                   "k_search_hex_learned_def": 0.47}
+VALU_ISSUE_FRAC = {"k_search_tet": 0.37, "k_search_hex": 0.59, "k_search_tet_learned_def": 0.33,
+                   "k_search_hex_learned_def": 0.34}
 VALU_ISSUE_BASIS = ("SQ_INSTS_VALU / kernel-trace duration / CUs over the calibrated mixed-instruction issue "
                     "ceiling (profiles/learned_vs_plain_tet40_hex48.md, profiles/valu_issue_calibration.md)")
 SURF_FLOP1D = {"tri": 3 * 8 * (149 + 59 * 6), "quad": 3 * 8 * (149 + 104 * 4)}
 WORKLOADS = {
     "tet40": {"kind": "tet", "flop": FLOP_TET, "cbrt": FULL_EVALS, "kernel": "k_search_tet<8>",
-              "traffic": 9_346_689, "learned_traffic": 6_482_023},
+              "traffic": 9_375_215, "learned_traffic": 6_956_080},
     "hex48": {"kind": "hex", "flop": FLOP_HEX, "cbrt": FULL_EVALS, "kernel": "k_search_hex<8>",
-              "traffic": 16_172_174, "learned_traffic": 10_517_734},
+              "traffic": 16_126_330, "learned_traffic": 10_674_340},
     # the 48^3 hex cube at jitter 0.15h: a valid mesh, so the surface and
     # feature passes run every iteration (the roofline is the inner kernel's)
     "hex48_surface": {"kind": "hex", "flop": FLOP_HEX, "cbrt": FULL_EVALS, "kernel": "k_search_hex<8>",
                       "traffic": None},
     "tri64": {"kind": "tri", "flop": 27_048, "cbrt": 0, "kernel": "k_search_flat<8>", "traffic": None},
     "surf_tri": {"kind": "tri", "surface": True, "flop": SURF_FLOP["tri"], "flop1d": SURF_FLOP1D["tri"], "cbrt": 0,
-                 "kernel": "k_search_fan2d<false>", "traffic": 18_791_143},
+                 "kernel": "k_search_fan2d<false>", "traffic": 18_974_770},
     "surf_quad": {"kind": "quad", "surface": True, "flop": SURF_FLOP["quad"], "flop1d": SURF_FLOP1D["quad"], "cbrt": 0,
-                  "kernel": "k_search_fan2d<true>", "traffic": 20_562_741},
+                  "kernel": "k_search_fan2d<true>", "traffic": 19_924_030},
     "batch256": {"kind": "batch", "flop": FLOP_TET, "cbrt": FULL_EVALS, "kernel": "k_batch_round", "traffic": None},
     # the default line: learned (+ batched) vs plain on tet40 and hex48
     "learned_vs_plain": {"kind": "tet", "flop": FLOP_TET, "cbrt": FULL_EVALS, "kernel": "k_search_tet_learned_def<8>",
@@ -283,7 +284,7 @@ def bench_batch(args):
                      "frac": achieved / PEAK_FP32_TFLOPS, "traffic": None, "kernel": "k_batch_typed (all rounds + "
                      "per-mesh quality, device time of the replayed iterations)",
                      "flop_basis": "canonical FP32 operations per tet update (13.125 per candidate and ring "
-                                   "element), 23 FLOP per flat-triangle evaluation"},
+                                   "element) of the full search, 23 FLOP per flat-triangle evaluation"},
         "cpu_baseline": cpu,
     }
     print(json.dumps(out), flush=True)
@@ -957,7 +958,7 @@ def main(argv=None):
                     help="iterations per autotuner trial (batch256); 0 skips the tuner and sets the configuration "
                          "it keeps on the 256-mesh mix")
     ap.add_argument("--mode", choices=["plain", "learned"], default="plain")
-    ap.add_argument("--waves", type=int, default=1, help="wavefronts per vertex search (1, 2, 4)")
+    ap.add_argument("--waves", type=int, default=1, help="the library's waves_per_vertex (accepted; the searches choose their wavefronts)")
     ap.add_argument("--compare-learned", type=int, default=None,
                     help="attach the learned-vs-plain comparison to the plain line (default: on for tet40)")
     ap.add_argument("--pairs", type=int, default=2_000_000, help="training pairs (learned mode)")
@@ -1060,7 +1061,8 @@ def main(argv=None):
             "mean_launch_us": 1e3 * st["kernel_ms"] / max(launches, 1),
             "flop_per_update": wl["flop"], "cbrt_per_update": wl["cbrt"],
             "flop_basis": ("canonical FP32 operations of a full search (candidates x ring elements x operations "
-                           "per pair)" if kind in ("tet", "hex") else "FLOP of the reference formulas")}
+                           "per pair); the searches leave out what their bounds rule out, so this is the rate of "
+                           "the work they stand for, and valu_issue_frac_profiled the executed one" if kind in ("tet", "hex") else "FLOP of the reference formulas")}
     if kind in ("tet", "hex") and not surface_mesh:
         roof["valu_issue_frac_profiled"] = VALU_ISSUE_FRAC[f"k_search_{kind}"]
         roof["valu_issue_basis"] = VALU_ISSUE_BASIS
@@ -1069,7 +1071,6 @@ def main(argv=None):
         threads = host_cpu()["threads_all"]
         cpu = cpu_baseline(kind, xyz, cells, args.cpu_iters, threads, not kw["fixed_boundary"] and not surface_mesh,
                            args.workload, surface_mesh)
-    desc += f"; {args.waves} wavefront(s) per vertex"
     learned = None
     if args.compare_learned and kind in ("tet", "hex"):
         learned = learned_comparison(args)

@@ -93,9 +93,9 @@ typedef struct vsdmo_params {
                                   one-rings of at most 40 vertices) */
     int32_t quality_guard;     /* 1: fail with VSDMO_QUALITY_DECREASED if min quality drops */
     float guard_tolerance;     /* relative slack of the guard (FP32 frame differences) */
-    int32_t waves_per_vertex;  /* 0, 1, 2 or 4 (dividing nq): accepted as before; a vertex search
-                                  runs on one wavefront whatever the value, and results do not
-                                  depend on it */
+    int32_t waves_per_vertex;  /* 0, 1, 2 or 4 (dividing nq): accepted as before; the library
+                                  chooses a search's wavefronts whatever the value, and results
+                                  do not depend on it */
     int32_t surface_path;      /* vsdmo_surface_path, triangle and quad meshes only; on the
                                   surface path fixed_boundary = 1 keeps the feature vertices */
     int32_t hex_metric;        /* vsdmo_hex_metric: the objective of the hex searches and the
@@ -335,7 +335,7 @@ typedef struct vsdmo_batch vsdmo_batch;
 typedef struct vsdmo_batch_params {
     int32_t nq;                /* candidates per axis: 2, 4, 6, 8 */
     int32_t depth;             /* refinement levels */
-    int32_t waves_per_vertex;  /* 1, 2, 4 (divides nq): accepted, one wavefront runs a search; results do
+    int32_t waves_per_vertex;  /* 1, 2, 4 (divides nq): accepted, the library chooses; results do
                                   not depend on it */
     float grid_scale;          /* first-level window scale (reference 0.5) */
     int32_t use_graph;         /* 1: replay a captured hipGraph of one iteration */
