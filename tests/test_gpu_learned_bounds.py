@@ -8,7 +8,7 @@ import pytest
 
 from test_gpu_learned_oracle import oracle_learned
 from test_gpu_search_bounds import _hex_fan
-from volumesurfacediscretemeshoptimization_amd import DMOHexClass, DMOMeshHexFactory, synth
+from volumesurfacediscretemeshoptimization_amd import DMOHexClass, DMOMeshHexFactory, DMOMLP, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -55,3 +55,27 @@ def test_rings(oracle, k):
     for metric in (0, 1):
         # the deferred policy takes rings of up to 21 hexes
         _compare(oracle, xyz, cells, 2, 0.5, "deferred" if 2 * k <= 21 else "immediate", metric=metric)
+
+
+@pytest.mark.parametrize("k", [4, 8, 12, 20])
+def test_neighbour_tables(oracle, k):
+    """the network's table of a ring's corners, 64 ring corners at a time: hubs
+    of 2k hexes, 56 to 280 corners, from below the table's 32 entries to above"""
+    xyz, cells = _hex_fan(k, 5)
+    policy = "deferred" if 2 * k <= 21 else "immediate"
+    mlp = DMOMLP(seed=5)
+    ref, fb = oracle_learned(oracle, "hex", xyz, cells, mlp, 1, 1, 0.5, policy, 2)
+    m = DMOMeshHexFactory.create(xyz, cells)
+    o = DMOHexClass(m, n_iter=2, fixed_boundary=True, quality_guard=False)
+    try:
+        o.set_proposal(mlp, mode=1, depth=1, window_frac=0.5, fallback=policy)
+        for it in range(2):
+            o.iterate(1)
+            gp = m.positions(original_order=False)
+            bad = (gp.view(np.uint32) != ref[it].view(np.uint32)).any(axis=1)
+            assert not bad.any(), (it, int(bad.sum()), np.nonzero(bad)[0][:5])
+        assert o.stats()["fallbacks"] == fb
+    finally:
+        o.close()
+        m.close()
+        mlp.close()
