@@ -59,7 +59,7 @@ public:
         for (;;) {
             for (size_t i = 0; i < pieces_.size(); ++i) {
                 if (pieces_[i].used || pieces_[i].n < bytes) continue;
-                const Piece rest{ pieces_[i].p + bytes, pieces_[i].n - bytes, false };
+                const Piece rest{ pieces_[i].p + bytes, pieces_[i].n - bytes, pieces_[i].chunk, false };
                 pieces_[i].n = bytes;
                 pieces_[i].used = true;
                 char* const p = pieces_[i].p;
@@ -81,7 +81,7 @@ public:
     }
 
 private:
-    struct Piece { char* p; size_t n; bool used; };
+    struct Piece { char* p; size_t n; size_t chunk; bool used; };
     void grow(size_t bytes)
     {
         bytes = std::max(bytes, size_t(1) << 20);
@@ -93,13 +93,14 @@ private:
             (void)hipFree(c);
             throw;
         }
-        pieces_.push_back({ static_cast<char*>(c), bytes, false });
+        pieces_.push_back({ static_cast<char*>(c), bytes, chunks_.size() - 1, false });
     }
-    // piece i with its successor, if both are free and contiguous
+    // piece i with its successor, if both are free and of one chunk.  (Two chunks
+    // can lie side by side, but a copy or a fill has to stay within one allocation.)
     void join(size_t i) noexcept
     {
         if (i + 1 >= pieces_.size() || pieces_[i].used || pieces_[i + 1].used) return;
-        if (pieces_[i].p + pieces_[i].n != pieces_[i + 1].p) return;
+        if (pieces_[i].chunk != pieces_[i + 1].chunk) return;
         pieces_[i].n += pieces_[i + 1].n;
         pieces_.erase(pieces_.begin() + (std::ptrdiff_t)i + 1);
     }
