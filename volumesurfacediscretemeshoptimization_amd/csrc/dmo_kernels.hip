@@ -1638,16 +1638,20 @@ __device__ void hex_window(const SearchArgs& a, const LearnArgs& la, int ringCap
     const auto group_bits = [&](bool b) { return (unsigned)(__ballot(b) >> gbase) & 0xffffu; };
     const auto select = [&](HexAcc& acc, bool hasAcc, bool accInRange, int n, auto pair) {
         bool ok = accInRange && n > 0 && n <= 4 * G;
-        float y[4], dm = FLT_MAX, fm = FLT_MAX, ym = FLT_MAX;
+        float y[4], d2[4], F3[4], dm = FLT_MAX, fm = FLT_MAX, ym = FLT_MAX;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             y[q] = FLT_MAX;
+            d2[q] = 1.0f;
+            F3[q] = 0.0f;   // a place without a pair replaces none
             if (s + q * G < n) {
                 const float2 v = pair(s + q * G);
                 ok = ok & sel_range(v.x, v.y);
                 dm = fminf(dm, v.x);
                 fm = fminf(fm, v.y);
-                y[q] = (v.x * v.x) * __builtin_amdgcn_rcpf((v.y * v.y) * v.y);
+                d2[q] = v.x * v.x;
+                F3[q] = (v.y * v.y) * v.y;
+                y[q] = d2[q] * __builtin_amdgcn_rcpf(F3[q]);
                 ym = fminf(ym, y[q]);
             }
         }
@@ -1667,12 +1671,17 @@ __device__ void hex_window(const SearchArgs& a, const LearnArgs& la, int ringCap
 #pragma unroll
         for (int q = 0; q < 4; ++q) band |= (unsigned long long)group_bits(y[q] <= lim) << (16 * q);
         if (!(ya <= lim)) { acc.bd2 = 1.0f; acc.bF3 = 0.0f; }   // replaced by the band's first
-        for (; band; band &= band - 1) {
-            const float2 v = pair(__builtin_ctzll(band));
-            const float d2 = v.x * v.x, F3 = (v.y * v.y) * v.y;
-            const bool take = d2 * acc.bF3 < acc.bd2 * F3;
-            acc.bd2 = take ? d2 : acc.bd2;
-            acc.bF3 = take ? F3 : acc.bF3;
+        for (;;) {   // on to the first that replaces the selected one, as select_lanes
+            unsigned long long m = 0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) m |= (unsigned long long)group_bits(d2[q] * acc.bF3 < acc.bd2 * F3[q]) << (16 * q);
+            m &= band;
+            if (m == 0) break;
+            const int t = __builtin_ctzll(m);
+            const float2 v = pair(t);
+            acc.bd2 = v.x * v.x;
+            acc.bF3 = (v.y * v.y) * v.y;
+            band &= ~((2ull << t) - 1ull);
         }
         return true;
     };
