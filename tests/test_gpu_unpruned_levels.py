@@ -16,3 +16,22 @@ def test_hex_rings_of_equal_elements(oracle, jitter, metric):
     that replaces the last to the next"""
     xyz, cells = _cube("hex", 8, 81, jitter)
     _compare(oracle, "hex", xyz, cells, hex_metric=metric)
+
+
+@pytest.mark.parametrize("nq", [2, 4, 6, 8])
+@pytest.mark.parametrize("jitter,grid_scale", [(0.0, 0.5), (0.02, 0.5), (0.25, 0.5), (0.25, 4.0), (0.45, 1.0)])
+def test_hex_windows_wider_than_the_bounds(oracle, nq, jitter, grid_scale):
+    """windows of the largest ring offset: none to all of the 40 (32) sub-tets
+    are left to a level, odd and even numbers of them"""
+    xyz, cells = _cube("hex", 7, 82, jitter)
+    for metric in (0, 1):
+        _compare(oracle, "hex", xyz, cells, iters=2, nq=nq, grid_scale=grid_scale, extent=0, hex_metric=metric)
+
+
+@pytest.mark.parametrize("k", [3, 6, 7, 13, 32])
+@pytest.mark.parametrize("grid_scale", [0.1, 0.5, 2.0])
+def test_hex_hubs(oracle, k, grid_scale):
+    """rings of 6 to 64 hexes, 24 to 320 sub-tets: lists of several lane loads"""
+    xyz, cells = _hex_fan(k, 6)
+    for metric in (0, 1):
+        _compare(oracle, "hex", xyz, cells, iters=2, grid_scale=grid_scale, extent=0, hex_metric=metric)

@@ -710,16 +710,69 @@ __device__ __forceinline__ HexBound hex_bound(const HexP& h, bool a3, float cx, 
     return b;
 }
 
-// one p-dependent sub-tet for the CPL candidates px[i] of a lane (shared y, z)
-template <bool A3, int CPL>
-__device__ __forceinline__ void hex_add_cpl(HexAcc* acc, const HexP& h, const float* px, const float* t3, float py,
-                                            float pz, float Q1, float Q3)
+// a = fminf(a, ..) without the canonicalising v_max per operand that fminf costs
+// here (no operand comes straight from a transcendental instruction)
+__device__ __forceinline__ void min_into(float& a, float b) { asm("v_min_f32 %0, %0, %1" : "+v"(a) : "v"(b)); }
+__device__ __forceinline__ void min_into(float& a, float b, float c)
 {
-    const float Tyz = fmaf(h.gy, py, fmaf(h.gz, pz, h.D));
-    const float Ryz = fmaf(h.sy, py, fmaf(h.sz, pz, h.K + (A3 ? Q3 : Q1)));
+    asm("v_min3_f32 %0, %0, %1, %2" : "+v"(a) : "v"(b), "v"(c));
+}
+// the selection of hex_acc_add
+__device__ __forceinline__ void hex_select(HexAcc& a, float det, float F)
+{
+    const float d2 = det * det, F3 = (F * F) * F;
+    const bool take = d2 * a.bF3 < a.bd2 * F3;
+    a.bd2 = take ? d2 : a.bd2;
+    a.bF3 = take ? F3 : a.bF3;
+}
+
+// A p-dependent sub-tet on a line of candidates along x (y, z fixed): det and F
+// of candidate px.  Al: alpha, 1 or 3, as a type (known to the compiler) or a float;
+// alpha * x is exact for 1 and rounds as 3 x for 3.
+template <class Al>
+struct HexLine {
+    const HexP& h;
+    Al al;
+    float T, R;
+    __device__ __forceinline__ HexLine(const HexP& hp, Al alpha, float py, float pz, float Q1) : h(hp), al(alpha)
+    {
+        T = fmaf(h.gy, py, fmaf(h.gz, pz, h.D));
+        R = fmaf(h.sy, py, fmaf(h.sz, pz, h.K + al * Q1));
+    }
+    __device__ __forceinline__ float det(float px) const { return fmaf(h.gx, px, T); }
+    __device__ __forceinline__ float F(float px) const { return fmaf(px, al * px + h.sx, R); }
+};
+struct Alpha1 { __device__ __forceinline__ float operator*(float x) const { return x; } };
+struct Alpha3 { __device__ __forceinline__ float operator*(float x) const { return 3.0f * x; } };
+
+// one sub-tet, or two in their order, added to the accumulators of the CPL
+// candidates px[i] of a lane
+template <int CPL, class Al>
+__device__ __forceinline__ void hex_add(HexAcc* acc, const HexP& h, Al al, const float* px, float py, float pz, float Q1)
+{
+    const HexLine<Al> l(h, al, py, pz, Q1);
 #pragma unroll
-    for (int i = 0; i < CPL; ++i)
-        hex_acc_add(acc[i], fmaf(h.gx, px[i], Tyz), fmaf(px[i], (A3 ? t3[i] : px[i]) + h.sx, Ryz));
+    for (int i = 0; i < CPL; ++i) {
+        const float det = l.det(px[i]), F = l.F(px[i]);
+        hex_select(acc[i], det, F);
+        min_into(acc[i].dmin, det);
+        min_into(acc[i].fmin, F);
+    }
+}
+template <int CPL, class Aa, class Ab>
+__device__ __forceinline__ void hex_add2(HexAcc* acc, const HexP& ha, Aa aa, const HexP& hb, Ab ab, const float* px,
+                                         float py, float pz, float Q1)
+{
+    const HexLine<Aa> la(ha, aa, py, pz, Q1);
+    const HexLine<Ab> lb(hb, ab, py, pz, Q1);
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) {
+        const float da = la.det(px[i]), Fa = la.F(px[i]), db = lb.det(px[i]), Fb = lb.F(px[i]);
+        hex_select(acc[i], da, Fa);
+        hex_select(acc[i], db, Fb);
+        min_into(acc[i].dmin, da, db);
+        min_into(acc[i].fmin, Fa, Fb);
+    }
 }
 
 // The nested grid search of a hex vertex, one wave: lane l = j + nq*k owns the
@@ -815,21 +868,43 @@ __device__ void hex_vertex(const SearchArgs& a, int vid, bool emin, HexLds* s_hx
         wave_lds_fence();
         const float py = (grid_coord(a.aff, j, NQ, gym, gyM) - f.x0y) * f.sg;
         const float pz = (grid_coord(a.aff, k, NQ, gzm, gzM) - f.x0z) * f.sg;
-        float px[NQ], t3[NQ];
+        float px[NQ];
 #pragma unroll
-        for (int i = 0; i < NQ; ++i) {
-            px[i] = (grid_coord(a.aff, i, NQ, gxm, gxM) - f.x0x) * f.sg;
-            t3[i] = 3.0f * px[i];
-        }
-        const float Q1 = fmaf(pz, pz, py * py), Q3 = 3.0f * Q1;
+        for (int i = 0; i < NQ; ++i) px[i] = (grid_coord(a.aff, i, NQ, gxm, gxM) - f.x0x) * f.sg;
+        const float Q1 = fmaf(pz, pz, py * py);
         HexAcc acc[NQ];
 #pragma unroll
         for (int i = 0; i < NQ; ++i) acc[i] = f.acc0;
-        for (int q = 0; q < nAct; ++q) {
-            const int code = uniform(s_act[q]);
-            const HexP h = s_hx[code >> 4].hp[(code >> 1) & 7];
-            if (code & 1) hex_add_cpl<true, NQ>(acc, h, px, t3, py, pz, Q1, Q3);
-            else hex_add_cpl<false, NQ>(acc, h, px, t3, py, pz, Q1, Q3);
+        // Most are left (windows much wider than the ring's smallest offset, regular
+        // rings): all of them, straight through the ring, 101 operations per sub-tet for
+        // the line's 8 candidates.  Through the list, two at a time, 113.  (One at a time
+        // with the code read from LDS it took 153: 40^3 hexes with the largest offset as
+        // extent 7.1 ms for 6 iterations, 5.7 so; without jitter 9.4 ms, 6.8 so.  The
+        // line at a half makes the former 5.9 ms, at 30 % 6.2.)
+        if (4 * nAct > 3 * nSub) {
+#pragma unroll 1
+            for (int e = 0; e < f.n; ++e) {
+                const HexP* hp = s_hx[e].hp;
+                hex_add2<NQ>(acc, hp[0], Alpha1{}, hp[1], Alpha3{}, px, py, pz, Q1);
+                hex_add2<NQ>(acc, hp[2], Alpha1{}, hp[3], Alpha1{}, px, py, pz, Q1);
+                if (!f.corner8) hex_add<NQ>(acc, hp[4], Alpha3{}, px, py, pz, Q1);
+            }
+        } else {
+            const auto sub = [&](int code) { return s_hx[code >> 4].hp[(code >> 1) & 7]; };
+            const auto alpha = [](int code) { return (code & 1) ? 3.0f : 1.0f; };
+            for (int q0 = 0; q0 < nAct; q0 += 64) {   // 64 codes at a time on the lanes
+                const int m = min(nAct - q0, 64), codes = s_act[q0 + min(lane, m - 1)];
+                for (int q = 0; q + 1 < m; q += 2) {
+                    const int ca = __builtin_amdgcn_readlane(codes, q), cb = __builtin_amdgcn_readlane(codes, q + 1);
+                    const HexP ha = sub(ca), hb = sub(cb);
+                    hex_add2<NQ>(acc, ha, alpha(ca), hb, alpha(cb), px, py, pz, Q1);
+                }
+                if (m & 1) {
+                    const int c = __builtin_amdgcn_readlane(codes, m - 1);
+                    const HexP h = sub(c);
+                    hex_add<NQ>(acc, h, alpha(c), px, py, pz, Q1);
+                }
+            }
         }
         wave_lds_fence();   // the next level rewrites the list
         // scores: only of candidates whose ratio is within rounding of the
@@ -1768,14 +1843,16 @@ __device__ void hex_window(const SearchArgs& a, const LearnArgs& la, int ringCap
 #pragma unroll
                 for (int i = 0; i < CPL; ++i) acc[i] = f.acc0;
                 const auto alpha = [&](int t) { return alpha3(t) ? 3.0f : 1.0f; };   // 1 * x is x, to the bit
-                const auto add = [&](const HexP h, float al) {
-                    const float Tyz = fmaf(h.gy, py, fmaf(h.gz, pz, h.D));
-                    const float Ryz = fmaf(h.sy, py, fmaf(h.sz, pz, h.K + al * Q1));
-#pragma unroll
-                    for (int i = 0; i < CPL; ++i)
-                        hex_acc_add(acc[i], fmaf(h.gx, px[i], Tyz), fmaf(px[i], al * px[i] + h.sx, Ryz));
-                };
-                if (bounded) {
+                const auto add = [&](const HexP h, float al) { hex_add<CPL>(acc, h, al, px, py, pz, Q1); };
+                if (!bounded || 4 * __popcll(act) > 3 * nSub) {   // most are left, as in hex_vertex
+#pragma unroll 1
+                    for (int e = 0; e < f.n; ++e) {
+                        const HexP* hp = hx[e].hp;
+                        hex_add2<CPL>(acc, hp[0], Alpha1{}, hp[1], Alpha3{}, px, py, pz, Q1);
+                        hex_add2<CPL>(acc, hp[2], Alpha1{}, hp[3], Alpha1{}, px, py, pz, Q1);
+                        if constexpr (!C8) hex_add<CPL>(acc, hp[4], Alpha3{}, px, py, pz, Q1);
+                    }
+                } else {
                     HexP h = sub(__builtin_ctzll(act));
                     float al = alpha(__builtin_ctzll(act));
                     for (unsigned long long m = act & (act - 1);; m &= m - 1) {   // the next one's loads ahead
@@ -1787,8 +1864,6 @@ __device__ void hex_window(const SearchArgs& a, const LearnArgs& la, int ringCap
                         h = hn;
                         al = an;
                     }
-                } else {
-                    for (int t = 0; t < nSub; ++t) add(sub(t), alpha(t));
                 }
                 // scores: only of candidates whose ratio is within rounding of the best one's
                 float y[CPL], ym = 0.0f;
