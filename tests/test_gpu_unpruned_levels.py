@@ -35,3 +35,41 @@ def test_hex_hubs(oracle, k, grid_scale):
     xyz, cells = _hex_fan(k, 6)
     for metric in (0, 1):
         _compare(oracle, "hex", xyz, cells, iters=2, grid_scale=grid_scale, extent=0, hex_metric=metric)
+
+
+@pytest.mark.parametrize("nq", [2, 4, 6, 8])
+@pytest.mark.parametrize("jitter,depth,extent,shift", [(0.3, 3, -1, 1000.0), (0.3, 7, -1, 0.0), (0.3, 3, 1, 0.0),
+                                                       (0.9, 3, -1, 0.0), (0.0, 5, -1, 0.0)])
+def test_tet_windows_that_the_planes_keep(oracle, nq, jitter, depth, extent, shift):
+    """every candidate of a level: windows smaller than the planes' margins, far
+    frames, inverted rings, regular ones; classes above the 4-wave form's 1,024"""
+    xyz, cells = _cube("tet", 20, 83, jitter)
+    xyz = (xyz.astype(np.float64) + shift).astype(np.float32)
+    _compare(oracle, "tet", xyz, cells, iters=2, nq=nq, depth=depth, extent=extent)
+
+
+@pytest.mark.parametrize("nq", [2, 4, 6, 8])
+def test_tet_hub_in_a_batch(oracle, nq):
+    """the one-wave search (a batch has no 4-wave form) on a ring of more
+    elements than lanes, in windows of every size"""
+    from volumesurfacediscretemeshoptimization_amd import DMOBatch, DMOMeshTetFactory
+    k = 40
+    t = 2.0 * np.pi * np.arange(k) / k
+    pts = np.array([[0.05, -0.03, 0.02]] + [[np.cos(a), np.sin(a), 0.0] for a in t] + [[0.0, 0.0, 1.0], [0.0, 0.0, -1.0]],
+                   np.float32)
+    cells = []
+    for i in range(k):
+        j = (i + 1) % k
+        cells += [[0, 1 + i, 1 + j, k + 1], [0, 1 + j, 1 + i, k + 2]]
+    cells = np.array(cells, np.int32)
+    mesh = DMOMeshTetFactory.create(pts, cells)
+    b = DMOBatch([mesh], persistent=False, nq=nq, depth=6, quality_guard=False)
+    o = oracle.OracleMesh("tet", pts, cells)
+    try:
+        b.iterate(2)
+        for _ in range(2):
+            o.iterate(nq=nq, depth=6, grid_scale=0.5)
+        assert np.array_equal(b.positions(0).view(np.uint32), o.positions().view(np.uint32))
+    finally:
+        b.close()
+        mesh.close()

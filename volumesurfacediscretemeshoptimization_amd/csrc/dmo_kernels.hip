@@ -21,6 +21,14 @@
 
 namespace vsdmo {
 
+// a = fminf(a, ..) without the canonicalising v_max per operand that fminf costs
+// here (no operand comes straight from a transcendental instruction)
+__device__ __forceinline__ void min_into(float& a, float b) { asm("v_min_f32 %0, %0, %1" : "+v"(a) : "v"(b)); }
+__device__ __forceinline__ void min_into(float& a, float b, float c)
+{
+    asm("v_min3_f32 %0, %0, %1, %2" : "+v"(a) : "v"(b), "v"(c));
+}
+
 // ------------------------------------------------------------------ tets
 // LDS of a tet vertex search: the ring's constants, the level's plane of each
 // element (4 floats: gradient, offset for cells; the offset for candidates in
@@ -192,7 +200,6 @@ __device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, unsigned cha
               kR * (c.K + P * (fabsf(c.m2sx) + fabsf(c.m2sy) + fabsf(c.m2sz) + 9.0f * P));
         return q;
     };
-    const Quad q0 = quad(c0);
     const int comp = lane >> 4, col = lane & 15;   // the lane's row (x, y, z, 1) and column of the products' operands
     const int nt = (f.n + 15) >> 4;
     bool fast = false;
@@ -202,8 +209,8 @@ __device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, unsigned cha
     const int myCell = (lane % NB) | ((lane / NB) % NB) << 8 | (lane / (NB * NB)) << 16;
     float cellU[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
     if constexpr (NC > 8) {
-        bool ok = P <= 32.0f && (!own0 || (q0.K >= kSelF && c0.K <= 4096.0f));
-        for (int e = lane + 64; e < f.n; e += 64) ok = ok && quad(s_tc[e]).K >= kSelF && s_tc[e].K <= 4096.0f;
+        bool ok = P <= 32.0f;
+        for (int e = lane; e < f.n; e += 64) ok = ok && quad(s_tc[e]).K >= kSelF && s_tc[e].K <= 4096.0f;
         fast = __ballot(!ok) == 0ull;
         // rows past the ring bound nothing
         if (lane < 16 * nt - f.n) {
@@ -239,10 +246,13 @@ __device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, unsigned cha
         const float s = yq * 5.1961524f;   // 3^1.5: against det / F^1.5
         unsigned long long mask = kAllCells, rest = 0ull;
         float o = 0.0f, D = 0.0f;   // the window's centre and half-width along the lane's axis
-        if constexpr (NC > 8) if (fast) {
-            // the window in frame coordinates: centre, half-widths
-            const float ox = (cx - f.x0x) * f.sg, oy = (cy - f.x0y) * f.sg, oz = (cz - f.x0z) * f.sg;
-            const float Dx = (ds * f.ex) * f.sg, Dy = (ds * f.ey) * f.sg, Dz = (ds * f.ez) * f.sg;
+        // the window's half-widths in frame coordinates.  Below kTiny the planes'
+        // margins keep it whole: every candidate is scored without them (32^3 at depth
+        // 8 5.3 -> 5.1 ms; lines from 2^-9 to 2^-7 measure the same)
+        constexpr float kTiny = 0x1p-8f;
+        const float Dx = (ds * f.ex) * f.sg, Dy = (ds * f.ey) * f.sg, Dz = (ds * f.ez) * f.sg;
+        if constexpr (NC > 8) if (fast && fmaxf(Dx, fmaxf(Dy, Dz)) > kTiny) {
+            const float ox = (cx - f.x0x) * f.sg, oy = (cy - f.x0y) * f.sg, oz = (cz - f.x0z) * f.sg;   // its centre
             const float dx = 1e-3f * kStep * Dx + 0x1p-20f * ((fabsf(cx) + ds * f.ex) * f.sg);
             const float dy = 1e-3f * kStep * Dy + 0x1p-20f * ((fabsf(cy) + ds * f.ey) * f.sg);
             const float dz = 1e-3f * kStep * Dz + 0x1p-20f * ((fabsf(cz) + ds * f.ez) * f.sg);
@@ -261,8 +271,7 @@ __device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, unsigned cha
                     make_float4(px, py, pz, fmaf(ax, kStep * Dx, fmaf(ay, kStep * Dy, fmaf(az, kStep * Dz, w))));
                 s_pw[e] = w;
             };
-            if (own0) plane(lane, c0, q0);
-            for (int e = lane + 64; e < f.n; e += 64) plane(e, s_tc[e], quad(s_tc[e]));
+            for (int e = lane; e < f.n; e += 64) plane(e, s_tc[e], quad(s_tc[e]));
             wave_lds_fence();
             o = comp == 0 ? ox : comp == 1 ? oy : comp == 2 ? oz : 1.0f;
             D = comp == 0 ? Dx : comp == 1 ? Dy : comp == 2 ? Dz : 0.0f;
@@ -285,11 +294,56 @@ __device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, unsigned cha
         auto better = [&](float q, int code) {   // uniform
             if (q > best || (q == best && code < cand)) { best = q; cand = code; }
         };
-        // the canonical scores of the first n (at most 64) buffered candidates,
-        // index i + nq (j + nq k)
+        // every candidate, index i + nq (j + nq k): a line along x per lane, half of
+        // it at a time (the whole line's accumulators would spill)
+        constexpr int H = NQ / 2;
+        auto score_all = [&]() {
+            const int j = lane % NQ, k = lane / NQ;
+            const float py = (grid_coord(a.aff, j, NQ, gym, gyM) - f.x0y) * f.sg;
+            const float pz = (grid_coord(a.aff, k, NQ, gzm, gzM) - f.x0z) * f.sg;
+            const float Qyz = 3.0f * fmaf(pz, pz, py * py);
+            float own = -FLT_MAX;
+            int bi = 0;
+#pragma unroll 1
+            for (int i0 = 0; i0 < NQ; i0 += H) {
+                float px[H], t3[H];
+                TetAcc acc[H];
+#pragma unroll
+                for (int i = 0; i < H; ++i) {
+                    px[i] = (grid_coord(a.aff, i0 + i, NQ, gxm, gxM) - f.x0x) * f.sg;
+                    t3[i] = 3.0f * px[i];
+                    acc[i] = tet_acc0();
+                }
+#pragma unroll 1
+                for (int e = 0; e < f.n; ++e) {
+                    const TetC t = s_tc[e];
+                    const float Tyz = fmaf(t.nny, py, fmaf(t.nnz, pz, t.D));
+                    const float Ryz = fmaf(t.m2sy, py, fmaf(t.m2sz, pz, t.K + Qyz));
+#pragma unroll
+                    for (int i = 0; i < H; ++i) {   // tet_acc_add
+                        const float det = fmaf(t.nnx, px[i], Tyz), L = fmaf(px[i], t3[i] + t.m2sx, Ryz);
+                        const float d2 = det * det, L3 = (L * L) * L;
+                        const bool take = d2 * acc[i].bL3 < acc[i].bd2 * L3;
+                        acc[i].bd2 = take ? d2 : acc[i].bd2;
+                        acc[i].bL3 = take ? L3 : acc[i].bL3;
+                        min_into(acc[i].dmin, det);
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < H; ++i) {
+                    const float q = tet_acc_score(acc[i], f.is3);
+                    if (lane < NQ * NQ && q > own) { own = q; bi = i0 + i; }
+                }
+            }
+            const float m = wave_max_u(own);
+            const int l = __builtin_ctzll(__ballot(own == m));
+            better(m, __builtin_amdgcn_readlane(bi, l) + NQ * l);
+        };
+        // the canonical scores of the first n (at most 64) buffered candidates
         auto score = [&](int n) {
             const int code = s_buf[min(lane, n - 1)];   // lanes past n repeat the last one
             if (n <= kTetFew && f.n <= 64) {
+                const TetC c0 = s_tc[own0 ? lane : 0];
                 bool told = true;
                 for (int c = 0; c < n && told; ++c) {
                     const int at = __builtin_amdgcn_readlane(code, c);
@@ -369,6 +423,17 @@ __device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, unsigned cha
         };
         while (mask != 0ull) {
             const int cnt = __popcll(mask);
+            // eight cells are a pass of one candidate per lane over the ring, all of
+            // them two passes of H: with more cells than the latter costs (windows so
+            // small that no plane tells their candidates apart, inverted rings) every
+            // candidate is scored.  (6 iterations, through the lists / so: 32^3 at depth
+            // 8 8.8 / 5.3 ms, 36^3 moved by 1,000 4.0 / 2.9 ms, 28^3 with jitter 0.9 2.4 /
+            // 1.8 ms.  With the line at a third of the cells the 40^3 cube takes 6.1 ms
+            // for 20 iterations, at a half 5.8.)
+            if (cnt > 8 * H) {
+                score_all();
+                break;
+            }
             if ((mask >> lane) & 1ull) s_cell[__popcll(mask & ((1ull << lane) - 1ull))] = myCell;
             wave_lds_fence();
             int nbuf = 0;
@@ -710,13 +775,6 @@ __device__ __forceinline__ HexBound hex_bound(const HexP& h, bool a3, float cx, 
     return b;
 }
 
-// a = fminf(a, ..) without the canonicalising v_max per operand that fminf costs
-// here (no operand comes straight from a transcendental instruction)
-__device__ __forceinline__ void min_into(float& a, float b) { asm("v_min_f32 %0, %0, %1" : "+v"(a) : "v"(b)); }
-__device__ __forceinline__ void min_into(float& a, float b, float c)
-{
-    asm("v_min3_f32 %0, %0, %1, %2" : "+v"(a) : "v"(b), "v"(c));
-}
 // the selection of hex_acc_add
 __device__ __forceinline__ void hex_select(HexAcc& a, float det, float F)
 {
