@@ -339,9 +339,10 @@ __device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, unsigned cha
             const int l = __builtin_ctzll(__ballot(own == m));
             better(m, __builtin_amdgcn_readlane(bi, l) + NQ * l);
         };
-        // the canonical scores of the first n (at most 64) buffered candidates
+        // the canonical scores of the first n (at most 64) buffered candidates; with
+        // no more than 64 in all, of candidate `lane`
         auto score = [&](int n) {
-            const int code = s_buf[min(lane, n - 1)];   // lanes past n repeat the last one
+            const int code = NC > 8 ? s_buf[min(lane, n - 1)] : min(lane, n - 1);   // lanes past n repeat the last one
             if (n <= kTetFew && f.n <= 64) {
                 const TetC c0 = s_tc[own0 ? lane : 0];
                 bool told = true;
@@ -415,12 +416,17 @@ __device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, unsigned cha
             const float m = wave_max_u(q);
             unsigned long long bal = __ballot(q == m);
             int lo = 0x7fffffff;
+            if (NC <= 8 && bal) { lo = __builtin_amdgcn_readlane(mine, __builtin_ctzll(bal)); bal = 0ull; }
             while (bal) {
                 lo = min(lo, __builtin_amdgcn_readlane(mine, __builtin_ctzll(bal)));
                 bal &= bal - 1;
             }
             better(m, lo);
         };
+        if constexpr (NC <= 8) {
+            score(NQ * NQ * NQ);
+            mask = 0ull;
+        }
         while (mask != 0ull) {
             const int cnt = __popcll(mask);
             // eight cells are a pass of one candidate per lane over the ring, all of
