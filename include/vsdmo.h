@@ -371,10 +371,11 @@ vsdmo_status vsdmo_batch_writeback(vsdmo_batch* b);
 vsdmo_status vsdmo_batch_restore(vsdmo_batch* b);
 vsdmo_status vsdmo_batch_get_params(vsdmo_batch* b, vsdmo_batch_params* p);
 vsdmo_status vsdmo_batch_set_params(vsdmo_batch* b, const vsdmo_batch_params* p);
-/* Autotuner over (nq, depth, waves_per_vertex, persistent): every trial starts
- * from the current positions and runs `iters` iterations; the schedule
- * (waves_per_vertex, persistent) is chosen by time at (8, 3), then (nq, depth) candidates are accepted when every
- * mesh's final min quality is >= the (8, 3) run's - tol; the fastest
+/* Autotuner over (nq, depth, persistent): every trial starts from the current
+ * positions and runs `iters` iterations; the schedule (persistent) is chosen by
+ * time at (8, 3), waves_per_vertex, which chooses nothing, is left at 1 (a
+ * schedule's log lines for 1, 2 and 4 hold one measurement); then (nq, depth)
+ * candidates are accepted when every mesh's final min quality is >= the (8, 3) run's - tol; the fastest
  * accepted configuration is set and returned, the positions are left as
  * they were, and each trial is written to log_path as one JSON line. */
 vsdmo_status vsdmo_batch_autotune(vsdmo_batch* b, int32_t iters, float tol, const char* log_path,
