@@ -73,3 +73,32 @@ def test_tet_hub_in_a_batch(oracle, nq):
     finally:
         b.close()
         mesh.close()
+
+
+@pytest.mark.parametrize("nq", [4, 8])
+@pytest.mark.parametrize("policy", ["immediate", "deferred"])
+@pytest.mark.parametrize("jitter", [0.0, 0.02, 0.3, 0.49])
+def test_hex_fallback_lists_on_4_waves(oracle, monkeypatch, nq, policy, jitter):
+    """learned hexes with the largest offset as extent: the fallbacks' full
+    searches take 4 waves per vertex"""
+    from test_gpu_learned_oracle import oracle_learned
+    from volumesurfacediscretemeshoptimization_amd import DMOHexClass, DMOMeshHexFactory
+    monkeypatch.setattr(oracle, "OR_EXTENT_MIN", oracle.OR_EXTENT_MAX)
+    full = oracle.OracleMesh.search_vertex
+    monkeypatch.setattr(oracle.OracleMesh, "search_vertex", lambda self, v, pos: full(self, v, pos, nq=nq))
+    for xyz, cells in (_cube("hex", 6, 84, jitter), _hex_fan(10, 7)):
+        for metric in (0, 1):
+            ref, fb = oracle_learned(oracle, "hex", xyz, cells, None, 2, 1, 0.03125, policy, 2, hex_metric=metric)
+            m = DMOMeshHexFactory.create(xyz, cells)
+            o = DMOHexClass(m, n_iter=2, nq=nq, extent_mode=0, fixed_boundary=True, hex_metric=metric, quality_guard=False)
+            try:
+                o.set_proposal(None, mode=2, depth=1, window_frac=0.03125, fallback=policy)
+                for it in range(2):
+                    o.iterate(1)
+                    gp = m.positions(original_order=False)
+                    bad = (gp.view(np.uint32) != ref[it].view(np.uint32)).any(axis=1)
+                    assert not bad.any(), (metric, it, int(bad.sum()), np.nonzero(bad)[0][:5])
+                assert o.stats()["fallbacks"] == fb
+            finally:
+                o.close()
+                m.close()

@@ -839,6 +839,20 @@ __device__ __forceinline__ void hex_add2(HexAcc* acc, const HexP& ha, Aa aa, con
     }
 }
 
+// all sub-tets of the ring, in its order
+template <int CPL>
+__device__ __forceinline__ void hex_add_ring(HexAcc* acc, const HexLds* hx, int n, bool corner8, const float* px, float py,
+                                             float pz, float Q1)
+{
+#pragma unroll 1
+    for (int e = 0; e < n; ++e) {
+        const HexP* hp = hx[e].hp;
+        hex_add2<CPL>(acc, hp[0], Alpha1{}, hp[1], Alpha3{}, px, py, pz, Q1);
+        hex_add2<CPL>(acc, hp[2], Alpha1{}, hp[3], Alpha1{}, px, py, pz, Q1);
+        if (!corner8) hex_add<CPL>(acc, hp[4], Alpha3{}, px, py, pz, Q1);
+    }
+}
+
 // The nested grid search of a hex vertex, one wave: lane l = j + nq*k owns the
 // candidates (i, j, k), i = 0..nq-1 (index i + nq*l; the lowest index wins).
 //
@@ -946,13 +960,7 @@ __device__ void hex_vertex(const SearchArgs& a, int vid, bool emin, HexLds* s_hx
         // extent 7.1 ms for 6 iterations, 5.7 so; without jitter 9.4 ms, 6.8 so.  The
         // line at a half makes the former 5.9 ms, at 30 % 6.2.)
         if (4 * nAct > 3 * nSub) {
-#pragma unroll 1
-            for (int e = 0; e < f.n; ++e) {
-                const HexP* hp = s_hx[e].hp;
-                hex_add2<NQ>(acc, hp[0], Alpha1{}, hp[1], Alpha3{}, px, py, pz, Q1);
-                hex_add2<NQ>(acc, hp[2], Alpha1{}, hp[3], Alpha1{}, px, py, pz, Q1);
-                if (!f.corner8) hex_add<NQ>(acc, hp[4], Alpha3{}, px, py, pz, Q1);
-            }
+            hex_add_ring<NQ>(acc, s_hx, f.n, f.corner8, px, py, pz, Q1);
         } else {
             const auto sub = [&](int code) { return s_hx[code >> 4].hp[(code >> 1) & 7]; };
             const auto alpha = [](int code) { return (code & 1) ? 3.0f : 1.0f; };
@@ -1009,6 +1017,82 @@ __device__ void hex_vertex(const SearchArgs& a, int vid, bool emin, HexLds* s_hx
         }
     }
     if (moved && lane == 0) { a.xw[vid] = cx; a.yw[vid] = cy; a.zw[vid] = cz; }
+}
+
+// The same search on the 4 waves of a block, every sub-tet scored, for fallback
+// lists with the largest offset as extent: lane l = j + nq k of wave w owns the
+// candidates (i, j, k), i = w nq / 4 and on.  Those windows leave the bounds little
+// to drop, and a short list waits for its slowest wave (24^3 cube, immediate
+// fallback, mode 1, 8 iterations: 9.7 ms with a wave per vertex, 5.9 so).  lds:
+// hex_wide_lds bytes.
+__host__ __device__ constexpr size_t hex_wide_lds(int ringCap)
+{
+    return sizeof(HexLds) * (size_t)ringCap + 8 * sizeof(TetBest) + sizeof(HexFrame);
+}
+template <int NQ>
+__device__ void hex_vertex_wide(const SearchArgs& a, int vid, unsigned char* lds, int ringCap)
+{
+    constexpr int W = 4, CPL = NQ / W;
+    static_assert(NQ % W == 0 && NQ * NQ <= 64, "nq 4 or 8");
+    const int lane = (int)(threadIdx.x & 63), wave = uniform((int)(threadIdx.x >> 6));
+    HexLds* s_hx = reinterpret_cast<HexLds*>(lds);
+    TetBest* s_best = reinterpret_cast<TetBest*>(s_hx + ringCap);   // [level parity][wave]
+    HexFrame* s_f = reinterpret_cast<HexFrame*>(s_best + 2 * W);
+    if (wave == 0) {
+        const HexFrame own = hex_stage(a, vid, a.extentMin != 0, s_hx);
+        if (lane == 0) *s_f = own;
+    }
+    __syncthreads();
+    const HexFrame f = *s_f;
+    float cx = f.x0x, cy = f.x0y, cz = f.x0z, ds = a.gridScale;
+    bool moved = false;
+    if (!hex_pinned(f)) {   // uniform over the block
+        float qcur = hex_start_lanes(s_hx, f.n, f.corner8, f.acc0, f.inRange, f.epsD, f.epsF);
+        const int j = lane % NQ, k = lane / NQ;
+        for (int d = 0; d < a.depth; ++d, ds = ds * a.shrink) {
+            const float gxM = cx + ds * f.ex, gxm = cx - ds * f.ex;
+            const float gyM = cy + ds * f.ey, gym = cy - ds * f.ey;
+            const float gzM = cz + ds * f.ez, gzm = cz - ds * f.ez;
+            const float py = (grid_coord(a.aff, j, NQ, gym, gyM) - f.x0y) * f.sg;
+            const float pz = (grid_coord(a.aff, k, NQ, gzm, gzM) - f.x0z) * f.sg;
+            const float Q1 = fmaf(pz, pz, py * py);
+            float px[CPL];
+            HexAcc acc[CPL];
+#pragma unroll
+            for (int i = 0; i < CPL; ++i) {
+                px[i] = (grid_coord(a.aff, wave * CPL + i, NQ, gxm, gxM) - f.x0x) * f.sg;
+                acc[i] = f.acc0;
+            }
+            hex_add_ring<CPL>(acc, s_hx, f.n, f.corner8, px, py, pz, Q1);
+            float own = -FLT_MAX;
+            int bi = 0;
+#pragma unroll
+            for (int i = 0; i < CPL; ++i) {
+                const float q = hex_acc_score(acc[i], f.epsD, f.epsF);
+                if (lane < NQ * NQ && q > own) { own = q; bi = i; }
+            }
+            const float m = wave_max_u(own);
+            const int l = __builtin_ctzll(__ballot(own == m));
+            if (lane == l) s_best[(d & 1) * W + wave] = { m, wave * CPL + bi + NQ * l };
+            __syncthreads();   // one a level: the next one's values go to the other half
+            float best = -FLT_MAX;
+            int cand = 0;
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                const TetBest b = s_best[(d & 1) * W + w];
+                if (b.q > best || (b.q == best && b.cand < cand)) { best = b.q; cand = b.cand; }
+            }
+            if (qcur < best) {
+                cx = grid_coord(a.aff, cand % NQ, NQ, gxm, gxM);
+                cy = grid_coord(a.aff, (cand / NQ) % NQ, NQ, gym, gyM);
+                cz = grid_coord(a.aff, cand / (NQ * NQ), NQ, gzm, gzM);
+                qcur = best;
+                moved = true;
+            }
+        }
+    }
+    if (moved && threadIdx.x == 0) { a.xw[vid] = cx; a.yw[vid] = cy; a.zw[vid] = cz; }
+    __syncthreads();   // the next vertex restages the ring
 }
 
 // ------------------------------------------------------------- flat tris
@@ -1810,7 +1894,17 @@ __device__ void hex_window(const SearchArgs& a, const LearnArgs& la, int ringCap
 #pragma unroll
         for (int q = 0; q < 4; ++q) band |= (unsigned long long)group_bits(y[q] <= lim) << (16 * q);
         if (!(ya <= lim)) { acc.bd2 = 1.0f; acc.bF3 = 0.0f; }   // replaced by the band's first
-        for (;;) {   // on to the first that replaces the selected one, as select_lanes
+        if (__popcll(band) <= 4) {   // a few: one after the other
+            for (; band; band &= band - 1) {
+                const float2 v = pair(__builtin_ctzll(band));
+                const float b2 = v.x * v.x, b3 = (v.y * v.y) * v.y;
+                const bool take = b2 * acc.bF3 < acc.bd2 * b3;
+                acc.bd2 = take ? b2 : acc.bd2;
+                acc.bF3 = take ? b3 : acc.bF3;
+            }
+            return true;
+        }
+        for (;;) {   // more: on to the first that replaces the selected one, as select_lanes
             unsigned long long m = 0;
 #pragma unroll
             for (int q = 0; q < 4; ++q) m |= (unsigned long long)group_bits(d2[q] * acc.bF3 < acc.bd2 * F3[q]) << (16 * q);
@@ -1908,14 +2002,10 @@ __device__ void hex_window(const SearchArgs& a, const LearnArgs& la, int ringCap
                 for (int i = 0; i < CPL; ++i) acc[i] = f.acc0;
                 const auto alpha = [&](int t) { return alpha3(t) ? 3.0f : 1.0f; };   // 1 * x is x, to the bit
                 const auto add = [&](const HexP h, float al) { hex_add<CPL>(acc, h, al, px, py, pz, Q1); };
-                if (!bounded || 4 * __popcll(act) > 3 * nSub) {   // most are left, as in hex_vertex
-#pragma unroll 1
-                    for (int e = 0; e < f.n; ++e) {
-                        const HexP* hp = hx[e].hp;
-                        hex_add2<CPL>(acc, hp[0], Alpha1{}, hp[1], Alpha3{}, px, py, pz, Q1);
-                        hex_add2<CPL>(acc, hp[2], Alpha1{}, hp[3], Alpha1{}, px, py, pz, Q1);
-                        if constexpr (!C8) hex_add<CPL>(acc, hp[4], Alpha3{}, px, py, pz, Q1);
-                    }
+                // where most are left to one of the wave's groups, all of them for all (as
+                // in hex_vertex; the groups' branches would run one after the other)
+                if (__ballot(!bounded || 4 * __popcll(act) > 3 * nSub) != 0ull) {
+                    hex_add_ring<CPL>(acc, hx, f.n, C8, px, py, pz, Q1);
                 } else {
                     HexP h = sub(__builtin_ctzll(act));
                     float al = alpha(__builtin_ctzll(act));
@@ -2043,6 +2133,10 @@ void k_search_hex_learned_def(SearchArgs a, LearnArgs la0, int ringCap, int nbLi
         // a full search alone takes as long as the windows' four rounds beside it:
         // it goes first (last wave of a class at 23 us instead of 31)
         __builtin_amdgcn_s_setprio(3);
+        if (!a.extentMin) {
+            for (int i = lb; i < n; i += nbList) hex_vertex_wide<NQ>(a, uniform(la.listIn[i]), s_hxd, ringCap);
+            return;
+        }
         const int w = uniform((int)(threadIdx.x >> 6));   // one vertex per wave, in the wave's own LDS
         unsigned char* lds = s_hxd + (size_t)w * hex_wave_lds(ringCap);
         for (int i = lb + w * nbList; i < n; i += 4 * nbList) {
@@ -2094,6 +2188,15 @@ __global__ __launch_bounds__(64) void k_search_list_hex(SearchArgs a, const int*
     }
 }
 template <int NQ>
+__global__ __launch_bounds__(256) void k_search_list_hex_wide(SearchArgs a, const int* __restrict__ list,
+                                                             const int* __restrict__ cnt, int* fallbacks, int ringCap)
+{
+    extern __shared__ __align__(16) unsigned char s_hxw[];
+    const int n = min(*cnt, a.cEnd - a.cStart);
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(fallbacks, n);
+    for (int i = blockIdx.x; i < n; i += gridDim.x) hex_vertex_wide<NQ>(a, uniform(list[i]), s_hxw, ringCap);
+}
+template <int NQ>
 static void list_nq(int kind, const SearchArgs& a, const int* list, const int* cnt, int* fallbacks, int grid,
                      int ringCap, hipStream_t s)
 {
@@ -2101,6 +2204,10 @@ static void list_nq(int kind, const SearchArgs& a, const int* list, const int* c
     if constexpr (NQ % 4 == 0) {
         if (kind == VSDMO_TET && 4 * lds <= 64 * 1024) {   // a vertex per wave fits a block's LDS
             launch_kernel(k_search_list_tet<NQ, true>, grid, 256, 4 * lds, s, a, list, cnt, fallbacks, ringCap);
+            return;
+        }
+        if (kind == VSDMO_HEX && !a.extentMin) {
+            launch_kernel(k_search_list_hex_wide<NQ>, grid, 256, hex_wide_lds(ringCap), s, a, list, cnt, fallbacks, ringCap);
             return;
         }
     }
