@@ -2490,8 +2490,9 @@ __device__ __forceinline__ void block_minsum256(float& m, double& s)
 // release of the whole L2 is needed.
 __device__ __forceinline__ bool last_block(int* ticket, int b, int nb)
 {
-    __builtin_amdgcn_s_waitcnt(0);
-    asm volatile("" ::: "memory");
+    // the wait and the compiler's fence in one: the builtin alone does not touch
+    // memory, so a relaxed store could be moved past it
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     const int g = b % kTicketGroups, ng = nb < kTicketGroups ? nb : kTicketGroups;
     const int members = nb / kTicketGroups + (g < nb % kTicketGroups);
     if (__hip_atomic_fetch_add(ticket + (g + 1) * kTicketStride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
