@@ -56,7 +56,7 @@ static vsdmo_status fail(vsdmo_status s, const std::string& msg)
 // largest one-ring each search kernel is built for (LDS per 64-thread block)
 static int max_ring_supported(int elem)
 {
-    return elem == VSDMO_HEX ? 256 : 1024;   // <= 48 KB of LDS per block
+    return elem == VSDMO_HEX ? kMaxRingHex : kMaxRingTet;
 }
 
 template <class T>

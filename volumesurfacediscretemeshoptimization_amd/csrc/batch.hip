@@ -539,7 +539,7 @@ vsdmo_status vsdmo_batch_create(vsdmo_mesh* const* meshes, int32_t n_meshes, con
             if ((long long)b->vOff[nm] >= (1LL << 30) || ringBase[nm] >= (1LL << 31) / 3 ||
                 hexBase[nm] >= (1LL << 31) / 7 || heBase[nm] >= (1LL << 31) || cellInts >= (1LL << 31))
                 throw StatusError{ VSDMO_INVALID_ARG, "batch too large for 32-bit indices" };
-            if (b->maxRingTet > 1024 || b->maxRingHex > 256 || b->maxHE > 1024)
+            if (b->maxRingTet > kMaxRingTet || b->maxRingHex > kMaxRingHex || b->maxHE > 1024)
                 throw StatusError{ VSDMO_LDS_OVERFLOW, "one-ring too large for the LDS staging" };
             b->totalV = b->vOff[nm];
             b->ringBaseTet = ringBase;

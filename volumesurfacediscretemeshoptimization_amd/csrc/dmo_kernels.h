@@ -175,10 +175,14 @@ struct BatchQArgs {
     int per;                   // elements per thread: chunks of <= 256 * per elements
 };
 
+// largest one-rings that a mesh may have: their LDS stays below 64 KB per block
+// (asserted beside the layouts), and the split rings' margin holds up to them
+constexpr int kMaxRingTet = 1024, kMaxRingHex = 256;
 size_t search_lds_bytes(int kind, int ringCap);
 bool waves_supported(int nq, int w);
-// the plain searches of one colour class, one wave per vertex (flat triangle
-// classes of 4,096 and more: 4 vertices per wave); ringCap >= the largest
+// the plain searches of one colour class, one wave per vertex (tet classes of up to
+// 1,024 at nq 4 and 8: 4 waves per vertex; flat triangle classes of 4,096 and more
+// at nq 8: 4 vertices per wave); ringCap >= the largest
 // one-ring (tet / hex) or fan (flat)
 void launch_search(int kind, int nq, const SearchArgs& a, int ringCap, hipStream_t s);
 // one colour round of a batch, persistent: grid one-wave blocks take the tet /

@@ -1,6 +1,7 @@
 // dmo_kernels.hip -- DMO vertex-search and quality kernels for gfx950.
 //
-// One wave64 per vertex.  The one-ring is staged in LDS as per-element
+// One wave64 per vertex; 4 of them where a launch or a list is short (*_vertex_wide),
+// a quarter of one for flat triangles of large classes (flat_group8).  The one-ring is staged in LDS as per-element
 // constants in a vertex-local frame.  A level of the 3D searches has nq^3
 // candidates, index i + nq (j + nq k), the lowest index winning ties; bounds
 // leave out what cannot decide it (tet_vertex: candidates no better than the
@@ -386,12 +387,15 @@ __device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, unsigned cha
                 // clearly smaller, the earlier one's where it is clearly larger;
                 // where neither, or the determinants leave the selection's range,
                 // the wave scores the ring in one piece.  Clearly: by more than
-                // kJoin, which exceeds the spread 2^-13 of a chain of near ties (gaps
-                // up to 2^-21, at most 256 elements) that could make the selection
-                // depend on where it starts.  (At 2^-8 two parts' minima often came
+                // kJoin, which exceeds what a chain of near ties can shift: a comparison
+                // of two rounded products takes or leaves a pair wrongly only within
+                // 2^-23 of the selected one, so over the at most 512 elements of a part a
+                // selection that starts elsewhere ends with the same pair, or within 514 x
+                // 2^-23 < 2^-13 of where it started.  (At 2^-8 two parts' minima often came
                 // too close and the ring was gone through again: 40^3 cube, 20
                 // iterations, 6.56 against 6.22 ms.)
                 constexpr float kJoin = 0x1p-12f;
+                static_assert(kJoin >= 2.0f * (kMaxRingTet / 2 + 2) * 0x1p-23f, "twice the shift of the largest part");
                 bool told = true;
                 auto join = [&](int far) {
                     const float od2 = __shfl_xor(acc.bd2, far), oL3 = __shfl_xor(acc.bL3, far), od = __shfl_xor(acc.dmin, far);
@@ -648,6 +652,7 @@ struct HexLds { float cd[4], cF[4]; HexP hp[5]; };
 constexpr size_t kHexLdsPer = sizeof(HexLds) + 5 * sizeof(int);
 // rounded up for a wave's slice of a block's LDS
 __host__ __device__ constexpr size_t hex_wave_lds(int ringCap) { return (kHexLdsPer * (size_t)ringCap + 15) / 16 * 16; }
+static_assert(tet_wave_lds(kMaxRingTet) <= 64 * 1024 && hex_wave_lds(kMaxRingHex) <= 64 * 1024, "a ring fits a block");
 __device__ __forceinline__ int* hex_act(unsigned char* lds, int ringCap)
 {
     return reinterpret_cast<int*>(lds + sizeof(HexLds) * (size_t)ringCap);
@@ -1029,6 +1034,8 @@ __host__ __device__ constexpr size_t hex_wide_lds(int ringCap)
 {
     return sizeof(HexLds) * (size_t)ringCap + 8 * sizeof(TetBest) + sizeof(HexFrame);
 }
+static_assert(hex_wide_lds(1) <= 4 * hex_wave_lds(1) && hex_wide_lds(kMaxRingHex) <= 64 * 1024,
+              "fits the four waves' slices of a block, and a block of its own");
 template <int NQ>
 __device__ void hex_vertex_wide(const SearchArgs& a, int vid, unsigned char* lds, int ringCap)
 {
@@ -2084,7 +2091,8 @@ __global__ __launch_bounds__(FUSED ? 256 : 64) void k_search_hex_learned(SearchA
 
 // deferred fallback: the first gridDim.x - nbList blocks take the windows of
 // 16 class vertices each (the vertices deferred last iteration excepted),
-// the last nbList blocks the full searches (4 waves per vertex) of the
+// the last nbList blocks the full searches (a wave per vertex; 4 for short tet
+// lists and for hexes with the largest offset as extent) of the
 // vertices the previous iteration deferred; both are vertices of one colour
 // class, so the two kinds run side by side.  The windows come first so that
 // the dispatcher starts them before the list blocks, most of which find no
@@ -2150,7 +2158,7 @@ void k_search_hex_learned_def(SearchArgs a, LearnArgs la0, int ringCap, int nbLi
 }
 
 // plain search of the vertices list[0 .. *cnt) (the fallbacks of a class),
-// one vertex per block of W waves at a time, blocks striding over the list
+// one vertex per wave at a time, waves striding over the list
 // (the grid is sized for a typical fallback share, the length is only known
 // on the device)
 // WIDE: blocks of 4 waves, which take a vertex together while the list is
@@ -2249,8 +2257,8 @@ bool learned_fused_ok(int kind, int ringCap)
     return fused_lds(kind, ringCap) <= 64 * 1024;
 }
 
-// the deferred policy's full searches run 4 waves per vertex, and its blocks
-// hold 16 rings in LDS with or without the network
+// the deferred policy's kernels hold the 4-wave full searches, which split a line of
+// candidates in four (nq 4 and 8), and 16 rings in LDS with or without the network
 bool learned_deferred_ok(int kind, int nq, int ringCap)
 {
     return (nq == 4 || nq == 8) && rings16_fit(kind, ringCap);
@@ -2290,7 +2298,7 @@ void launch_search_learned(int kind, int nq, const SearchArgs& a, const LearnNet
         const int nb = (nc + kMlpRows - 1) / kMlpRows;
         const size_t wave = kind == VSDMO_TET ? tet_wave_lds(ringCap) : hex_wave_lds(ringCap);
         const size_t lds = std::max(fused ? fused_lds(kind, ringCap) : (size_t)kMlpRows * ringCap * per, 4 * wave);
-        switch (nq) {   // the full searches use 4 waves: nq 4 and 8 (learned_deferred_ok)
+        switch (nq) {   // learned_deferred_ok
         case 4: fused ? learned_def_nq<4, true>(kind, a, la, ringCap, nbList, nb, lds, s)
                       : learned_def_nq<4, false>(kind, a, la, ringCap, nbList, nb, lds, s); break;
         case 8: fused ? learned_def_nq<8, true>(kind, a, la, ringCap, nbList, nb, lds, s)
