@@ -107,16 +107,15 @@ __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirs
 // ------------------------------------------- correctly rounded, fewer steps
 // 1 / x for x in [2^-126, 2^126): the hardware's reciprocal and one Newton
 // step in fused arithmetic (Markstein, IBM J. Res. Dev. 34, 1990), 3
-// instructions where the division takes 11.  Equal to 1.0f / x for every
-// mantissa at exponents across the range.
+// instructions where the division takes 11.  Equal to 1.0f / x for every value of
+// the range (tests/test_gpu_rounding.py).
 __device__ __forceinline__ float recip_rn(float x)
 {
     const float y = __builtin_amdgcn_rcpf(x);
     return fmaf(fmaf(-x, y, 1.0f), y, y);
 }
 // sqrt(x) for x in [2^-96, 2^128): g = x * rsqrt(x), one step on the exact
-// residual x - g^2.  Equal to sqrtf(x) for every mantissa at exponents across
-// the range, both parities.
+// residual x - g^2.  Equal to sqrtf(x) for every value of the range (the same test).
 __device__ __forceinline__ float sqrt_rn(float x)
 {
     const float y = __builtin_amdgcn_rsqf(x);
