@@ -201,6 +201,7 @@ __device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, unsigned cha
               kR * (c.K + P * (fabsf(c.m2sx) + fabsf(c.m2sy) + fabsf(c.m2sz) + 9.0f * P));
         return q;
     };
+    const Quad q0 = quad(c0);
     const int comp = lane >> 4, col = lane & 15;   // the lane's row (x, y, z, 1) and column of the products' operands
     const int nt = (f.n + 15) >> 4;
     bool fast = false;
@@ -211,7 +212,8 @@ __device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, unsigned cha
     float cellU[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
     if constexpr (NC > 8) {
         bool ok = P <= 32.0f;
-        for (int e = lane; e < f.n; e += 64) ok = ok && quad(s_tc[e]).K >= kSelF && s_tc[e].K <= 4096.0f;
+        ok = ok && (!own0 || (q0.K >= kSelF && c0.K <= 4096.0f));
+        for (int e = lane + 64; e < f.n; e += 64) ok = ok && quad(s_tc[e]).K >= kSelF && s_tc[e].K <= 4096.0f;
         fast = __ballot(!ok) == 0ull;
         // rows past the ring bound nothing
         if (lane < 16 * nt - f.n) {
@@ -248,11 +250,13 @@ __device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, unsigned cha
         unsigned long long mask = kAllCells, rest = 0ull;
         float o = 0.0f, D = 0.0f;   // the window's centre and half-width along the lane's axis
         // the window's half-widths in frame coordinates.  Below kTiny the planes'
-        // margins keep it whole: every candidate is scored without them (32^3 at depth
-        // 8 5.3 -> 5.1 ms; lines from 2^-9 to 2^-7 measure the same)
-        constexpr float kTiny = 0x1p-8f;
+        // margins keep it whole: every candidate is scored without them (6 iterations
+        // at depth 8: 32^3 5.3 -> 5.1 ms at any line from 2^-9 to 2^-7, 20^3 at nq 6 2.57 ms
+        // at 2^-8, 2.42 at 2^-7)
+        constexpr float kTiny = 0x1p-7f;
         const float Dx = (ds * f.ex) * f.sg, Dy = (ds * f.ey) * f.sg, Dz = (ds * f.ez) * f.sg;
-        if constexpr (NC > 8) if (fast && fmaxf(Dx, fmaxf(Dy, Dz)) > kTiny) {
+        const bool planes = NC > 8 && fast && fmaxf(Dx, fmaxf(Dy, Dz)) > kTiny;
+        if constexpr (NC > 8) if (planes) {
             const float ox = (cx - f.x0x) * f.sg, oy = (cy - f.x0y) * f.sg, oz = (cz - f.x0z) * f.sg;   // its centre
             const float dx = 1e-3f * kStep * Dx + 0x1p-20f * ((fabsf(cx) + ds * f.ex) * f.sg);
             const float dy = 1e-3f * kStep * Dy + 0x1p-20f * ((fabsf(cy) + ds * f.ey) * f.sg);
@@ -272,7 +276,8 @@ __device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, unsigned cha
                     make_float4(px, py, pz, fmaf(ax, kStep * Dx, fmaf(ay, kStep * Dy, fmaf(az, kStep * Dz, w))));
                 s_pw[e] = w;
             };
-            for (int e = lane; e < f.n; e += 64) plane(e, s_tc[e], quad(s_tc[e]));
+            if (own0) plane(lane, s_tc[lane], q0);
+            for (int e = lane + 64; e < f.n; e += 64) plane(e, s_tc[e], quad(s_tc[e]));
             wave_lds_fence();
             o = comp == 0 ? ox : comp == 1 ? oy : comp == 2 ? oz : 1.0f;
             D = comp == 0 ? Dx : comp == 1 ? Dy : comp == 2 ? Dz : 0.0f;
@@ -439,8 +444,10 @@ __device__ void tet_vertex(const SearchArgs& a, int vid, bool emin, unsigned cha
             // candidate is scored.  (6 iterations, through the lists / so: 32^3 at depth
             // 8 8.8 / 5.3 ms, 36^3 moved by 1,000 4.0 / 2.9 ms, 28^3 with jitter 0.9 2.4 /
             // 1.8 ms.  With the line at a third of the cells the 40^3 cube takes 6.1 ms
-            // for 20 iterations, at a half 5.8.)
-            if (cnt > 8 * H) {
+            // for 20 iterations, at a half 5.8.)  The coarser cells of nq 6 say less of their
+            // candidates: there the lists are only left out with the planes (28^3 at nq 6,
+            // 12 iterations 2.66 ms, with the line at 24 of 27 cells 2.69).
+            if (NQ == 8 ? cnt > 8 * H : !planes) {
                 score_all();
                 break;
             }
