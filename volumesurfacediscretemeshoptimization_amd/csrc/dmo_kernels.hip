@@ -1186,8 +1186,10 @@ __device__ void flat_vertex(const SearchArgs& a, int vid, TriC* s_tr)
 }
 
 // one vertex per wave and block, vertices [cStart, cEnd) of one colour class.
-// The tet search asks for 6 waves per SIMD (79 VGPRs, no spill): 40^3 cube, 20
-// iterations, 6.53 ms against 6.64 at 5, 6.66 at 7 and 6.84 at 8 (both spill)
+// The tet search asks for 6 waves per SIMD (80 VGPRs, 2 of them spilled outside the
+// loops): 40^3 cube, 20 iterations, 6.15 ms; reading the spilled quadric back from
+// LDS instead 6.28.  Before the levels that score every candidate 6.53 ms (no
+// spill) against 6.64 at 5, 6.66 at 7 and 6.84 at 8 waves
 #ifndef VSDMO_TET_MIN_WAVES
 #define VSDMO_TET_MIN_WAVES 6
 #endif
